@@ -7,7 +7,8 @@ import cpu_kernels
 from synaptix_amd.cache import SequenceCache
 from synaptix_amd.engine.generate import generate, plan_batch, GenerationConfig
 from synaptix_amd.parts import KvNeed
-from synaptix_amd.sampling import Philox4x32, SequenceSampler, filter_batch
+from synaptix_amd.kernels import ops
+from synaptix_amd.sampling import Philox4x32, SequenceSampler, filter_batch, sample_batch
 import plain_qwen3 as P
 
 V = 50
@@ -180,6 +181,44 @@ def test_philox_matches_the_known_answer_and_the_plain_stream():
     assert Philox4x32(1).next_multinomial_uniform() == P.uniform_for_multinomial(P.PlainPhilox(1))
     u = Philox4x32(3).next_f32_uniform()
     assert 0.0 <= u < 1.0
+
+
+@pytest.mark.parametrize("last_n", [0, 3])
+def test_the_penalties_see_the_context_as_it_is_at_the_step(monkeypatch, last_n):
+    """`context` is the caller's to change: an entry replaced, entries taken away and put back, a new list of the same
+    length, and tokens that are no Python integers, each between two steps of sample_batch."""
+    import cpu_kernels
+    cpu_kernels.install(monkeypatch)
+    seen = []
+    plain = ops.filter_rows
+    monkeypatch.setattr(ops, "filter_rows", lambda *a: (seen.append(None if a[9] is None else a[9].tolist()), plain(*a))[1])
+    cfg = GenerationConfig(repetition_penalty=1.3, repeat_last_n=last_n)
+    s = SequenceSampler(cfg, [1, 2, 3, 4])
+
+    def step():
+        sample_batch(torch.linspace(0, 1, 20)[None], [s])
+        want = [int(t) for t in (s.context[:-1] if last_n == 0 else s.context[:-1][-last_n:])]
+        assert seen.pop() == want
+    step()
+    s.context[-1] = 9
+    step()
+    s.context[0] = 11
+    step()
+    del s.context[-2:]
+    s.context += [5, 6]
+    step()
+    s.context = [7] * len(s.context)
+    step()
+    s.context.clear()
+    s.commit(12)
+    step()
+    s.context[-1] = 3.0
+    step()
+    step()
+    assert filter_batch(torch.zeros(1, 20), [cfg], [iter([2.0, 3])]).shape == (1, 20) and seen.pop() == [2, 3]
+    far = SequenceSampler(GenerationConfig(repetition_penalty=1.3, repeat_last_n=2), [1 << 40, 1.0, 4])
+    sample_batch(torch.zeros(1, 20), [far])
+    assert seen.pop() == [1, 4]
 
 
 def test_options_reach_the_filters_as_the_plain_ones_apply_them(monkeypatch):
