@@ -364,7 +364,7 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out, int V,
   float* x = out + (size_t)row * V;
   const float* src = in + (size_t)row * V;    // the row as it comes, until the first pass that writes has copied it
 
-  // ---- penalties: occurrences counted in the row's scratch counters, which are zero before and after
+  // ---- penalties: occurrences counted in the row's scratch counters, of which those of its tokens are zeroed before and after
   const int n_ids = id_start ? id_start[row + 1] - id_start[row] : 0;
   const float rep = repetition[row], pres = presence[row], freq = frequency[row];
   if (n_ids > 0 && (rep != 1.f || pres != 0.f || freq != 0.f)) {
@@ -375,6 +375,11 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out, int V,
     }
     int* cnt = counts + (size_t)row * V;
     const int* mine = ids + id_start[row];
+    for (int i = tid; i < n_ids; i += nt) {
+      const int t = mine[i];
+      if (t >= 0 && t < V) cnt[t] = 0;
+    }
+    __syncthreads();
     for (int i = tid; i < n_ids; i += nt) {
       const int t = mine[i];
       if (t >= 0 && t < V) atomicAdd(&cnt[t], 1);
@@ -576,7 +581,7 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out, int V,
 
 // in, out [n_rows, V] float (may be the same); one entry a row of every option (top_k 0 and top_p >= 1: off);
 // ids, id_start [n_rows + 1]: the tokens that the penalties look at, row after row (null: none);
-// counts [n_rows * V] int, zero (needed with ids; the kernel leaves them zero)
+// counts [n_rows * V] int, any content: this call's own (needed with ids)
 SYN_EXPORT int syn_filter_rows(const float* in, float* out, int n_rows, int V, const float* temperature, const int* top_k,
                                const float* top_p, const float* min_p, const float* repetition, const float* presence,
                                const float* frequency, const int* ids, const int* id_start, int* counts,

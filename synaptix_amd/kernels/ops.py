@@ -1346,7 +1346,7 @@ def filter_rows(logits, out, temperature, top_k, top_p, min_p, repetition, prese
     in `out` (which may be `logits`).  Every option is an array with one entry a row: temperature (<= 0 or 1:
     the row is not divided), top_k (int32; 0: off), top_p (>= 1: off), min_p (0: off), repetition (1: off),
     presence, frequency (0: off).  ids (int32, flat) and id_start (int32 [R + 1]) give each row the tokens that
-    the penalties look at; counts (int32 [R * V], zero) is their scratch memory, left zero."""
+    the penalties look at; counts (int32 [R * V], any content) is this call's scratch memory."""
     _need(logits, "filter_rows.logits", _F32, (None, None))
     R, V = logits.shape
     _need(out, "filter_rows.out", _F32, (R, V))

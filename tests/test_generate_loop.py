@@ -221,6 +221,19 @@ def test_the_penalties_see_the_context_as_it_is_at_the_step(monkeypatch, last_n)
     assert seen.pop() == [1, 4]
 
 
+def test_every_call_counts_the_penalties_tokens_in_memory_of_its_own(monkeypatch):
+    """Calls on other streams or threads may be under way: no two of them may share counters."""
+    import cpu_kernels
+    cpu_kernels.install(monkeypatch)
+    held = []
+    plain = ops.filter_rows
+    monkeypatch.setattr(ops, "filter_rows", lambda *a: (held.append(a[11]), plain(*a))[1])
+    cfg = GenerationConfig(repetition_penalty=1.3)
+    for _ in range(3):
+        sample_batch(torch.linspace(0, 1, 40).view(2, 20), [SequenceSampler(cfg, [1, 2]), SequenceSampler(cfg, [3])])
+    assert all(c.numel() >= 40 for c in held) and len({c.data_ptr() for c in held}) == 3
+
+
 def test_options_reach_the_filters_as_the_plain_ones_apply_them(monkeypatch):
     """What a GenerationConfig and a context become on their way to the filter kernel (here its stand-in on the
     CPU): which tokens the penalties see (the last repeat_last_n), which options are on, row by row of a batch

@@ -1309,6 +1309,37 @@ def test_filter_rows_against_the_plain_processors(ops, V):
     assert torch.equal(torch.nan_to_num(again, neginf=-1e30), torch.nan_to_num(got, neginf=-1e30)), "in place, and the same bits twice"
 
 
+def test_filter_rows_counts_in_memory_of_any_content(ops):
+    """The penalties' counters need not be zero, and calls on two streams from two threads give what they give one after another."""
+    import threading
+    from synaptix_amd.sampling import GenerationConfig, SequenceSampler, sample_batch
+    V, R = 5000, 4
+    x, g = rnd((R, V), 150, scale=3.0).to(DEV), torch.Generator().manual_seed(151)
+    ids = torch.randint(0, 40, (R * 300,), generator=g).to(I32).to(DEV)
+    starts = torch.arange(0, R * 300 + 1, 300, dtype=I32, device=DEV)
+    one, off = torch.ones(R, device=DEV), torch.zeros(R, device=DEV)
+    outs = []
+    for counts in (torch.zeros(R * V, dtype=I32, device=DEV), torch.randint(-9, 9, (R * V,), generator=g).to(I32).to(DEV)):
+        outs.append(torch.empty_like(x))
+        ops.filter_rows(x, outs[-1], one, off.to(I32), one, off, 1.1 * one, 0.2 * one, 0.1 * one, ids, starts, counts)
+    assert torch.equal(*outs)
+
+    cfg = GenerationConfig(temperature=0.8, top_k=40, repetition_penalty=1.3, frequency_penalty=0.2)
+    rows = [rnd((8, 33000), 160 + i, scale=3.0).to(DEV) for i in range(2)]
+    batches = lambda: [[SequenceSampler(cfg, list(range(50 * i, 50 * i + 400)), 7 * i + r) for r in range(8)] for i in range(2)]
+    steps = lambda i, samplers: [sample_batch(rows[i], samplers) for _ in range(20)]
+    want = [steps(i, b) for i, b in enumerate(batches())]
+    got, side = [None, None], batches()
+    torch.cuda.synchronize()
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got[i] = steps(i, side[i])
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads], [t.join() for t in threads]
+    assert got == want
+
+
 def test_filter_rows_with_equal_values(ops):
     """Equal values at the k-th place and at the boundary of the probability mass: of equal entries the first in
     index order stay, so that top-k keeps exactly k; rows of one value only; rows that are -inf but for a few."""
