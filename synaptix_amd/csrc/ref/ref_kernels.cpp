@@ -138,7 +138,7 @@ REF_API void ref_attention(const float* q, const float* k_pages, const float* v_
 }
 
 // out[r] = the last of the largest logits where temperature is null or <= 0, else the first index whose
-// cumulated softmax(logits / temperature) exceeds uniform[r] (the last index if none does).
+// cumulated softmax(logits / temperature) exceeds uniform[r] (if none does, the last one that is not -inf, else the last).
 REF_API void ref_sample_rows(const float* logits, const float* temperature, const float* uniform, int* out, int rows,
                              int vocab) {
   for (int r = 0; r < rows; ++r) {
@@ -155,6 +155,11 @@ REF_API void ref_sample_rows(const float* logits, const float* temperature, cons
     for (int i = 0; i < vocab; ++i) sum += std::exp((double)(x[i] / t - top));
     double cum = 0.0;
     int pick = vocab - 1;
+    for (int i = vocab - 1; i >= 0; --i)
+      if (x[i] != -INFINITY) {
+        pick = i;
+        break;
+      }
     for (int i = 0; i < vocab; ++i) {
       cum += std::exp((double)(x[i] / t - top)) / sum;
       if ((double)uniform[r] < cum) {

@@ -2,8 +2,8 @@
 //   temperature <= 0: argmax, the last of equal maxima
 //                     (crates/synaptix-infer/src/sampling/greedy.rs:7-13: Rust's max_by keeps the last)
 //   temperature  > 0: x = logit / T (skipped for T == 1), p = softmax(x), the first i with u < cumsum_i,
-//                     else the last index (crates/synaptix-infer/src/sampling/multinomial.rs:7-28,
-//                     logit_processor.rs:8-18)
+//                     else the last index that is not -inf (crates/synaptix-infer/src/sampling/multinomial.rs:7-28,
+//                     logit_processor.rs:8-18; a dropped entry is never drawn, where the reference falls back to the last index)
 // The uniform number u comes from the host (a Philox stream per sequence).
 // The reference samples on the host from a downloaded vector; the arithmetic is the same,
 // only the order of the two sums differs (parallel instead of sequential).
@@ -143,8 +143,8 @@ sample_rows_kernel(const float* __restrict__ logits, const float* __restrict__ t
       for (int q = 0; q < 16; ++q) v[q] = i0 + q < hi ? x[i0 + q] : -INFINITY;
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
-        if (hit == V && i0 + q < hi) {
-          if (v[q] != -INFINITY) c += weight(v[q]) / total;
+        if (hit == V && v[q] != -INFINITY) {      // (a dropped entry is never drawn, wherever the roundings of two chunks leave u)
+          c += weight(v[q]) / total;
           if (u < c) hit = i0 + q;
         }
       }
@@ -155,11 +155,23 @@ sample_rows_kernel(const float* __restrict__ logits, const float* __restrict__ t
   for (int off = 32; off > 0; off >>= 1) hit = min(hit, __shfl_xor(hit, off, SYN_WAVE));
   if (tid % SYN_WAVE == 0) found[tid / SYN_WAVE] = hit;
   __syncthreads();
-  if (tid == 0) {
-    int r = V;
-    for (int w = 0; w < (int)blockDim.x / SYN_WAVE; ++w) r = min(r, found[w]);
-    out[row] = r >= V ? V - 1 : r;
+  int r = V;
+  for (int w = 0; w < SAMPLE_THREADS / SYN_WAVE; ++w) r = min(r, found[w]);
+  if (r == V) {
+    // nothing passes u (the rounded sum ends below it, or is NaN): the last entry that is not dropped, of all of them the last
+    int last = -1;
+    for (int i = hi - 1; i >= lo && last < 0; --i)
+      if (x[i] != -INFINITY) last = i;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, SYN_WAVE));
+    __syncthreads();
+    if (tid % SYN_WAVE == 0) found[tid / SYN_WAVE] = last;
+    __syncthreads();
+    r = -1;
+    for (int w = 0; w < SAMPLE_THREADS / SYN_WAVE; ++w) r = max(r, found[w]);
+    if (r < 0) r = V - 1;
   }
+  if (tid == 0) out[row] = r;
 }
 
 SYN_EXPORT int syn_sample_rows(const float* logits, const float* temperature, const float* uniform, int* out,

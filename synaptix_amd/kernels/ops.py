@@ -1328,7 +1328,8 @@ def diff_heads(a, out, lam, eps, post, n_kv_heads, heads_per_kv, vdim):
 
 def sample_rows(logits, temperature, uniform, out):
     """out[r] = argmax (last of equal maxima) where temperature[r] <= 0 or temperature is None,
-    else a draw from softmax(logits[r] / temperature[r]) by inverse CDF with uniform[r]."""
+    else a draw from softmax(logits[r] / temperature[r]) by inverse CDF with uniform[r] (-inf is never drawn where
+    anything else is left)."""
     _need(logits, "sample_rows.logits", _F32, (None, None))
     R, V = logits.shape
     if temperature is not None:

@@ -243,7 +243,8 @@ def sample_rows(logits, temperature, uniform, out):
             x = x / torch.tensor(T, dtype=F32)
         p = torch.softmax(x, 0)
         hit = torch.nonzero(float(uniform[r]) < torch.cumsum(p, 0))
-        out[r] = int(hit[0]) if hit.numel() else x.numel() - 1
+        kept = torch.nonzero(x != float("-inf"))
+        out[r] = int(hit[0]) if hit.numel() else int(kept[-1]) if kept.numel() else x.numel() - 1
 
 
 def filter_rows(logits, out, temperature, top_k, top_p, min_p, repetition, presence, frequency,

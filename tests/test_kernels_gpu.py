@@ -1144,9 +1144,29 @@ def test_sample_rows_draws_where_the_sum_passes_u(ops, V, left):
     cum, off = p.cumsum(-1), 2 ** -24 * (V // 1024 + 1 + 1024)
     for r, i in enumerate(out.tolist()):
         before = float(cum[r, i] - p[r, i])
-        if i == V - 1 and float(u[r]) >= 1 - off:
-            continue                                        # u at the top: the last index where nothing passes it
         assert p[r, i] > 0 and before <= float(u[r]) + off and float(u[r]) <= float(cum[r, i]) + off, (r, i)
+
+
+@pytest.mark.parametrize("V,left", [(2000, 700), (33000, 900), (151936, 50)])
+def test_sample_rows_draws_no_dropped_entry(ops, V, left):
+    """u within a few steps of 2^-24 of every place where the running sum may pass it, and beyond its end: the chunks' sums
+    are rounded apart from each other, and what they leave between them belongs to no dropped entry."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.full((V,), -math.inf)
+    keep = torch.randperm(V, generator=g)[:left].sort().values
+    x[keep] = 2 * torch.randn(left, generator=g)
+    cum = torch.softmax(x.double(), 0)[keep].cumsum(0).float()
+    steps = torch.arange(-4, 5, dtype=F32) * 2 ** -24
+    u = torch.cat([(cum[:: max(1, left // 60), None] + steps).flatten(), torch.tensor([0.0, 1 - 2 ** -24, 1.0, 1.5])])
+    rows = x.expand(u.numel(), V).contiguous().to(DEV)
+    out = torch.empty(u.numel(), dtype=I32, device=DEV)
+    ops.sample_rows(rows, torch.ones(u.numel(), device=DEV), u.to(DEV), out)
+    got = out.cpu().long()
+    assert torch.isfinite(x[got]).all() and got[-1] == keep[-1]
+    nan = torch.full((2, 1000), float("nan"), device=DEV)
+    nan[1] = -math.inf
+    ops.sample_rows(nan, torch.ones(2, device=DEV), torch.full((2,), 0.5, device=DEV), out[:2])
+    assert out[:2].tolist() == [999, 999]
 
 
 def test_sample_rows_frequencies(ops):

@@ -108,6 +108,12 @@ def test_sampling(twins):
     for r in range(6):
         want = P.greedy(x[r]) if temps[r] <= 0 else P.multinomial(x[r] / temps[r], float(us[r]))
         assert int(out[r]) == want
+    # where nothing passes u: the last entry that is not dropped
+    x[:, 40:] = float("-inf")
+    x[5, 30:] = float("-inf")
+    x[1] = float("-inf")
+    twins.sample_rows(x, torch.ones(6), torch.full((6,), 1.5), out)
+    assert out.tolist() == [39, 49, 39, 39, 39, 29]
 
 
 @pytest.mark.gpu
