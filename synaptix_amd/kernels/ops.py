@@ -528,6 +528,18 @@ def gemm_slices(M, N, K, dtype):
     return slices
 
 
+def gemm_keeps_sums(M, N, K, dtype) -> bool:
+    """Whether a bf16 product whose reader takes 32-bit sums (q, k and v in front of their norm and rotation) hands them on,
+    in as many slices as gemm_slices finds fastest, rather than round them to 16 bits.  Decided by the sizes alone, not by the
+    number of slices: the sums stay wherever 256 x 256 tiles fill at most half of the compute units.  Wider or longer products
+    would pay for the doubled bytes (2,048 rows, N = 6144: 25 MB more written and read a layer)."""
+    if dtype != _BF16 or K % 8 != 0 or N > 16384 or K < 2048:
+        return False
+    if M > 64 and K % 128 == 0 and 2 * -(-M // 256) * -(-N // 256) <= compute_units():
+        return True
+    return gemm_slices(M, N, K, dtype) > 1
+
+
 # ----------------------------------------------------------------------------- attention
 
 def v_pages_to_kernel_order(v):

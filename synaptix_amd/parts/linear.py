@@ -244,6 +244,13 @@ def product_slices(n_rows, w, dtype) -> int:
     return ops.gemm_slices(n_rows, w.shape[0], w.shape[1], dtype)
 
 
+def keeps_sums(n_rows, w, dtype) -> bool:
+    """Whether the product of n_rows rows with w goes to a reader of partial sums as 32-bit sums (linear_for_sum), whatever their number."""
+    if product_slices(n_rows, w, dtype) > 1:
+        return True
+    return w.dtype == dtype and (w.packed is None or w.shape[1] % 128 == 0) and ops.gemm_keeps_sums(n_rows, w.shape[0], w.shape[1], dtype)
+
+
 def linear_for_sum(x, w):
     """The product as float partial sums for a consumer that adds them up (the residual sum fused
     into the next norm): [S, M, N] when cutting K into S slices gives a small product more

@@ -15,7 +15,7 @@ import torch
 from ..kernels import ops
 from ..weights.source import TensorSpec
 from .base import Part, KvNeed
-from .linear import (Matrix, linear, linear_for_sum, product_slices, deferred_product, as_rows, ScaledRows,
+from .linear import (Matrix, linear, linear_for_sum, keeps_sums, deferred_product, as_rows, ScaledRows,
                      WeightedDeltas)
 from .position import Position, NoPosition
 
@@ -130,17 +130,17 @@ class GqaAttention(Mixer):
         cap = self.position.capacity
         if cap is not None and ctx.max_position >= cap:
             raise ValueError(f"position {ctx.max_position} is beyond the position encoding's capacity {cap}")
-        # single tokens: partial sums over slices of K, which the attention kernel adds; prompts: the plain product
-        if self.w_qkv.packed is not None and N <= ops.PACKED_MAX_ROWS and act == torch.bfloat16:
-            qkv = linear_for_sum(h, self.w_qkv)       # float partial sums [S, N, width]
+        # single tokens and short prompts: float sums [S, N, width] over one or several slices of K, which every kernel behind
+        # adds itself; long prompts: the plain product in the activation type (ops.gemm_keeps_sums)
+        few = self.w_qkv.packed is not None and N <= ops.PACKED_MAX_ROWS and act == torch.bfloat16
+        if not few:
+            h = as_rows(h)
+        if few or keeps_sums(N, self.w_qkv, act):
+            qkv = linear_for_sum(h, self.w_qkv)
             if qkv.dim() == 2:
                 qkv = qkv.unsqueeze(0)
         else:
-            h = as_rows(h)
-            # (every kernel behind it adds partial sums itself; ops.gemm_slices cuts where the product would
-            # otherwise leave compute units without work: single tokens and prompts up to about 1,200 tokens)
-            sliced = product_slices(N, self.w_qkv, act) > 1
-            qkv = linear_for_sum(h, self.w_qkv) if sliced else linear(h, self.w_qkv, act)
+            qkv = linear(h, self.w_qkv, act)
         cos, sin = self.position.tables(h.device)
         table = ctx.page_table(cache.group)
         o = torch.empty((N, nh * hd), dtype=act, device=h.device)

@@ -128,6 +128,10 @@ def gemm_slices(M, N, K, dtype):
     return 2 if (dtype == torch.bfloat16 and M <= 16 and K >= 64 and K % 8 == 0) else 1
 
 
+def gemm_keeps_sums(M, N, K, dtype):
+    return gemm_slices(M, N, K, dtype) > 1
+
+
 def qk_norm_rope_kv_write(qkv, q_out, k_pages, v_pages, page_table, tok_seq, tok_pos, q_gain, k_gain, eps,
                           cos, sin, n_heads, n_kv_heads, head_dim, write_kv=True, gain_offset=0.0):
     nh, nkv, hd = n_heads, n_kv_heads, head_dim
@@ -282,7 +286,7 @@ def filter_rows(logits, out, temperature, top_k, top_p, min_p, repetition, prese
         out[r] = x
 
 
-ALL = ["embed", "add_rmsnorm", "rmsnorm_rows", "swiglu", "gemm", "gemm_swiglu", "gemm_packed", "stream_scope", "gemm_slices", "qk_norm_rope_kv_write", "attention_f32",
+ALL = ["embed", "add_rmsnorm", "rmsnorm_rows", "swiglu", "gemm", "gemm_swiglu", "gemm_packed", "stream_scope", "gemm_slices", "gemm_keeps_sums", "qk_norm_rope_kv_write", "attention_f32",
        "attention_prefill_bf16", "decode_splits", "attention_decode_bf16", "attention_decode_fused_bf16", "sample_rows", "filter_rows"]
 
 

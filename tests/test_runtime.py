@@ -94,6 +94,28 @@ def test_decode_tables_pad_with_a_spare_page():
                                           rt.ints(spare), None, None, None, host.ctypes.data))
 
 
+def test_sums_of_short_prompts_stay_in_32_bits_whatever_the_number_of_slices():
+    """q, k and v of prompts whose product fills at most half of the compute units reach their norm as 32-bit sums, also at the
+    sizes where one slice of K is the fastest: the number of slices decides the speed, not the precision."""
+    import torch
+    from synaptix_amd.kernels import ops
+    from synaptix_amd.parts.linear import Matrix, keeps_sums, product_slices
+    one = 0
+    for N, K, tokens in ((6144, 2560, (258, 320, 540, 640, 961, 1280)), (4096, 2048, (713, 1024, 1153, 1408, 1537, 2048)),
+                         (3072, 1024 * 2, (321, 2560)), (6144, 4096, (66, 129, 250, 300, 700, 1280)), (10240, 5120, (256, 700))):
+        w = Matrix(torch.zeros((N, K), dtype=torch.bfloat16), keep_rows=True)
+        for M in tokens:
+            assert ops.gemm_keeps_sums(M, N, K, torch.bfloat16) and keeps_sums(M, w, torch.bfloat16), (M, N, K)
+            one += product_slices(M, w, torch.bfloat16) == 1
+    assert one          # (sizes of one slice were among them)
+    for M in (2048, 5000):
+        assert not ops.gemm_keeps_sums(M, 6144, 4096, torch.bfloat16)
+    for M in (1, 64, 300, 5000):
+        for N, K in ((6144, 4096), (64, 64), (4096, 2052), (30000, 4096)):
+            assert not ops.gemm_keeps_sums(M, N, K, torch.float32)
+            assert ops.gemm_keeps_sums(M, N, K, torch.bfloat16) >= (ops.gemm_slices(M, N, K, torch.bfloat16) > 1)
+
+
 def test_host_side_rules_of_the_kernels_stay_within_their_kernels_limits():
     """The numbers of splits and slices that the host picks: pure functions, checked over a grid of sizes."""
     import torch
