@@ -519,6 +519,55 @@ def test_gated_activations_of_many_rows(ops, act, M, I, K):
     close(out[rows.to(DEV), cols.to(DEV)], want.float(), 1e-4 * math.sqrt(K), 2 ** -8 + 1e-4, f"{act} {M}x{I}x{K}")
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
+def test_gated_epilogue_of_streamed_tiles_is_no_less_exact(ops, act):
+    """The epilogue that the streamed tiles make of the hardware's base-2 functions, stored as 32-bit numbers, against 64 bits and
+    beside the library functions of the plain kernel, on the same sums: rows of x hold a 1 and a power of two, so the sums
+    are exact, gates from -120 to 120 (beyond e^88, where the library's exponential overflows) and from -3 to 3, and infinities."""
+    K, J, P = 256, 1024, 512
+    g = torch.Generator().manual_seed(7)
+    x = torch.zeros(P, K)
+    x[torch.arange(P), torch.arange(P) % K] = 1.0
+    x[torch.arange(P), (torch.arange(P) * 7 + 3) % K] = 2.0 ** -9
+    w = torch.empty(1, J, K)
+    w[0, 0::2] = torch.where(torch.rand(J // 2, 1, generator=g) < 0.5, 240 * torch.rand(J // 2, K, generator=g) - 120,
+                             6 * torch.rand(J // 2, K, generator=g) - 3)
+    w[0, 1::2] = torch.randn(J // 2, K, generator=g)
+    x, w = x.to(BF16), ((64 * w).round() / 64).to(BF16)
+    z = x.double() @ w[0].double().T
+    gt, up = z[:, 0::2], z[:, 1::2]
+    assert torch.equal(z.float().double(), z)
+    if act == "silu":
+        want = gt * torch.sigmoid(gt) * up
+    elif act == "gelu_tanh":
+        t = 2 * math.sqrt(2 / math.pi) * (gt + 0.044715 * gt ** 3)
+        want = gt * torch.sigmoid(t) * up
+    else:
+        gl, ul = gt.clamp(max=7.0), up.clamp(-7.0, 7.0)
+        want = gl * torch.sigmoid(1.702 * gl) * (ul + 1)
+    d = lambda t: t.to(DEV)
+    ids = torch.arange(P, dtype=I32, device=DEV)
+    seg = torch.tensor([0, P], dtype=I32, device=DEV)
+    outs = []
+    for plain in (False, True):
+        out = torch.full((P, J // 2), float("nan"), dtype=F32, device=DEV)
+        ops.experts_product(d(x), d(w) if plain else ops.pack_expert_weights(d(w)), out, seg, ids, ids, gated=act, force_simt=plain)
+        outs.append(out.cpu().double())
+    # (results below the smallest normal number, and where the plain kernel's overflow gave nothing, tell nothing about rounding)
+    tell = (want.abs() > 1e-30) & (outs[1] != 0)
+    off = [((o - want).abs() / want.abs())[tell] for o in outs]
+    assert float(tell.float().mean()) > 0.7
+    assert float(off[0].max()) <= float(off[1].max()) and float(off[0].norm()) <= float(off[1].norm()), [float(o.max()) * 2 ** 24 for o in off]
+    assert ((outs[0] - want).abs() <= (outs[1] - want).abs() + 1e-29)[~tell].all()
+    # infinite sums: what the plain kernel makes of them
+    w[0, 0, :], w[0, 2, :] = float("inf"), -float("inf")
+    a, b = torch.empty(P, J // 2, device=DEV), torch.empty(P, J // 2, device=DEV)
+    one = torch.ones(P, K, dtype=BF16, device=DEV)
+    ops.experts_product(one, ops.pack_expert_weights(d(w)), a, seg, ids, ids, gated=act)
+    ops.experts_product(one, d(w), b, seg, ids, ids, gated=act, force_simt=True)
+    assert torch.equal(torch.nan_to_num(a[:, :2]), torch.nan_to_num(b[:, :2])) and torch.equal(a[:, :2].isnan(), b[:, :2].isnan())
+
+
 @pytest.mark.parametrize("counts,J,K", [([0, 1, 63, 64, 129, 300, 0, 43], 544, 320), ([48], 32, 256), ([600, 0, 5], 256, 512),
                                         ([130] * 70, 288, 256)])
 @pytest.mark.parametrize("act,gated,out_dtype", [(None, None, F32), ("gelu", None, BF16), ("gelu", None, F32), ("relu_squared", None, BF16),
