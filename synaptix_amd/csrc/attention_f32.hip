@@ -1,5 +1,5 @@
 // Attention over the paged cache in true 32-bit: one wave, or four, for each (token, head), plain FMA,
-// online softmax over blocks of 64 keys.  Any head size up to 256, prefill and decode alike.
+// four online softmaxes over blocks of 64 keys in turns.  Any head size up to 256, prefill and decode alike.
 //
 //   query of token t sits at position p = tok_pos[t] of sequence tok_seq[t];
 //   key j is visible iff j <= p and (window <= 0 or j > p - window);
@@ -12,9 +12,11 @@
 
 #define ATTN32_MAX_HD 256
 
-// WAVES waves a workgroup.  SPLIT: they take the blocks of keys of one (token, head) in turns and merge what they have in LDS, in
-// the order of the waves (few tokens: a wave alone would walk a sequence's keys one block after another); else each has a head
-// of its own, the heads of one kv head side by side, which then share its keys and values in the compute unit's cache.
+// The blocks of keys of a (token, head) fall into four classes in turns, each with a running softmax of its own, merged in the order
+// of the classes.  WAVES waves a workgroup.  SPLIT: a wave a class (few tokens: a wave alone would walk a sequence's keys one block
+// after another); else each wave has a head of its own and takes the classes one after another, the heads of one kv head
+// side by side, which then share its keys and values in the compute unit's cache.  The sums are the same either way: a
+// token's result does not depend on how many others are in the step.
 // VEC: head sizes that are a multiple of 4 take keys, queries and values 16 bytes at a time (a lane has a key's row, then a
 // dimension's row, to itself: each 128-byte line is asked for 8 times instead of 32).  490 tokens of 120, 137 and 233 with 32
 // heads of 128 over 8: 839 -> 265 us.
@@ -24,9 +26,12 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
                 const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
                 const int* __restrict__ tok_pos, float* __restrict__ out, float scale, int window, int nh, int nkv,
                 int hd, ScoreTerms terms) {
+#pragma clang fp contract(off)      // (fused where it says so, the same in every variant)
   __shared__ __attribute__((aligned(16))) float qs_all[WAVES][ATTN32_MAX_HD];
   __shared__ __attribute__((aligned(16))) float ps_all[WAVES][SYN_PAGE];
-  __shared__ float stat[SPLIT ? WAVES : 1][2];
+  constexpr int CLASSES = 4;
+  static_assert(!SPLIT || WAVES == CLASSES, "a wave a class");
+  __shared__ float part_all[SPLIT ? 1 : WAVES][CLASSES][ATTN32_MAX_HD], stat_all[SPLIT ? 1 : WAVES][CLASSES][2];
   const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
   const int tok = blockIdx.x, head = SPLIT ? (int)blockIdx.y : (int)blockIdx.y * WAVES + wave;
   float* qs = qs_all[wave];
@@ -41,95 +46,98 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
   const int lo = window > 0 ? max(0, pos - window + 1) : 0;
   const bool with_terms = score_terms_on(terms);
   const float slope = terms.slopes ? terms.slopes[head] : 0.f;
-  float m = -INFINITY, l = 0.f;
-  float o[ATTN32_MAX_HD / SYN_WAVE] = {0.f, 0.f, 0.f, 0.f};
-  for (int kb = lo / SYN_PAGE + (SPLIT ? wave : 0); kb <= pos / SYN_PAGE; kb += SPLIT ? WAVES : 1) {
-    const int page = page_table[(size_t)seq * table_stride + kb];
-    const size_t base = ((size_t)page * nkv + kvh) * SYN_PAGE * hd;
-    const int key = kb * SYN_PAGE + lane;
-    const bool valid = key >= lo && key <= pos;
-    float s = -INFINITY;
-    if (valid) {
-      const float* kr = k_pages + base + (size_t)lane * hd;
-      float dot = 0.f;
-      if constexpr (VEC) {
-        f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-        for (int d = 0; d < hd; d += 4) {
-          const f32x4 kk = *(const f32x4*)(kr + d), qq = *(const f32x4*)(qs + d);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) d4[e] = fmaf(qq[e], kk[e], d4[e]);
-        }
-        dot = (d4[0] + d4[1]) + (d4[2] + d4[3]);
-      } else {
-        for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], kr[d], dot);
-      }
-      s = dot * scale;
-      if (with_terms) s = score_with_terms(s, slope, terms.softcap, pos, key);
-    }
-    const float m_new = fmaxf(m, wave_max(s));  // every block of the range holds a visible key
-    const float alpha = expf(m - m_new);
-    const float p = valid ? expf(s - m_new) : 0.f;
-    l = l * alpha + wave_sum(p);
-    m = m_new;
-    ps[lane] = p;
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < ATTN32_MAX_HD / SYN_WAVE; ++i) {
-      const int d = lane + i * SYN_WAVE;
-      if (d < hd) {
-        const float* vr = v_pages + base + (size_t)d * SYN_PAGE;
-        // (slots past the sequence's end may hold anything: a weight of zero takes nothing from them)
+  auto part = part_all[SPLIT ? 0 : wave];
+  auto stat = stat_all[SPLIT ? 0 : wave];
+  for (int c = SPLIT ? wave : 0; c < (SPLIT ? wave + 1 : CLASSES); ++c) {
+    float m = -INFINITY, l = 0.f;
+    float o[ATTN32_MAX_HD / SYN_WAVE] = {0.f, 0.f, 0.f, 0.f};
+    for (int kb = lo / SYN_PAGE + c; kb <= pos / SYN_PAGE; kb += CLASSES) {
+      const int page = page_table[(size_t)seq * table_stride + kb];
+      const size_t base = ((size_t)page * nkv + kvh) * SYN_PAGE * hd;
+      const int key = kb * SYN_PAGE + lane;
+      const bool valid = key >= lo && key <= pos;
+      float s = -INFINITY;
+      if (valid) {
+        const float* kr = k_pages + base + (size_t)lane * hd;
+        float dot = 0.f;
         if constexpr (VEC) {
-          f32x4 a4 = {o[i] * alpha, 0.f, 0.f, 0.f};
+          f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
-          for (int j = 0; j < SYN_PAGE; j += 4) {
-            const f32x4 vv = *(const f32x4*)(vr + j), pp = *(const f32x4*)(ps + j);
+          for (int d = 0; d < hd; d += 4) {
+            const f32x4 kk = *(const f32x4*)(kr + d), qq = *(const f32x4*)(qs + d);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) a4[e] = fmaf(pp[e], pp[e] != 0.f ? vv[e] : 0.f, a4[e]);
+            for (int e = 0; e < 4; ++e) d4[e] = fmaf(qq[e], kk[e], d4[e]);
           }
-          o[i] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
+          dot = (d4[0] + d4[1]) + (d4[2] + d4[3]);
         } else {
-          float acc = o[i] * alpha;
-          for (int j = 0; j < SYN_PAGE; ++j) {
-            const float pj = ps[j];
-            if (pj != 0.f) acc = fmaf(pj, vr[j], acc);
+          for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], kr[d], dot);
+        }
+        s = dot * scale;
+        if (with_terms) s = score_with_terms(s, slope, terms.softcap, pos, key);
+      }
+      const float m_new = fmaxf(m, wave_max(s));  // every block of the range holds a visible key
+      const float alpha = expf(m - m_new);
+      const float p = valid ? expf(s - m_new) : 0.f;
+      l = fmaf(l, alpha, wave_sum(p));
+      m = m_new;
+      ps[lane] = p;
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < ATTN32_MAX_HD / SYN_WAVE; ++i) {
+        const int d = lane + i * SYN_WAVE;
+        if (d < hd) {
+          const float* vr = v_pages + base + (size_t)d * SYN_PAGE;
+          // (slots past the sequence's end may hold anything: a weight of zero takes nothing from them)
+          if constexpr (VEC) {
+            f32x4 a4 = {o[i] * alpha, 0.f, 0.f, 0.f};
+#pragma unroll 8
+            for (int j = 0; j < SYN_PAGE; j += 4) {
+              const f32x4 vv = *(const f32x4*)(vr + j), pp = *(const f32x4*)(ps + j);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) a4[e] = fmaf(pp[e], pp[e] != 0.f ? vv[e] : 0.f, a4[e]);
+            }
+            o[i] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
+          } else {
+            float acc = o[i] * alpha;
+            for (int j = 0; j < SYN_PAGE; ++j) {
+              const float pj = ps[j];
+              if (pj != 0.f) acc = fmaf(pj, vr[j], acc);
+            }
+            o[i] = acc;
           }
-          o[i] = acc;
         }
       }
+      __builtin_amdgcn_wave_barrier();
     }
-    __builtin_amdgcn_wave_barrier();
-  }
-  if constexpr (SPLIT) {
-    // the waves' results: the common maximum first, then sums in the order of the waves (a wave without a block has m = -inf, l = 0)
-    if (lane == 0) stat[wave][0] = m, stat[wave][1] = l;
+    if (lane == 0) stat[c][0] = m, stat[c][1] = l;
+#pragma unroll
     for (int i = 0; i < ATTN32_MAX_HD / SYN_WAVE; ++i) {
       const int d = lane + i * SYN_WAVE;
-      if (d < hd) qs[d] = o[i];
+      if (d < hd) part[c][d] = o[i];
     }
+  }
+  // the common maximum first, then sums in the order of the classes (one without a block has m = -inf, l = 0)
+  if constexpr (SPLIT) {
     __syncthreads();
     if (wave != 0) return;
-    float top = stat[0][0];
+  } else {
+    __builtin_amdgcn_wave_barrier();
+  }
+  float top = stat[0][0], l = 0.f, f[CLASSES], o[ATTN32_MAX_HD / SYN_WAVE];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) top = fmaxf(top, stat[w][0]);
-    float f[WAVES];
-    l = 0.f;
+  for (int c = 1; c < CLASSES; ++c) top = fmaxf(top, stat[c][0]);
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      f[w] = stat[w][0] == -INFINITY ? 0.f : expf(stat[w][0] - top);
-      l += f[w] * stat[w][1];
-    }
+  for (int c = 0; c < CLASSES; ++c) {
+    f[c] = stat[c][0] == -INFINITY ? 0.f : expf(stat[c][0] - top);
+    l = fmaf(f[c], stat[c][1], l);
+  }
 #pragma unroll
-    for (int i = 0; i < ATTN32_MAX_HD / SYN_WAVE; ++i) {
-      const int d = lane + i * SYN_WAVE;
-      if (d < hd) {
-        float acc = 0.f;
+  for (int i = 0; i < ATTN32_MAX_HD / SYN_WAVE; ++i) {
+    const int d = lane + i * SYN_WAVE;
+    o[i] = 0.f;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) acc += f[w] == 0.f ? 0.f : f[w] * qs_all[w][d];
-        o[i] = acc;
-      }
-    }
+    for (int c = 0; c < CLASSES; ++c)
+      if (d < hd && f[c] != 0.f) o[i] = fmaf(f[c], part[c][d], o[i]);
   }
   float* orow = out + ((size_t)tok * nh + head) * hd;
 #pragma unroll

@@ -1,7 +1,7 @@
 // out[M, N] = x[M, K] . W[N, K]^T with 32-bit accumulation (both operands K-contiguous).
 //
-//   gemm_simt      any shape and type; plain FMA: what the MFMA kernels refuse (K not a multiple of 8, or of 4 for
-//                  few rows in 32 bits; unaligned rows).
+//   gemm_simt      any shape and type; plain FMA: what the MFMA kernels refuse (K not a multiple of 8, or of 4 in 32 bits;
+//                  unaligned rows).
 //   gemm_f32_few   32-bit, up to 64 rows: v_mfma_f32_16x16x4_f32 over W streamed once, K over the waves.
 //   gemm_f32_tiles 32-bit, more rows: tiles of 64 x 64 or 64 x 32 through LDS.
 //   gemm_skinny    bf16, M == 1: the weight matrix is streamed once from HBM through
@@ -464,16 +464,19 @@ static int tile_grid(int M, int N, int BM, int BN) {
 }
 
 // ------------------------------------------------------------------ 32-bit products on the matrix units
-// v_mfma_f32_16x16x4 and v_mfma_f32_32x32x2 multiply and add in 32 bits, as the plain kernel's fused multiply-adds do, at 256 of them
-// a clock and compute unit (a large library product reaches 149 TFLOP/s here; the plain kernel 20).  Which four (two) k-values a
-// step multiplies is free as long as both operands agree: a lane loads four neighbouring ones (16 bytes) and gives them
-// to four steps one after another.
+// v_mfma_f32_16x16x4 multiplies and adds in 32 bits, as the plain kernel's fused multiply-adds do, at 256 of them a clock and
+// compute unit (a large library product reaches 149 TFLOP/s here; the plain kernel 20).  Which four k-values a step multiplies
+// is free as long as both operands agree: a lane loads four neighbouring ones (16 bytes) and gives them to four steps one
+// after another.
+// The order of the sums is the same whatever the number of rows, so a row's results do not depend on what else is in the
+// batch: K in chunks of 32, chunk c of class c % 16; the chunks of a class one after another in ascending order, each in eight steps
+// (16 values in four steps of every fourth one, twice); then the sixteen sums in the order of the classes.
 //
-// Up to 64 rows of x: bound by reading W, which no cache holds.  A workgroup owns 16 rows of W; its 16 waves take k-chunks of
-// 16 in turns, eight (four with many rows of x) at a time, so that the workgroup has up to 128 KB of W under way, and
-// their partial tiles are added in LDS in the order of the waves.  D[n = 4 (lane / 16) + j][m = lane % 16].
+// Up to 64 rows of x: bound by reading W, which no cache holds.  A workgroup owns 16 rows of W; its 16 waves take a class
+// each, eight loads of 16 k-values (four with many rows of x) at a time, so that the workgroup has up to 128 KB of W under way,
+// and their partial tiles are added in LDS in the order of the waves.  D[n = 4 (lane / 16) + j][m = lane % 16].
 // W of 2,560 x 9,728: 1 row 1,604 -> 38 us, 16 rows 1,655 -> 52 (plain kernel, this one); of 151,936 x 2,560: 1 row 1,225 ->
-// 415 us (3.8 TB/s).  The sums' error against 64 bits is a quarter of the plain kernel's (4.5e-7, 1.8e-6), since a wave adds a
+// 415 us (3.8 TB/s).  The sums' error against 64 bits is a quarter of the plain kernel's (4.5e-7, 1.8e-6), since a class is a
 // sixteenth of K.
 template <int FM, int U>
 __global__ void __launch_bounds__(16 * SYN_WAVE)
@@ -491,11 +494,11 @@ gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, fl
 #pragma unroll
   for (int i = 0; i < FM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = wave * 16; k0 < K; k0 += WAVES * 16 * U) {
+  for (int k0 = wave * 32; k0 < K; k0 += WAVES * 16 * U) {
     f32x4 b[U], a[U][FM];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * WAVES * 16;
+      const int k = k0 + u / 2 * WAVES * 32 + u % 2 * 16;
       const bool in = k + k4 < K;      // (K is a multiple of 4)
       b[u] = in ? __builtin_nontemporal_load((const f32x4*)(wr + k)) : zero;
 #pragma unroll
@@ -527,13 +530,13 @@ gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, fl
 
 // More rows: tiles of 64 x BN (BN = 64, 32), 4 waves of 32 x BN / 2, k-tiles of 32 in a ring of three LDS buffers that loads
 // fill without passing through registers; a row's eight 16-byte chunks are swizzled as in gemm_direct.  Three to five
-// workgroups share a compute unit.  D[m = 8 (e / 4) + 4 (lane / 32) + e % 4][n = lane % 32] with 32 x 32, and the tiles of 16
-// columns D[m = 4 (lane / 16) + e][n = lane % 16].
-// M = 490: N = 19,456, K = 2,560 1,257 -> 492 us (99 TFLOP/s), N = 2,560, K = 9,728 1,820 -> 337; the error is the plain kernel's.
+// workgroups share a compute unit.  A k-tile is a chunk of the order above, and they come class by class.
+// D[n = 4 (lane / 16) + e][m = lane % 16].
 template <int BN>
 __global__ void __launch_bounds__(256)
 gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K, int point) {
   constexpr int BM = 64, BK = 32, STAGES = 3, ROWS = BM + BN, RPI = 8, WAVES = 4, PASSES = ROWS / (RPI * WAVES);
+  constexpr int CLASSES = 16, FN = BN / 32;
   static_assert(BN == 64 || BN == 32, "tile shape");
   __shared__ __attribute__((aligned(16))) float smem[STAGES * ROWS * BK];
   const int lane = threadIdx.x % SYN_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE);
@@ -557,70 +560,69 @@ gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     for (int p = 0; p < PASSES; ++p)
       buffer_to_lds16(p * WAVES * RPI < BM ? vx : vw, smem + ((size_t)buf * ROWS + (p * WAVES + wave) * RPI) * BK, src[p], kt * BK * 4);
   };
-  constexpr bool WIDE = BN == 64;
-  f32x16 acc = {};
-  f32x4 half[2] = {};
+  struct Place {      // in the order of the k-tiles
+    int kt, of_class;
+  };
+  auto next = [&](Place p) { return p.kt + CLASSES < nk ? Place{p.kt + CLASSES, p.of_class} : Place{p.of_class + 1, p.of_class + 1}; };
+  f32x4 acc[2][FN] = {}, total[2][FN] = {};
+  Place load = {0, 0}, at = {0, 0};
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t)
-    if (t < nk) fetch(t, t);
-  for (int kt = 0; kt < nk; ++kt) {
-    // this wave's loads of tile kt have landed (all but the youngest tile's), and behind the barrier everyone's
-    if (kt + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f70 | PASSES);
+    if (t < nk) fetch(load.kt, t), load = next(load);
+  const int r16 = lane % 16, q = lane / 16;
+  for (int i = 0; i < nk; ++i) {
+    // this wave's loads of the i-th k-tile have landed (all but the youngest tile's), and behind the barrier everyone's
+    if (i + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f70 | PASSES);
     else __builtin_amdgcn_s_waitcnt(0x0f70);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (kt + STAGES - 1 < nk) fetch(kt + STAGES - 1, (kt + STAGES - 1) % STAGES);   // that buffer was read before the barrier
-    const float* xs = smem + (size_t)(kt % STAGES) * ROWS * BK;
+    if (i + STAGES - 1 < nk) fetch(load.kt, (i + STAGES - 1) % STAGES), load = next(load);   // that buffer was read before the barrier
+    const float* xs = smem + (size_t)(i % STAGES) * ROWS * BK;
     const float* ws = xs + BM * BK;
-    const int steps = min(BK, K - kt * BK);
-    if constexpr (WIDE) {
-      const int rx = wm + lane % 32, rw = wn + lane % 32, h = lane / 32;
-      auto eight = [&](int c) {       // eight k-values: two chunks, one for each half of the wave
-        const f32x4 a = *(const f32x4*)(xs + rx * BK + (((c + h) ^ (rx >> 1)) & 7) * 4);
-        const f32x4 b = *(const f32x4*)(ws + rw * BK + (((c + h) ^ ((BM + rw) >> 1)) & 7) * 4);
+    const int steps = min(BK, K - at.kt * BK);
+    auto sixteen = [&](int c, bool in) {     // sixteen k-values: four chunks of 4, one for each quarter of the wave
+      f32x4 a[2], b[FN];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], acc, 0, 0, 0);
-      };
-      if (steps == BK) {
+      for (int j = 0; j < 2; ++j) a[j] = *(const f32x4*)(xs + (wm + 16 * j + r16) * BK + (((c + q) ^ ((wm + 16 * j + r16) >> 1)) & 7) * 4);
 #pragma unroll
-        for (int c = 0; c < 8; c += 2) eight(c);
-      } else {
-        for (int c = 0; 4 * c < steps; c += 2) eight(c);
+      for (int j = 0; j < FN; ++j) b[j] = *(const f32x4*)(ws + (wn + 16 * j + r16) * BK + (((c + q) ^ ((BM + wn + 16 * j + r16) >> 1)) & 7) * 4);
+      if (!in) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ia = 0; ia < 2; ++ia)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[ia][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][e], a[ia][e], acc[ia][j], 0, 0, 0);
+    };
+    if (steps == BK) {
+      sixteen(0, true), sixteen(4, true);
     } else {
-      const int rx = wm + lane % 16, rw = wn + lane % 16, q = lane / 16;
-      auto sixteen = [&](int c) {     // sixteen k-values: four chunks, one for each quarter of the wave
-        const bool in = 4 * (c + q) < steps;
-        f32x4 a0 = *(const f32x4*)(xs + rx * BK + (((c + q) ^ (rx >> 1)) & 7) * 4);
-        f32x4 a1 = *(const f32x4*)(xs + (rx + 16) * BK + (((c + q) ^ ((rx + 16) >> 1)) & 7) * 4);
-        f32x4 b = *(const f32x4*)(ws + rw * BK + (((c + q) ^ ((BM + rw) >> 1)) & 7) * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          half[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a0[e] : 0.f, in ? b[e] : 0.f, half[0], 0, 0, 0);
-          half[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a1[e] : 0.f, in ? b[e] : 0.f, half[1], 0, 0, 0);
-        }
-      };
-#pragma unroll
-      for (int c = 0; c < 8; c += 4)
-        if (4 * c < steps) sixteen(c);
+      for (int c = 0; 4 * c < steps; c += 4) sixteen(c, 4 * (c + q) < steps);
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this tile's reads are done when the next barrier is reached
-  }
-  if constexpr (WIDE) {
+    const Place behind = next(at);
+    if (behind.of_class != at.of_class) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = m0 + wm + 8 * (e / 4) + 4 * (lane / 32) + e % 4, n = n0 + wn + lane % 32;
-      if (m < M && n < N) out[(size_t)m * N + n] = point_activation(point, acc[e]);
+      for (int ia = 0; ia < 2; ++ia)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) total[ia][j] += acc[ia][j], acc[ia][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-  } else {
+    at = behind;
+  }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+  for (int ia = 0; ia < 2; ++ia)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + wm + 16 * i + 4 * (lane / 16) + e, n = n0 + wn + lane % 16;
-        if (m < M && n < N) out[(size_t)m * N + n] = point_activation(point, half[i][e]);
+        const int m = m0 + wm + 16 * ia + r16, n = n0 + wn + 16 * j + 4 * q + e;
+        if (m < M && n < N) out[(size_t)m * N + n] = point_activation(point, total[ia][j][e]);
       }
-  }
 }
 
 // The accumulators of a wave (TM x TN tiles of MFMA 32x32: D[m = 8*(e/4) + 4*(lane/32) + e%4][n = lane%32])
@@ -1357,10 +1359,9 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   if (dtype == 0) {
     const float *xf = (const float*)x, *wf = (const float*)w;
     float* of = (float*)out;
-    // loads of 16 bytes; eight k-values a step of the tiles
     const bool loads16 = !force_simt && K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
     // (a wide W of 33 to 64 rows: one tile of x, and W by the tiles; N = 19,456, K = 2,560: 182 -> 143 us)
-    if (loads16 && (M <= 32 || (M <= 64 && (N < 8192 || K % 8)))) {
+    if (loads16 && (M <= 32 || (M <= 64 && N < 8192))) {
       const int groups = (N + 15) / 16;
       if (M <= 16) gemm_f32_few_kernel<1, 8><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
       else if (M <= 32) gemm_f32_few_kernel<2, 4><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
@@ -1368,7 +1369,7 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
       SYN_LAUNCH_CHECK("gemm_f32_few");
       return 0;
     }
-    if (loads16 && K % 8 == 0) {
+    if (loads16) {
       // whichever leaves less of the last round empty
       const long cus = syn_compute_units(), wide = (long)((M + 63) / 64) * ((N + 63) / 64), slim = (long)((M + 63) / 64) * ((N + 31) / 32);
       if (2 * ((wide + cus - 1) / cus) <= (slim + cus - 1) / cus)

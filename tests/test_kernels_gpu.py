@@ -220,6 +220,44 @@ def test_gemm_f32_on_the_matrix_units(ops, M, N, K):
     close(out, want.float(), 2 ** -24 * K * 4, 1e-6, f"gemm f32 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("N,K", [(48, 4), (33, 68), (100, 260), (2560, 1000), (1000, 2052), (8200, 544), (9000, 612)])
+def test_gemm_f32_rows_do_not_depend_on_the_batch(ops, N, K):
+    """Every split of the 32-bit products adds in the same order: a row has the same bits alone, among few and among many rows."""
+    M = 300
+    x, w = rnd((M, K), 10).to(DEV), rnd((N, K), 11).to(DEV)
+    whole = torch.empty((M, N), device=DEV)
+    ops.gemm(x, w, whole)
+    for m in (1, 3, 16, 17, 32, 33, 64, 65, 128, 200):
+        for lo in {0, M - m}:
+            out = torch.empty((m, N), device=DEV)
+            ops.gemm(x[lo:lo + m].contiguous(), w, out)
+            assert torch.equal(out, whole[lo:lo + m]), (m, lo)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,window", [(8, 2, 64, 0), (8, 4, 32, 100), (4, 4, 6, 0), (8, 1, 128, 64)])
+def test_attention_f32_does_not_depend_on_the_batch(ops, nh, nkv, hd, window):
+    """Many tokens (a wave a head) and few of the same (the keys over four waves): the same bits."""
+    past, new = [300, 0, 64], [4, 500, 129]
+    lens = [p + n for p, n in zip(past, new)]
+    width = max((T + 63) // 64 for T in lens)
+    table = shuffled_table(len(past), width, 4)
+    k, v = make_cache(len(past) * width, nkv, hd, F32, 33, fill="nan")
+    fill_sequences(k, v, table, lens, nkv, hd, F32, 34)
+    tok_seq, tok_pos, _, _, _ = step_arrays(past, new)
+    q = rnd((len(tok_seq), nh * hd), 35, scale=2.0)
+    d = lambda t: t.to(DEV)
+    k, v, table = d(k), dv(v), d(table)
+
+    def run(rows):
+        out = torch.empty((len(rows), nh * hd), device=DEV)
+        ops.attention_f32(d(q[rows]), k, v, table, d(tok_seq[rows]), d(tok_pos[rows]), out, 0.3, window, nh, nkv, hd)
+        return out
+    whole = run(torch.arange(len(tok_seq)))
+    assert torch.isfinite(whole).all()
+    for rows in (torch.tensor([0]), torch.tensor([3, 4, 503, 504, 632]), torch.arange(200, 330)):
+        assert torch.equal(run(rows), whole[d(rows)])
+
+
 @pytest.mark.parametrize("hd,past,new", [(6, [300, 0], [1, 2]), (6, [0, 70], [200, 150]), (32, [1000], [1]), (128, [70], [3])])
 def test_attention_f32_splits_and_head_sizes(ops, hd, past, new):
     """Few tokens (the keys over four waves, more waves than blocks of keys among them) and many, head sizes that 16-byte loads
