@@ -1,7 +1,9 @@
-"""The streamed products issue their matrix instructions as inline assembly with the sums in place: the compiler does not
-know them for matrix instructions and would read a sum right behind one without the wait that takes.  So no sum may be
-moved between a kernel's first matrix instruction and the wait behind its last: read from the assembly of these two sources."""
+"""The streamed products and latent attention's prompts issue their matrix instructions as inline assembly: the compiler does not
+know them for matrix instructions and would read a sum right behind one without the wait that takes.  So in the streamed
+products no sum may be moved between a kernel's first matrix instruction and the wait behind its last, and in all three no
+vector instruction may come too close: read from the assembly of these sources."""
 
+import functools
 import os
 import re
 import subprocess
@@ -12,13 +14,23 @@ from synaptix_amd.kernels import build
 
 
 
-def kernels_of(source, kernel, tmp_path):
+@functools.lru_cache(maxsize=None)
+def assembly_of(source, folder):
     _, defines = build._spec("core")
     flags = [f for f in build.FLAGS if f != "-shared"]
-    listing = tmp_path / "out.s"
+    listing = folder / (source + ".s")
     subprocess.check_call([build.find_hipcc(), "-w", *flags, *defines, "-S", "--cuda-device-only",
                            os.path.join(build.CSRC, source), "-o", str(listing)])
-    lines = listing.read_text().split("\n")
+    return listing.read_text().split("\n")
+
+
+@pytest.fixture(scope="module")
+def folder(tmp_path_factory):
+    return tmp_path_factory.mktemp("assembly")
+
+
+def kernels_of(source, kernel, folder):
+    lines = assembly_of(source, folder)
     starts = [i for i, l in enumerate(lines) if re.match(rf"_Z\d+{kernel}\w*:", l)]
     assert starts
     for start in starts:
@@ -26,9 +38,12 @@ def kernels_of(source, kernel, tmp_path):
         yield lines[start], [l.split(";")[0].strip() for l in lines[start:end]]
 
 
-@pytest.mark.parametrize("source,kernel", [("gemm.hip", "gemm_stream_kernel"), ("grouped.hip", "grouped_stream_kernel")])
-def test_no_sum_moves_between_matrix_instructions(source, kernel, tmp_path):
-    for name, body in kernels_of(source, kernel, tmp_path):
+STREAMED = [("gemm.hip", "gemm_stream_kernel"), ("grouped.hip", "grouped_stream_kernel")]
+
+
+@pytest.mark.parametrize("source,kernel", STREAMED)
+def test_no_sum_moves_between_matrix_instructions(source, kernel, folder):
+    for name, body in kernels_of(source, kernel, folder):
         matrix = [i for i, l in enumerate(body) if "v_mfma" in l]
         behind = next(i for i in range(matrix[-1], len(body)) if "s_nop 15" in body[i])
         moves = [l for l in body[matrix[0]:behind] if "v_accvgpr" in l or "scratch_" in l]
@@ -42,10 +57,11 @@ def registers(operand):
     return {(m[4], int(m[5]))} if m[4] else {(m[1], k) for k in range(int(m[2]), int(m[3]) + 1)}
 
 
-def test_vector_instructions_keep_away_from_matrix_instructions(tmp_path):
-    """Latent attention's prompts mix both: no vector instruction may write what a matrix instruction reads one or two states
-    later, nor touch a result within eighteen of its start."""
-    for name, body in kernels_of("latent_attention.hip", "latent_prompt_bf16_kernel", tmp_path):
+@pytest.mark.parametrize("source,kernel", STREAMED + [("latent_attention.hip", "latent_prompt_bf16_kernel")])
+def test_vector_instructions_keep_away_from_matrix_instructions(source, kernel, folder):
+    """No vector instruction may write what a matrix instruction reads one or two states later, nor touch a result within
+    eighteen of its start (latent attention mixes both on every page; the streamed products at the ends of their tiles)."""
+    for name, body in kernels_of(source, kernel, folder):
         body = [l for l in body if re.match(r"[a-z]+_", l)]
         for i, line in enumerate(body):
             if not line.startswith("v_"):
