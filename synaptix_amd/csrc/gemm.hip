@@ -9,11 +9,12 @@
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
 //   gemm_packed    bf16, M <= 16 (used up to 8): the same over a copy of W kept in the order of the MFMA
 //                  fragments, so that every load of a wave is 1 KB of consecutive bytes.
-//   gemm_stream    bf16, M > 128, K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
+//   gemm_stream    bf16, M > 64, K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
 //                  stream of k-steps over all tiles of a workgroup.
-//   gemm_direct    bf16, up to 128 rows: 32 to 128 rows of x, 64 to 128 rows of W, 64 or 128 deep, straight into LDS: the rows
-//                  of W arrive as whole 256-byte pieces, which streams them faster than loading MFMA fragments (64
-//                  bytes a row) straight from memory.
+//   gemm_direct    bf16, up to 64 rows, and up to 256 where its tiles go round once or their reader adds partial sums: 32 to 256
+//                  rows of x, 64 to 128 rows of W, 64 to 256 deep, straight into LDS: the rows of W arrive as whole
+//                  256-byte pieces, which streams them faster than loading MFMA fragments (64 bytes a row) straight
+//                  from memory.
 //   gemm_tiled     bf16, any K that is a multiple of 8: the tiles pass through registers on their way to LDS.
 //                  The last three: K may be cut into slices whose partial sums the reader adds; with paired rows W holds
 //                  those of a gate and of an up projection in turns of 16 and the kernel stores act(gate) * up,
@@ -1323,6 +1324,15 @@ static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, 
   return launch_tiled<128, 128, 64, 2, 2, PAIRED>(x, w.p, out, ep, M, N, K, stream);
 }
 
+// Whether an uncut product of 65 to 256 rows goes through the 64 x 128 tiles with k-tiles of 128 (gemm_direct): where they go round once
+// (tile_grid, which counts what each XCD gets), W arrives in longer pieces than the streamed tiles ask for.  Weights that no cache
+// holds, direct against streamed: 4096 x 4096 96 rows 26.6 us against 28.8, 128 rows 29.1, 35.4, 256 rows 29.2, 35.2; 10,240 x 5,120
+// 128 rows 39.6, 48.4; 4096 x 12288 192 rows 80.5, 101.2.  Not where the last 64 rows are few (4096 x 12288: 65 rows 71.5, 66.4; 81
+// rows 69.2, 71.3; 193 rows 76.9, 66.3; 208 rows 71.7, 71.2), and not in two rounds (10,240 x 4,096 129 rows 50.1, 27.7).
+static bool direct_one_round(int M, int N) {
+  return M <= 256 && (M - 1) % 64 >= 16 && tile_grid(M, N, 64, 128) <= syn_compute_units();
+}
+
 // Into how many slices of K a product of more than 64 rows is cut when its reader adds partial sums: the smallest estimate of
 // the product's time and of what its reader pays for the slices beyond the first (M x N floats each, half of them from caches).
 SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
@@ -1427,6 +1437,9 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     // round (N = 4096): down_proj 38 us with 256 rows, 37 with 224 and 35 with 192 (the streamed tiles 42, 39 and 37); q/k/v
     // with N = 6144 in two slices 26, 25.5 and 25 (the streamed tiles 25, 24 and 23, which it therefore takes).
     rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
+  } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N)) {
+    // the same of up to 256 rows whose reader takes the finished product
+    rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream);
   } else if (M <= 64) {
     rc = launch_tiled<64, 64, 128, 2, 2>(xb, wb, out, ep, M, N, K, stream, slices);
   } else {

@@ -510,6 +510,20 @@ def test_products_of_a_prompt_at_the_sizes_of_an_8b_layer(ops):
     close(q[rows.to(DEV), cols.to(DEV)], want, 0.02, 1e-2, "q/k/v at 8B sizes")
 
 
+@pytest.mark.parametrize("M", [65, 80, 81, 128, 129, 145, 192, 208, 209, 256])
+@pytest.mark.parametrize("N,K,packed", [(16, 128, True), (1008, 384, True), (8192, 256, True), (16384, 256, True), (333, 256, False)])
+def test_products_of_65_to_256_rows_at_the_lines_of_their_tiles(ops, M, N, K, packed):
+    """Both sides of the line between the 64 x 128 tiles and the streamed ones, ragged in both directions, W in fragment order and in
+    plain rows: every value against 64 bits."""
+    x, w = rnd((M, K), 86, BF16).to(DEV), rnd((N, K), 87, BF16).to(DEV)
+    want = (x.double() @ w.double().T).float()
+    for dt in (F32, BF16):
+        out = torch.full((M, N), float("nan"), dtype=dt, device=DEV)
+        ops.gemm(x, ops.pack_weight(w) if packed else w, out)
+        # exact products, 32-bit sums of K terms of size one; bf16: half a unit in the last of 8 bits on top
+        close(out, want, 1e-4 * math.sqrt(K), 0 if dt == F32 else 2 ** -8, f"{M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("M,N,K,S", [
     (129, 16, 128, 1), (300, 1040, 160 * 2, 1),              # fewer columns than a tile; the ring's shortest K
     (2305, 24592, 256, 1), (5000, 4112, 512, 1),             # several tiles a workgroup, ragged in both directions
