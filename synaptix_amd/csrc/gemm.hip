@@ -1190,9 +1190,9 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
       }
     };
     if constexpr (OUT == SYN_OUT_GATED) {
-      if (ep.act == SYN_ACT_SILU) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SILU>(g, u, 0.f); });
-      else if (ep.act == SYN_ACT_SWIGLU_LIMIT) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SWIGLU_LIMIT>(g, u, ep.limit); });
-      else store_all([&](float g, float u) { return gated_quick<SYN_ACT_GELU_TANH>(g, u, 0.f); });
+      if (ep.act == SYN_ACT_SILU) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SILU, false>(g, u, 0.f); });
+      else if (ep.act == SYN_ACT_SWIGLU_LIMIT) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SWIGLU_LIMIT, false>(g, u, ep.limit); });
+      else store_all([&](float g, float u) { return gated_quick<SYN_ACT_GELU_TANH, false>(g, u, 0.f); });
     } else {
       if (ep.point == SYN_POINT_NONE) store_all([&](float v, float) { return v; });
       else store_all([&](float v, float) { return point_activation(SYN_POINT_RELU_SQUARED, v); });

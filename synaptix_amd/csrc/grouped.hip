@@ -571,9 +571,9 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
       }
     };
     if constexpr (PAIR) {
-      if (g.pair - 1 == SYN_ACT_SILU) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SILU>(gt, up, 0.f); });
-      else if (g.pair - 1 == SYN_ACT_SWIGLU_LIMIT) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SWIGLU_LIMIT>(gt, up, g.limit); });
-      else store_all([&](float gt, float up) { return gated_quick<SYN_ACT_GELU_TANH>(gt, up, 0.f); });
+      if (g.pair - 1 == SYN_ACT_SILU) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SILU, F32>(gt, up, 0.f); });
+      else if (g.pair - 1 == SYN_ACT_SWIGLU_LIMIT) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SWIGLU_LIMIT, F32>(gt, up, g.limit); });
+      else store_all([&](float gt, float up) { return gated_quick<SYN_ACT_GELU_TANH, F32>(gt, up, 0.f); });
     } else {
       if (g.act == 0) store_all([&](float v, float) { return v; });
       else if (g.act == 2) store_all([&](float v, float) { return point_activation(SYN_POINT_RELU_SQUARED, v); });

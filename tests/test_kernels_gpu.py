@@ -571,10 +571,11 @@ def test_gated_activations_of_many_rows(ops, act, M, I, K):
     close(out[rows.to(DEV), cols.to(DEV)], want.float(), 1e-4 * math.sqrt(K), 2 ** -8 + 1e-4, f"{act} {M}x{I}x{K}")
 
 
+@pytest.mark.parametrize("out_dtype", [F32, BF16])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
-def test_gated_epilogue_of_streamed_tiles_is_no_less_exact(ops, act):
-    """The epilogue that the streamed tiles make of the hardware's base-2 functions, stored as 32-bit numbers, against 64 bits and
-    beside the library functions of the plain kernel, on the same sums: rows of x hold a 1 and a power of two, so the sums
+def test_gated_epilogue_of_streamed_tiles_is_no_less_exact(ops, act, out_dtype):
+    """The epilogue that the streamed tiles make of the hardware's base-2 functions, against 64 bits and beside the
+    library functions of the plain kernel, on the same sums: rows of x hold a 1 and a power of two, so the sums
     are exact, gates from -120 to 120 (beyond e^88, where the library's exponential overflows) and from -3 to 3, and infinities."""
     K, J, P = 256, 1024, 512
     g = torch.Generator().manual_seed(7)
@@ -602,15 +603,19 @@ def test_gated_epilogue_of_streamed_tiles_is_no_less_exact(ops, act):
     seg = torch.tensor([0, P], dtype=I32, device=DEV)
     outs = []
     for plain in (False, True):
-        out = torch.full((P, J // 2), float("nan"), dtype=F32, device=DEV)
+        out = torch.full((P, J // 2), float("nan"), dtype=out_dtype, device=DEV)
         ops.experts_product(d(x), d(w) if plain else ops.pack_expert_weights(d(w)), out, seg, ids, ids, gated=act, force_simt=plain)
         outs.append(out.cpu().double())
     # (results below the smallest normal number, and where the plain kernel's overflow gave nothing, tell nothing about rounding)
     tell = (want.abs() > 1e-30) & (outs[1] != 0)
     off = [((o - want).abs() / want.abs())[tell] for o in outs]
     assert float(tell.float().mean()) > 0.7
-    assert float(off[0].max()) <= float(off[1].max()) and float(off[0].norm()) <= float(off[1].norm()), [float(o.max()) * 2 ** 24 for o in off]
-    assert ((outs[0] - want).abs() <= (outs[1] - want).abs() + 1e-29)[~tell].all()
+    if out_dtype == F32:
+        assert float(off[0].max()) <= float(off[1].max()) and float(off[0].norm()) <= float(off[1].norm()), [float(o.max()) * 2 ** 24 for o in off]
+    else:
+        # half a unit in the last of 8 bits, and what a few ulp of 32 bits (|t| of them in 1.702 t, which both round) can add where that is a tie
+        assert float(off[0].max()) <= 2 ** -8 * (1 + 2 ** -8) and float(off[0].norm()) <= float(off[1].norm()) * (1 + 1e-5)
+    assert ((outs[0] - want).abs() <= (outs[1] - want).abs() + (1e-29 if out_dtype == F32 else 1e-29 + 2 ** -8 * want.abs()))[~tell].all()
     # infinite sums: what the plain kernel makes of them
     w[0, 0, :], w[0, 2, :] = float("inf"), -float("inf")
     a, b = torch.empty(P, J // 2, device=DEV), torch.empty(P, J // 2, device=DEV)
