@@ -1288,7 +1288,8 @@ static int launch_stream_as(int tile, const bf16* x, Weight w, void* out, Epilog
     case 6: return launch_stream<192, 192, OUT, false>(x, w, out, ep, M, N, K, stream, slices);
     case 7: return launch_stream<128, 192, OUT, false>(x, w, out, ep, M, N, K, stream, slices);
     case 8: return launch_stream<64, 128, OUT, true>(x, w, out, ep, M, N, K, stream, slices);
-    default: return launch_stream<64, 192, OUT, false>(x, w, out, ep, M, N, K, stream, slices);
+    case 9: return launch_stream<64, 192, OUT, false>(x, w, out, ep, M, N, K, stream, slices);
+    default: SYN_CHECK(false, "gemm: there is no streamed tile %d", tile);
   }
 }
 
@@ -1309,8 +1310,8 @@ static int pick_register_tile(int M, int N) {
 // M > 64.  A K that the kernel above does not take goes through the tiles that pass through registers (any K that is a multiple
 // of 8, one slice) or, in slices, through the smallest of those that load straight into LDS.
 template <bool PAIRED>
-static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1) {
-  const int tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
+static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1, int tile = -1) {
+  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
   if (tile >= 0) {
     if (PAIRED) return launch_stream_as<SYN_OUT_GATED>(tile, x, w, out, ep, M, N, K, stream, slices);
     if (ep.out_is_f32) return launch_stream_as<SYN_OUT_F32>(tile, x, w, out, ep, M, N, K, stream, slices);
@@ -1355,8 +1356,11 @@ SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
 // w_packed: w is the weight in fragment order (pack_weight; bf16, N a multiple of 16, K of 128): for the tiles that
 // load straight into LDS; the other kernels read plain rows only.
 // point: what the finished sums pass before they are stored (point_activation; one slice).
+// tile: -1, or for tests and measurements one of STREAM_TILES, whatever the rules below would take (bf16 operands).
 SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int M, int N, int K, int force_simt,
-                        int slices, int w_packed, int point, hipStream_t stream) {
+                        int slices, int w_packed, int point, int tile, hipStream_t stream) {
+  SYN_CHECK(tile < 0 || (dtype != 0 && !force_simt && K % 64 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0),
+            "gemm: the streamed tiles take aligned bf16 operands and a K that is a multiple of 64 (K = %d)", K);
   SYN_CHECK(point >= 0 && point < SYN_POINT_COUNT && (point == SYN_POINT_NONE || slices == 1),
             "gemm: activation code %d over %d slices", point, slices);
   SYN_CHECK(M > 0 && N > 0 && K > 0, "gemm: empty shape M=%d N=%d K=%d", M, N, K);
@@ -1412,7 +1416,9 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   const bool few_row_tiles = M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units();
   // From sweeps at the shapes of an 8B model (N = 4096 .. 151936, K = 4096 and 12288).
   int rc = 0;
-  if (M == 1 && slices == 1 && !w_packed) {
+  if (tile >= 0) {
+    rc = launch_large<false>(xb, wt, out, ep, M, N, K, stream, slices, tile);
+  } else if (M == 1 && slices == 1 && !w_packed) {
     // one row: fragments of W straight from memory, K split over the waves
     if (N <= 8192) launch_skinny<1, 16, 4>(xb, wb, out, ep, M, N, K, stream);
     else launch_skinny<1, 8, 4>(xb, wb, out, ep, M, N, K, stream);
@@ -1453,9 +1459,10 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
 // out[M, N/2] = silu(x . Wg^T) * (x . Wu^T), bf16, where w [N, K] holds the rows of Wg and of Wu in
 // turns of 16: rows 32b .. 32b+15 are rows 16b .. 16b+15 of Wg, rows 32b+16 .. 32b+31 those of Wu.
 // The activation is applied to the 32-bit sums and rounded once.
-// w_packed: as for syn_gemm
+// w_packed, tile: as for syn_gemm
 SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, int N, int K, int act, float limit,
-                               int w_packed, hipStream_t stream) {
+                               int w_packed, int tile, hipStream_t stream) {
+  SYN_CHECK(tile < 0 || K % 64 == 0, "gemm_swiglu: the streamed tiles take a K that is a multiple of 64 (K = %d)", K);
   SYN_CHECK(M > 0 && N > 0 && K > 0, "gemm_swiglu: empty shape M=%d N=%d K=%d", M, N, K);
   SYN_CHECK(!w_packed || K % 128 == 0, "gemm_swiglu: a weight in fragment order needs K = %d a multiple of 128", K);
   SYN_CHECK(act >= 0 && act < SYN_ACT_COUNT, "gemm_swiglu: unknown activation code %d", act);
@@ -1467,7 +1474,9 @@ SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, i
   const bf16* wb = (const bf16*)w;
   int rc = 0;
   const Weight wt = {wb, w_packed != 0};
-  if (M == 1 && !w_packed) {
+  if (tile >= 0) {
+    rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream, 1, tile);
+  } else if (M == 1 && !w_packed) {
     // one row: fragments of W straight from memory; eight waves on the gate rows, eight on the up rows
     launch_skinny<2, 8, 4, true>(xb, wb, out, ep, M, N, K, stream);
   } else if (M <= 32) {

@@ -272,14 +272,15 @@ def point_code(name) -> int:
     return POINT_ACTIVATIONS[name]
 
 
-def gemm(x, w, out, force_simt=False, point=None):
+def gemm(x, w, out, force_simt=False, point=None, tile=-1):
     """out[M, N] = x[M, K] . w[N, K]^T with 32-bit accumulation.
     float x float -> float; bf16 x bf16 -> bf16 or float (MFMA, plain FMA for shapes it does not take).
     A float out of shape [S, M, N] (bf16 operands) receives S partial sums over slices of K
     instead; their sum over S is the product.
     w may be the weight in fragment order (pack_weight: four dimensions): the tiles for 9 rows and more read it
     where K is a multiple of 128; for other K the product runs in blocks of 16 rows through gemm_packed.
-    point: a name of POINT_ACTIVATIONS, applied to the finished sums before they are stored (not to partial sums)."""
+    point: a name of POINT_ACTIVATIONS, applied to the finished sums before they are stored (not to partial sums).
+    tile: for tests and measurements, a streamed tile of csrc/gemm.hip by its number whatever the rules there would take."""
     point_of = point_code(point)
     _need(x, "gemm.x", (_BF16, _F32), (None, None))
     M, K = x.shape
@@ -317,7 +318,7 @@ def gemm(x, w, out, force_simt=False, point=None):
         _need(out, "gemm.out", (_BF16, _F32), (M, N))
         code = 2 if out.dtype == _F32 else 1
     _call(load_library("core"), "syn_gemm", _ptr(x), _ptr(w), _ptr(out), code, M, N, K, 1 if force_simt else 0,
-          slices, 1 if packed else 0, point_of, _stream())
+          slices, 1 if packed else 0, point_of, tile, _stream())
 
 
 PAIR = 16   # rows of the gate and of the up projection alternate in turns of this many
@@ -331,10 +332,10 @@ def pair_rows(gate, up):
     return torch.stack([gate.view(I // PAIR, PAIR, K), up.view(I // PAIR, PAIR, K)], 1).reshape(2 * I, K).contiguous()
 
 
-def gemm_swiglu(x, w_paired, out, activation="silu"):
+def gemm_swiglu(x, w_paired, out, activation="silu", tile=-1):
     """out[M, I] = act(x . Wg^T) * (x . Wu^T) in bf16 with w_paired = pair_rows(Wg, Wu): the
     activation on the 32-bit sums inside the product, so that the two products are never stored.
-    w_paired may be in fragment order (pack_weight of the paired rows), as for gemm."""
+    w_paired may be in fragment order (pack_weight of the paired rows), as for gemm; tile: as there."""
     _need(x, "gemm_swiglu.x", _BF16, (None, None))
     M, K = x.shape
     packed = isinstance(w_paired, torch.Tensor) and w_paired.dim() == 4
@@ -352,7 +353,7 @@ def gemm_swiglu(x, w_paired, out, activation="silu"):
                         activation=activation)
         return
     _call(load_library("core"), "syn_gemm_swiglu", _ptr(x), _ptr(w_paired), _ptr(out), M, N, K,
-          *_activation_args(activation), 1 if packed else 0, _stream())
+          *_activation_args(activation), 1 if packed else 0, tile, _stream())
 
 
 PACKED_BLOCK_ROWS = 16   # the most rows that a product of gemm_packed takes

@@ -549,6 +549,77 @@ def test_streamed_tiles_run_on_into_the_next_tile(ops, M, N, K, S):
             close(got, want, 1e-3 * math.sqrt(K), 0 if dt == F32 else 2 ** -8, f"{M}x{N}x{K}, slice {s} of {S}")
 
 
+PLAIN_TILES = (0, 1, 2, 8)          # the streamed tiles that also read W in plain rows
+
+
+@pytest.mark.parametrize("kind", ["float", "bf16", "gated", "slices"])
+@pytest.mark.parametrize("tile", range(10))
+def test_every_streamed_tile(ops, tile, kind):
+    """Each tile by its number, whatever the rules would take, with every output that it is compiled for: W in fragment order and
+    (where compiled) in plain rows of a width that is no multiple of 16; ragged M and N, one tile and several tiles a workgroup, the
+    shortest K that its ring allows, and slices whose last one is shorter.  Every value against 64 bits."""
+    for M, N, K, S in ((70, 48, 256, 1), (1100, 2064, 256, 1), (5000, 4112, 256, 1), (300, 1040, 640, 2), (1300, 2576, 1024, 3)):
+        if (kind == "slices") != (S > 1):
+            continue
+        if kind == "gated":
+            N = (N + 31) // 32 * 32
+        x, w = rnd((M, K), 88, BF16).to(DEV), rnd((N, K), 89, BF16).to(DEV)
+        step = ((K + S - 1) // S + 127) // 128 * 128
+        for packed in (True, False):
+            if not packed and tile not in PLAIN_TILES:
+                continue
+            n = N if packed or kind == "gated" else N - 7
+            wn = w[:n].contiguous()
+            want = torch.stack([x[:, k:k + step].double() @ wn[:, k:k + step].double().T for k in range(0, K, step)])
+            wk = ops.pack_weight(wn) if packed else wn
+            tol = 1e-4 * math.sqrt(K)          # exact products, 32-bit sums of K terms of size one
+            if kind == "gated":
+                out = torch.full((M, N // 2), float("nan"), dtype=BF16, device=DEV)
+                ops.gemm_swiglu(x, wk, out, tile=tile)
+                z = want[0].view(M, N // 32, 2, 16)
+                g, u = z[:, :, 0].reshape(M, -1), z[:, :, 1].reshape(M, -1)
+                # (both factors carry the sums' error)
+                off = (out.double() - g * torch.sigmoid(g) * u).abs() - 2 ** -8 * (g * torch.sigmoid(g) * u).abs() - tol * (g.abs() + u.abs() + 1)
+            else:
+                dt = BF16 if kind == "bf16" else F32
+                out = torch.full((S, M, n) if S > 1 else (M, n), float("nan"), dtype=dt, device=DEV)
+                ops.gemm(x, wk, out, tile=tile)
+                off = (out.double().view(want.shape) - want).abs() - (2 ** -8 if dt == BF16 else 0) * want.abs() - tol
+            assert torch.isfinite(out).all() and float(off.max()) <= 0, (M, N, K, S, packed, float(off.max()))
+
+
+def test_there_are_ten_streamed_tiles_and_they_refuse_what_they_do_not_take(ops):
+    from synaptix_amd.kernels.ops import KernelError
+    x, w, out = (torch.zeros(s, dtype=BF16, device=DEV) for s in ((70, 256), (48, 256), (70, 48)))
+    packed = ops.pack_weight(w)
+    for tile, weight in [(10, packed), (11, packed)] + [(t, w) for t in range(10) if t not in PLAIN_TILES]:
+        with pytest.raises(KernelError):
+            ops.gemm(x, weight, out, tile=tile)
+    with pytest.raises(KernelError):      # a ring of eight k-tiles needs a K of 256
+        ops.gemm(x[:, :128].contiguous(), w[:, :128].contiguous(), out, tile=8)
+    with pytest.raises(KernelError):
+        ops.gemm(x.float(), w.float(), out.float(), tile=0)
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("N,K", [(800, 192), (24576, 256), (28672, 256), (32800, 256)])
+@pytest.mark.parametrize("M", [128, 129, 192, 193, 256, 257])
+def test_gated_products_of_129_to_256_rows(ops, M, N, K, packed):
+    """At the lines between the streamed tiles and those that hold all rows of x, which go round once or not at all (N = 32,800), W in
+    fragment order and in plain rows: every value against 64 bits."""
+    x, w = rnd((M, K), 92, BF16).to(DEV), rnd((N, K), 93, BF16).to(DEV)
+    if packed and K % 128:
+        pytest.skip("in fragment order K is a multiple of 128")
+    out = torch.full((M, N // 2), float("nan"), dtype=BF16, device=DEV)
+    ops.gemm_swiglu(x, ops.pack_weight(w) if packed else w, out)
+    z = (x.double() @ w.double().T).view(M, N // 32, 2, 16)
+    g, u = z[:, :, 0].reshape(M, -1), z[:, :, 1].reshape(M, -1)
+    want = g * torch.sigmoid(g) * u
+    # the sums are off by at most 1e-4 sqrt(K) (products exact, 32-bit sums of K terms of size one), and both factors carry that; one rounding
+    off = (out.double() - want).abs() - 2 ** -8 * want.abs() - 1e-4 * math.sqrt(K) * (g.abs() + u.abs() + 1)
+    assert torch.isfinite(out).all() and float(off.max()) <= 0, float(off.max())
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
 @pytest.mark.parametrize("M,I,K", [(300, 1200, 256), (2100, 4112, 512)])
 def test_gated_activations_of_many_rows(ops, act, M, I, K):
