@@ -1205,40 +1205,51 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
 }
 
 // The tiles that the kernel comes in, and the estimate of a product's time that picks one of them and the slices of K.  Three
-// things run side by side, and the longest counts most (a norm of order 2.3): rounds of tiles over the chip at `round` us for
-// 4,096 of K; the matrix units' power, at `power` us for 4,096 of K with a tile on every compute unit; and the way of W from
-// memory, which is longer where fewer compute units ask for it.  The stores of the output come on top.  The figures are
-// fitted to 6,400 products measured with weights that no cache held: M = 66 .. 3,270, N x K = 6144 x 4096, 4096 x 4096, 4096
-// x 12288, 24576 x 4096 (gated), 2560 x 9728, 2560 x 4096, 19456 x 2560 (gated), 5120 x 25600, 3072 x 1024, 1024 x 4096, 8192 x
-// 1024 (gated), every tile in 1 to 8 slices of K.  What the estimate picks takes 2 % longer than the fastest on average
-// (20 % at the worst of 198 sizes), and a factor of 1.38 less (geometric mean) than the tiles before this kernel.
+// things run side by side, and the longest counts most (a norm of order 2): rounds of tiles over the chip at `round` us for 4,096
+// of K, a quarter of them whatever stands in the tiles; the matrix units' power, at `power` us for 4,096 of K with a tile on every
+// compute unit; and the way of W from memory, which is longer where fewer compute units ask for it.  Rows and columns beyond M
+// and N are zeros, which draw next to no power: with 129 rows 19,456 x 2,560 takes 34 us, with 256, the same tiles, 48.  So
+// both count by the share of a tile that is filled.  The stores of the output come on top.
+// The figures are fitted to 9,200 products measured with weights that no cache held: 72 to 3,000 rows, multiples of the tiles and
+// others, through N x K = 6144 x 4096, 4096 x 4096, 4096 x 12288, 2560 x 9728, 10240 x 5120, 32768 x 4096, 12288 x 4096, 8192 x 2048,
+// 5120 x 17408, 2048 x 8192, 6144 x 2560 (32-bit sums in 1, 2 and 4 slices of K) and, gated, 24576 x 4096, 19456 x 2560, 51200 x
+// 5120, 16384 x 2048, 28672 x 4096, 32768 x 4096, 20480 x 8192, 22016 x 4096, 17408 x 5120, 8192 x 1024, every tile.  What
+// the estimate picks takes 0.6 % longer than the fastest on average; 4 % of the sizes lose more than 5 %, 2 % more than 10 %.
 struct StreamTile {
   int bm, bn;
   double round, power;
   bool plain;       // also over W in plain rows (the others are compiled for fragment order alone)
 };
 static const StreamTile STREAM_TILES[] = {
-    {256, 256, 74.6, 46.9, true},  {256, 192, 61.6, 44.9, true},  {128, 128, 33.1, 17.3, true},  {192, 256, 60.6, 36.3, false},
-    {128, 256, 52.1, 28.2, false}, {256, 128, 47.8, 38.5, false}, {192, 192, 52.5, 30.3, false}, {128, 192, 44.2, 19.4, false},
-    {64, 128, 20.0, 21.0, true},   {64, 192, 31.2, 20.8, false}};
+    {256, 256, 82.9, 33.2, true},  {256, 192, 74.7, 20.6, true},  {128, 128, 38.0, 14.4, true},  {192, 256, 67.0, 24.9, false},
+    {128, 256, 56.0, 25.9, false}, {256, 128, 66.6, 22.0, false}, {192, 192, 59.0, 26.9, false}, {128, 192, 45.3, 16.3, false},
+    {64, 128, 23.5, 12.2, true},   {64, 192, 38.1, 5.3, false},
+    // of gemm_direct, for gated products of one tile of rows that go round once (W arrives in longer pieces; 28,672 x 4,096 with 224
+    // rows 69.5 us through the best streamed tile, 65.7 so; 32,768 x 4,096 75.9, 69.5)
+    {192, 128, 49.5, 0.0, true},   {256, 128, 46.2, 20.7, true}};
+constexpr int STREAMED_TILES = 10;
 static int stream_slice(int K, int slices) { return ((K + slices - 1) / slices + 127) / 128 * 128; }
 static int stream_last_slice(int K, int slices) { return K - (slices - 1) * stream_slice(K, slices); }
 struct StreamPlan {
   int tile;        // -1: none takes this K (k-steps come in pairs, and a slice holds a ring of them at least)
   double us;
 };
-static StreamPlan plan_stream(int M, int N, int K, int slices, bool packed, int out_bytes) {
+static StreamPlan plan_stream(int M, int N, int K, int slices, bool packed, int out_bytes, bool gated) {
   StreamPlan best = {-1, 1e30};
   if (K % 64) return best;
   const long cus = syn_compute_units();
   const double k = stream_slice(K, slices) / 4096.0;
   for (int i = 0; i < (int)(sizeof(STREAM_TILES) / sizeof(STREAM_TILES[0])); ++i) {
     const StreamTile& s = STREAM_TILES[i];
-    if ((!packed && !s.plain) || stream_last_slice(K, slices) < 32 * stream_stages(s.bm, s.bn)) continue;
-    const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * slices;
-    const double work = (double)((tiles + cus - 1) / cus) * s.round * k + 4.6, power = (double)tiles / cus * s.power * k;
-    const double way = 0.143e-6 * 2.0 * N * K * pow((double)cus / (double)(tiles < cus ? tiles : cus), 0.59);
-    const double us = pow(pow(work, 2.28) + pow(way, 2.28) + pow(power, 2.28), 1.0 / 2.28) + 0.234e-6 * M * N * slices * out_bytes;
+    if (i < STREAMED_TILES ? (!packed && !s.plain) || stream_last_slice(K, slices) < 32 * stream_stages(s.bm, s.bn)
+                           : !gated || M > s.bm || M <= s.bm - 64 || tile_grid(M, N, s.bm, s.bn) > cus)
+      continue;
+    const long down = (M + s.bm - 1) / s.bm, across = (N + s.bn - 1) / s.bn, tiles = down * across * slices;
+    const double filled = (double)M / (double)(down * s.bm) * (double)N / (double)(across * s.bn);
+    const double work = (double)((tiles + cus - 1) / cus) * s.round * k * (0.255 + 0.745 * filled) + 4.5;
+    const double power = (double)tiles / cus * s.power * k * filled;
+    const double ask = tiles < cus ? cbrt((double)cus / (double)tiles) : 1.0, way = 0.146e-6 * 2.0 * N * K * ask * ask;
+    const double us = sqrt(work * work + way * way + power * power) + 0.229e-6 * M * N * slices * out_bytes;
     if (us < best.us) best = {i, us};
   }
   return best;
@@ -1311,7 +1322,11 @@ static int pick_register_tile(int M, int N) {
 // of 8, one slice) or, in slices, through the smallest of those that load straight into LDS.
 template <bool PAIRED>
 static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1, int tile = -1) {
-  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
+  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2, PAIRED).tile;
+  if constexpr (PAIRED) {
+    if (tile == STREAMED_TILES) return launch_direct<192, 128, 64, 2, 2, true, 3>(x, w, out, ep, M, N, K, stream);
+    if (tile == STREAMED_TILES + 1) return launch_direct<256, 128, 64, 4, 2, true, 3>(x, w, out, ep, M, N, K, stream);
+  }
   if (tile >= 0) {
     if (PAIRED) return launch_stream_as<SYN_OUT_GATED>(tile, x, w, out, ep, M, N, K, stream, slices);
     if (ep.out_is_f32) return launch_stream_as<SYN_OUT_F32>(tile, x, w, out, ep, M, N, K, stream, slices);
@@ -1341,7 +1356,7 @@ SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
   double least = 1e30;
   if (M <= 0 || N <= 0 || K <= 0) return 1;
   for (int s : {1, 2, 3, 4, 6, 8}) {
-    const StreamPlan p = plan_stream(M, N, K, s, true, 4);
+    const StreamPlan p = plan_stream(M, N, K, s, true, 4, false);
     if (p.tile < 0) break;
     const double us = p.us + (s - 1) * 0.12e-6 * 4.0 * M * N;
     if (us < least) least = us, best = s;
@@ -1414,7 +1429,7 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   const bf16* wb = (const bf16*)w;
   const Weight wt = {wb, w_packed != 0};
   const bool few_row_tiles = M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units();
-  // From sweeps at the shapes of an 8B model (N = 4096 .. 151936, K = 4096 and 12288).
+  // (from sweeps at the shapes of an 8B model, N = 4096 .. 151936, K = 4096 and 12288, where no other are named)
   int rc = 0;
   if (tile >= 0) {
     rc = launch_large<false>(xb, wt, out, ep, M, N, K, stream, slices, tile);

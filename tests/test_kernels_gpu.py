@@ -281,10 +281,10 @@ def test_attention_f32_splits_and_head_sizes(ops, hd, past, new):
 @pytest.mark.parametrize("M,N,K", [
     (1, 48, 64), (3, 1000, 176), (16, 100, 320), (17, 40, 72), (33, 1000, 128), (48, 70, 2048), (64, 4096, 512),
     (65, 130, 104), (128, 128, 32), (200, 300, 1000), (513, 257, 4096),
-    (1700, 5120, 128),                  # the 256 x 160 tile: 32 tiles along N where 256 x 192 makes 27
+    (1700, 5120, 128),                  # several tiles a workgroup, the shortest K that the streamed tiles take
     (5, 30, 20), (70, 50, 36),          # K no multiple of 8: the plain kernel takes them
-    (2048, 6144, 512), (1000, 12300, 136),   # large enough for the 256 x 256 tiles with 8 waves, ragged edges
-    (1000, 12544, 128), (300, 200, 64),   # K a multiple of 64: loads straight into LDS, every tile shape
+    (2048, 6144, 512), (1000, 12300, 136),   # many rows, ragged edges: streamed, and through registers (K = 136)
+    (1000, 12544, 128), (300, 200, 64),   # K a multiple of 64: loads straight into LDS, streamed and (K = 64) in tiles of 128 x 128
     (8, 40000, 256), (40, 33000, 72), (64, 50000, 1000),   # wide
     (1, 9000, 520), (1, 70000, 136),                       # one row: W straight from memory, K over the waves
     (8, 70000, 264), (20, 66000, 72),                      # few rows, very wide: 32-row tiles, 256 deep
@@ -304,7 +304,7 @@ def test_gemm_bf16(ops, out_dtype, M, N, K):
                                      (40, 70, 2048, 2), (64, 130, 520, 5), (8, 96, 1536, 5), (50, 200, 3072, 7),
                                      (300, 520, 1024, 2), (130, 260, 640, 3), (65, 33, 4096, 4),
                                      (200, 4096, 1024, 2), (256, 1000, 2048, 4),
-                                     # short prompts cut along K: tiles of 128 x 128 up to 256 rows, of 256 x 128 beyond
+                                     # short prompts cut along K: tiles of 128 x 128 up to 128 rows (to 256 in four slices and more), streamed ones beyond
                                      (66, 6144, 4096, 4), (128, 200, 4096, 8), (129, 4100, 1024, 2), (256, 1000, 2560, 4),
                                      (257, 520, 4096, 8), (400, 2000, 1152, 2), (512, 4096, 1024, 2)])
 def test_gemm_bf16_partial_sums_over_slices_of_k(ops, M, N, K, S):
@@ -341,7 +341,7 @@ def test_gemm_bf16_partial_sums_over_slices_of_k(ops, M, N, K, S):
 @pytest.mark.parametrize("M,I,K", [(1, 48, 64), (1, 2560, 4096), (1, 1008, 1096), (8, 2560, 4096), (7, 112, 1000), (33, 80, 136), (64, 1024, 512),
                                    (300, 400, 264), (2048, 3072, 256), (1000, 6272, 136), (8, 32784, 72),
                                    (1000, 6272, 128), (300, 400, 192),
-                                   # 65 to 256 rows: all of x in one tile of 128, 192 or 256 rows and 96 or 128 rows of W
+                                   # 65 to 256 rows: all of x in one tile of 128, 192 or 256 rows and 96 or 128 rows of W, or streamed
                                    (65, 48, 64), (100, 1040, 448), (128, 12288, 512), (129, 400, 192), (192, 2000, 320),
                                    (193, 80, 1024), (256, 4864, 640), (200, 400, 72), (1700, 2560, 192)])
 def test_gemm_with_the_gated_activation_inside(ops, M, I, K):
@@ -754,7 +754,7 @@ def test_slices_fill_the_compute_units(ops):
     (9, 48, 128, 1), (16, 4096, 4096, 1), (33, 208, 256, 1), (64, 6144, 4096, 1), (64, 144, 384, 3),
     (100, 4112, 384, 1), (128, 208, 4096, 8), (130, 6144, 1024, 1), (200, 4096, 1024, 2), (256, 1008, 2560, 4),
     (257, 528, 4096, 8), (300, 96, 128, 1), (512, 4096, 1024, 2), (700, 272, 640, 1),
-    (1700, 5120, 128, 1),               # the 256 x 160 tile
+    (1700, 5120, 128, 1),               # several tiles a workgroup, the shortest K of the streamed tiles
     (2053, 528, 256, 1), (1000, 12304, 128, 1), (2048, 6144, 512, 1),   # the large tiles, ragged edges
     (8, 70000 // 16 * 16, 256, 1), (20, 66000 // 16 * 16, 128, 1),      # few rows, very wide
     (40, 80, 96, 1), (300, 48, 160, 1),                                   # K no multiple of 128: in blocks of 16 rows
