@@ -11,6 +11,7 @@
 
 #define SAMPLE_THREADS 1024
 #define DRAW_PART 32
+#define DRAW_DIRECT 16      // entries of a chunk up to which it is not passed through LDS
 
 struct ArgBest {
   float v;
@@ -86,16 +87,23 @@ sample_rows_kernel(const float* __restrict__ logits, const float* __restrict__ t
   const bool scale = T != 1.f;
   const float m = scale ? best.v / T : best.v;  // T > 0: the largest logit stays the largest
 
-  // Each thread owns one contiguous chunk, so that prefix sums follow the index order.  Read straight from memory, chunk after
-  // chunk beside each other, every load of a wave would touch 64 lines, more than the caches of the compute unit keep; the
+  // Each thread owns one contiguous chunk, so that prefix sums follow the index order.  Read straight from memory, long chunks
+  // beside each other, every load of a wave would touch 64 lines, more than the caches of the compute unit keep; the
   // chunks therefore pass through LDS, DRAW_PART entries of each at a time, 32 neighbours a load (rows of 151,936 logits,
-  // with filters in front: 202 -> 45 us).
+  // with filters in front: 205 us read straight, 94 so).  Short chunks are read as they lie (8 rows of 5,000: 16.6 us, through
+  // LDS 24; of 16,384: 22 and 38; of 24,000: 40 straight, 39 through LDS, filtered 40 and 29).
   extern __shared__ float part[];            // [SAMPLE_THREADS][DRAW_PART + 1]
   const int per = (V + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
   const int lo = min(V, tid * per), hi = min(V, lo + per);
-  // (what the processors in front have dropped adds nothing; a wave whose entries are all dropped skips the arithmetic)
+  // (what the processors in front have dropped adds nothing; on the way through LDS a wave whose entries are all dropped skips the
+  // arithmetic, which short chunks, whose loads are under way together, do not gain by)
   auto weight = [&](float v) { return expf((scale ? v / T : v) - m); };
-  auto each_of_chunk = [&](auto f) {
+  auto add_chunk = [&](float& sum, auto of) {
+    if (per <= DRAW_DIRECT) {
+#pragma unroll 8
+      for (int i = lo; i < hi; ++i) sum += of(x[i]);
+      return;
+    }
     for (int at = 0; at < per; at += DRAW_PART) {
       __syncthreads();                       // (the part before has been read)
 #pragma unroll
@@ -105,37 +113,43 @@ sample_rows_kernel(const float* __restrict__ logits, const float* __restrict__ t
       }
       __syncthreads();
       const int n = min(DRAW_PART, hi - lo - at);
-      for (int k = 0; k < n; ++k) f(part[tid * (DRAW_PART + 1) + k]);
+      for (int k = 0; k < n; ++k) {
+        const float v = part[tid * (DRAW_PART + 1) + k];
+        if (v != -INFINITY) sum += of(v);
+      }
     }
   };
   float s = 0.f;
-  each_of_chunk([&](float v) {
-    if (v != -INFINITY) s += weight(v);
-  });
+  add_chunk(s, [&](float v) { return weight(v); });
   const float total = block_sum(s, red);
   float ps = 0.f;
-  each_of_chunk([&](float v) {
-    if (v != -INFINITY) ps += weight(v) / total;
-  });
+  add_chunk(ps, [&](float v) { return weight(v) / total; });
   chunk_sum[tid] = ps;
   __syncthreads();
-  // prefix[t] = the sum of the chunks before t, added one after another in their order
-  if (tid == 0) {
-    float sum = 0.f;
+  // the sum of the chunks before this one, added one after another in their order: by every thread for itself, with long chunks
+  // by one for all
+  const int chunks = (V + per - 1) / per;
+  float prefix = 0.f;
+  if (per <= DRAW_DIRECT) {
+    for (int t = 0; t < min(tid, chunks); ++t) prefix += chunk_sum[t];
+  } else {
+    if (tid == 0) {
+      float sum = 0.f;
 #pragma unroll 16
-    for (int t = 0; t < SAMPLE_THREADS; ++t) {
-      const float c = chunk_sum[t];
-      chunk_sum[t] = sum;
-      sum += c;
+      for (int t = 0; t < chunks; ++t) {
+        const float c = chunk_sum[t];
+        chunk_sum[t] = sum;
+        sum += c;
+      }
     }
+    __syncthreads();
+    prefix = chunk_sum[tid];
   }
-  __syncthreads();
-  const float prefix = chunk_sum[tid];
   const float u = uniform[row];
   int hit = V;  // none
   // A chunk whose end lies clearly below u has no hit (its entries added to `prefix` one by one and its own sum differ by no
-  // more than the roundings of `per` additions below 2), and of the chunks that begin above u only the first entry counts.
-  if (lo < hi && u < prefix + ps + 2.4e-7f * (float)(per + 1)) {
+  // more than the roundings of `per` additions below 2); those that begin above u come into question only if none before them has one.
+  if (lo < hi && prefix <= u && u < prefix + ps + 2.4e-7f * (float)(per + 1)) {
     float c = prefix;
     for (int i0 = lo; i0 < hi && hit == V; i0 += 16) {
       float v[16];
@@ -150,25 +164,29 @@ sample_rows_kernel(const float* __restrict__ logits, const float* __restrict__ t
       }
     }
   }
-  // smallest hit of the block
+  // the smallest (largest) of the threads' numbers, in all of them
+  auto block_first = [&](int n, bool last) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) hit = min(hit, __shfl_xor(hit, off, SYN_WAVE));
-  if (tid % SYN_WAVE == 0) found[tid / SYN_WAVE] = hit;
-  __syncthreads();
-  int r = V;
-  for (int w = 0; w < SAMPLE_THREADS / SYN_WAVE; ++w) r = min(r, found[w]);
+    for (int off = 32; off > 0; off >>= 1) {
+      const int o = __shfl_xor(n, off, SYN_WAVE);
+      n = last ? max(n, o) : min(n, o);
+    }
+    __syncthreads();
+    if (tid % SYN_WAVE == 0) found[tid / SYN_WAVE] = n;
+    __syncthreads();
+    n = found[0];
+    for (int w = 1; w < SAMPLE_THREADS / SYN_WAVE; ++w) n = last ? max(n, found[w]) : min(n, found[w]);
+    return n;
+  };
+  int r = block_first(hit, false);
   if (r == V) {
-    // nothing passes u (the rounded sum ends below it, or is NaN): the last entry that is not dropped, of all of them the last
-    int last = -1;
-    for (int i = hi - 1; i >= lo && last < 0; --i)
-      if (x[i] != -INFINITY) last = i;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, SYN_WAVE));
-    __syncthreads();
-    if (tid % SYN_WAVE == 0) found[tid / SYN_WAVE] = last;
-    __syncthreads();
-    r = -1;
-    for (int w = 0; w < SAMPLE_THREADS / SYN_WAVE; ++w) r = max(r, found[w]);
+    // u lies between two chunks: the first entry behind it that is not dropped.  Or nothing passes u (the rounded sum ends below it, or
+    // is NaN): the last entry that is not dropped, of all of them the last.
+    int first = V, last = -1;
+    for (int i = lo; i < hi; ++i)
+      if (x[i] != -INFINITY) last = i, first = min(first, i);
+    r = block_first(prefix > u ? first : V, false);
+    if (r == V) r = block_first(last, true);
     if (r < 0) r = V - 1;
   }
   if (tid == 0) out[row] = r;
@@ -178,7 +196,7 @@ SYN_EXPORT int syn_sample_rows(const float* logits, const float* temperature, co
                                int n_rows, int V, hipStream_t stream) {
   SYN_CHECK(n_rows > 0 && V > 0, "sample_rows: empty input (%d rows, vocabulary %d)", n_rows, V);
   SYN_CHECK(temperature == nullptr || uniform != nullptr, "sample_rows: temperatures need uniform numbers");
-  const size_t lds = temperature ? (size_t)SAMPLE_THREADS * (DRAW_PART + 1) * sizeof(float) : 0;     // (a draw's)
+  const size_t lds = temperature && V > DRAW_DIRECT * SAMPLE_THREADS ? (size_t)SAMPLE_THREADS * (DRAW_PART + 1) * sizeof(float) : 0;     // (a draw's)
   static OncePerDevice raised;
   if (lds) {
     const hipError_t e = once_per_device(raised, [&] {

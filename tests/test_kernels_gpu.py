@@ -1304,7 +1304,7 @@ def test_sample_rows_temperature(ops):
     assert out.cpu().tolist() == [V - 1] * R
 
 
-@pytest.mark.parametrize("V,left", [(1, 1), (31, 5), (1023, 1023), (1025, 40), (33000, 33000), (151936, 50), (151937, 3)])
+@pytest.mark.parametrize("V,left", [(1, 1), (31, 5), (1023, 1023), (1025, 40), (16384, 16384), (16385, 16385), (33000, 33000), (151936, 50), (151937, 3)])
 def test_sample_rows_draws_where_the_sum_passes_u(ops, V, left):
     """Chunks of every length, with most entries dropped and with none, and u at both ends: the drawn entry is where the 64-bit
     running sum passes u, up to the roundings of V additions in 32 bits (2^-24 each), and never a dropped one."""
@@ -1324,7 +1324,7 @@ def test_sample_rows_draws_where_the_sum_passes_u(ops, V, left):
         assert p[r, i] > 0 and before <= float(u[r]) + off and float(u[r]) <= float(cum[r, i]) + off, (r, i)
 
 
-@pytest.mark.parametrize("V,left", [(2000, 700), (33000, 900), (151936, 50)])
+@pytest.mark.parametrize("V,left", [(2000, 700), (16384, 16000), (16385, 500), (33000, 900), (151936, 50)])
 def test_sample_rows_draws_no_dropped_entry(ops, V, left):
     """u within a few steps of 2^-24 of every place where the running sum may pass it, and beyond its end: the chunks' sums
     are rounded apart from each other, and what they leave between them belongs to no dropped entry."""
