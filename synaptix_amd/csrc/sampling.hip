@@ -7,6 +7,8 @@
 // The uniform number u comes from the host (a Philox stream per sequence).
 // The reference samples on the host from a downloaded vector; the arithmetic is the same,
 // only the order of the two sums differs (parallel instead of sequential).
+#include <type_traits>
+
 #include "common.h"
 
 #define SAMPLE_THREADS 1024
@@ -442,25 +444,31 @@ filter_rows_kernel(const float* __restrict__ in, float* __restrict__ out, int V,
   const bool scale = T > 0.f && T != 1.f;
   const int k = top_k[row];
   const bool cut = k > 0 && k < V;
-  for (int b = tid; b < 256; b += nt) sh.cnt[b] = 0;
-  if (tid == 0) sh.n_cand = 0;
-  __syncthreads();
-  float m = -INFINITY;
-  BinCache top;
-  if (scale || src != x) {
-    map_entries(src, x, V, [&](int, float v) {
-      if (scale) v = v / T;
-      m = fmaxf(m, v);
-      if (cut) top.add(sh, order_key(v) >> 24, 0, false);
-      return v;
-    });
-  } else {
-    for_each_entry(x, V, [&](int, float v) {
-      m = fmaxf(m, v);
-      if (cut) top.add(sh, order_key(v) >> 24, 0, false);
-    });
+  if (cut) {
+    for (int b = tid; b < 256; b += nt) sh.cnt[b] = 0;
+    if (tid == 0) sh.n_cand = 0;
+    __syncthreads();
   }
-  top.flush(sh, false);
+  float m = -INFINITY;
+  auto first_pass = [&](auto with_histogram) {      // (two loops: rows without top-k pay nothing for it)
+    BinCache top;
+    auto seen = [&](float v) {
+      m = fmaxf(m, v);
+      if constexpr (decltype(with_histogram)::value) top.add(sh, order_key(v) >> 24, 0, false);
+    };
+    if (scale || src != x) {
+      map_entries(src, x, V, [&](int, float v) {
+        if (scale) v = v / T;
+        seen(v);
+        return v;
+      });
+    } else {
+      for_each_entry(x, V, [&](int, float v) { seen(v); });
+    }
+    if constexpr (decltype(with_histogram)::value) top.flush(sh, false);
+  };
+  if (cut) first_pass(std::true_type{});
+  else first_pass(std::false_type{});
   m = block_max_all(m, sh.redf);   // (its barriers also stand between the writes above and the reads below)
 
   // ---- top-k: the key of the k-th largest, a byte at a time.  Once few enough entries can still be among the k (after two
