@@ -1428,7 +1428,7 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
   const Weight wt = {wb, w_packed != 0};
-  const bool few_row_tiles = M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units();
+  const bool few_row_tiles = M > 176 && M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units();
   // (from sweeps at the shapes of an 8B model, N = 4096 .. 151936, K = 4096 and 12288, where no other are named)
   int rc = 0;
   if (tile >= 0) {
@@ -1451,12 +1451,13 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     // as well (though that product then has only 192 workgroups); 64 x 64 tiles in a ring of four: 8.08.
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
   } else if (M > 64 && K % 128 == 0 && (M <= 128 ? slices > 1 : few_row_tiles)) {
-    // 65 rows and more of a narrow product whose reader adds partial sums, still bound by reading W: k-tiles of 64 in a ring
+    // 65 to 128 rows of a narrow product whose reader adds partial sums, still bound by reading W: k-tiles of 64 in a ring
     // of three, all of x beside 128 rows of W, and as many slices of K as fill the compute units (ops.gemm_slices).  128
     // rows: q/k/v of an 8B layer in 4 slices 17 us, down_proj in 8 slices 26; in a prompt step o_proj and down_proj together
-    // take 42 us with 128 rows, and 43 with 96 over the tiles for more rows.  129 to 256 rows where four slices and more go
-    // round (N = 4096): down_proj 38 us with 256 rows, 37 with 224 and 35 with 192 (the streamed tiles 42, 39 and 37); q/k/v
-    // with N = 6144 in two slices 26, 25.5 and 25 (the streamed tiles 25, 24 and 23, which it therefore takes).
+    // take 42 us with 128 rows, and 43 with 96 over the streamed tiles.  177 to 256 rows where the two rows of tiles
+    // go round once in four slices and more.  In four slices, against the streamed tile of the estimate: 4096 x 12288 160 rows
+    // 34.3 us, 32.0; 192 rows 34.2, 36.5; 256 rows 37.0, 42.9; 4096 x 4096 160 rows 15.3, 14.9; 192 rows 15.6, 16.3; 256 rows
+    // 17.0, 18.6; 2560 x 9728 160 rows 26.1, 21.6; 192 rows 27.1, 25.8; 256 rows 28.9, 31.3.
     rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
   } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N)) {
     // the same of up to 256 rows whose reader takes the finished product
