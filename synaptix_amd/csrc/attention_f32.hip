@@ -12,14 +12,18 @@
 
 #define ATTN32_MAX_HD 256
 
+// (16 bytes that start at any float: one load all the same)
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // The blocks of keys of a (token, head) fall into four classes in turns, each with a running softmax of its own, merged in the order
 // of the classes.  WAVES waves a workgroup.  SPLIT: a wave a class (few tokens: a wave alone would walk a sequence's keys one block
 // after another); else each wave has a head of its own and takes the classes one after another, the heads of one kv head
 // side by side, which then share its keys and values in the compute unit's cache.  The sums are the same either way: a
 // token's result does not depend on how many others are in the step.
-// VEC: head sizes that are a multiple of 4 take keys, queries and values 16 bytes at a time (a lane has a key's row, then a
-// dimension's row, to itself: each 128-byte line is asked for 8 times instead of 32).  490 tokens of 120, 137 and 233 with 32
-// heads of 128 over 8: 839 -> 265 us.
+// A lane has a key's row, then a dimension's row, to itself: 16 bytes at a time each 128-byte line is asked for 8 times instead of
+// 32.  The values' rows (64 floats) are always read so, keys and queries where the head size is a multiple of 4 (VEC).  490 tokens of
+// 120, 137 and 233 with 32 heads of 128 over 8: 839 -> 265 us.  Values one at a time behind a branch on their weight: three
+// times 400 tokens with 7 heads of 63 take 809 us, so 424.
 template <int WAVES, bool SPLIT, bool VEC>
 __global__ void __launch_bounds__(WAVES * SYN_WAVE)
 attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
@@ -88,23 +92,14 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
         if (d < hd) {
           const float* vr = v_pages + base + (size_t)d * SYN_PAGE;
           // (slots past the sequence's end may hold anything: a weight of zero takes nothing from them)
-          if constexpr (VEC) {
-            f32x4 a4 = {o[i] * alpha, 0.f, 0.f, 0.f};
+          f32x4 a4 = {o[i] * alpha, 0.f, 0.f, 0.f};
 #pragma unroll 8
-            for (int j = 0; j < SYN_PAGE; j += 4) {
-              const f32x4 vv = *(const f32x4*)(vr + j), pp = *(const f32x4*)(ps + j);
+          for (int j = 0; j < SYN_PAGE; j += 4) {
+            const f32x4 vv = *(const f32x4_any*)(vr + j), pp = *(const f32x4*)(ps + j);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) a4[e] = fmaf(pp[e], pp[e] != 0.f ? vv[e] : 0.f, a4[e]);
-            }
-            o[i] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
-          } else {
-            float acc = o[i] * alpha;
-            for (int j = 0; j < SYN_PAGE; ++j) {
-              const float pj = ps[j];
-              if (pj != 0.f) acc = fmaf(pj, vr[j], acc);
-            }
-            o[i] = acc;
+            for (int e = 0; e < 4; ++e) a4[e] = fmaf(pp[e], pp[e] != 0.f ? vv[e] : 0.f, a4[e]);
           }
+          o[i] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
         }
       }
       __builtin_amdgcn_wave_barrier();

@@ -258,7 +258,8 @@ def test_attention_f32_does_not_depend_on_the_batch(ops, nh, nkv, hd, window):
         assert torch.equal(run(rows), whole[d(rows)])
 
 
-@pytest.mark.parametrize("hd,past,new", [(6, [300, 0], [1, 2]), (6, [0, 70], [200, 150]), (32, [1000], [1]), (128, [70], [3])])
+@pytest.mark.parametrize("hd,past,new", [(6, [300, 0], [1, 2]), (6, [0, 70], [200, 150]), (32, [1000], [1]), (128, [70], [3]),
+                                         (71, [70, 0], [200, 130]), (255, [130], [2])])
 def test_attention_f32_splits_and_head_sizes(ops, hd, past, new):
     """Few tokens (the keys over four waves, more waves than blocks of keys among them) and many, head sizes that 16-byte loads
     do not divide, NaN in every slot behind a sequence's end."""
