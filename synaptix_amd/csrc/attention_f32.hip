@@ -79,9 +79,10 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
         s = dot * scale;
         if (with_terms) s = score_with_terms(s, slope, terms.softcap, pos, key);
       }
-      const float m_new = fmaxf(m, wave_max(s));  // every block of the range holds a visible key
-      const float alpha = expf(m - m_new);
-      const float p = valid ? expf(s - m_new) : 0.f;
+      // (a score of -inf weighs nothing, also among none but such; one that is no number stays one in p and l)
+      const float m_new = fmaxf(m, wave_max(s));
+      const float alpha = m == m_new ? 1.f : expf(m - m_new);
+      const float p = s == -INFINITY ? 0.f : expf(s - m_new);
       l = fmaf(l, alpha, wave_sum(p));
       m = m_new;
       ps[lane] = p;
@@ -111,7 +112,8 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
       if (d < hd) part[c][d] = o[i];
     }
   }
-  // the common maximum first, then sums in the order of the classes (one without a block has m = -inf, l = 0)
+  // the common maximum first, then sums in the order of the classes (one without a weight has m = -inf and l = 0, or an l that is
+  // no number where a score was none)
   if constexpr (SPLIT) {
     __syncthreads();
     if (wave != 0) return;
@@ -123,7 +125,7 @@ attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, 
   for (int c = 1; c < CLASSES; ++c) top = fmaxf(top, stat[c][0]);
 #pragma unroll
   for (int c = 0; c < CLASSES; ++c) {
-    f[c] = stat[c][0] == -INFINITY ? 0.f : expf(stat[c][0] - top);
+    f[c] = stat[c][0] == -INFINITY ? stat[c][1] : expf(stat[c][0] - top);
     l = fmaf(f[c], stat[c][1], l);
   }
 #pragma unroll

@@ -278,6 +278,37 @@ def test_attention_f32_splits_and_head_sizes(ops, hd, past, new):
     close(out, want, 1e-5, 1e-5, "attention f32")
 
 
+@pytest.mark.parametrize("new", [1, 600])
+def test_attention_f32_keeps_what_is_no_number(ops, new):
+    """A key that is no number makes every result that sees it one, also where no other key stands in its block of 64; scores of
+    -inf, a block full of them among others, weigh nothing.  With few tokens (the keys over four waves) and many."""
+    nh, nkv, hd, T = 4, 2, 16, 700
+    pages = (T + 63) // 64
+    k, v, q = rnd((pages, nkv, 64, hd), 36), rnd((pages, nkv, hd, 64), 37), rnd((new, nh * hd), 38)
+    table = torch.arange(pages, dtype=I32).view(1, pages)
+    tok_seq, tok_pos = torch.zeros(new, dtype=I32), torch.arange(T - new, T, dtype=I32)
+    d = lambda t: t.to(DEV)
+
+    def run(k, pos=tok_pos):
+        out = torch.empty((new, nh * hd), device=DEV)
+        ops.attention_f32(d(q), d(k), d(v), d(table), d(tok_seq), d(pos), out, 0.3, 0, nh, nkv, hd)
+        return out.cpu()
+    bad = k.clone()
+    bad[5, :, 0, 3] = float("nan")                       # position 320, the first of its block
+    seen = torch.full((new,), 320, dtype=I32)            # ... and the last that is seen
+    assert torch.isnan(run(bad, seen)).all() and torch.isfinite(run(bad, seen - 1)).all()
+    assert torch.equal(torch.isnan(run(bad)).all(1), tok_pos >= 320) and torch.equal(torch.isnan(run(bad)).any(1), tok_pos >= 320)
+    q = q.view(new, nh, hd)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.1
+    q = q.view(new, nh * hd)
+    low = k.clone()
+    low[2, :, :, 0] = float("-inf")                      # every score of positions 128 to 191
+    got, pos = run(low), tok_pos.clamp(max=127)
+    assert torch.isfinite(got).all()
+    low[3:, :, :, 0] = float("-inf")
+    close(run(low).to(DEV), run(k, pos), 1e-5, 1e-5, "blocks that weigh nothing")
+
+
 @pytest.mark.parametrize("out_dtype", [BF16, F32])
 @pytest.mark.parametrize("M,N,K", [
     (1, 48, 64), (3, 1000, 176), (16, 100, 320), (17, 40, 72), (33, 1000, 128), (48, 70, 2048), (64, 4096, 512),
