@@ -1095,7 +1095,7 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     }
   };
   // Before the barrier that ends a step a wave waits until its reads have returned and all but its youngest loads, those of
-  // the last two steps, have landed: behind it the k-tile after the next is whole, and the buffer of this step's tile free.
+  // the last STAGES - 2 steps, have landed: behind it the k-tile after the next is whole, and the buffer of this step's tile free.
   // (A tile's stores are younger than the loads that the step behind them waits for, and count like loads.)
   constexpr int YOUNGER = (STAGES - 2) * PASSES;
   auto landed = [&] {
@@ -1349,12 +1349,25 @@ static bool direct_one_round(int M, int N) {
   return M <= 256 && (M - 1) % 64 >= 16 && tile_grid(M, N, 64, 128) <= syn_compute_units();
 }
 
+// Whether a product of 177 to 256 rows whose reader adds partial sums takes the tiles of 128 x 128 that hold k-tiles of 64
+// (gemm_direct) in two slices: where they go round once and leave few compute units without work, since what they take hardly
+// depends on N.  Against the streamed tiles in the slices of the estimate, what the reader pays for further slices included, weights
+// that no cache holds: 6144 x 2560 177 rows 18.1 us against 19.7, 256 rows 18.6, 21.9; 6144 x 4096 177 rows 24.0, 23.5, 256 rows 24.4,
+// 26.9; 7168 x 8192 200 rows 43.1, 46.1; 8192 x 5120 256 rows 32.6, 36.3.  Not with three quarters of the compute units and longer
+// sums (6144 x 6144 192 rows 34.3, 32.2), nor with fewer (5120 x 4096 192 rows 23.7, 21.1), nor in short ones (8192 x 2048 192 rows
+// 17.1, 16.8; 200 rows 17.2, 15.8).
+static bool direct_two_slices(int M, int N, int K) {
+  const long tiles = 4L * ((N + 127) / 128), cus = syn_compute_units();
+  return M > 176 && M <= 256 && K % 128 == 0 && K >= 2560 && tiles <= cus && 4 * tiles >= 3 * cus && (K <= 4096 || 20 * tiles >= 17 * cus);
+}
+
 // Into how many slices of K a product of more than 64 rows is cut when its reader adds partial sums: the smallest estimate of
 // the product's time and of what its reader pays for the slices beyond the first (M x N floats each, half of them from caches).
 SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
   int best = 1;
   double least = 1e30;
   if (M <= 0 || N <= 0 || K <= 0) return 1;
+  if (direct_two_slices(M, N, K)) return 2;
   for (int s : {1, 2, 3, 4, 6, 8}) {
     const StreamPlan p = plan_stream(M, N, K, s, true, 4, false);
     if (p.tile < 0) break;
@@ -1428,7 +1441,8 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
   const Weight wt = {wb, w_packed != 0};
-  const bool few_row_tiles = M > 176 && M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units();
+  const bool few_row_tiles = (M > 176 && M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units()) ||
+                             (slices == 2 && direct_two_slices(M, N, K));
   // (from sweeps at the shapes of an 8B model, N = 4096 .. 151936, K = 4096 and 12288, where no other are named)
   int rc = 0;
   if (tile >= 0) {
@@ -1455,7 +1469,7 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     // of three, all of x beside 128 rows of W, and as many slices of K as fill the compute units (ops.gemm_slices).  128
     // rows: q/k/v of an 8B layer in 4 slices 17 us, down_proj in 8 slices 26; in a prompt step o_proj and down_proj together
     // take 42 us with 128 rows, and 43 with 96 over the streamed tiles.  177 to 256 rows where the two rows of tiles
-    // go round once in four slices and more.  In four slices, against the streamed tile of the estimate: 4096 x 12288 160 rows
+    // go round once in four slices and more, or in two (direct_two_slices).  In four slices, against the streamed tile of the estimate: 4096 x 12288 160 rows
     // 34.3 us, 32.0; 192 rows 34.2, 36.5; 256 rows 37.0, 42.9; 4096 x 4096 160 rows 15.3, 14.9; 192 rows 15.6, 16.3; 256 rows
     // 17.0, 18.6; 2560 x 9728 160 rows 26.1, 21.6; 192 rows 27.1, 25.8; 256 rows 28.9, 31.3.
     rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);

@@ -508,8 +508,8 @@ def gemm_slices(M, N, K, dtype):
         if K % 128:
             return 1
         if M <= 128 or 176 < M <= 256:
-            # still bound by reading W: tiles of 128 x 128, cut until they fill the compute units (from 177 rows on only
-            # where that takes four slices: csrc/gemm.hip)
+            # still bound by reading W: tiles of 128 x 128, cut until they fill the compute units (from 177 rows on here
+            # only where that takes four slices; where it takes two, csrc/gemm.hip knows)
             most, slices = min(8, units // (-(-M // 128) * -(-N // 128)), K // 512), 1
             while slices * 2 <= most:
                 slices *= 2

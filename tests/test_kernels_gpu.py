@@ -338,7 +338,9 @@ def test_gemm_bf16(ops, out_dtype, M, N, K):
                                      (200, 4096, 1024, 2), (256, 1000, 2048, 4),
                                      # short prompts cut along K: tiles of 128 x 128 up to 128 rows (to 256 in four slices and more), streamed ones beyond
                                      (66, 6144, 4096, 4), (128, 200, 4096, 8), (129, 4100, 1024, 2), (256, 1000, 2560, 4),
-                                     (257, 520, 4096, 8), (400, 2000, 1152, 2), (512, 4096, 1024, 2)])
+                                     (257, 520, 4096, 8), (400, 2000, 1152, 2), (512, 4096, 1024, 2),
+                                     # ... to 256 in two slices where they leave few compute units without work, and beside that line
+                                     (177, 6144, 2560, 2), (256, 8192, 2688, 2), (250, 7100, 4224, 2), (176, 6144, 2560, 2), (200, 6000, 2560, 2)])
 def test_gemm_bf16_partial_sums_over_slices_of_k(ops, M, N, K, S):
     """[S, M, N]: slice s holds the sum over its part of K; the slices add up to the product, also
     when K is no multiple of the slice and the last slices are short or empty."""
