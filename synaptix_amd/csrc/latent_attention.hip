@@ -238,7 +238,9 @@ latent_attention_bf16_kernel(const bf16* __restrict__ q, const bf16* __restrict_
 // A page is 72 + 128 matrix instructions a wave with rows of 512 + 64 values, a quarter of what it takes: the phases follow
 // each other with one wave a SIMD (scores, weights, their exchange, second product), and 140 KB a page come from L2.  Against a
 // wave a tile of 16 rows with the page staged through LDS between two barriers, every load waited for: 1,500 tokens, 32 heads,
-// 627 -> 218 us; eight sequences, 3,270 tokens in all: 584 -> 240 us.
+// 627 -> 218 us; eight sequences, 3,270 tokens in all: 584 -> 240 us.  Other rows, the same 1,500 tokens: 128 + 16 values 138 -> 52 us,
+// 128 + 64 163 -> 119, 256 + 32 240 -> 122, 256 + 64 258 -> 127, 512 + 16 713 -> 221, 512 + 128 671 -> 237; 128 tokens behind 4,096 with
+// 128 + 16 260 -> 121, 512 + 128 1,130 -> 323.
 // The matrix instructions stand as inline assembly to keep the accumulators in vector registers and the fragments in the
 // accumulation registers (left to itself the compiler moves 128 of them back and forth on every page, or spills); it does not
 // know them for what they are, so their results are waited for by hand.
