@@ -34,11 +34,13 @@ __device__ __forceinline__ ArgBest block_argmax(ArgBest best, ArgBest* red) {
     o.i = __shfl_xor(best.i, off, SYN_WAVE);
     best = arg_better(best, o);
   }
-  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE, nw = blockDim.x / SYN_WAVE;
+  constexpr int nw = SAMPLE_THREADS / SYN_WAVE;     // (known, so that the reads below are under way together)
+  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
   __syncthreads();
   if (lane == 0) red[wave] = best;
   __syncthreads();
   ArgBest r = red[0];
+#pragma unroll
   for (int w = 1; w < nw; ++w) r = arg_better(r, red[w]);
   return r;
 }
@@ -255,23 +257,25 @@ struct FilterShared {
 __device__ __forceinline__ float block_max_all(float v, float* red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, SYN_WAVE));
-  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE, nw = blockDim.x / SYN_WAVE;
+  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
   float t = red[0];
-  for (int i = 1; i < nw; ++i) t = fmaxf(t, red[i]);
+#pragma unroll
+  for (int i = 1; i < FILTER_THREADS / SYN_WAVE; ++i) t = fmaxf(t, red[i]);
   return t;
 }
 __device__ __forceinline__ u64 block_sum_all(u64 v, u64* red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, SYN_WAVE);
-  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE, nw = blockDim.x / SYN_WAVE;
+  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
   u64 t = 0;
-  for (int i = 0; i < nw; ++i) t += red[i];
+#pragma unroll
+  for (int i = 0; i < FILTER_THREADS / SYN_WAVE; ++i) t += red[i];
   return t;
 }
 
@@ -632,5 +636,386 @@ SYN_EXPORT int syn_filter_rows(const float* in, float* out, int n_rows, int V, c
   filter_rows_kernel<<<n_rows, FILTER_THREADS, 0, stream>>>(in, out, V, temperature, top_k, top_p, min_p, repetition,
                                                             presence, frequency, ids, id_start, counts);
   SYN_LAUNCH_CHECK("filter_rows");
+  return 0;
+}
+
+// ------------------------------------------------------------------ filters and draw of rows with a top-k, many workgroups a row
+// With a top-k the processors keep few entries, and a token can be drawn from those alone: no row is written, and the row is
+// read once, by as many workgroups as it has slices.  What bounds it: the start of two kernels and the walk of a slice of some
+// thousand entries through LDS, then of the slices' candidates by one workgroup.
+//   1  topk_slices: a workgroup takes a slice of the row into LDS, applies the penalties (their tokens counted in LDS) and the
+//      temperature, finds the slice's own k largest and stores them in index order;
+//   2  topk_draw: a workgroup a row finds the k largest of these, which are the row's (of equal values the first in index order:
+//      the slices and what they store lie in that order), then top-p, min-p and the draw on the at most TOPK_MAX that are left.
+// Every step takes the same roundings in the same order as the kernels above (the sums of top-p are whole numbers, those of the
+// draw go chunk by chunk as there), so a row's token is the one that they give.  8 rows of 151,936 logits with penalties,
+// top-k 50 and top-p: 104 + 95 us as two kernels of a workgroup a row, 18 + 19 so; a call with its upload and the token's way back
+// 305 -> 150 us.
+#define TOPK_MAX 512         // of a row's k; with TOPK_SLICES slices their candidates fill 128 KB of LDS
+#define TOPK_SLICES 32
+#define TOPK_SLICE_MAX 8192  // entries of a slice: 32 KB of values and as much for the counters
+#define SLICE_THREADS 512
+
+template <int NT>
+struct SelectShared {
+  unsigned hist[2048];
+  unsigned wave_n[2][NT / SYN_WAVE];
+  unsigned bin, need, ties;
+};
+
+// Of the n keys that `key` returns those above `prefix` and the first `need` that equal it are the k largest (1 <= k <= n): 11, 11
+// and 10 bits of the keys at a time from the top, with a histogram each.
+template <int NT, typename F>
+__device__ __forceinline__ void kth_key(F key, int n, unsigned k, SelectShared<NT>& sh, unsigned& prefix, unsigned& need) {
+  constexpr int BINS = 2048 / NT;
+  const int tid = threadIdx.x, wave = tid / SYN_WAVE, lane = tid % SYN_WAVE;
+  unsigned ties;
+  prefix = 0, need = k;
+  for (int pass = 0; pass < 3; ++pass) {
+    const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0;
+    const unsigned low = pass == 2 ? 1023u : 2047u, himask = pass == 0 ? 0u : pass == 1 ? 0xffe00000u : 0xfffffc00u;
+    for (int b = tid; b < 2048; b += NT) sh.hist[b] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += NT) {
+      const unsigned q = key(i);
+      if ((q & himask) == prefix) atomicAdd(&sh.hist[(q >> shift) & low], 1u);
+    }
+    __syncthreads();
+    unsigned mine[BINS], own = 0;
+#pragma unroll
+    for (int i = 0; i < BINS; ++i) mine[i] = sh.hist[BINS * tid + i], own += mine[i];
+    unsigned from_here = own;       // becomes the sum over this lane's bins and those of all higher lanes
+#pragma unroll
+    for (int off = 1; off < SYN_WAVE; off <<= 1) {
+      const unsigned o = __shfl_down(from_here, off, SYN_WAVE);
+      if (lane + off < SYN_WAVE) from_here += o;
+    }
+    if (lane == 0) sh.wave_n[0][wave] = from_here;
+    __syncthreads();
+    unsigned above = from_here - own;
+#pragma unroll
+    for (int w = 0; w < NT / SYN_WAVE; ++w) above += w > wave ? sh.wave_n[0][w] : 0u;
+#pragma unroll
+    for (int i = BINS - 1; i >= 0; --i) {
+      if (above < need && need <= above + mine[i]) sh.bin = BINS * tid + i, sh.need = need - above, sh.ties = mine[i];
+      above += mine[i];
+    }
+    __syncthreads();
+    prefix |= sh.bin << shift, need = sh.need, ties = sh.ties;
+    __syncthreads();
+    if (need == ties && prefix > 0) {      // everything from here up belongs to them: no need to look at the bits below
+      --prefix, need = 0;
+      return;
+    }
+  }
+}
+
+// put(i, place) for the entries i < n above `prefix` and the first `need` that equal it, in index order; returns how many.  Each wave
+// takes a run of neighbours, counts what is in it, and places them behind those of the waves before it.
+template <int NT, typename F, typename G>
+__device__ __forceinline__ int keep_largest(F key, int n, unsigned prefix, unsigned need, SelectShared<NT>& sh, G put) {
+  constexpr int NW = NT / SYN_WAVE;
+  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
+  const int run = (n + NT - 1) / NT * SYN_WAVE, lo = wave * run, hi = min(n, lo + run);
+  const u64 below = (1ull << lane) - 1ull;
+  unsigned more_n = 0, ties_n = 0;
+  for (int i0 = lo; i0 < hi; i0 += SYN_WAVE) {
+    const int i = i0 + lane;
+    const unsigned q = i < hi ? key(i) : 0u;
+    more_n += __popcll(__ballot(i < hi && q > prefix));
+    ties_n += __popcll(__ballot(i < hi && q == prefix));
+  }
+  if (lane == 0) sh.wave_n[0][wave] = ties_n, sh.wave_n[1][wave] = more_n;
+  __syncthreads();
+  unsigned ties = 0, more = 0, ties_all = 0, more_all = 0;      // in front of this wave's run; everywhere
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const unsigned t = sh.wave_n[0][w], m = sh.wave_n[1][w];
+    if (w < wave) ties += t, more += m;
+    ties_all += t, more_all += m;
+  }
+  if (more_n + ties_n > 0) {
+    for (int i0 = lo; i0 < hi; i0 += SYN_WAVE) {
+      const int i = i0 + lane;
+      const unsigned q = i < hi ? key(i) : 0u;
+      const bool is_more = i < hi && q > prefix, is_tie = i < hi && q == prefix;
+      const u64 v_more = __ballot(is_more), v_tie = __ballot(is_tie);
+      const unsigned ties_at = ties + __popcll(v_tie & below);
+      // (in front of an entry stay the larger ones, and of its equals no more than `need`)
+      if (is_more || (is_tie && ties_at < need)) put(i, (int)(more + __popcll(v_more & below) + min(ties_at, need)));
+      more += __popcll(v_more), ties += __popcll(v_tie);
+    }
+  }
+  return (int)(more_all + min(ties_all, need));
+}
+
+__global__ void __launch_bounds__(SLICE_THREADS)
+topk_slices_kernel(const float* __restrict__ in, int V, int slice, const float* __restrict__ temperature,
+                   const int* __restrict__ top_k, const float* __restrict__ repetition, const float* __restrict__ presence,
+                   const float* __restrict__ frequency, const int* __restrict__ ids, const int* __restrict__ id_start,
+                   float* __restrict__ cand_v, int* __restrict__ cand_i, int* __restrict__ cand_n) {
+  __shared__ SelectShared<SLICE_THREADS> sh;
+  extern __shared__ __align__(16) float val[];   // [slice], and behind them the counters [slice]
+  int* cnt = (int*)(val + slice);
+  const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
+  const int lo = part * slice, n = min(slice, V - lo);
+  const float* x = in + (size_t)row * V + lo;
+  if (V % 4 == 0 && (uintptr_t)in % 16 == 0) {   // (a slice is a multiple of four entries)
+    const float4* x4 = (const float4*)x;
+    float4* d4 = (float4*)val;
+    const int n4 = n / 4;
+    for (int i0 = tid; i0 < n4; i0 += 4 * SLICE_THREADS) {
+      float4 v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (i0 + q * SLICE_THREADS < n4) v[q] = x4[i0 + q * SLICE_THREADS];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (i0 + q * SLICE_THREADS < n4) d4[i0 + q * SLICE_THREADS] = v[q];
+    }
+  } else {
+    for (int j = tid; j < n; j += SLICE_THREADS) val[j] = x[j];
+  }
+  const int first = id_start ? id_start[row] : 0, n_ids = id_start ? id_start[row + 1] - first : 0;
+  const float rep = repetition[row], pres = presence[row], freq = frequency[row];
+  const bool penalties = n_ids > 0 && (rep != 1.f || pres != 0.f || freq != 0.f);
+  if (penalties) {
+    for (int j = tid; j < n; j += SLICE_THREADS) cnt[j] = 0;
+    __syncthreads();
+    for (int i = tid; i < n_ids; i += SLICE_THREADS) {
+      const int t = ids[first + i];
+      if (t >= lo && t < lo + n) atomicAdd(&cnt[t - lo], 1);
+    }
+  }
+  __syncthreads();
+  const float T = temperature[row];
+  const bool scale = T > 0.f && T != 1.f;
+  if (penalties || scale) {
+    for (int j = tid; j < n; j += SLICE_THREADS) {
+      float v = val[j];
+      const int c = penalties ? cnt[j] : 0;
+      if (c > 0) {
+        if (rep != 1.f) {
+          const float f = powf(rep, (float)c);
+          v = v > 0.f ? v / f : v * f;
+        }
+        if (pres != 0.f || freq != 0.f) v -= pres + freq * (float)c;
+      }
+      val[j] = scale ? v / T : v;
+    }
+    __syncthreads();
+  }
+  const int k = max(1, min(top_k[row], TOPK_MAX));
+  auto key = [&](int i) { return order_key(val[i]); };
+  unsigned prefix = 0, need = 0;
+  if (k < n) kth_key<SLICE_THREADS>(key, n, (unsigned)k, sh, prefix, need);      // (else prefix 0: all of them stay)
+  const size_t at = ((size_t)row * gridDim.x + part) * TOPK_MAX;
+  const int kept = keep_largest<SLICE_THREADS>(key, n, prefix, k < n ? need : (unsigned)n, sh, [&](int i, int place) {
+    cand_v[at + place] = val[i];
+    cand_i[at + place] = lo + i;
+  });
+  if (tid == 0) cand_n[row * gridDim.x + part] = kept;
+}
+
+__global__ void __launch_bounds__(SAMPLE_THREADS)
+topk_draw_kernel(const float* __restrict__ cand_v, const int* __restrict__ cand_i, const int* __restrict__ cand_n, int parts,
+                 int V, const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ min_p,
+                 const float* __restrict__ draw, const float* __restrict__ uniform, int* __restrict__ out) {
+  __shared__ SelectShared<SAMPLE_THREADS> sh;
+  __shared__ float kept_v[TOPK_MAX], chunk_at[TOPK_MAX];
+  __shared__ int kept_i[TOPK_MAX];
+  __shared__ u64 mass[TOPK_MAX];
+  __shared__ unsigned keys[TOPK_MAX];
+  __shared__ u64 red64[SAMPLE_THREADS / SYN_WAVE];
+  __shared__ float redf[SAMPLE_THREADS / SYN_WAVE];
+  __shared__ ArgBest red_arg[SAMPLE_THREADS / SYN_WAVE];
+  __shared__ float chunk_sum[SAMPLE_THREADS];
+  __shared__ int starts[TOPK_SLICES + 1];
+  __shared__ int found[2];
+  extern __shared__ float all_v[];               // [parts * TOPK_MAX] values, and behind them their places in the row
+  int* all_i = (int*)(all_v + parts * TOPK_MAX);
+  const int row = blockIdx.x, tid = threadIdx.x;
+
+  if (tid < SYN_WAVE) {
+    int n = tid < parts ? cand_n[row * parts + tid] : 0;
+    const int own = n;
+#pragma unroll
+    for (int off = 1; off < TOPK_SLICES; off <<= 1) {
+      const int o = __shfl_up(n, off, SYN_WAVE);
+      if (tid >= off) n += o;
+    }
+    if (tid < parts) starts[tid] = n - own;
+    if (tid == parts - 1) starts[parts] = n;
+  }
+  __syncthreads();
+  const int n_all = starts[parts];
+  for (int p = tid / SYN_WAVE; p < parts; p += SAMPLE_THREADS / SYN_WAVE) {
+    const size_t at = ((size_t)row * parts + p) * TOPK_MAX;
+    for (int i = tid % SYN_WAVE; i < starts[p + 1] - starts[p]; i += SYN_WAVE)
+      all_v[starts[p] + i] = cand_v[at + i], all_i[starts[p] + i] = cand_i[at + i];
+  }
+  __syncthreads();
+
+  // ---- top-k
+  // (k < V and a slice has left out entries only if it kept k, so there are k of them)
+  const unsigned k = (unsigned)max(1, min(min(top_k[row], TOPK_MAX), n_all));
+  unsigned prefix, need;
+  auto key = [&](int i) { return order_key(all_v[i]); };
+  kth_key<SAMPLE_THREADS>(key, n_all, k, sh, prefix, need);
+  const int n = keep_largest<SAMPLE_THREADS>(key, n_all, prefix, need, sh, [&](int i, int place) {
+    kept_v[place] = all_v[i], kept_i[place] = all_i[i];
+  });
+  __syncthreads();
+
+  // ---- top-p and min-p, an entry a thread: an entry stays while the mass of those before it (larger, or equal and earlier) is
+  // at most p * all mass, which is what the radix search above finds the boundary of
+  const float p = top_p[row], mp = min_p[row];
+  float mine = tid < n ? kept_v[tid] : -INFINITY;
+  const float m = block_max_all(mine, redf);
+  if (p < 1.f) {
+    const bool counts = tid < n && is_finite(mine);
+    const u64 own = counts ? mass_of(mine, m) : 0;
+    const unsigned mk = order_key(mine);
+    if (tid < n) mass[tid] = own, keys[tid] = mk;
+    const u64 total = block_sum_all(own, red64);
+    const u64 limit = (u64)((double)p * (double)total);
+    if (counts) {
+      u64 before = 0;
+#pragma unroll 8
+      for (int j = 0; j < n; ++j) {
+        const unsigned q = keys[j];
+        const u64 w = mass[j];
+        before += (q > mk) | ((q == mk) & (j < tid)) ? w : 0;
+      }
+      if (before > limit) mine = -INFINITY;
+    }
+  }
+  if (mp > 0.f && is_finite(mine) && expf(mine - m) < mp) mine = -INFINITY;
+  __syncthreads();
+  if (tid < n) kept_v[tid] = mine;
+  if (tid < 2) found[tid] = tid == 0 ? V : -1;
+  chunk_sum[tid] = 0.f;
+  // (a NaN is larger than nothing; the barriers inside end the writes above)
+  const ArgBest best = block_argmax(arg_better(ArgBest{-INFINITY, -1}, ArgBest{mine, tid < n ? kept_i[tid] : -1}), red_arg);
+
+  if (!(draw[row] > 0.f)) {
+    if (tid == 0) {
+      int r = best.i;
+      if (!(best.v > -INFINITY)) {     // nothing is larger than -inf: the last entry that is -inf, among all entries of the row
+        r = V - 1;
+        for (int j = n - 1; j >= 0 && kept_i[j] == r && kept_v[j] != -INFINITY; --j) --r;
+        if (r < 0) r = V - 1;
+      }
+      out[row] = r;
+    }
+    return;
+  }
+
+  // ---- the draw, as sample_rows takes it at temperature 1: chunks of the row, each by the thread of its first entry
+  const float top = best.v;
+  const int per = (V + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
+  const int chunk = tid < n ? kept_i[tid] / per : -1;
+  const bool opens = tid < n && (tid == 0 || kept_i[tid - 1] / per != chunk);
+  int end = tid;
+  if (opens) {
+    float s = 0.f;
+    for (; end < n && kept_i[end] / per == chunk; ++end)
+      if (kept_v[end] != -INFINITY) s += expf(kept_v[end] - top);
+    chunk_sum[chunk] = s;
+  }
+  __syncthreads();
+  const float total = block_sum(chunk_sum[tid], redf);
+  float ps = 0.f;
+  if (opens)
+    for (int j = tid; j < end; ++j)
+      if (kept_v[j] != -INFINITY) ps += expf(kept_v[j] - top) / total;
+  if (tid < n) chunk_at[tid] = opens ? ps : 0.f;
+  __syncthreads();
+  if (tid == 0) {
+    float sum = 0.f;      // (chunks without entries add nothing)
+    for (int j0 = 0; j0 < n; j0 += 16) {
+      float c[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) c[q] = j0 + q < n ? chunk_at[j0 + q] : 0.f;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        if (j0 + q < n) chunk_at[j0 + q] = sum;
+        sum += c[q];
+      }
+    }
+  }
+  __syncthreads();
+  const float u = uniform[row];
+  const float before = opens ? chunk_at[tid] : 0.f;
+  if (opens && before <= u && u < before + ps + 2.4e-7f * (float)(per + 1)) {
+    float c = before;
+    for (int j = tid; j < end; ++j)
+      if (kept_v[j] != -INFINITY) {
+        c += expf(kept_v[j] - top) / total;
+        if (u < c) {
+          atomicMin(&found[0], kept_i[j]);
+          break;
+        }
+      }
+  }
+  __syncthreads();
+  int r = found[0];
+  if (r == V) {
+    // as in sample_rows: the first entry that is left in a chunk behind u, else the last one that is left
+    __syncthreads();
+    if (opens)
+      for (int j = tid; j < end; ++j)
+        if (kept_v[j] != -INFINITY) {
+          if (before > u) atomicMin(&found[0], kept_i[j]);
+          atomicMax(&found[1], kept_i[j]);
+        }
+    __syncthreads();
+    r = found[0] < V ? found[0] : found[1] >= 0 ? found[1] : V - 1;
+  }
+  if (tid == 0) out[row] = r;
+}
+
+// Slices of a row: as many as the chip has room for at few rows, of at least 1,024 entries.
+static int topk_slice(int V) {
+  const int parts = V / 1024 < 1 ? 1 : V / 1024 > TOPK_SLICES ? TOPK_SLICES : V / 1024;
+  return ((V + parts - 1) / parts + 3) / 4 * 4;
+}
+// Four-byte words of scratch memory that syn_draw_top_k needs for n_rows rows of V logits; 0: it does not take rows of this size.
+SYN_EXPORT long syn_draw_top_k_words(int n_rows, int V) {
+  const int slice = V > 0 ? topk_slice(V) : 0;
+  if (n_rows <= 0 || n_rows > 65535 || V <= 0 || slice > TOPK_SLICE_MAX) return 0;
+  return (long)n_rows * ((V + slice - 1) / slice) * (2 * TOPK_MAX + 1);
+}
+
+// filter_rows and sample_rows in one for rows that all have a top-k (1 <= top_k <= TOPK_MAX, top_k < V; the rows' largest is max_k):
+// the token of every row to out.  draw: greedy where <= 0, else the row is drawn from with `uniform`.  words: syn_draw_top_k_words of
+// scratch memory with any content.
+SYN_EXPORT int syn_draw_top_k(const float* logits, int n_rows, int V, int max_k, const float* temperature, const int* top_k,
+                              const float* top_p, const float* min_p, const float* repetition, const float* presence,
+                              const float* frequency, const int* ids, const int* id_start, const float* draw,
+                              const float* uniform, float* words, int* out, hipStream_t stream) {
+  SYN_CHECK(syn_draw_top_k_words(n_rows, V) > 0, "draw_top_k: %d rows of %d logits", n_rows, V);
+  SYN_CHECK(logits && temperature && top_k && top_p && min_p && repetition && presence && frequency && draw && uniform && words && out,
+            "draw_top_k: an array is missing");
+  SYN_CHECK((ids == nullptr) == (id_start == nullptr), "draw_top_k: the penalties' tokens come with their row offsets");
+  SYN_CHECK(max_k >= 1 && max_k <= TOPK_MAX && max_k < V, "draw_top_k: top-k up to %d of %d logits (at most %d)", max_k, V, TOPK_MAX);
+  const int slice = topk_slice(V), parts = (V + slice - 1) / slice;
+  const size_t lds_slice = (size_t)slice * 8, lds_draw = (size_t)parts * TOPK_MAX * 8;
+  static OncePerDevice raised;
+  const hipError_t e = once_per_device(raised, [&] {
+    const hipError_t a = hipFuncSetAttribute((const void*)topk_slices_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             TOPK_SLICE_MAX * 8);
+    return a != hipSuccess ? a : hipFuncSetAttribute((const void*)topk_draw_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     TOPK_SLICES * TOPK_MAX * 8);
+  });
+  SYN_CHECK(e == hipSuccess, "draw_top_k: %zu and %zu bytes of LDS refused: %s", lds_slice, lds_draw, hipGetErrorString(e));
+  const size_t n_cand = (size_t)n_rows * parts * TOPK_MAX;
+  int* cand_i = (int*)(words + n_cand);
+  int* cand_n = (int*)(words + 2 * n_cand);
+  topk_slices_kernel<<<dim3(parts, n_rows), SLICE_THREADS, lds_slice, stream>>>(logits, V, slice, temperature, top_k, repetition,
+                                                                               presence, frequency, ids, id_start, words, cand_i, cand_n);
+  SYN_LAUNCH_CHECK("draw_top_k");
+  topk_draw_kernel<<<n_rows, SAMPLE_THREADS, lds_draw, stream>>>(words, cand_i, cand_n, parts, V, top_k, top_p, min_p, draw, uniform, out);
+  SYN_LAUNCH_CHECK("draw_top_k");
   return 0;
 }

@@ -1381,6 +1381,39 @@ def filter_rows(logits, out, temperature, top_k, top_p, min_p, repetition, prese
           _ptr(counts), _stream())
 
 
+DRAW_TOP_K_MAX = 512         # largest top-k of draw_top_k (TOPK_MAX of csrc/sampling.hip)
+
+
+@functools.lru_cache(maxsize=None)
+def draw_top_k_words(n_rows: int, V: int) -> int:
+    """Four-byte words of scratch memory for draw_top_k, 0 for rows that it does not take."""
+    lib = load_library("core")
+    lib.syn_draw_top_k_words.restype = ctypes.c_long
+    return int(lib.syn_draw_top_k_words(n_rows, V))
+
+
+def draw_top_k(logits, out, max_k, temperature, top_k, top_p, min_p, repetition, presence, frequency, draw, uniform, ids=None,
+               id_start=None):
+    """filter_rows and sample_rows(temperature=draw) in one for rows that all have a top-k (1 <= top_k <= max_k <= DRAW_TOP_K_MAX,
+    max_k < V), spread over many workgroups a row; the options as in filter_rows.  draw [R]: 1 where the row is drawn from with
+    uniform[r], 0 where its largest is taken.  out [R] int32: the tokens that those two give."""
+    _need(logits, "draw_top_k.logits", _F32, (None, None))
+    R, V = logits.shape
+    for name, t, dt in (("temperature", temperature, _F32), ("top_k", top_k, _I32), ("top_p", top_p, _F32),
+                        ("min_p", min_p, _F32), ("repetition", repetition, _F32), ("presence", presence, _F32),
+                        ("frequency", frequency, _F32), ("draw", draw, _F32), ("uniform", uniform, _F32), ("out", out, _I32)):
+        _need(t, f"draw_top_k.{name}", dt, (R,))
+    if (ids is None) != (id_start is None):
+        raise KernelError("draw_top_k: ids and id_start come together")
+    if ids is not None:
+        _need(ids, "draw_top_k.ids", _I32, (None,))
+        _need(id_start, "draw_top_k.id_start", _I32, (R + 1,))
+    words = torch.empty(max(1, draw_top_k_words(R, V)), dtype=_F32, device=logits.device)
+    _call(load_library("core"), "syn_draw_top_k", _ptr(logits), R, V, int(max_k), _ptr(temperature), _ptr(top_k), _ptr(top_p),
+          _ptr(min_p), _ptr(repetition), _ptr(presence), _ptr(frequency), _ptr(ids), _ptr(id_start), _ptr(draw), _ptr(uniform),
+          _ptr(words), _ptr(out), _stream())
+
+
 # ----------------------------------------------------------------------------- what the machine gives
 
 def measure_ceilings(device="cuda:0", read_bytes=1 << 30, repeats=5):

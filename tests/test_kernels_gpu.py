@@ -1540,6 +1540,55 @@ def test_filter_rows_against_the_plain_processors(ops, V):
     assert torch.equal(torch.nan_to_num(again, neginf=-1e30), torch.nan_to_num(got, neginf=-1e30)), "in place, and the same bits twice"
 
 
+@pytest.mark.parametrize("V,shift", [(3, 0), (1000, 0), (1027, 0), (8192, 0), (33001, 0), (33004, 1), (151936, 0), (262144, 0)])
+def test_draw_top_k_gives_what_the_filters_and_the_draw_give(ops, V, shift):
+    """The one path against the two kernels it stands for, token by token: k from 1 to the largest, one value in many places, rows of
+    -inf but for a few, infinities and NaN, penalties with tokens outside the row, u at both ends, rows whose memory begins
+    `shift` entries into a 16-byte line."""
+    top = min(ops.DRAW_TOP_K_MAX, V - 1)
+    ks = sorted({1, min(2, top), min(50, top), min(257, top), top})
+    options = [dict(k=k, **o) for k in ks for o in (dict(), dict(T=0.7, p=0.9), dict(mp=0.05), dict(T=0.0, p=0.5),
+                                                    dict(T=1.5, p=0.8, mp=0.02, rep=1.2, pres=0.3, freq=0.1))]
+    g = torch.Generator().manual_seed(V)
+    kinds = []
+    for i in range(len(options)):
+        x = torch.randn(V, generator=g) * 2.5
+        kind = i % 8
+        if kind == 1:
+            x = x.round()                                        # ties at every cut
+        elif kind == 2:
+            x = torch.full((V,), 1.5)
+        elif kind == 3:
+            x[torch.randperm(V, generator=g)[:V - max(1, V // 4000)]] = float("-inf")
+        elif kind == 4:
+            x[torch.randint(0, V, (3,), generator=g)] = float("inf")
+        elif kind == 5:
+            x[torch.randint(0, V, (2,), generator=g)] = float("nan")
+        elif kind == 6:
+            x[:] = float("-inf")
+            x[V - 1] = float("nan")
+        kinds.append(x)
+    R = len(options)
+    whole = torch.empty(R * V + 4, dtype=F32, device=DEV)
+    x = whole[shift:shift + R * V].view(R, V)
+    x.copy_(torch.stack(kinds))
+    col = lambda key, default, dt=F32: torch.tensor([o.get(key, default) for o in options], dtype=dt).to(DEV)
+    ids = [torch.randint(-2, V + 3, (1 + 40 * (r % 6),), generator=g).tolist() * (1 + r % 2) for r in range(R)]
+    flat = torch.tensor(sum(ids, []), dtype=I32).to(DEV)
+    starts = torch.tensor([0] + torch.tensor([len(i) for i in ids]).cumsum(0).tolist(), dtype=I32).to(DEV)
+    args = [col("T", 1.0), col("k", 0, I32), col("p", 1.0), col("mp", 0.0), col("rep", 1.0), col("pres", 0.0), col("freq", 0.0)]
+    draw = torch.tensor([1.0 if o.get("T", 1.0) > 0 else 0.0 for o in options]).to(DEV)
+    for with_ids in (True, False):
+        left = torch.empty_like(x)
+        counts = torch.zeros(R * V, dtype=I32, device=DEV)
+        ops.filter_rows(x, left, *args, *((flat, starts, counts) if with_ids else ()))
+        for u in (torch.rand(R, generator=g), torch.zeros(R), torch.full((R,), 0.99999994), torch.ones(R)):
+            want, got = torch.full((R,), -1, dtype=I32, device=DEV), torch.full((R,), -2, dtype=I32, device=DEV)
+            ops.sample_rows(left, draw, u.to(DEV), want)
+            ops.draw_top_k(x, got, max(ks), *args, draw, u.to(DEV), *((flat, starts) if with_ids else ()))
+            assert got.tolist() == want.tolist(), (V, with_ids, [(i, options[i], i % 8) for i in range(R) if got[i] != want[i]])
+
+
 def test_filter_rows_counts_in_memory_of_any_content(ops):
     """The penalties' counters need not be zero, and calls on two streams from two threads give what they give one after another."""
     import threading
