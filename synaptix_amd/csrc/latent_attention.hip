@@ -559,3 +559,307 @@ SYN_EXPORT int syn_latent_attention_bf16(const void* q, const void* k_pages, con
   }
   return 0;
 }
+
+// ------------------------------------------------------------------ prompts over keys and values of the heads' own
+// The products with W_uk and W_uv at the keys' side after all: keys and values of every head are made from the latents once a step
+// (two products over the sequences' rows), and a query then meets dim + rot instead of rank + rot values and sums v_dim instead
+// of rank: with heads of 128 + 64 and a latent of 512 a (query, key) pair is 640 + 256 multiplications less 2,176 + 1,024 (the second
+// numbers: a weight counts as two bf16 numbers, as above), which pays where a step brings as many tokens as a prompt.
+//   latent_rows      the rows [latent | rotated part] of all sequences out of their pages, one after another, each sequence's first
+//                    visible page first; what lies behind a sequence's end is zero
+//   latent_expanded  the attention itself: 128 queries of a head a workgroup, four waves of 32, 32x32x16 matrix instructions,
+//                    blocks of 64 keys through two LDS buffers, as csrc/attention_bf16.hip has them for 128 + 128
+// Two workgroups a compute unit (80 KB of LDS each).  1,500 tokens, 32 heads of 128 + 64, a latent of 512: 61 + 220 + 55 us a
+// layer with the up-projections absorbed (queries, attention, values), 5 + 37 + 73 so (rows, keys and values, attention).
+#define LX_ROWS 128
+#define LX_DIM 128           // of a head's unrotated keys and of its values
+#define LX_ROT 64
+#define LX_LAZY 8.f          // a row's sums are rescaled where its maximum has grown by more than 2^LX_LAZY
+
+// rows of the sequences in front of `seq`, and the first page of `seq` that some new token sees
+__device__ __forceinline__ int lx_rows_before(const int* seq_start, const int* seq_past, int seq, int window, int& first_page) {
+  const int lane = threadIdx.x % SYN_WAVE;
+  int pages = 0;
+  for (int b = lane; b < seq; b += SYN_WAVE) {
+    const int past = seq_past[b], len = past + seq_start[b + 1] - seq_start[b];
+    pages += (len + SYN_PAGE - 1) / SYN_PAGE - (window > 0 ? max(0, past - window + 1) / SYN_PAGE : 0);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) pages += __shfl_xor(pages, off, SYN_WAVE);
+  first_page = (window > 0 ? max(0, seq_past[seq] - window + 1) : 0) / SYN_PAGE;
+  return pages * SYN_PAGE;
+}
+
+__global__ void __launch_bounds__(256)
+latent_rows_kernel(const bf16* __restrict__ k_pages, const int* __restrict__ page_table, int table_stride,
+                   const int* __restrict__ seq_start, const int* __restrict__ seq_past, int n_seqs, int window, int rank, int rot,
+                   bf16* __restrict__ latent, bf16* __restrict__ rotated) {
+  // a quarter of a page a workgroup; which page this is: the sequences one after another
+  int t = blockIdx.x / 4, seq = 0, page = 0, len = 0;
+  for (; seq < n_seqs; ++seq) {
+    const int past = seq_past[seq];
+    len = past + seq_start[seq + 1] - seq_start[seq];
+    const int lo = (window > 0 ? max(0, past - window + 1) : 0) / SYN_PAGE, n = (len + SYN_PAGE - 1) / SYN_PAGE - lo;
+    if (t < n) {
+      page = lo + t;
+      break;
+    }
+    t -= n;
+  }
+  if (seq == n_seqs) return;
+  const int R = rank + rot, per = R / 8, left = len - page * SYN_PAGE;
+  const bf16* src = k_pages + (size_t)page_table[(size_t)seq * table_stride + page] * SYN_PAGE * R;
+  const bf16x8 zero = {};
+  for (int c = threadIdx.x; c < SYN_PAGE / 4 * per; c += blockDim.x) {
+    const int r = blockIdx.x % 4 * (SYN_PAGE / 4) + c / per, d = c % per * 8;
+    const bf16x8 v = r < left ? *(const bf16x8*)(src + (size_t)r * R + d) : zero;
+    const size_t row = (size_t)(blockIdx.x / 4) * SYN_PAGE + r;
+    *(bf16x8*)(d < rank ? latent + row * rank + d : rotated + row * rot + d - rank) = v;
+  }
+}
+
+__global__ void __launch_bounds__(256, 2)
+latent_expanded_kernel(const bf16* __restrict__ q_nope, const bf16* __restrict__ q_rot, int q_rot_stride, const bf16* __restrict__ keys,
+                       const bf16* __restrict__ rotated, const bf16* __restrict__ values, int n_rows,
+                       const int* __restrict__ seq_start, const int* __restrict__ seq_past, int n_seqs, bf16* __restrict__ out,
+                       float scale, int nh, int window, const float* __restrict__ gate, int gate_stride, int gate_per_value) {
+  constexpr int KS = (LX_DIM + LX_ROT) / 16, NOPE = SYN_PAGE * LX_DIM * 2, ROT = SYN_PAGE * LX_ROT * 2, BUF = 2 * NOPE + ROT;
+  constexpr int DT = LX_DIM / 16, D32 = LX_DIM / 32, NLOAD = BUF / 1024 / 4, AHEAD = 6;
+  extern __shared__ __attribute__((aligned(16))) char lds[];      // [2][unrotated keys | rotated keys | values]
+  // late tiles of a sequence see the most keys: they come first, and a late and an early one meet on a compute unit
+  int total = 0;
+  for (int s = 0; s < n_seqs; ++s) total += (seq_start[s + 1] - seq_start[s] + LX_ROWS - 1) / LX_ROWS;
+  const int y = blockIdx.y, half = (total + 1) / 2;
+  if (y >= total) return;
+  int seq, tile, tok0, n_new;
+  if (!la_find_unit(y < half ? total - 1 - y : y - half, LX_ROWS, seq_start, n_seqs, 1, seq, tile, tok0, n_new)) return;
+  seq = __builtin_amdgcn_readfirstlane(seq), tile = __builtin_amdgcn_readfirstlane(tile);
+  tok0 = __builtin_amdgcn_readfirstlane(tok0), n_new = __builtin_amdgcn_readfirstlane(n_new);
+  const int lane = threadIdx.x % SYN_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE);
+  const int n32 = lane % 32, hh = lane / 32;
+  const int hx = blockIdx.x, head = nh % 8 == 0 ? (hx % 8) * (nh / 8) + hx / 8 : hx;      // neighbouring heads on one die
+  const int past = seq_past[seq], q0 = tile * LX_ROWS;
+  int page0;
+  const int row0 = __builtin_amdgcn_readfirstlane(lx_rows_before(seq_start, seq_past, seq, window, page0));
+  const int kb_hi = (past + min(q0 + LX_ROWS, n_new) - 1) / SYN_PAGE;
+  const int kb_lo = (window > 0 ? max(0, past + q0 - window + 1) : 0) / SYN_PAGE;
+  if (row0 + (kb_hi - page0 + 1) * SYN_PAGE > n_rows) return;      // (the caller's rows are not those of these sequences)
+  const int r0 = q0 + wave * 32, row = r0 + n32;
+  const bool wave_on = r0 < n_new, valid = row < n_new;
+  const int qpos = valid ? past + row : -1, lo = (window > 0 && valid) ? max(0, qpos - window + 1) : 0;
+  const int w_kmax = past + min(r0 + 31, n_new - 1), w_qmin = past + r0, w_kmin = window > 0 ? max(0, w_qmin - window + 1) : 0;
+  const float scale2 = scale * 1.4426950408889634f;
+  const bf16x8 zero8 = {};
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = 16 * ks + 8 * hh;
+    const size_t at = (size_t)(tok0 + row) * nh + head;
+    qf[ks] = !valid ? zero8 : ks < LX_DIM / 16 ? *(const bf16x8*)(q_nope + at * LX_DIM + d) : *(const bf16x8*)(q_rot + at * q_rot_stride + d - LX_DIM);
+  }
+  f32x16 o[D32];
+#pragma unroll
+  for (int d = 0; d < D32; ++d)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[d][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+
+  struct Views {
+    BufferView k, r, v;
+  };
+  auto views_of = [&](int kb) {
+    const size_t at = row0 + (size_t)(kb - page0) * SYN_PAGE;
+    return Views{buffer_view(keys + (at * nh + head) * LX_DIM, ((size_t)(SYN_PAGE - 1) * nh + 1) * LX_DIM * 2),
+                 buffer_view(rotated + at * LX_ROT, ROT),
+                 buffer_view(values + (size_t)head * LX_DIM * n_rows + at, ((size_t)(LX_DIM - 1) * n_rows + SYN_PAGE) * 2)};
+  };
+  // load j of a wave for a block: 1 KB straight into LDS, 16-byte chunks of a key's row swizzled (a fragment reads 32 rows at the same
+  // column), values in the order of their fragments
+  auto fetch_one = [&](const Views& v, int buf, int j) {
+    char* dst = lds + buf * BUF;
+    const int i = j * 4 + wave;
+    if (j < 4) {
+      const int at = 64 * i + lane, r = at / 16, slot = at % 16;
+      buffer_to_lds16(v.k, dst + 1024 * i, (unsigned)(r * nh * LX_DIM * 2 + (slot ^ (r & 15)) * 16), 0);
+    } else if (j < 6) {
+      const int at = 64 * (i - 16) + lane, r = at / 8, slot = at % 8;
+      buffer_to_lds16(v.r, dst + 1024 * i, (unsigned)((r * 8 + (slot ^ ((r >> 1) & 7))) * 16), 0);
+    } else {
+      const int f = i - 24, d = (f % DT) * 16 + lane % 16, key = (f / DT) * 32 + (lane / 16) * 8;
+      buffer_to_lds16(v.v, dst + 1024 * i, (unsigned)((d * n_rows + key) * 2), 0);
+    }
+  };
+  auto landed = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's loads have written LDS; behind the barrier all have
+    __syncthreads();
+  };
+  const int krow0 = 16 * (n32 / 16) + 8 * ((n32 % 8) / 4) + 4 * ((n32 % 16) / 8) + n32 % 4;      // (so that a lane's scores are 8 consecutive keys)
+
+  auto block = [&](int kb, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    const int buf = (kb - kb_lo) & 1, key0 = kb * SYN_PAGE;
+    Views next;
+    if constexpr (MORE) next = views_of(kb + 1);
+    const char* ks_ = lds + buf * BUF;
+    const char* rs_ = ks_ + NOPE;
+    const char* vs_ = rs_ + ROT;
+    if (wave_on && key0 <= w_kmax && key0 + SYN_PAGE > w_kmin) {
+      constexpr int NQK = 2 * KS, NPV = 4 * D32;
+      static_assert(NLOAD <= NQK / 2, "a load behind every second MFMA of the scores");
+      f32x16 s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[t][e] = 0.f;
+      auto k_frag = [&](int i) {   // read i: k-step i / 2 of score tile i % 2
+        const int ks = i / 2, r = 32 * (i % 2) + krow0;
+        return ks < LX_DIM / 16 ? *(const bf16x8*)(ks_ + (r * 16 + ((2 * ks + hh) ^ (r & 15))) * 16)
+                                : *(const bf16x8*)(rs_ + (r * 8 + ((2 * (ks - LX_DIM / 16) + hh) ^ ((r >> 1) & 7))) * 16);
+      };
+      auto v_frag = [&](int i) {   // read i: output tile i % D32 of k-step i / D32 = 2 t + j
+        const int d = i % D32, tj = i / D32, t = tj / 2, j = tj % 2;
+        return *(const bf16x8*)(vs_ + (((t * DT + 2 * d + n32 / 16) * 64 + (2 * j + hh) * 16 + n32 % 16)) * 16);
+      };
+      bf16x8 kf[NQK], vf[NPV];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) kf[i] = k_frag(i);
+#pragma unroll
+      for (int i = 0; i < NQK; ++i) {
+        s[i % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i / 2], s[i % 2], 0, 0, 0);
+        if (i + AHEAD < NQK) kf[i + AHEAD] = k_frag(i + AHEAD);
+        else if (i + AHEAD - NQK < AHEAD) vf[i + AHEAD - NQK] = v_frag(i + AHEAD - NQK);
+        if (MORE && i % 2 == 1 && i / 2 < NLOAD) fetch_one(next, buf ^ 1, i / 2);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+      for (int i = 0; i < NQK; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA,
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one read behind it,
+        if (MORE && i % 2 == 1 && i / 2 < NLOAD) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);      // a load behind every second
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (key0 + SYN_PAGE - 1 > w_qmin || (window > 0 && key0 < w_kmax - window + 1) || r0 + 32 > n_new) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int key = key0 + 32 * t + 16 * (e / 8) + 8 * hh + e % 8;
+            if (key > qpos || key < lo) s[t][e] = -INFINITY;
+          }
+      }
+      float mloc = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[t][e]);
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 32, SYN_WAVE)) * scale2;
+      const bool raise = mloc > m_run + LX_LAZY || (m_run == -INFINITY && mloc > -INFINITY);
+      if (__any(raise)) {
+        const float m_new = raise ? mloc : m_run;
+        const float alpha = raise ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;  // from -inf: 0
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < D32; ++d) o[d] *= alpha;
+      }
+      const float neg_m = m_run == -INFINITY ? 0.f : -m_run;  // a column that has seen no key yet
+      float lsum = 0.f;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        bf16x8 hi, rest;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(s[tj / 2][8 * (tj % 2) + e], scale2, neg_m));   // a masked score: 2^-inf = 0
+          lsum += p;
+          hi[e] = (bf16)p;
+          rest[e] = (bf16)(p - (float)hi[e]);
+        }
+#pragma unroll
+        for (int d = 0; d < D32; ++d) {
+          const int i = tj * D32 + d;
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], hi, o[d], 0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], rest, o[d], 0, 0, 0);
+          if (i + AHEAD < NPV) vf[i + AHEAD] = v_frag(i + AHEAD);
+        }
+      }
+      l_run += lsum;
+    } else if constexpr (MORE) {
+#pragma unroll
+      for (int j = 0; j < NLOAD; ++j) fetch_one(next, buf ^ 1, j);
+    }
+    landed();
+  };
+  {
+    const Views v = views_of(kb_lo);
+#pragma unroll
+    for (int j = 0; j < NLOAD; ++j) fetch_one(v, 0, j);
+  }
+  landed();
+  for (int kb = kb_lo; kb < kb_hi; ++kb) block(kb, std::true_type{});
+  block(kb_hi, std::false_type{});
+  if (!wave_on) return;
+  const float l = l_run + __shfl_xor(l_run, 32, SYN_WAVE);
+  if (!valid) return;
+  const float inv = 1.f / l;
+  const size_t at = (size_t)(tok0 + row) * nh + head;
+  const float* grow = gate ? gate + (size_t)(tok0 + row) * gate_stride + (gate_per_value ? head * LX_DIM : head) : nullptr;
+  auto sigmoid = [](float z) { return 1.f / (1.f + expf(-z)); };
+  const float of_head = gate && !gate_per_value ? sigmoid(grow[0]) : 1.f;
+  bf16* orow = out + at * LX_DIM + 4 * hh;
+#pragma unroll
+  for (int d = 0; d < D32; ++d)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      bf16x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x = o[d][4 * b + e] * inv;
+        if (gate) x *= gate_per_value ? sigmoid(grow[32 * d + 8 * b + 4 * hh + e]) : of_head;
+        v[e] = (bf16)x;
+      }
+      *(bf16x4*)(orow + 32 * d + 8 * b) = v;
+    }
+}
+
+// The rows of a step's sequences out of their pages: latent [n_rows][rank], rotated [n_rows][rot], n_rows = 64 times the pages that some
+// new token of its sequence sees (window 0: all).
+SYN_EXPORT int syn_latent_rows(const void* k_pages, const int* page_table, int table_stride, const int* seq_start, const int* seq_past,
+                               int n_seqs, int window, int rank, int rot, void* latent, void* rotated, int n_rows, hipStream_t stream) {
+  SYN_CHECK(n_seqs > 0 && n_rows > 0 && n_rows % SYN_PAGE == 0 && window >= 0, "latent_rows: %d rows of %d sequences", n_rows, n_seqs);
+  SYN_CHECK(rank > 0 && rot >= 0 && rank % 8 == 0 && rot % 8 == 0 && ((uintptr_t)k_pages | (uintptr_t)latent | (uintptr_t)rotated) % 16 == 0,
+            "latent_rows: rows of %d + %d values (multiples of 8, 16-byte aligned)", rank, rot);
+  latent_rows_kernel<<<4 * (n_rows / SYN_PAGE), 256, 0, stream>>>((const bf16*)k_pages, page_table, table_stride, seq_start, seq_past, n_seqs,
+                                                            window, rank, rot, (bf16*)latent, (bf16*)rotated);
+  SYN_LAUNCH_CHECK("latent_rows");
+  return 0;
+}
+
+// q_nope [N][nh][128]; q_rot: the rotated parts, 64 values every q_rot_stride; keys [n_rows][nh][128], rotated [n_rows][64], values
+// [nh][128][n_rows] (rows as syn_latent_rows leaves them); out [N][nh][128] times sigmoid(gate), gate float rows every gate_stride: one
+// number a head or (gate_per_value) a value, or null.
+SYN_EXPORT int syn_latent_expanded(const void* q_nope, const void* q_rot, int q_rot_stride, const void* keys, const void* rotated,
+                                   const void* values, int n_rows, const int* seq_start, const int* seq_past, int n_seqs, int n_tokens,
+                                   void* out, float scale, int nh, int dim, int rot, int window, const float* gate, int gate_stride,
+                                   int gate_per_value, hipStream_t stream) {
+  SYN_CHECK(dim == LX_DIM && rot == LX_ROT, "latent_expanded: heads of %d + %d values (%d + %d)", dim, rot, LX_DIM, LX_ROT);
+  SYN_CHECK(n_seqs > 0 && n_tokens >= n_seqs && nh > 0 && n_rows > 0 && n_rows % SYN_PAGE == 0 && window >= 0 && scale > 0.f,
+            "latent_expanded: %d tokens, %d rows, scale %g", n_tokens, n_rows, (double)scale);
+  SYN_CHECK(q_rot_stride % 8 == 0 && ((uintptr_t)q_nope | (uintptr_t)q_rot | (uintptr_t)keys | (uintptr_t)rotated | (uintptr_t)values | (uintptr_t)out) % 16 == 0,
+            "latent_expanded: operands must be 16-byte aligned");
+  SYN_CHECK((size_t)n_rows * LX_DIM * 2 < 0x7fffffffull && (size_t)nh * LX_DIM * 2 * SYN_PAGE < 0x7fffffffull, "latent_expanded: %d rows of %d heads", n_rows, nh);
+  constexpr int LDS = 2 * (2 * SYN_PAGE * LX_DIM + SYN_PAGE * LX_ROT) * 2;
+  static OncePerDevice raised;
+  const hipError_t e = once_per_device(raised, [&] {
+    return hipFuncSetAttribute((const void*)latent_expanded_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  });
+  SYN_CHECK(e == hipSuccess, "latent_expanded: %d bytes of LDS refused: %s", LDS, hipGetErrorString(e));
+  const int tiles = n_tokens / LX_ROWS + n_seqs;      // a bound; surplus workgroups leave at once
+  SYN_CHECK(tiles <= 65535, "latent_expanded: %d tiles", tiles);
+  latent_expanded_kernel<<<dim3(nh, tiles), 256, LDS, stream>>>((const bf16*)q_nope, (const bf16*)q_rot, q_rot_stride, (const bf16*)keys,
+                                                                (const bf16*)rotated, (const bf16*)values, n_rows, seq_start, seq_past,
+                                                                n_seqs, (bf16*)out, scale, nh, window, gate, gate_stride, gate_per_value);
+  SYN_LAUNCH_CHECK("latent_expanded");
+  return 0;
+}

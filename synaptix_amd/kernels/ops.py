@@ -1721,6 +1721,63 @@ def latent_intake(proj, gain, eps, cos, sin, q_nope, q_full, k_pages, v_pages, p
 
 # ----------------------------------------------------------------------------- latent attention
 
+def latent_expanded_takes(dim, rot_dim, v_dim, rank) -> bool:
+    """Whether latent_expanded_attention takes heads of these sizes (and its two products a latent of this rank)."""
+    return dim == v_dim == 128 and rot_dim == 64 and rank % 128 == 0
+
+
+def latent_expanded_rows(past, new, window=0) -> int:
+    """Rows of latent_rows for sequences of past[b] cached and new[b] new tokens: whole pages, from the first that some new token sees."""
+    return PAGE_TOKENS * sum((p + n + PAGE_TOKENS - 1) // PAGE_TOKENS - (max(0, p - window + 1) // PAGE_TOKENS if window else 0)
+                             for p, n in zip(past, new))
+
+
+def latent_rows(k_pages, page_table, seqs, rank, rot_dim, n_rows, window=0):
+    """The step's sequences' cache rows out of their pages k_pages [pages, 1, 64, rank + rot_dim] bf16: (latents [n_rows, rank], rotated
+    key parts [n_rows, rot_dim]), the sequences one after another in whole pages, zeros behind their ends; n_rows:
+    latent_expanded_rows."""
+    seq_start, seq_past = seqs
+    _need(k_pages, "latent_rows.k_pages", _BF16, (None, 1, PAGE_TOKENS, rank + rot_dim))
+    _need(page_table, "latent_rows.page_table", _I32, (None, None))
+    _need(seq_past, "latent_rows.seq_past", _I32, (None,))
+    B = seq_past.shape[0]
+    _need(seq_start, "latent_rows.seq_start", _I32, (B + 1,))
+    if page_table.shape[0] < B:
+        raise KernelError(f"latent_rows: page table has {page_table.shape[0]} rows for {B} sequences")
+    latent = torch.empty((n_rows, rank), dtype=_BF16, device=k_pages.device)
+    rotated = torch.empty((n_rows, rot_dim), dtype=_BF16, device=k_pages.device)
+    _call(load_library("core"), "syn_latent_rows", _ptr(k_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_start), _ptr(seq_past),
+          B, int(window or 0), rank, rot_dim, _ptr(latent), _ptr(rotated), n_rows, _stream())
+    return latent, rotated
+
+
+def latent_expanded_attention(q_nope, q_full, rank, keys, rotated, values, seqs, out, scale, window=0, gate=None, gate_per_value=True):
+    """Attention of prompts with keys and values of every head's own: q_nope [N, heads, 128] and the rotated parts q_full [N, heads,
+    rank + 64] behind each row's first `rank` places, keys [rows, heads, 128], rotated [rows, 64] (shared by the heads), values
+    [heads, 128, rows], all bf16, rows as latent_rows leaves them; out [N, heads, 128] = sum_j softmax_j(scale (q_nope . k_j + q_rot . r_j))
+    v_j  [* sigmoid(gate)] over the keys at or before the query's position (window > 0: the last `window` of them).  gate as in
+    heads_product."""
+    _need(q_nope, "latent_expanded.q_nope", _BF16, (None, None, 128))
+    N, Hn, D = q_nope.shape
+    _need(q_full, "latent_expanded.q_full", _BF16, (N, Hn, rank + 64))
+    _need(keys, "latent_expanded.keys", _BF16, (None, Hn, D))
+    n_rows = keys.shape[0]
+    _need(rotated, "latent_expanded.rotated", _BF16, (n_rows, 64))
+    _need(values, "latent_expanded.values", _BF16, (Hn, D, n_rows))
+    seq_start, seq_past = seqs
+    _need(seq_past, "latent_expanded.seq_past", _I32, (None,))
+    B = seq_past.shape[0]
+    _need(seq_start, "latent_expanded.seq_start", _I32, (B + 1,))
+    _need(out, "latent_expanded.out", _BF16, (N, Hn, D))
+    ld = 0
+    if gate is not None:
+        ld = _float_rows_view(gate, "latent_expanded.gate", N, Hn * D if gate_per_value else Hn)
+    rot_parts = ctypes.c_void_p(q_full.data_ptr() + rank * q_full.element_size())
+    _call(load_library("core"), "syn_latent_expanded", _ptr(q_nope), rot_parts, rank + 64, _ptr(keys), _ptr(rotated), _ptr(values), n_rows,
+          _ptr(seq_start), _ptr(seq_past), B, N, _ptr(out), ctypes.c_float(scale), Hn, D, 64, int(window or 0), _ptr(gate), ld,
+          int(bool(gate_per_value)), _stream())
+
+
 LATENT_ATTENTION_MAX_ROW = WINDOW_ATTENTION_MAX_DIM      # plain FMA: 32-bit, and sizes that the tiles do not take
 LATENT_TILED_MAX_RANK, LATENT_TILED_MAX_ROW = 512, 640
 

@@ -12,7 +12,8 @@ Computed with the up-projections moved to the query's side, which is the same su
     q_nope . (W_uk[h] c_j) = (W_uk[h]^T q_nope) . c_j          the query in the latent's space ("absorbed")
     sum_j p_j W_uv[h] c_j  = W_uv[h] (sum_j p_j c_j)           the weights meet the latents, then one small product
 so that attention is one shared key row [c | k_rot] of rank + rot_dim values a token for all heads, whose first
-`rank` values are also its value.  The cache group has one kv head with rows [c | k_rot] and the latent once more
+`rank` values are also its value.  (Steps of many tokens take the formula as it stands above, with keys and values of every
+head made from the cached latents once a step: `_expanded`.)  The cache group has one kv head with rows [c | k_rot] and the latent once more
 transposed as the value page (what the attention kernels' second product reads along the keys).
 Scores, weights, the latent's norm, the rotation and the gates are 32-bit in both engine types.
 """
@@ -58,7 +59,7 @@ class LatentAttention(Mixer):
         if q_rank is not None and q_rank <= 0:
             raise ValueError(f"{prefix}: a query latent of {q_rank} values")
         self.names = dict(self.NAMES, **(names or {}))
-        self.w_in = self.w_q_up = self.w_o = self.w_uk_t = self.w_uv = self.gain = self.q_gain = None
+        self.w_in = self.w_q_up = self.w_o = self.w_uk_t = self.w_uk = self.w_uv = self.gain = self.q_gain = None
 
     def _n(self, key):
         return self.prefix + self.names[key]
@@ -95,6 +96,9 @@ class LatentAttention(Mixer):
         # W_uk[h] as [rank, dim]: the query's product with it runs along dim
         self.w_uk_t = get(self._n("up_k")).view(self.nh, self.dim, self.rank).transpose(1, 2).contiguous()
         self.w_uv = get(self._n("up_v")).view(self.nh, self.vdim, self.rank).contiguous()
+        # ... and for prompts as it is: the latents' product with it runs along the rank
+        self.w_uk = (_projection(get(self._n("up_k")))
+                     if self.w_uv.dtype == torch.bfloat16 and ops.latent_expanded_takes(self.dim, self.rot, self.vdim, self.rank) else None)
 
     def cache_need(self):
         return KvNeed(1, self.rank + self.rot, self.window, v_dim=self.rank)
@@ -128,6 +132,10 @@ class LatentAttention(Mixer):
         ops.latent_intake(queries, self.gain, self.norm_eps, cos, sin, q_nope, q_full, cache.k_pages, cache.v_pages, table,
                           ctx.tok_seq, ctx.tok_pos, nh, dim, rot, rank, ctx.max_position, write_kv=owner, v_fragments=tiled,
                           down=proj[:, at:])
+        gate = proj[:, at + R:] if self.gate else None
+        rows = self._expanded_rows(ctx) if tiled else 0
+        if rows:
+            return deferred_product(self._expanded(q_nope, q_full, cache, table, ctx, rows, gate), self.w_o)
         # the query in the latent's space, into the first `rank` places of each head's row
         ops.heads_product(q_nope.view(N, nh, dim), self.w_uk_t, q_full.view(N, nh, R))
         o_lat = torch.empty((N, nh * rank), dtype=act, device=dev)
@@ -136,7 +144,30 @@ class LatentAttention(Mixer):
                              rank, rot, window=self.window or 0, seqs=(ctx.seq_start, ctx.seq_past) if tiled else None,
                              workspace=ctx.scratch("latent_attention", floats) if floats else None)
         o = torch.empty((N, nh * vdim), dtype=act, device=dev)
-        gate = proj[:, at + R:] if self.gate else None
         ops.heads_product(o_lat.view(N, nh, rank), self.w_uv, o.view(N, nh, vdim), gate=gate,
                           gate_per_value=self.gate == "value")
         return deferred_product(o, self.w_o)
+
+    def _expanded_rows(self, ctx) -> int:
+        """Rows of keys and values that the step makes for every head, or 0 where it absorbs the up-projections instead.  Keys and
+        values of a cached token cost two products with all heads' up-projections, which the new tokens' smaller attention
+        pays back while there are few cached tokens to each new one: steps of one layer (4,096 wide, 32 heads, a latent of 512), us
+        with and without: 1,500 tokens 881 and 1,091, behind 6,000 cached ones 1,191 and 2,292; 200 behind 3,200 805 and 957; 16
+        sequences of 30 behind 200 676 and 678 (8.5 rows a new token); 8 single tokens behind 2,000 beside a prompt of 1,500 1,105 and
+        1,103 (11.9), beside one of 300 1,237 and 1,178 (54).  Steps replayed from graphs (up to 128 tokens of prompts, or single
+        ones) know no lengths on the host and absorb."""
+        if self.w_uk is None or self.scale <= 0 or ctx.n_tokens <= 128 or min(ctx.slots) < 0:
+            return 0
+        rows = ops.latent_expanded_rows(ctx.past, ctx.new_counts, self.window or 0)
+        return rows if rows <= 8 * ctx.n_tokens else 0
+
+    def _expanded(self, q_nope, q_full, cache, table, ctx, rows, gate):
+        N, nh, dim, vdim, seqs = q_nope.shape[0], self.nh, self.dim, self.vdim, (ctx.seq_start, ctx.seq_past)
+        latent, rotated = ops.latent_rows(cache.k_pages, table, seqs, self.rank, self.rot, rows, self.window or 0)
+        keys = linear(latent, self.w_uk, latent.dtype)
+        values = torch.empty((nh * vdim, rows), dtype=latent.dtype, device=latent.device)
+        ops.gemm(self.w_uv.view(nh * vdim, self.rank), latent, values)      # (along the keys, as the second product reads them)
+        o = torch.empty((N, nh, vdim), dtype=latent.dtype, device=latent.device)
+        ops.latent_expanded_attention(q_nope.view(N, nh, dim), q_full.view(N, nh, -1), self.rank, keys.view(rows, nh, dim), rotated,
+                                      values.view(nh, vdim, rows), seqs, o, self.scale, self.window or 0, gate, self.gate == "value")
+        return o.view(N, nh * vdim)

@@ -309,6 +309,58 @@ def test_latent_attention_of_prompts_at_the_edges_of_its_tiles(window, H, C, B):
     assert float(off.max()) <= 0, (float(off.max()), int((off > 0).sum()))
 
 
+@pytest.mark.parametrize("H,past,new", [(1, [0], [1]), (3, [0, 5, 67, 0], [129, 1, 61, 64]), (8, [500, 0], [300, 63]), (5, [63, 64, 1], [128, 257, 2])])
+@pytest.mark.parametrize("window,gate", [(0, None), (1, "head"), (64, "value"), (65, None), (200, "head")])
+def test_latent_attention_over_keys_and_values_of_the_heads(H, past, new, window, gate):
+    """The rows that come out of the pages, and the attention of 128 + 64 values over 128: sequences that begin and end inside pages
+    and tiles, windows down to one key, pages behind a window left out, NaN in the pages behind the sequences' ends.  The bound as
+    above: results are rounded to bf16, weights count with 16 bits, scores are 32-bit sums of 192 products."""
+    from synaptix_amd.kernels import ops
+    D, B, C, dt = 128, 64, 128, torch.bfloat16
+    g = torch.Generator().manual_seed(H + window)
+    pages, table = [], torch.zeros((len(past), (max(p + n for p, n in zip(past, new)) + 63) // 64), dtype=torch.int32)
+    rows, qs = [], []
+    for b, (p, n) in enumerate(zip(past, new)):
+        rows.append(torch.randn(p + n, C + B, generator=g).to(dt))
+        qs.append((2 * torch.randn(n, H, D + B, generator=g)).to(dt))
+        padded = torch.full(((p + n + 63) // 64 * 64, C + B), float("nan"), dtype=dt)
+        padded[:p + n] = rows[b]
+        for i in range(padded.shape[0] // 64):
+            table[b, i] = len(pages)
+            pages.append(padded[64 * i:64 * i + 64])
+    kp = torch.stack(pages)[:, None].contiguous().to(DEV)
+    seqs = (torch.tensor([0] + torch.tensor(new).cumsum(0).tolist(), dtype=torch.int32, device=DEV), torch.tensor(past, dtype=torch.int32, device=DEV))
+    n_rows = ops.latent_expanded_rows(past, new, window)
+    latent, rotated = ops.latent_rows(kp, table.to(DEV), seqs, C, B, n_rows, window)
+    firsts = [max(0, p - window + 1) // 64 * 64 if window else 0 for p in past]
+    cut = [torch.cat([r[f:], torch.zeros(-len(r) % 64, C + B, dtype=dt)]) for r, f in zip(rows, firsts)]
+    assert torch.equal(torch.cat([latent, rotated], 1).cpu(), torch.cat(cut)) and len(latent) == n_rows
+    N = sum(new)
+    keys, values = torch.randn(n_rows, H, D, generator=g).to(dt), torch.randn(H, D, n_rows, generator=g).to(dt)
+    gates = None if gate is None else torch.randn(N, H * D + 3, generator=g)
+    q = torch.cat(qs)
+    q_full = torch.full((N, H, C + B), float("nan"), dtype=dt)
+    q_full[:, :, C:] = q[:, :, D:]
+    out = torch.full((N, H, D), float("nan"), dtype=dt, device=DEV)
+    ops.latent_expanded_attention(q[:, :, :D].contiguous().to(DEV), q_full.to(DEV), C, keys.to(DEV), rotated, values.to(DEV), seqs, out, 0.07,
+                                  window, None if gate is None else gates.to(DEV)[:, 2:], gate == "value")
+    wants, at = [], 0
+    for b, (p, n) in enumerate(zip(past, new)):
+        T = p + n - firsts[b]
+        k = torch.cat([keys[at:at + T].double(), rotated[at:at + T].cpu().double()[:, None].expand(T, H, B)], -1)
+        s = 0.07 * torch.einsum("qhd,khd->hqk", qs[b].double(), k)
+        pos, key = torch.arange(p, p + n)[:, None], torch.arange(firsts[b], p + n)[None]
+        s = s.masked_fill((key > pos) | ((pos - key >= window) if window else False), float("-inf"))
+        wants.append(torch.einsum("hqk,hdk->qhd", s.softmax(-1), values[:, :, at:at + T].double()))
+        at += len(cut[b])
+    want = torch.cat(wants)
+    if gate is not None:
+        z = gates[:, 2:].double()
+        want = want * torch.sigmoid(z[:, :H * D].view(N, H, D) if gate == "value" else z[:, :H, None])
+    off = (out.cpu().double() - want).abs() - (2 ** -8 * want.abs() + 1e-3)
+    assert float(off.max()) <= 0, (float(off.max()), int((off > 0).sum()))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,D,B,C,pairs", [(3, 8, 6, 20, 3), (2, 16, 8, 32, 2), (1, 4, 0, 6, 0), (4, 32, 16, 64, 8)])
 def test_latent_intake_norms_turns_and_writes_the_pages(H, D, B, C, pairs, dtype):
