@@ -81,8 +81,8 @@ class StepContext:
         self.max_position = max(p + n for p, n in zip(past, new_counts)) - 1
         self._scratch = scratch_pool
         for name, (o, n) in layout.off.items():
-            setattr(self, name, buffer[o:o + n])
-        self._tables = [buffer[o:o + n].view(layout.B, w) for (o, n), w in zip(layout.table_off, layout.widths)]
+            setattr(self, name, buffer.narrow(0, o, n))
+        self._tables = [buffer.narrow(0, o, n).view(layout.B, w) for (o, n), w in zip(layout.table_off, layout.widths)]
         self.items = None       # a work list of decode attention for each group, where the step's owner keeps them
 
     def page_table(self, group: int) -> torch.Tensor:

@@ -11,6 +11,8 @@ their reuse are this engine's own.
 """
 from __future__ import annotations
 
+import itertools
+
 import numpy as np
 import torch
 
@@ -135,22 +137,25 @@ class Engine:
         if len(set(slots)) != len(slots):
             raise StepError("a slot appears twice in one step")
         past = []
+        flat = token_lists[0] if len(token_lists) == 1 else np.concatenate(token_lists)
+        in_vocab = flat.size > 0 and flat.min() >= 0 and flat.max() < self.vocab     # (one look at all; at each for the message)
         for sid, toks in zip(slots, token_lists):
             past.append(self.cache.length(sid))          # raises CacheError for an unknown slot
             if toks.size == 0:
                 raise StepError(f"slot {sid}: a step brings at least one token for each of its sequences")
-            if toks.min() < 0 or toks.max() >= self.vocab:
+            if not in_vocab and (toks.min() < 0 or toks.max() >= self.vocab):
                 raise StepError(f"slot {sid}: token id outside the vocabulary [0, {self.vocab})")
             if self.max_positions is not None and past[-1] + toks.size > self.max_positions:
                 raise CacheError(f"KV overflow: slot {sid} holds {past[-1]} tokens, {toks.size} more exceed "
                                  f"the position range {self.max_positions}")
-        starts = np.concatenate([[0], np.cumsum([t.size for t in token_lists])])
+        counts = [t.size for t in token_lists]
+        starts = [0, *itertools.accumulate(counts)]
         if want is None:
             want_rows = []
         elif isinstance(want, str) and want == "last":
-            want_rows = [int(starts[i + 1]) - 1 for i in range(len(entries))]
+            want_rows = [e - 1 for e in starts[1:]]
         elif isinstance(want, str) and want == "all":
-            want_rows = list(range(int(starts[-1])))
+            want_rows = list(range(starts[-1]))
         else:
             if len(want) != len(entries):
                 raise StepError("`want` needs one list of places for each sequence of the step")
@@ -159,8 +164,7 @@ class Engine:
                 for p in places:
                     if not (0 <= p < token_lists[i].size):
                         raise StepError(f"slot {slots[i]}: wanted place {p} is outside its {token_lists[i].size} tokens")
-                    want_rows.append(int(starts[i]) + int(p))
-        counts = [int(t.size) for t in token_lists]
+                    want_rows.append(starts[i] + int(p))
         return slots, token_lists, past, counts, want_rows
 
     def prepare(self, entries, want) -> tuple:
@@ -180,7 +184,8 @@ class Engine:
         i, host, dev = self._buffers(layout.total)
         fill_host_buffer(layout, host.numpy(), self.cache, slots, tokens_flat, counts, want_rows)
         dev[:layout.total].copy_(host[:layout.total], non_blocking=True)
-        self._copied[i] = torch.cuda.Event()
+        if self._copied[i] is None:
+            self._copied[i] = torch.cuda.Event()
         self._copied[i].record()
         return dev
 

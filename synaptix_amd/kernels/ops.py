@@ -27,9 +27,14 @@ class KernelError(RuntimeError):
 _scope = threading.local()
 
 
+def _current_stream():
+    """The handle of torch's current stream (0.2 us; through a torch.cuda.Stream made for it 2.8)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+
+
 def _stream():
     held = getattr(_scope, "stream", None)
-    return held if held is not None else ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return held if held is not None else _current_stream()
 
 
 @contextlib.contextmanager
@@ -39,7 +44,7 @@ def stream_scope():
     stream; asking torch each time costs more than the launch).  Scopes nest; code that switches streams
     inside one opens a new one."""
     before = getattr(_scope, "stream", None)
-    _scope.stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _scope.stream = _current_stream()
     try:
         yield
     finally:
@@ -642,6 +647,63 @@ def attention_f32(q, k_pages, v_pages, page_table, tok_seq, tok_pos, out, scale,
     _call(load_library("core"), "syn_attention_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table),
           page_table.shape[1], _ptr(tok_seq), _ptr(tok_pos), _ptr(out), ctypes.c_float(scale), int(window or 0),
           N, nh, nkv, hd, *_score_terms("attention_f32", slopes, softcap, nh), _stream())
+
+
+def _fits(t, dtype, shape) -> bool:
+    return t.dtype is dtype and t.is_cuda and t.shape == shape and t.is_contiguous()
+
+
+def block_f32(resid, delta, norm1, attention, norm2, feed, cache, table, tok_seq, tok_pos, write_kv):
+    """A pre-norm layer of the 32-bit path in one call (csrc/block_f32.hip): add_rmsnorm, gemm, qk_norm_rope_kv_write, attention_f32,
+    gemm, add_rmsnorm, gemm, swiglu, gemm, with the same results.  resid [N, H] gets delta ([N, H] or None) and the attention's result;
+    returns what the feed-forward adds, or None where something is not as these take it (the caller then calls them one by one, and
+    the one that refuses says why).  norm1, norm2: (gain, eps, gain offset); attention: (w_qkv, q_gain, k_gain, eps, gain offset, cos, sin,
+    w_o, scale, window, soft cap, slopes, heads, kv heads, head size); feed: (w_gate_up, w_down, inner width, activation)."""
+    w_qkv, q_gain, k_gain, qk_eps, qk_offset, cos, sin, w_o, scale, window, softcap, slopes, nh, nkv, hd = attention
+    w_gate_up, w_down, inner, activation = feed
+    (gain1, eps1, offset1), (gain2, eps2, offset2) = norm1, norm2
+    N, H = resid.shape
+    k_pages, v_pages = cache
+    pages, width = k_pages.shape[0], table.shape[1]
+    row, gains, rot = (N, H), (_F32, _BF16), 0
+    if not (_fits(resid, _F32, row) and (delta is None or _fits(delta, _F32, row)) and gain1.dtype in gains and gain2.dtype in gains
+            and _fits(gain1, gain1.dtype, (H,)) and _fits(gain2, gain2.dtype, (H,))
+            and _fits(w_qkv, _F32, ((nh + 2 * nkv) * hd, H)) and _fits(w_o, _F32, (H, nh * hd)) and _fits(w_gate_up, _F32, (2 * inner, H))
+            and _fits(w_down, _F32, (H, inner)) and _fits(k_pages, _F32, (pages, nkv, PAGE_TOKENS, hd))
+            and _fits(v_pages, _F32, (pages, nkv, hd, PAGE_TOKENS)) and _fits(table, _I32, (table.shape[0], width))
+            and _fits(tok_seq, _I32, (N,)) and _fits(tok_pos, _I32, (N,)) and hd <= MAX_HEAD_DIM and softcap >= 0.0
+            and (slopes is None or _fits(slopes, _F32, (nh,)))):
+        return None
+    if (q_gain is None) != (k_gain is None) or (cos is None) != (sin is None):
+        return None
+    if q_gain is not None and not (q_gain.dtype in gains and _fits(q_gain, q_gain.dtype, (hd,)) and _fits(k_gain, q_gain.dtype, (hd,))):
+        return None
+    if cos is not None:
+        rot = 2 * cos.shape[1]
+        if rot > hd or not (_fits(cos, _F32, cos.shape) and _fits(sin, _F32, cos.shape)):
+            return None
+    act, limit = _activation_args(activation)
+    lib = _block_lib()
+    work = torch.empty(lib.syn_block_f32_floats(N, H, nh, nkv, hd, inner), dtype=_F32, device=resid.device)
+    out = torch.empty(row, dtype=_F32, device=resid.device)
+    at = lambda t: 0 if t is None else t.data_ptr()
+    words = _BlockWords(at(resid), at(delta), at(out), at(work), at(gain1), at(w_qkv), at(q_gain), at(k_gain), at(cos), at(sin), at(k_pages),
+                        at(v_pages), at(table), at(tok_seq), at(tok_pos), at(slopes), at(w_o), at(gain2), at(w_gate_up), at(w_down),
+                        gain1.dtype is _F32, q_gain is not None and q_gain.dtype is _F32, gain2.dtype is _F32, width, N, H, nh, nkv, hd, rot,
+                        window, bool(write_kv), inner, act)
+    reals = _BlockReals(eps1, offset1, qk_eps, qk_offset, scale, softcap, eps2, offset2, limit.value)
+    _call(lib, "syn_block_f32", words, reals, _stream())
+    return out
+
+
+_BlockWords, _BlockReals = ctypes.c_int64 * 34, ctypes.c_double * 9      # (BlockF32 and its reals)
+
+
+@functools.lru_cache(maxsize=None)
+def _block_lib():
+    lib = load_library("core")
+    lib.syn_block_f32_floats.restype, lib.syn_block_f32_floats.argtypes = ctypes.c_int64, [ctypes.c_int64] * 6
+    return lib
 
 
 def _attn_lib(hd):

@@ -7,8 +7,14 @@ unsummed and takes the previous block's.
 """
 from __future__ import annotations
 
+import torch
+
+from ..kernels import ops
 from .base import Part
+from .feedforward import GatedMlp
 from .linear import as_rows, as_delta
+from .mixer import GqaAttention
+from .norm import RmsNorm
 
 
 class Block(Part):
@@ -83,7 +89,37 @@ class PreNormBlock(Block):
             return delta.scaled(scale)
         return ChannelScaledDeltas([(delta, scale)])
 
+    # what _whole_layer stands for: these parts as they are, not what derives from them or was put in their place
+    _STANDS_FOR = ((RmsNorm, "add_apply", RmsNorm.add_apply), (GqaAttention, "forward", GqaAttention.forward),
+                   (GatedMlp, "forward", GatedMlp.forward))
+
+    def _whole_layer(self, resid, pending, ctx, cache, owner):
+        """The layer in one call of the native library where it is a plain one in 32 bits (the same kernels with the same
+        results; a launch at a time, steps of few tokens wait for the host), or None."""
+        n1, a, n2, f = self.norm1, self.mixer, self.norm2, self.feed_forward
+        if self.scale_prefix is not None or not resid.is_cuda or ops.timing_active() or not (pending is None or isinstance(pending, torch.Tensor)):
+            return None
+        for part, (kind, name, method) in zip((n1, n2, a, f), (self._STANDS_FOR[0],) + self._STANDS_FOR):
+            if type(part) is not kind or getattr(getattr(part, name), "__func__", None) is not method:
+                return None
+        cap = a.position.capacity
+        if f.paired or (cap is not None and ctx.max_position >= cap):
+            return None
+        if any(w.plain is None for w in (a.w_qkv, a.w_o, f.w_gate_up, f.w_down)):
+            return None
+        terms = a._score_terms(resid.device)
+        cos, sin = a.position.tables(resid.device)
+        return ops.block_f32(resid, pending, (n1.gain, n1.eps, n1.gain_offset),
+                             (a.w_qkv.plain, a.q_gain, a.k_gain, a.qk_norm_eps or 0.0, a.qk_gain_offset, cos, sin, a.w_o.plain, a.scale,
+                              a.window or 0, terms["softcap"], terms["slopes"], a.nh, a.nkv, a.hd),
+                             (n2.gain, n2.eps, n2.gain_offset), (f.w_gate_up.plain, f.w_down.plain, f.intermediate, f.activation),
+                             (cache.k_pages, cache.v_pages), ctx.page_table(cache.group), ctx.tok_seq, ctx.tok_pos, owner)
+
     def forward(self, resid, pending, ctx, cache, owner=True):
+        if ctx.act_dtype == torch.float32:
+            out = self._whole_layer(resid, pending, ctx, cache, owner)
+            if out is not None:
+                return out
         # a norm may hand on rows whose last step a product finishes, and take a product that has not been run
         # (parts.linear.ScaledRows, DeferredProduct); parts that do not say they take them get plain tensors
         h = self.norm1.add_apply(resid, _norm_input(self.norm1, pending), ctx.act_dtype)

@@ -726,3 +726,40 @@ def test_toy_block_arrangement_and_toy_norm_register_build_and_step(tmp_path):
         cut = [eng.step([(a, ids[:5])], want="all"), eng.step([(a, ids[5:9])], want="all")]
         cut += [eng.step([(a, [tok])], want="last") for tok in ids[9:]]
         assert (torch.cat(cut).cpu() - whole).abs().max() <= (1e-4 if dtype == "float32" else 5e-2 * max(1.0, float(whole.abs().max())))
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(num_key_value_heads=1, head_dim=6), dict(hidden_size=66, intermediate_size=50, head_dim=34)])
+def test_a_plain_32_bit_layer_in_one_call_gives_what_its_parts_give(kw, monkeypatch):
+    """Prompts, a portion behind them and single tokens through the layers' one call, and through their parts one by one: the same
+    bits.  A part that derives from a plain one, or whose method was replaced, runs as it is."""
+    from synaptix_amd import Engine, Qwen3Config
+    from synaptix_amd.parts import GatedMlp, PreNormBlock
+    cfg = Qwen3Config(**dict(dict(vocab_size=300, hidden_size=64, intermediate_size=176, num_hidden_layers=2, num_attention_heads=4,
+                                  num_key_value_heads=2, head_dim=16, max_position_embeddings=256, rope_theta=1e4, rms_norm_eps=1e-6,
+                                  tie_word_embeddings=False, eos_token_id=None), **kw))
+    eng = Engine.from_config(cfg, seed=3, dtype="float32", max_tokens=1024)
+    g = torch.Generator().manual_seed(5)
+    steps = [[torch.randint(0, 300, (n,), generator=g).tolist() for n in lens] for lens in ((5, 70, 131), (1, 40, 1), (1, 1, 1))]
+
+    def run():
+        slots = [eng.acquire() for _ in range(3)]
+        out = [eng.step(list(zip(slots, s)), want="all").cpu() for s in steps]
+        [eng.release(s) for s in slots]
+        return out
+    whole, calls = run(), []
+    one = PreNormBlock._whole_layer
+    monkeypatch.setattr(PreNormBlock, "_whole_layer", lambda *a: (calls.append(one(*a)), calls[-1])[1])
+    assert all(torch.equal(a, b) for a, b in zip(run(), whole)) and len(calls) == 6 and all(c is not None for c in calls)
+    monkeypatch.setattr(PreNormBlock, "_whole_layer", lambda *a: None)
+    assert all(torch.equal(a, b) for a, b in zip(run(), whole))
+    monkeypatch.setattr(PreNormBlock, "_whole_layer", one)
+
+    class Twice(GatedMlp):
+        def forward(self, h, ctx):
+            return 2 * super().forward(h, ctx)
+    eng.model.blocks[1].feed_forward.__class__ = Twice
+    other = run()
+    assert not torch.equal(other[0], whole[0])
+    eng.model.blocks[1].feed_forward.__class__ = GatedMlp
+    eng.model.blocks[1].feed_forward.forward = lambda h, ctx: 2 * GatedMlp.forward(eng.model.blocks[1].feed_forward, h, ctx)
+    assert all(torch.equal(a, b) for a, b in zip(run(), other))
