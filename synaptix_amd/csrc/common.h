@@ -223,9 +223,10 @@ __device__ __forceinline__ void buffer_to_lds16(const BufferView& v, void* lds, 
 // loads and stores through a view; a lane whose offset lies beyond its end gets zeros, and stores nothing
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+template <bool STREAMED = false>
 __device__ __forceinline__ bf16x8 buffer_load16(const BufferView& v, unsigned off) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(v.r, off, 0, 0));
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(v.r, off, 0, STREAMED ? 2 : 0));
 #else
   return bf16x8{};
 #endif

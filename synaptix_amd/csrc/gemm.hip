@@ -976,6 +976,161 @@ static int launch_direct(const bf16* x, Weight w, void* out, Epilogue ep, int M,
   return 0;
 }
 
+// ------------------------------------------------------------------ 17 to 128 rows, W in fragment order: operands straight to registers
+// What bounds it: the stream of W, of which a compute unit has to keep some 64 KB under way.  Through a ring of LDS buffers W shares
+// the room with x (36 KB of it under way beside 96 rows of x), and every k-tile ends in a barrier.  Here the four waves of a workgroup
+// (one a SIMD, all 512 registers) split K, and each takes all rows of x and all 16 NF rows of W of the workgroup: a fragment of
+// either is loaded once a workgroup, straight into the registers of the one wave that multiplies it, S steps of 32 k-values ahead;
+// no barrier and no LDS until the waves' sums are added at the end, in the order of the waves.  x comes from the L2s, as many
+// bytes as W with 16 NF rows of it.
+// W: a step's fragment is 1 KB of consecutive bytes; x: 16 rows of 64 bytes, the two steps of a 128-byte line asked for together.
+// A wave takes every fourth pair of steps.  Rows of x beyond M, rows of W beyond N and steps beyond the slice lie behind the views'
+// ends: zeros without traffic.  D[n = 4 (lane / 16) + e][m = lane % 16] of fragments (n, m).
+template <int NF, int FM, int S, bool PAIRED>
+__global__ void __launch_bounds__(256, 1)
+gemm_rows_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void* __restrict__ out, Epilogue ep, int M, int N, int K,
+                 int k_slice) {
+  static_assert(NF % 2 == 0 && S % 2 == 0, "fragments of W in pairs (gate and up), steps in pairs (a line of x)");
+  constexpr int FRAGS = NF * FM, CHUNK = FRAGS <= 36 ? FRAGS : FRAGS / 2;      // fragments of sums that pass through LDS at a time
+  static_assert(FRAGS % CHUNK == 0 && CHUNK % 2 == 0 && CHUNK <= 36, "the waves' sums in LDS");
+  extern __shared__ f32x4 part[];      // [4][CHUNK][64]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE), lane = threadIdx.x % SYN_WAVE, r16 = lane % 16, g = lane / 16;
+  const int n0 = (int)blockIdx.x * 16 * NF, k_begin = (int)blockIdx.y * k_slice;
+  const int pairs = max(0, min(K - k_begin, k_slice)) / 64, steps = 2 * max(0, (pairs - wave + 3) / 4);
+  const size_t row_bytes = (size_t)K * sizeof(bf16);
+  const BufferView vw = buffer_view(wp + (size_t)n0 * K, (size_t)(N - n0) * row_bytes), vx = buffer_view(x, (size_t)M * row_bytes);
+  const unsigned w_frag = (unsigned)(16 * row_bytes);
+  const unsigned w_at = (unsigned)(k_begin / 32 + 2 * wave) * 1024 + lane * 16, x_at = (unsigned)(r16 * row_bytes) + (k_begin + 64 * wave + 8 * g) * 2;
+  bf16x8 wf[S][NF], xf[S][FM];
+  f32x4 acc[NF][FM];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // step s of this wave: pair wave + 4 (s / 2), half s % 2
+  auto load_w = [&](int s, bf16x8 (&f)[NF]) {
+    const unsigned at = w_at + (unsigned)((s / 2) * 8 + s % 2) * 1024;
+#pragma unroll
+    for (int i = 0; i < NF; ++i) f[i] = buffer_load16<true>(vw, s < steps ? at + i * w_frag : SYN_NOWHERE);
+  };
+  auto load_x = [&](int s, bf16x8 (&f)[FM]) {
+    const unsigned at = x_at + (unsigned)((s / 2) * 256 + (s % 2) * 32) * 2;
+#pragma unroll
+    for (int j = 0; j < FM; ++j) f[j] = buffer_load16(vx, s < steps ? at + j * w_frag : SYN_NOWHERE);
+  };
+#pragma unroll
+  for (int s = 0; s < S; s += 2) {
+    // (in this order: the loop waits for no load that is younger than those it takes, on any way into it)
+    load_w(s, wf[s]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_x(s, xf[s]), load_x(s + 1, xf[s + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(s + 1, wf[s + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int s0 = 0; s0 < steps; s0 += S) {
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+#pragma unroll
+      for (int i = 0; i < NF; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[u][i]), "v"(xf[u][j]));
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(s0 + S + u, wf[u]);
+      if (u % 2 == 1) load_x(s0 + S + u - 1, xf[u - 1]), load_x(s0 + S + u, xf[u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // (the compiler does not know the matrix instructions for what they are: their results are waited for by hand)
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+  for (int c = 0; c < FRAGS / CHUNK; ++c) {
+    // fragment f: rows 2 (f / 2 / FM) + f % 2 of W (gate and up side by side), rows f / 2 % FM of x
+    if (c) __syncthreads();
+#pragma unroll
+    for (int f = 0; f < CHUNK; ++f) {
+      const int q = (c * CHUNK + f) / 2;
+      part[(wave * CHUNK + f) * SYN_WAVE + lane] = acc[2 * (q / FM) + f % 2][q % FM];
+    }
+    __syncthreads();
+    for (int q = wave; q < CHUNK / 2; q += 4) {
+      f32x4 v[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        v[h] = part[(2 * q + h) * SYN_WAVE + lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) v[h] += part[(w * CHUNK + 2 * q + h) * SYN_WAVE + lane];
+      }
+      const int pair = c * CHUNK / 2 + q, m = 16 * (pair % FM) + r16, n = n0 + 32 * (pair / FM) + 4 * g;
+      if (m >= M) continue;
+      if constexpr (PAIRED) {
+        bf16x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = (bf16)gated(ep.act, v[0][e], v[1][e], ep.limit);
+        const int col = n0 / 2 + 16 * (pair / FM) + 4 * g;
+        if (n < N) *(bf16x4*)((bf16*)out + (size_t)m * (N / 2) + col) = r;
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (n + 16 * h >= N) continue;
+          const size_t at = ((size_t)blockIdx.y * M + m) * N + n + 16 * h;
+          f32x4 o;
+          bf16x4 r;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = point_activation(ep.point, v[h][e]), r[e] = (bf16)o[e];
+          if (ep.out_is_f32) *(f32x4*)((float*)out + at) = o;
+          else *(bf16x4*)((bf16*)out + at) = r;
+        }
+      }
+    }
+  }
+}
+
+template <int NF, int FM, int S, bool PAIRED>
+static int launch_rows_tile(const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K, int slices, hipStream_t stream) {
+  constexpr int CHUNK = NF * FM <= 36 ? NF * FM : NF * FM / 2, LDS = 4 * CHUNK * SYN_WAVE * 16;
+  static OncePerDevice raised;
+  const hipError_t e = once_per_device(raised, [&] {
+    return hipFuncSetAttribute((const void*)gemm_rows_kernel<NF, FM, S, PAIRED>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  });
+  SYN_CHECK(e == hipSuccess, "gemm: %d bytes of LDS refused: %s", LDS, hipGetErrorString(e));
+  const int k_slice = ((K / 64 + slices - 1) / slices) * 64;
+  gemm_rows_kernel<NF, FM, S, PAIRED><<<dim3((N + 16 * NF - 1) / (16 * NF), slices), 256, LDS, stream>>>(x, wp, out, ep, M, N, K, k_slice);
+  return 0;
+}
+// nf: 16-row groups of W a workgroup (2, 4 or 6), picked by the host's rule (ops.rows_tile).  Deeper where few rows of x leave room; six
+// groups beside more than 48 rows of x, or four beside more than 96, do not fit the registers with nothing moved between them.
+template <bool PAIRED>
+static int launch_rows(int nf, const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K, int slices, hipStream_t stream) {
+  SYN_CHECK(M <= (nf == 6 ? 48 : nf == 4 ? 96 : 128) && (nf == 2 || nf == 4 || nf == 6) && K % 64 == 0 && N % (PAIRED ? 32 : 16) == 0 &&
+            (size_t)K * 2 * 128 < 0x7fffffffull, "gemm: %d rows beside %d x 16 of W, N = %d, K = %d", M, nf, N, K);
+#define SYN_ROWS(NF, FM, S) return launch_rows_tile<NF, FM, S, PAIRED>(x, wp, out, ep, M, N, K, slices, stream)
+  if (nf == 6) {
+    if (M <= 16) SYN_ROWS(6, 1, 8);
+    if (M <= 32) SYN_ROWS(6, 2, 6);
+    SYN_ROWS(6, 3, 4);
+  }
+  if (nf == 4) {
+    if (M <= 16) SYN_ROWS(4, 1, 8);
+    if (M <= 32) SYN_ROWS(4, 2, 6);
+    if (M <= 48) SYN_ROWS(4, 3, 6);
+    if (M <= 64) SYN_ROWS(4, 4, 6);
+    SYN_ROWS(4, 6, 4);
+  }
+  if (M <= 16) SYN_ROWS(2, 1, 8);
+  if (M <= 32) SYN_ROWS(2, 2, 6);
+  if (M <= 48) SYN_ROWS(2, 3, 6);
+  if (M <= 64) SYN_ROWS(2, 4, 6);
+  if (M <= 96) SYN_ROWS(2, 6, 4);
+  SYN_ROWS(2, 8, 4);
+#undef SYN_ROWS
+}
+
 // ------------------------------------------------------------------ tiled, M > 64: one stream of k-steps over all tiles
 // What bounds it: the matrix units, and under random operands the power that they draw (a product of zeros of
 // 2,048 x 24,576 x 4,096 takes 209 us, of random numbers 278).  The kernel therefore spends as little as it can on
@@ -1386,7 +1541,7 @@ SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
 // point: what the finished sums pass before they are stored (point_activation; one slice).
 // tile: -1, or for tests and measurements one of STREAM_TILES, whatever the rules below would take (bf16 operands).
 SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int M, int N, int K, int force_simt,
-                        int slices, int w_packed, int point, int tile, hipStream_t stream) {
+                        int slices, int w_packed, int point, int tile, int rows, hipStream_t stream) {
   SYN_CHECK(tile < 0 || (dtype != 0 && !force_simt && K % 64 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0),
             "gemm: the streamed tiles take aligned bf16 operands and a K that is a multiple of 64 (K = %d)", K);
   SYN_CHECK(point >= 0 && point < SYN_POINT_COUNT && (point == SYN_POINT_NONE || slices == 1),
@@ -1447,6 +1602,8 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   int rc = 0;
   if (tile >= 0) {
     rc = launch_large<false>(xb, wt, out, ep, M, N, K, stream, slices, tile);
+  } else if (rows && w_packed) {
+    rc = launch_rows<false>(rows, xb, wb, out, ep, M, N, K, slices, stream);
   } else if (M == 1 && slices == 1 && !w_packed) {
     // one row: fragments of W straight from memory, K split over the waves
     if (N <= 8192) launch_skinny<1, 16, 4>(xb, wb, out, ep, M, N, K, stream);
@@ -1489,9 +1646,9 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
 // out[M, N/2] = silu(x . Wg^T) * (x . Wu^T), bf16, where w [N, K] holds the rows of Wg and of Wu in
 // turns of 16: rows 32b .. 32b+15 are rows 16b .. 16b+15 of Wg, rows 32b+16 .. 32b+31 those of Wu.
 // The activation is applied to the 32-bit sums and rounded once.
-// w_packed, tile: as for syn_gemm
+// w_packed, tile, rows: as for syn_gemm
 SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, int N, int K, int act, float limit,
-                               int w_packed, int tile, hipStream_t stream) {
+                               int w_packed, int tile, int rows, hipStream_t stream) {
   SYN_CHECK(tile < 0 || K % 64 == 0, "gemm_swiglu: the streamed tiles take a K that is a multiple of 64 (K = %d)", K);
   SYN_CHECK(M > 0 && N > 0 && K > 0, "gemm_swiglu: empty shape M=%d N=%d K=%d", M, N, K);
   SYN_CHECK(!w_packed || K % 128 == 0, "gemm_swiglu: a weight in fragment order needs K = %d a multiple of 128", K);
@@ -1506,6 +1663,8 @@ SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, i
   const Weight wt = {wb, w_packed != 0};
   if (tile >= 0) {
     rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream, 1, tile);
+  } else if (rows && w_packed) {
+    rc = launch_rows<true>(rows, xb, wb, out, ep, M, N, K, 1, stream);
   } else if (M == 1 && !w_packed) {
     // one row: fragments of W straight from memory; eight waves on the gate rows, eight on the up rows
     launch_skinny<2, 8, 4, true>(xb, wb, out, ep, M, N, K, stream);

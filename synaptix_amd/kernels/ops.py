@@ -277,7 +277,7 @@ def point_code(name) -> int:
     return POINT_ACTIVATIONS[name]
 
 
-def gemm(x, w, out, force_simt=False, point=None, tile=-1):
+def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
     """out[M, N] = x[M, K] . w[N, K]^T with 32-bit accumulation.
     float x float -> float; bf16 x bf16 -> bf16 or float (MFMA, plain FMA for shapes it does not take).
     A float out of shape [S, M, N] (bf16 operands) receives S partial sums over slices of K
@@ -285,7 +285,8 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1):
     w may be the weight in fragment order (pack_weight: four dimensions): the tiles for 9 rows and more read it
     where K is a multiple of 128; for other K the product runs in blocks of 16 rows through gemm_packed.
     point: a name of POINT_ACTIVATIONS, applied to the finished sums before they are stored (not to partial sums).
-    tile: for tests and measurements, a streamed tile of csrc/gemm.hip by its number whatever the rules there would take."""
+    tile: for tests and measurements, a streamed tile of csrc/gemm.hip by its number whatever the rules there would take.
+    rows: rows_tile of the sizes (with a weight in fragment order), or 0 for the tiles that plain rows take as well."""
     point_of = point_code(point)
     _need(x, "gemm.x", (_BF16, _F32), (None, None))
     M, K = x.shape
@@ -323,7 +324,72 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1):
         _need(out, "gemm.out", (_BF16, _F32), (M, N))
         code = 2 if out.dtype == _F32 else 1
     _call(load_library("core"), "syn_gemm", _ptr(x), _ptr(w), _ptr(out), code, M, N, K, 1 if force_simt else 0,
-          slices, 1 if packed else 0, point_of, tile, _stream())
+          slices, 1 if packed else 0, point_of, tile, rows, _stream())
+
+
+# Products of up to this many rows over a weight in fragment order may take the kernel whose operands go straight to registers
+# (gemm_rows_kernel in csrc/gemm.hip).
+ROWS_MAX = 128
+
+
+def _bytes_a_unit(M, tile, K, slices, tiles, units, shared):
+    """What a compute unit has to bring in, a workgroup holding `tile` rows of W beside all M rows of x over a slice of K, and its share
+    of the partial sums that are written and read again; shared: workgroups share a compute unit (else they come in rounds)."""
+    wgs = tiles * slices
+    rounds = max(1.0, wgs / units) if shared else -(-wgs // units)
+    return rounds * (tile + M) * (-(-K // (64 * slices)) * 64) * 2 + (8 * slices * M * tile * tiles / units if slices > 1 else 0)
+
+
+def _rows_choice(M, N, K, slices, gated):
+    """(bytes a compute unit, groups of 16 rows of W a workgroup, slices of K) of gemm_rows_kernel for a product in `slices` slices (None:
+    the best), its workgroups going round once; None where it does not."""
+    units, best = compute_units(), None
+    for nf in (2, 4, 6):
+        if M > {2: 128, 4: 96, 6: 48}[nf]:
+            continue
+        tiles = -(-N // (16 * nf))
+        for s in (range(1, 9) if slices is None else (slices,)):
+            if tiles * s <= units and (s == 1 or K >= 512 * s):
+                cost = (_bytes_a_unit(M, 16 * nf, K, s, tiles, units, False), nf, s)
+                best = cost if best is None or cost < best else best
+    return best
+
+
+def _tiles_bytes(M, N, K, slices, gated):
+    """The same of the tiles that gemm_direct_kernel takes."""
+    tile = 64 if M <= 32 else 96 if gated and M > 64 else 128
+    return _bytes_a_unit(M, tile, K, slices, -(-N // tile), compute_units(), M <= 32)
+
+
+def _rows_pay(new, old, M, gated):
+    """Both are bound by the bytes that a compute unit brings in, W's stream and x from the L2s; through a ring of LDS buffers they come
+    in a little faster from 33 rows of x on, where the registers hold fewer steps.  Measured, us (this kernel, tiles, ratio of the
+    bytes): gated 24,576 x 4,096 with 24 rows 39.2, 43.7, 0.91, with 48 42.4, 43.0, 0.82, with 64 46.3, 45.7; 16,384 x 2,048 with 64 20.5,
+    22.7, 0.67, with 128 28.7, 27.5, 0.86; 8,192 x 1,024 with 128 14.3, 17.8, 0.71; plain 2,560 x 9,728 with 24 11.9, 15.1, 0.68, with
+    64 17.0, 16.3, 0.85; 6,144 x 2,560 with 32 9.7, 10.2, 0.9; 4,096 x 12,288 with 32 20.5, 19.6, 1.0; 2,048 x 2,048 with 48 5.8, 7.5, 0.45, with
+    128 9.2, 10.6, 0.63; 1,024 x 4,096 with 96 7.8, 10.2, 0.57; 6,144 x 2,048 with 48 10.1, 9.5, 0.82."""
+    return new <= (0.95 if M <= 32 and gated else 0.9 if M <= 32 else 0.75 if gated else 0.65) * old
+
+
+@functools.lru_cache(maxsize=4096)
+def rows_tile(M, N, K, slices, gated=False) -> int:
+    """Groups of 16 rows of W that a workgroup of gemm_rows_kernel takes for this product in so many slices, 0: it takes other tiles."""
+    if M > ROWS_MAX or M <= (PACKED_MAX_ROWS_GATED if gated else PACKED_MAX_ROWS) or K % 128 or N % 16:
+        return 0
+    new = _rows_choice(M, N, K, slices, gated)
+    if new is None or slices > 1 and slices != rows_slices(M, N, K):
+        return 0
+    return new[1] if slices > 1 or _rows_pay(new[0], _tiles_bytes(M, N, K, 1, gated), M, gated) else 0
+
+
+@functools.lru_cache(maxsize=4096)
+def rows_slices(M, N, K) -> int:
+    """Into how many slices of K a plain product over a weight in fragment order is cut for gemm_rows_kernel, 0: it takes other tiles (and
+    the slices of gemm_slices)."""
+    if M > ROWS_MAX or M <= PACKED_MAX_ROWS or K % 128 or N % 16:
+        return 0
+    new = _rows_choice(M, N, K, None, False)
+    return new[2] if new is not None and _rows_pay(new[0], _tiles_bytes(M, N, K, gemm_slices(M, N, K, _BF16), False), M, False) else 0
 
 
 PAIR = 16   # rows of the gate and of the up projection alternate in turns of this many
@@ -337,10 +403,10 @@ def pair_rows(gate, up):
     return torch.stack([gate.view(I // PAIR, PAIR, K), up.view(I // PAIR, PAIR, K)], 1).reshape(2 * I, K).contiguous()
 
 
-def gemm_swiglu(x, w_paired, out, activation="silu", tile=-1):
+def gemm_swiglu(x, w_paired, out, activation="silu", tile=-1, rows=0):
     """out[M, I] = act(x . Wg^T) * (x . Wu^T) in bf16 with w_paired = pair_rows(Wg, Wu): the
     activation on the 32-bit sums inside the product, so that the two products are never stored.
-    w_paired may be in fragment order (pack_weight of the paired rows), as for gemm; tile: as there."""
+    w_paired may be in fragment order (pack_weight of the paired rows), as for gemm; tile, rows: as there."""
     _need(x, "gemm_swiglu.x", _BF16, (None, None))
     M, K = x.shape
     packed = isinstance(w_paired, torch.Tensor) and w_paired.dim() == 4
@@ -358,7 +424,7 @@ def gemm_swiglu(x, w_paired, out, activation="silu", tile=-1):
                         activation=activation)
         return
     _call(load_library("core"), "syn_gemm_swiglu", _ptr(x), _ptr(w_paired), _ptr(out), M, N, K,
-          *_activation_args(activation), 1 if packed else 0, tile, _stream())
+          *_activation_args(activation), 1 if packed else 0, tile, rows, _stream())
 
 
 PACKED_BLOCK_ROWS = 16   # the most rows that a product of gemm_packed takes

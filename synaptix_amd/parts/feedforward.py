@@ -10,7 +10,7 @@ import torch
 from ..kernels import ops
 from ..weights.source import TensorSpec
 from .base import Part
-from .linear import Matrix, linear, linear_for_sum, deferred_product, as_rows, ScaledRows
+from .linear import Matrix, linear, linear_for_sum, deferred_product, as_rows, rows_kernel, ScaledRows
 
 
 class FeedForward(Part):
@@ -65,7 +65,8 @@ class GatedMlp(FeedForward):
                 else:
                     ops.gemm_packed(h, self.w_gate_up.packed, m, paired=True, activation=self.activation)
             else:
-                ops.gemm_swiglu(as_rows(h), self.w_gate_up.data, m, self.activation)
+                h = as_rows(h)
+                ops.gemm_swiglu(h, self.w_gate_up.data, m, self.activation, **rows_kernel(h, self.w_gate_up, gated=True))
         else:
             h = as_rows(h)
             ops.swiglu(linear(h, self.w_gate_up, h.dtype), m, self.activation)

@@ -39,6 +39,14 @@ def _use_packed(x, m):
     return m.packed is not None and x.dtype == torch.bfloat16 and x.shape[0] <= ops.packed_max_rows(m.shape[0])
 
 
+def rows_kernel(x, w, slices=1, gated=False) -> dict:
+    """What ops.gemm and ops.gemm_swiglu are told beside the operands where few rows meet a weight in fragment order (ops.rows_tile)."""
+    if w.packed is None or x.shape[0] > ops.ROWS_MAX or x.dtype != torch.bfloat16 or not x.is_cuda:
+        return {}
+    rows = ops.rows_tile(x.shape[0], *w.shape, slices, gated)
+    return {"rows": rows} if rows else {}
+
+
 def _matrix(w):
     """The products below take a Matrix; a tensor [N, K] in plain rows is taken as it is."""
     return w if isinstance(w, Matrix) else Matrix(w, keep_rows=True)
@@ -233,7 +241,7 @@ def linear(x, w, out_dtype, point=None):
             raise TypeError(f"linear: activation {x.dtype} with weight {w.dtype}")
     out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32 if x.dtype == torch.float32 else out_dtype,
                       device=x.device)
-    ops.gemm(x, w.data, out, point=point)
+    ops.gemm(x, w.data, out, point=point, **rows_kernel(x, w))
     return out if out.dtype == out_dtype else out.to(out_dtype)
 
 
@@ -241,6 +249,10 @@ def product_slices(n_rows, w, dtype) -> int:
     """Into how many slices of K the product of n_rows rows with w is cut for a reader that adds partial sums."""
     if w.dtype != dtype or (w.packed is not None and w.shape[1] % 128):
         return 1            # (in fragment order the tiles for many rows take a K that is a multiple of 128 only)
+    if w.packed is not None and dtype == torch.bfloat16 and n_rows <= ops.ROWS_MAX and w.device.type == "cuda":
+        slices = ops.rows_slices(n_rows, *w.shape)
+        if slices:
+            return slices
     return ops.gemm_slices(n_rows, w.shape[0], w.shape[1], dtype)
 
 
@@ -272,5 +284,5 @@ def linear_for_sum(x, w):
     if slices <= 1:
         return linear(x, w, torch.float32)
     out = torch.empty((slices, M, w.shape[0]), dtype=torch.float32, device=x.device)
-    ops.gemm(x, w.data, out)
+    ops.gemm(x, w.data, out, **rows_kernel(x, w, slices))
     return out

@@ -1452,6 +1452,48 @@ def test_attention_of_random_shapes(ops):
                                               r.choice([0, 0, 2, 4, 8]), r.random() < 0.8)
 
 
+@pytest.mark.parametrize("nf", [2, 4, 6])
+@pytest.mark.parametrize("M", [9, 16, 17, 33, 48, 49, 64, 65, 96, 97, 128])
+def test_products_of_few_rows_straight_to_registers(ops, nf, M):
+    """gemm_rows_kernel by the number of its rows of W, wherever that many rows of x fit: N that is no multiple of a workgroup's rows, K whose
+    pairs of steps do not divide by four waves nor by the slices (some empty), every output, against 64 bits at every place.  The
+    bounds: 32-bit sums of K products of bf16 numbers, 2^-8 of a result that is rounded."""
+    if M > {2: 128, 4: 96, 6: 48}[nf]:
+        pytest.skip("not compiled: more sums than registers")
+    for N, K, slices in ((32, 128, 1), (224, 640, 1), (208, 384, 2), (1008, 2176, 3), (96, 1024, 8), (16, 256, 5)):
+        x, w = rnd((M, K), M + K, BF16), rnd((N, K), N + K, BF16, 0.05)
+        full, wp = x.double() @ w.double().T, ops.pack_weight(w.to(DEV))
+        bound = 2 ** -24 * 8 * math.sqrt(K) + 2 ** -22 * (x.double().abs() @ w.double().abs().T)
+        for dt in (F32, BF16) if slices == 1 else (F32,):
+            out = torch.full((slices, M, N) if slices > 1 else (M, N), float("nan"), dtype=dt, device=DEV)
+            ops.gemm(x.to(DEV), wp, out, rows=nf)
+            got = (out.double().sum(0) if slices > 1 else out.double()).cpu()
+            assert bool(((got - full).abs() <= bound + (2 ** -8 * full.abs() if dt == BF16 else 0)).all()), (N, K, slices, dt)
+        if slices == 1:
+            out = torch.full((M, N), float("nan"), device=DEV)
+            ops.gemm(x.to(DEV), wp, out, point="relu_squared", rows=nf)
+            assert bool(((out.cpu().double() - full.clamp(min=0) ** 2).abs() <= 2 * full.abs() * bound + bound ** 2 + 2 ** -22 * full ** 2).all())
+        if N % 32 == 0 and slices == 1:
+            paired = ops.pack_weight(ops.pair_rows(w[:N // 2].contiguous(), w[N // 2:].contiguous()).to(DEV))
+            out = torch.full((M, N // 2), float("nan"), dtype=BF16, device=DEV)
+            ops.gemm_swiglu(x.to(DEV), paired, out, rows=nf)
+            g, u = full[:, :N // 2], full[:, N // 2:]
+            want = g * torch.sigmoid(g) * u
+            assert bool(((out.cpu().double() - want).abs() <= 2 ** -7 * want.abs() + 4 * bound.amax() * (1 + u.abs() + g.abs())).all()), (N, K)
+
+
+def test_the_rule_for_products_of_few_rows_gives_sizes_that_run(ops):
+    """Whatever the sizes, what the rule picks goes round once, fits the registers and leaves every slice work of its own."""
+    for M in range(1, 140, 3):
+        for N in (16, 48, 1024, 2560, 4096, 6144, 9728, 24576, 51200):
+            for K in (128, 1024, 2560, 4096, 9728, 25600):
+                for gated in (False, True):
+                    s = 1 if gated else max(1, ops.rows_slices(M, N, K))
+                    nf = ops.rows_tile(M, N, K, s, gated)
+                    assert nf == 0 or (M <= {2: 128, 4: 96, 6: 48}[nf] and -(-N // (16 * nf)) * s <= ops.compute_units() and (s == 1 or K >= 512 * s))
+                    assert nf or s == 1
+
+
 def _filter(ops, x, options, ids=None, in_place=False):
     """ops.filter_rows over rows x [R, V] with options = list of dicts (k, p, mp, T, rep, pres, freq) and ids = list of lists."""
     R, V = x.shape

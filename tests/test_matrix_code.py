@@ -1,7 +1,8 @@
 """The streamed products and latent attention's prompts issue their matrix instructions as inline assembly: the compiler does not
 know them for matrix instructions and would read a sum right behind one without the wait that takes.  So in the streamed
-products no sum may be moved between a kernel's first matrix instruction and the wait behind its last, and in all three no
-vector instruction may come too close: read from the assembly of these sources."""
+products no sum may be moved between a kernel's first matrix instruction and the wait behind its last, and in all of them (the
+products of few rows whose operands go straight to registers among them) no vector instruction may come too close: read from
+the assembly of these sources."""
 
 import functools
 import os
@@ -57,7 +58,7 @@ def registers(operand):
     return {(m[4], int(m[5]))} if m[4] else {(m[1], k) for k in range(int(m[2]), int(m[3]) + 1)}
 
 
-@pytest.mark.parametrize("source,kernel", STREAMED + [("latent_attention.hip", "latent_prompt_bf16_kernel")])
+@pytest.mark.parametrize("source,kernel", STREAMED + [("gemm.hip", "gemm_rows_kernel"), ("latent_attention.hip", "latent_prompt_bf16_kernel")])
 def test_vector_instructions_keep_away_from_matrix_instructions(source, kernel, folder):
     """No vector instruction may write what a matrix instruction reads one or two states later, nor touch a result within
     eighteen of its start (latent attention mixes both on every page; the streamed products at the ends of their tiles)."""
