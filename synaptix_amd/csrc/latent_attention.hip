@@ -499,9 +499,18 @@ latent_attention_merge_kernel(const float* __restrict__ part_o, const float* __r
   bf16* orow = out + ((size_t)(start + flat / nh) * nh + flat % nh) * rank;
   for (int d = threadIdx.x; d < rank; d += blockDim.x) {
     float o = 0.f;
-    for (int s = 0; s < n_splits; ++s) {
-      const float f = factor[s];
-      if (f != 0.f) o += f * part_o[(at0 + (size_t)s * LA_ROWS) * rank + d];
+    // eight splits' values on their way together, added in their order (8 rows of 32 heads, 42 splits: 12.2 ->
+    // 6.8 us); a split without keys
+    // weighs nothing and may hold anything
+    for (int s0 = 0; s0 < n_splits; s0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part_o[(at0 + (size_t)min(s0 + u, n_splits - 1) * LA_ROWS) * rank + d];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float f = s0 + u < n_splits ? factor[s0 + u] : 0.f;
+        if (f != 0.f) o += f * v[u];
+      }
     }
     orow[d] = (bf16)(o / l);
   }

@@ -344,6 +344,8 @@ def _rows_choice(M, N, K, slices, gated):
     """(bytes a compute unit, groups of 16 rows of W a workgroup, slices of K) of gemm_rows_kernel for a product in `slices` slices (None:
     the best), its workgroups going round once; None where it does not."""
     units, best = compute_units(), None
+    if N * K < 1 << 19:      # (less than 1 MB of W: a launch's time whatever the tiles)
+        return None
     for nf in (2, 4, 6):
         if M > {2: 128, 4: 96, 6: 48}[nf]:
             continue
@@ -1657,11 +1659,12 @@ ROUTE_MAX_EXPERTS, ROUTE_MAX_TOP = 1024, 64
 
 
 def route_topk(logits, bias, ids, weights):
-    """The choice of a mixture's router: logits [N, E] float (the 32-bit sums of the router's product) + bias [E];
-    ids [N, top] int32 the experts with the largest logits (largest first, the lower index of equal ones), weights
+    """The choice of a mixture's router: logits [N, E] float (the 32-bit sums of the router's product, or partial sums [S, N, E] of
+    them, which are added here) + bias [E]; ids [N, top] int32 the experts with the largest logits (largest first, the lower index of equal ones), weights
     [N, top] float the softmax over those logits alone."""
-    _need(logits, "route_topk.logits", _F32, (None, None))
-    N, E = logits.shape
+    parts = logits.shape[0] if isinstance(logits, torch.Tensor) and logits.dim() == 3 else 1
+    _need(logits, "route_topk.logits", _F32, (None, None) if parts == 1 and logits.dim() != 3 else (parts, None, None))
+    N, E = logits.shape[-2:]
     if bias is not None:
         _need(bias, "route_topk.bias", _F32, (E,))
     _need(ids, "route_topk.ids", _I32, (N, None))
@@ -1669,7 +1672,7 @@ def route_topk(logits, bias, ids, weights):
     _need(weights, "route_topk.weights", _F32, (N, top))
     if not (0 < top <= min(E, ROUTE_MAX_TOP)) or E > ROUTE_MAX_EXPERTS:
         raise KernelError(f"route_topk: the {top} largest of {E} experts (at most {ROUTE_MAX_TOP} of {ROUTE_MAX_EXPERTS})")
-    _call(load_library("core"), "syn_route_topk", _ptr(logits), _ptr(bias), _ptr(ids), _ptr(weights), N, E, top, _stream())
+    _call(load_library("core"), "syn_route_topk", _ptr(logits), _ptr(bias), _ptr(ids), _ptr(weights), N, E, top, parts, _stream())
 
 
 def route_sort(ids, weights, n_experts):

@@ -235,7 +235,10 @@ class RoutedExperts(FeedForward):
         N, dev = h.shape[0], h.device
         ids = torch.empty((N, self.top), dtype=torch.int32, device=dev)
         weights = torch.empty((N, self.top), dtype=torch.float32, device=dev)
-        logits = linear(h, self.w_router, torch.float32)
+        # (few rows of W: the choice adds the sums over slices of K itself; 1,500 tokens, 48 experts of 4,096: 25 -> 8.2 us, the
+        # choice 9 -> 11)
+        takes_parts = self.router == "top_logits" and self.shared_gate is None and h.dtype == self.w_router.dtype
+        logits = (linear_for_sum if takes_parts else linear)(h, self.w_router, *(() if takes_parts else (torch.float32,)))
         shared_gate = None
         if self.shared_gate is not None:
             logits, shared_gate = logits[:, :self.total], logits[:, self.total:self.total + 1]

@@ -652,3 +652,30 @@ def test_command_line_and_trace_replay_as_a_user_starts_them(tmp_path):
             want = plain.forward(toks)
             rows = np.stack([got[where[(rid, p)][0]][where[(rid, p)][1]] for p in range(len(toks))])
             assert_logits_close(rows, want, dtype, f"trace_run {dtype} request {rid}", sharp=False)
+
+
+@pytest.mark.parametrize("N,top,E", [(1, 1, 1), (1025, 1, 3), (171, 6, 48), (3000, 6, 48), (20000, 8, 1024)])
+def test_choices_sorted_by_many_workgroups(N, top, E):
+    """Every pair once, in its expert's segment, whatever the number of workgroups that place them; ids outside the experts count as the
+    nearest one; the partial sums of a router's product are added in their order."""
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(N + E)
+    ids = (torch.rand(N, top, generator=g) ** 2 * E).int().clamp(max=E - 1)
+    ids[0, 0], ids[-1, -1] = -3, E + 5
+    weights = torch.rand(N, top, generator=g)
+    seg, tok_of, pair_of, part_of, weight_of = (t.cpu().long() if t.dtype == torch.int32 else t.cpu()
+                                                for t in ops.route_sort(ids.to(DEV), weights.to(DEV), E))
+    flat = ids.view(-1).long().clamp(0, E - 1)
+    assert torch.equal(seg, torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(flat, minlength=E).cumsum(0)]))
+    assert torch.equal(pair_of.sort().values, torch.arange(N * top))
+    assert torch.equal(flat[pair_of], torch.arange(E).repeat_interleave(seg[1:] - seg[:-1]))
+    assert torch.equal(tok_of, pair_of // top) and torch.equal(part_of, pair_of % top * N + pair_of // top)
+    assert torch.equal(weight_of, weights.view(-1)[pair_of])
+    parts, bias = torch.randn(5, min(N, 300), E, generator=g), torch.randn(E, generator=g)
+    whole = parts[0].clone()
+    for p in parts[1:]:
+        whole += p
+    got = [(torch.empty((whole.shape[0], top), dtype=torch.int32, device=DEV), torch.empty((whole.shape[0], top), device=DEV)) for _ in range(2)]
+    ops.route_topk(parts.to(DEV), bias.to(DEV), *got[0])
+    ops.route_topk(whole.to(DEV), bias.to(DEV), *got[1])
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
