@@ -9,7 +9,7 @@ SYN_EXPORT int syn_gemm(const void*, const void*, void*, int, int, int, int, int
 SYN_EXPORT int syn_qk_norm_rope_kv_write(const void*, int, void*, void*, void*, int, const int*, int, const int*, const int*, const void*,
                                          const void*, int, float, float, const float*, const float*, int, int, int, int, int, int, hipStream_t);
 SYN_EXPORT int syn_attention_f32(const float*, const float*, const float*, const int*, int, const int*, const int*, float*, float, int, int,
-                                 int, int, int, const float*, float, hipStream_t);
+                                 int, int, int, const float*, float, int, hipStream_t);
 SYN_EXPORT int syn_swiglu(const void*, void*, int, int, int, int, float, hipStream_t);
 
 // The layer as the host hands it over: pointers and whole numbers as 64-bit words, in this order.
@@ -19,7 +19,7 @@ struct BlockF32 {
   int *page_table, *tok_seq, *tok_pos;
   float* slopes;
   void *w_o, *gain2, *w_gate_up, *w_down;
-  int64_t gain1_f32, qk_gain_f32, gain2_f32, table_stride, n, hidden, nh, nkv, hd, rot, window, write_kv, inner, act;
+  int64_t gain1_f32, qk_gain_f32, gain2_f32, table_stride, n, hidden, nh, nkv, hd, rot, window, write_kv, inner, act, prompts;
 };
 
 static int64_t block_piece(int64_t floats) { return (floats + 63) / 64 * 64; }
@@ -52,7 +52,7 @@ SYN_EXPORT int syn_block_f32(const void* words, const double* reals, hipStream_t
                                    (const float*)b.sin_t, (int)b.rot, n, nh, nkv, hd, (int)b.write_kv, stream);
   if (!rc)
     rc = syn_attention_f32(last, (const float*)b.k_pages, (const float*)b.v_pages, b.page_table, (int)b.table_stride, b.tok_seq, b.tok_pos, rows,
-                           (float)reals[4], (int)b.window, n, nh, nkv, hd, b.slopes, (float)reals[5], stream);
+                           (float)reals[4], (int)b.window, n, nh, nkv, hd, b.slopes, (float)reals[5], (int)b.prompts, stream);
   if (!rc) rc = syn_gemm(rows, b.w_o, last, 0, n, H, nh * hd, 0, 1, 0, 0, -1, 0, stream);
   if (!rc) rc = syn_add_rmsnorm(b.resid, last, 1, n, nullptr, n, b.gain2, (int)b.gain2_f32, (float)reals[7], (float)reals[6], rows, 1, H, stream);
   if (!rc) rc = syn_gemm(rows, b.w_gate_up, wide, 0, n, 2 * I, H, 0, 1, 0, 0, -1, 0, stream);

@@ -714,7 +714,12 @@ def attention_f32(q, k_pages, v_pages, page_table, tok_seq, tok_pos, out, scale,
     _need(out, "attention_f32.out", _F32, (N, nh * hd))
     _call(load_library("core"), "syn_attention_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table),
           page_table.shape[1], _ptr(tok_seq), _ptr(tok_pos), _ptr(out), ctypes.c_float(scale), int(window or 0),
-          N, nh, nkv, hd, *_score_terms("attention_f32", slopes, softcap, nh), _stream())
+          N, nh, nkv, hd, *_score_terms("attention_f32", slopes, softcap, nh), int(_mostly_prompts(N, page_table)), _stream())
+
+
+def _mostly_prompts(n_tokens, page_table) -> bool:
+    """Whether tokens stand beside others of their sequence, so that 16 (token, head) rows share the keys that they see."""
+    return n_tokens >= 16 * page_table.shape[0]
 
 
 def _fits(t, dtype, shape) -> bool:
@@ -758,13 +763,13 @@ def block_f32(resid, delta, norm1, attention, norm2, feed, cache, table, tok_seq
     words = _BlockWords(at(resid), at(delta), at(out), at(work), at(gain1), at(w_qkv), at(q_gain), at(k_gain), at(cos), at(sin), at(k_pages),
                         at(v_pages), at(table), at(tok_seq), at(tok_pos), at(slopes), at(w_o), at(gain2), at(w_gate_up), at(w_down),
                         gain1.dtype is _F32, q_gain is not None and q_gain.dtype is _F32, gain2.dtype is _F32, width, N, H, nh, nkv, hd, rot,
-                        window, bool(write_kv), inner, act)
+                        window, bool(write_kv), inner, act, _mostly_prompts(N, table))
     reals = _BlockReals(eps1, offset1, qk_eps, qk_offset, scale, softcap, eps2, offset2, limit.value)
     _call(lib, "syn_block_f32", words, reals, _stream())
     return out
 
 
-_BlockWords, _BlockReals = ctypes.c_int64 * 34, ctypes.c_double * 9      # (BlockF32 and its reals)
+_BlockWords, _BlockReals = ctypes.c_int64 * 35, ctypes.c_double * 9      # (BlockF32 and its reals)
 
 
 @functools.lru_cache(maxsize=None)

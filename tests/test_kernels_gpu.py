@@ -278,6 +278,38 @@ def test_attention_f32_splits_and_head_sizes(ops, hd, past, new):
     close(out, want, 1e-5, 1e-5, "attention f32")
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (8, 2, 64), (12, 4, 16), (20, 2, 96), (8, 8, 32), (17, 1, 112), (10, 2, 48), (6, 3, 80)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_attention_f32_of_prompts_has_the_bits_of_single_tokens(ops, nh, nkv, hd, odd):
+    """16 (token, head) rows a workgroup on the matrix units against a wave a row (a page table with a row a token looks like single tokens):
+    tiles over the ends of sequences, heads that do not divide 16, NaN behind the sequences' ends; `odd`: keys and values among the cached
+    ones that are infinite, no number, or below the normal range."""
+    past, new = [300, 0, 64, 7], [90, 200, 129, 1]
+    lens = [p + n for p, n in zip(past, new)]
+    width = max((T + 63) // 64 for T in lens)
+    table = shuffled_table(len(past), width, 4)
+    k, v = make_cache(len(past) * width, nkv, hd, F32, 33, fill="nan")
+    fill_sequences(k, v, table, lens, nkv, hd, F32, 34)
+    if odd:
+        for b, at, x in ((0, 350, float("inf")), (1, 120, float("nan")), (1, 150, -float("inf")), (2, 100, 1e-39), (2, 170, 3e38)):
+            page = int(table[b, at // 64])
+            v[page, at % nkv, at % hd, at % 64] = x
+            k[page, (at + 1) % nkv, at % 64, at % hd] = x
+    tok_seq, tok_pos, _, _, _ = step_arrays(past, new)
+    q = rnd((len(tok_seq), nh * hd), 35, scale=2.0)
+    d = lambda t: t.to(DEV)
+    k, v, n = d(k), dv(v), len(tok_seq)
+    tall = torch.cat([table, torch.zeros((n, width), dtype=I32)])
+    assert ops._mostly_prompts(n, table) and not ops._mostly_prompts(n, tall) and n * nh > 8 * ops.compute_units()
+    outs = []
+    for t in (table, tall):
+        outs.append(torch.full((n, nh * hd), 7.0, device=DEV))
+        ops.attention_f32(d(q), k, v, d(t), d(tok_seq), d(tok_pos), outs[-1], 0.3, 0, nh, nkv, hd)
+    a, b = outs
+    assert torch.equal(torch.isnan(a), torch.isnan(b)) and bool(torch.isnan(a).any()) == odd
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)), int((torch.nan_to_num(a) != torch.nan_to_num(b)).sum())
+
+
 @pytest.mark.parametrize("new", [1, 600])
 def test_attention_f32_keeps_what_is_no_number(ops, new):
     """A key that is no number makes every result that sees it one, also where no other key stands in its block of 64; scores of
