@@ -2,8 +2,8 @@
 //
 //   gemm_simt      any shape and type; plain FMA: what the MFMA kernels refuse (K not a multiple of 8, or of 4 in 32 bits;
 //                  unaligned rows).
-//   gemm_f32_few   32-bit, up to 64 rows: v_mfma_f32_16x16x4_f32 over W streamed once, K over the waves.
-//   gemm_f32_tiles 32-bit, more rows: tiles of 64 x 64 or 64 x 32 through LDS.
+//   gemm_f32_few   32-bit, up to 64 rows of a W that is not wide: v_mfma_f32_16x16x4_f32 over W streamed once, K over the waves.
+//   gemm_f32_tiles 32-bit, more rows or a wide W: tiles of 64 x 32, 32 x 64 or 32 x 32 through LDS.
 //   gemm_skinny    bf16, M == 1: the weight matrix is streamed once from HBM through
 //                  v_mfma_f32_16x16x32_bf16; the waves of a workgroup split K and sum in LDS
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
@@ -473,11 +473,10 @@ static int tile_grid(int M, int N, int BM, int BN) {
 // batch: K in chunks of 32, chunk c of class c % 16; the chunks of a class one after another in ascending order, each in eight steps
 // (16 values in four steps of every fourth one, twice); then the sixteen sums in the order of the classes.
 //
-// Up to 64 rows of x: bound by reading W, which no cache holds.  A workgroup owns 16 rows of W; its 16 waves take a class
+// Up to 64 rows of x and a W that is not wide: bound by reading W, which no cache holds.  A workgroup owns 16 rows of W; its 16 waves take a class
 // each, eight loads of 16 k-values (four with many rows of x) at a time, so that the workgroup has up to 128 KB of W under way,
 // and their partial tiles are added in LDS in the order of the waves.  D[n = 4 (lane / 16) + j][m = lane % 16].
-// W of 2,560 x 9,728: 1 row 1,604 -> 38 us, 16 rows 1,655 -> 52 (plain kernel, this one); of 151,936 x 2,560: 1 row 1,225 ->
-// 415 us (3.8 TB/s).  The sums' error against 64 bits is a quarter of the plain kernel's (4.5e-7, 1.8e-6), since a class is a
+// W of 2,560 x 9,728: 1 row 1,604 -> 38 us, 16 rows 1,655 -> 52 (plain kernel, this one).  The sums' error against 64 bits is a quarter of the plain kernel's (4.5e-7, 1.8e-6), since a class is a
 // sixteenth of K.
 template <int FM, int U>
 __global__ void __launch_bounds__(16 * SYN_WAVE)
@@ -529,21 +528,41 @@ gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, fl
   }
 }
 
-// More rows: tiles of 64 x BN (BN = 64, 32), 4 waves of 32 x BN / 2, k-tiles of 32 in a ring of three LDS buffers that loads
-// fill without passing through registers; a row's eight 16-byte chunks are swizzled as in gemm_direct.  Three to five
-// workgroups share a compute unit.  A k-tile is a chunk of the order above, and they come class by class.
+// Which tile of a product that the matrix units bound: every XCD gets as many as every other (to one tile), a run of the tiles in
+// bands of at most eight rows of tiles, all bands alike, column after column of a band.  In panels of 8 x 4 (tile_of_workgroup) the
+// XCDs' shares differ by a panel, and all panels of a short last band can go to the same ones: 640 rows of 19,456 x 2,560 837 ->
+// 524 us, 384 rows of 2,560 x 9,728 263 -> 180, 192 rows 180 -> 147.
+__device__ __forceinline__ bool tile_of_share(int M, int N, int BM, int BN, int& tm, int& tn) {
+  const int tiles_n = (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM, tiles = tiles_m * tiles_n;
+  const int bands = (tiles_m + 7) / 8, high = (tiles_m + bands - 1) / bands;
+  const int xcd = (int)blockIdx.x % 8, local = (int)blockIdx.x / 8, more = tiles % 8;
+  if (local >= tiles / 8 + (xcd < more)) return false;
+  const int t = xcd * (tiles / 8) + min(xcd, more) + local, band = t / (high * tiles_n), in_band = t - band * high * tiles_n;
+  const int rows = min(high, tiles_m - band * high);
+  tm = band * high + in_band % rows;
+  tn = in_band / rows;
+  return true;
+}
+
+static int share_grid(int M, int N, int BM, int BN) { return (((M + BM - 1) / BM) * ((N + BN - 1) / BN) + 7) / 8 * 8; }
+
+// More rows, or a wide W: tiles of BM x BN, 4 waves of BM / 2 x BN / 2, k-tiles of 32 in a ring of three LDS buffers that loads
+// fill without passing through registers; a row's eight 16-byte chunks are swizzled as in gemm_direct.  Bound by the matrix units
+// (1,000 rows of 19,456 x 2,560: 121 TFLOP/s of some 150), alone on a compute unit by a k-tile's chain from load to sum (0.5 us a k-tile of
+// 64 x 32, 0.4 of 32 x 32), and with few rows by W (151,936 x 2,560, 1 row: 5.7 TB/s).  Four to six workgroups share a compute
+// unit; 64 x 64 was as fast at best, 128 x 64 and larger slower.  A k-tile is a chunk of the order above, and they come class by class.
 // D[n = 4 (lane / 16) + e][m = lane % 16].
-template <int BN>
+template <int BM, int BN>
 __global__ void __launch_bounds__(256)
 gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K, int point) {
-  constexpr int BM = 64, BK = 32, STAGES = 3, ROWS = BM + BN, RPI = 8, WAVES = 4, PASSES = ROWS / (RPI * WAVES);
-  constexpr int CLASSES = 16, FN = BN / 32;
-  static_assert(BN == 64 || BN == 32, "tile shape");
+  constexpr int BK = 32, STAGES = 3, ROWS = BM + BN, RPI = 8, WAVES = 4, PASSES = ROWS / (RPI * WAVES);
+  constexpr int CLASSES = 16, FM = BM / 32, FN = BN / 32;
+  static_assert((BM == 64 || BM == 32) && (BN == 64 || BN == 32), "tile shape");
   __shared__ __attribute__((aligned(16))) float smem[STAGES * ROWS * BK];
   const int lane = threadIdx.x % SYN_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE);
-  const int wm = (wave / 2) * 32, wn = (wave % 2) * (BN / 2);
+  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * (BN / 2);
   int tm, tn;
-  if (!tile_of_workgroup(M, N, BM, BN, tm, tn)) return;
+  if (!tile_of_share(M, N, BM, BN, tm, tn)) return;
   const int m0 = tm * BM, n0 = tn * BN, nk = (K + BK - 1) / BK;
   const size_t row_bytes = (size_t)K * sizeof(float);
   const BufferView vx = buffer_view(x + (size_t)m0 * K, (size_t)(M - m0) * row_bytes);
@@ -565,7 +584,7 @@ gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     int kt, of_class;
   };
   auto next = [&](Place p) { return p.kt + CLASSES < nk ? Place{p.kt + CLASSES, p.of_class} : Place{p.of_class + 1, p.of_class + 1}; };
-  f32x4 acc[2][FN] = {}, total[2][FN] = {};
+  f32x4 acc[FM][FN] = {}, total[FM][FN] = {};
   Place load = {0, 0}, at = {0, 0};
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t)
@@ -582,21 +601,21 @@ gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     const float* ws = xs + BM * BK;
     const int steps = min(BK, K - at.kt * BK);
     auto sixteen = [&](int c, bool in) {     // sixteen k-values: four chunks of 4, one for each quarter of the wave
-      f32x4 a[2], b[FN];
+      f32x4 a[FM], b[FN];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) a[j] = *(const f32x4*)(xs + (wm + 16 * j + r16) * BK + (((c + q) ^ ((wm + 16 * j + r16) >> 1)) & 7) * 4);
+      for (int j = 0; j < FM; ++j) a[j] = *(const f32x4*)(xs + (wm + 16 * j + r16) * BK + (((c + q) ^ ((wm + 16 * j + r16) >> 1)) & 7) * 4);
 #pragma unroll
       for (int j = 0; j < FN; ++j) b[j] = *(const f32x4*)(ws + (wn + 16 * j + r16) * BK + (((c + q) ^ ((BM + wn + 16 * j + r16) >> 1)) & 7) * 4);
       if (!in) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < FM; ++j) a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < FN; ++j) b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int ia = 0; ia < 2; ++ia)
+        for (int ia = 0; ia < FM; ++ia)
 #pragma unroll
           for (int j = 0; j < FN; ++j) acc[ia][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][e], a[ia][e], acc[ia][j], 0, 0, 0);
     };
@@ -609,14 +628,14 @@ gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     const Place behind = next(at);
     if (behind.of_class != at.of_class) {
 #pragma unroll
-      for (int ia = 0; ia < 2; ++ia)
+      for (int ia = 0; ia < FM; ++ia)
 #pragma unroll
         for (int j = 0; j < FN; ++j) total[ia][j] += acc[ia][j], acc[ia][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     at = behind;
   }
 #pragma unroll
-  for (int ia = 0; ia < 2; ++ia)
+  for (int ia = 0; ia < FM; ++ia)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
@@ -1557,8 +1576,12 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     const float *xf = (const float*)x, *wf = (const float*)w;
     float* of = (float*)out;
     const bool loads16 = !force_simt && K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
-    // (a wide W of 33 to 64 rows: one tile of x, and W by the tiles; N = 19,456, K = 2,560: 182 -> 143 us)
-    if (loads16 && (M <= 32 || (M <= 64 && N < 8192))) {
+    // Few rows take the tiles from where their W makes tiles for most of the chip: up to 16 rows from 64 rows of W a compute unit on
+    // (few-row kernel, tiles, at 1 row: 12,288 x 1,024 16.6, 19.6 us; 19,456 x 2,560 59, 56; 151,936 x 2,560 425, 274), up to 64 from
+    // 24 on (17 rows: 4,096 x 4,096 28, 54; 6,144 x 2,560 37, 36; 19,456 x 2,560 91, 58; 33 rows: 4,096 x 4,096 45, 55; 6,144 x 2,560
+    // 63, 42; 64 rows: 2,560 x 9,728 132, 124; 4,096 x 4,096 56, 55).
+    const long cus = syn_compute_units(), across = (N + 31) / 32, down = (M + 31) / 32;
+    if (loads16 && (M <= 16 ? N < 64 * cus : M <= 64 && N < 24 * cus)) {
       const int groups = (N + 15) / 16;
       if (M <= 16) gemm_f32_few_kernel<1, 8><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
       else if (M <= 32) gemm_f32_few_kernel<2, 4><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
@@ -1567,12 +1590,16 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
       return 0;
     }
     if (loads16) {
-      // whichever leaves less of the last round empty
-      const long cus = syn_compute_units(), wide = (long)((M + 63) / 64) * ((N + 63) / 64), slim = (long)((M + 63) / 64) * ((N + 31) / 32);
-      if (2 * ((wide + cus - 1) / cus) <= (slim + cus - 1) / cus)
-        gemm_f32_tiles_kernel<64><<<tile_grid(M, N, 64, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
+      // 32 x 32 where each has a compute unit to itself, so that a tile's time is the product's (65 rows, 2,560 x 9,728: 124 us,
+      // 149 in 32 x 64, 147 in 64 x 32); otherwise 64 x 32 in up to four rounds of an even number of 32 rows (384 rows: 181, 184),
+      // and 32 x 64, which asks L2 for less of W's share and pads to 32 rows only (65 rows, 19,456 x 2,560: 97, 64 x 32 133; 256
+      // rows 227, 234; 1,000 rows 841, 843)
+      if (down * across <= cus)
+        gemm_f32_tiles_kernel<32, 32><<<share_grid(M, N, 32, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
+      else if (down % 2 == 0 && down / 2 * across <= 4 * cus)
+        gemm_f32_tiles_kernel<64, 32><<<share_grid(M, N, 64, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
       else
-        gemm_f32_tiles_kernel<32><<<tile_grid(M, N, 64, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
+        gemm_f32_tiles_kernel<32, 64><<<share_grid(M, N, 32, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
       SYN_LAUNCH_CHECK("gemm_f32_tiles");
       return 0;
     }

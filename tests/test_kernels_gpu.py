@@ -220,6 +220,18 @@ def test_gemm_f32_on_the_matrix_units(ops, M, N, K):
     close(out, want.float(), 2 ** -24 * K * 4, 1e-6, f"gemm f32 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16384, 36), (16, 16500, 68), (17, 6144, 40), (64, 6200, 36),       # a wide W with few rows
+                                   (65, 40, 36), (320, 2560, 64), (640, 96, 32), (530, 1100, 36),         # bands of unequal height,
+                                   (577, 2600, 36), (1100, 33, 40), (2100, 700, 36), (257, 8200, 32)])    # counts that 8 does not divide
+def test_gemm_f32_tiles_cover_the_product(ops, M, N, K):
+    """Tiles of 64 x 32, 32 x 64 and 32 x 32 dealt out to the XCDs in equal runs: every one is computed, and by its rows and columns."""
+    x, w = rnd((M, K), 12), rnd((N, K), 13)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm(x.to(DEV), w.to(DEV), out)
+    # K fused steps of 2^-24 each at most, on products of size one
+    close(out, (x.double() @ w.double().T).float(), 2 ** -24 * K * 4, 1e-6, f"gemm f32 {M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("N,K", [(48, 4), (33, 68), (100, 260), (2560, 1000), (1000, 2052), (8200, 544), (9000, 612)])
 def test_gemm_f32_rows_do_not_depend_on_the_batch(ops, N, K):
     """Every split of the 32-bit products adds in the same order: a row has the same bits alone, among few and among many rows."""
