@@ -1,5 +1,6 @@
-// Attention over the paged cache in true 32-bit: one wave, or four, for each (token, head), plain FMA,
-// four online softmaxes over blocks of 64 keys in turns.  Any head size up to 256, prefill and decode alike.
+// Attention over the paged cache in true 32-bit: four online softmaxes over blocks of 64 keys in turns.  Any
+// head size up to 256, prefill and decode alike: one wave, or four, for each (token, head) with plain FMA; for prompts 16 (token,
+// head) rows a workgroup on the matrix units, with the same bits.
 //
 //   query of token t sits at position p = tok_pos[t] of sequence tok_seq[t];
 //   key j is visible iff j <= p and (window <= 0 or j > p - window);
