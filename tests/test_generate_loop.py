@@ -221,6 +221,18 @@ def test_the_penalties_see_the_context_as_it_is_at_the_step(monkeypatch, last_n)
     assert seen.pop() == [1, 4]
 
 
+@pytest.mark.parametrize("top_k", [float("inf"), float("nan"), 1 << 40, 8192.0, 0, -1])
+def test_a_top_k_that_leaves_nothing_out_is_off_for_long_rows_too(monkeypatch, top_k):
+    import cpu_kernels
+    cpu_kernels.install(monkeypatch)
+    seen, plain = [], ops.filter_rows
+    monkeypatch.setattr(ops, "filter_rows", lambda *a: (seen.append(a[3].tolist()), plain(*a))[1])
+    cfg = GenerationConfig(temperature=0.7, top_k=top_k)
+    rows = torch.linspace(0, 1, 2 * 8192).view(2, 8192)
+    tokens = sample_batch(rows, [SequenceSampler(cfg, [1]), SequenceSampler(GenerationConfig(temperature=0.0, top_p=0.9), [2])])
+    assert seen == [[0, 0]] and tokens[1] == 8191
+
+
 def test_every_call_counts_the_penalties_tokens_in_memory_of_its_own(monkeypatch):
     """Calls on other streams or threads may be under way: no two of them may share counters."""
     import cpu_kernels
