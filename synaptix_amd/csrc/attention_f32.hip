@@ -321,7 +321,8 @@ attn_f32_tiles_kernel(const float* __restrict__ q, const float* __restrict__ k_p
   }
 }
 
-// slopes [nh] float or null, softcap (0: none): see ScoreTerms; prompts: most tokens stand beside others of their sequence
+// slopes [nh] float or null, softcap (0: none): see ScoreTerms; prompts: 16 rows a workgroup may take the step (the host's rule, which
+// knows the lengths: a workgroup walks the sequences of its rows one after another, ops.prompt_rows_pay)
 SYN_EXPORT int syn_attention_f32(const float* q, const float* k_pages, const float* v_pages, const int* page_table,
                                  int table_stride, const int* tok_seq, const int* tok_pos, float* out, float scale,
                                  int window, int n_tokens, int nh, int nkv, int hd, const float* slopes, float softcap,

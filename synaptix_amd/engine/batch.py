@@ -83,6 +83,7 @@ class StepContext:
         for name, (o, n) in layout.off.items():
             setattr(self, name, buffer.narrow(0, o, n))
         self._tables = [buffer.narrow(0, o, n).view(layout.B, w) for (o, n), w in zip(layout.table_off, layout.widths)]
+        self._prompt_rows = {}
         self.items = None       # a work list of decode attention for each group, where the step's owner keeps them
 
     def page_table(self, group: int) -> torch.Tensor:
@@ -90,6 +91,14 @@ class StepContext:
 
     def decode_splits(self, n_kv_heads: int, group: int) -> int:
         return ops.decode_splits(self.n_seqs, n_kv_heads, self.layout.widths[group])
+
+    def prompt_rows_pay(self, *heads) -> bool:
+        """ops.prompt_rows_pay of the step's lengths and a layer's (heads, kv heads, head size), looked at once a step."""
+        known = self._prompt_rows.get(heads)
+        if known is None:
+            known = not self.one_token_each and ops.prompt_rows_pay(self.past, self.new_counts, *heads)
+            self._prompt_rows[heads] = known
+        return known
 
     def decode_items(self, group: int):
         """The group's work list for decode attention (int32 [n_seqs * decode_splits, 4]) or None."""

@@ -702,8 +702,9 @@ def _score_terms(name, slopes, softcap, n_heads):
 
 
 def attention_f32(q, k_pages, v_pages, page_table, tok_seq, tok_pos, out, scale, window, n_heads, n_kv_heads,
-                  head_dim, slopes=None, softcap=0.0):
-    """True 32-bit attention of every token (prefill and decode alike).  slopes, softcap: see _score_terms."""
+                  head_dim, slopes=None, softcap=0.0, prompts=None):
+    """True 32-bit attention of every token (prefill and decode alike).  slopes, softcap: see _score_terms.  prompts: whether the kernel
+    for prompts may take the step (prompt_rows_pay of its lengths; the results have the same bits); None: as far as the tables tell."""
     nh, nkv, hd = n_heads, n_kv_heads, head_dim
     _need(q, "attention_f32.q", _F32, (None, nh * hd))
     N = q.shape[0]
@@ -714,7 +715,8 @@ def attention_f32(q, k_pages, v_pages, page_table, tok_seq, tok_pos, out, scale,
     _need(out, "attention_f32.out", _F32, (N, nh * hd))
     _call(load_library("core"), "syn_attention_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table),
           page_table.shape[1], _ptr(tok_seq), _ptr(tok_pos), _ptr(out), ctypes.c_float(scale), int(window or 0),
-          N, nh, nkv, hd, *_score_terms("attention_f32", slopes, softcap, nh), int(_mostly_prompts(N, page_table)), _stream())
+          N, nh, nkv, hd, *_score_terms("attention_f32", slopes, softcap, nh),
+          int(_mostly_prompts(N, page_table) if prompts is None else bool(prompts)), _stream())
 
 
 def _mostly_prompts(n_tokens, page_table) -> bool:
@@ -722,16 +724,52 @@ def _mostly_prompts(n_tokens, page_table) -> bool:
     return n_tokens >= 16 * page_table.shape[0]
 
 
+def prompt_rows_pay(past, new, n_heads, n_kv_heads, head_dim) -> bool:
+    """Whether 32-bit attention of sequences with past[b] cached and new[b] new tokens is faster 16 (token, head) rows a workgroup than a
+    wave a row, which it is where it looks a seventh faster in estimates that are wrong by a tenth at the median and by a quarter in one
+    case of ten.  A wave a row: so many blocks of 64 keys a microsecond for all rows, and the longest row's own.  16 rows: a block is
+    read once for all of them that see it, but a workgroup walks its rows' sequences one after another, four blocks at a time, and
+    one with fewer than four leaves waves without work.  Measured, us (a wave a row, 16 rows): 400 new tokens beside 20 single ones
+    behind 1,500, 12 heads of 96 232 and 1,474, 32 of 128 over 8 kv heads 700 and 550; 100 beside 3 behind 2,000, 32 of 128 over 8
+    250 and 389, 64 over 8 378 and 277; up to 64 keys, 32 of 128 over 8: 2 times 33 tokens 22 and 35, 8 times 33 53 and 68, 16 times 17 51 and 70,
+    4 times 64 61 and 37; behind 100, 8 times 17 74 and 51; 120, 137 and 233 tokens 228 and 87."""
+    group, n = n_heads // n_kv_heads, sum(new)
+    if n * n_heads <= 8 * compute_units():
+        return False
+    blocks_before = lambda x: 32 * (x // 64) * (x // 64 + 1) + x % 64 * (x // 64 + 1)      # of the tokens in front of place x, their blocks
+    row = seen = visits = most = 0
+    shared, walk, longest = -1, 0, 0        # the workgroup that the last sequence ended in, the turns of four blocks it has to walk
+    for p, m in zip(past, new):
+        first, last = row // 16, (row + m * group - 1) // 16
+        row += m * group
+        blocks = blocks_before(p + m) - blocks_before(p)
+        seen += blocks
+        visits += (last - first + 1) * blocks / m
+        most = max(most, (p + m + 63) // 64)
+        turns = (p + m + 255) // 256
+        if first == shared:
+            walk += turns if first == last else p // 256 + 1
+            longest = max(longest, walk)
+        if first != shared or first != last:
+            shared, walk = last, turns
+            longest = max(longest, walk)
+    size, idle = head_dim / 128, 1 - min(seen / n, 4) / 4
+    a_row = 4.5 + size * (seen * n_heads * (7.3e-3 - 1.9e-3 * size) + 6 * most)
+    sixteen = 5.7 + size * (10.6 * longest + visits * n_kv_heads * (15e-3 + 1.7e-3 * size) * (1 + 2.7 * idle))
+    return sixteen < 0.86 * a_row
+
+
 def _fits(t, dtype, shape) -> bool:
     return t.dtype is dtype and t.is_cuda and t.shape == shape and t.is_contiguous()
 
 
-def block_f32(resid, delta, norm1, attention, norm2, feed, cache, table, tok_seq, tok_pos, write_kv):
+def block_f32(resid, delta, norm1, attention, norm2, feed, cache, table, tok_seq, tok_pos, write_kv, prompts):
     """A pre-norm layer of the 32-bit path in one call (csrc/block_f32.hip): add_rmsnorm, gemm, qk_norm_rope_kv_write, attention_f32,
     gemm, add_rmsnorm, gemm, swiglu, gemm, with the same results.  resid [N, H] gets delta ([N, H] or None) and the attention's result;
     returns what the feed-forward adds, or None where something is not as these take it (the caller then calls them one by one, and
     the one that refuses says why).  norm1, norm2: (gain, eps, gain offset); attention: (w_qkv, q_gain, k_gain, eps, gain offset, cos, sin,
-    w_o, scale, window, soft cap, slopes, heads, kv heads, head size); feed: (w_gate_up, w_down, inner width, activation)."""
+    w_o, scale, window, soft cap, slopes, heads, kv heads, head size); feed: (w_gate_up, w_down, inner width, activation); prompts: as in
+    attention_f32."""
     w_qkv, q_gain, k_gain, qk_eps, qk_offset, cos, sin, w_o, scale, window, softcap, slopes, nh, nkv, hd = attention
     w_gate_up, w_down, inner, activation = feed
     (gain1, eps1, offset1), (gain2, eps2, offset2) = norm1, norm2
@@ -763,7 +801,7 @@ def block_f32(resid, delta, norm1, attention, norm2, feed, cache, table, tok_seq
     words = _BlockWords(at(resid), at(delta), at(out), at(work), at(gain1), at(w_qkv), at(q_gain), at(k_gain), at(cos), at(sin), at(k_pages),
                         at(v_pages), at(table), at(tok_seq), at(tok_pos), at(slopes), at(w_o), at(gain2), at(w_gate_up), at(w_down),
                         gain1.dtype is _F32, q_gain is not None and q_gain.dtype is _F32, gain2.dtype is _F32, width, N, H, nh, nkv, hd, rot,
-                        window, bool(write_kv), inner, act, _mostly_prompts(N, table))
+                        window, bool(write_kv), inner, act, bool(prompts))
     reals = _BlockReals(eps1, offset1, qk_eps, qk_offset, scale, softcap, eps2, offset2, limit.value)
     _call(lib, "syn_block_f32", words, reals, _stream())
     return out

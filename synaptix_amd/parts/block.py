@@ -113,7 +113,8 @@ class PreNormBlock(Block):
                              (a.w_qkv.plain, a.q_gain, a.k_gain, a.qk_norm_eps or 0.0, a.qk_gain_offset, cos, sin, a.w_o.plain, a.scale,
                               a.window or 0, terms["softcap"], terms["slopes"], a.nh, a.nkv, a.hd),
                              (n2.gain, n2.eps, n2.gain_offset), (f.w_gate_up.plain, f.w_down.plain, f.intermediate, f.activation),
-                             (cache.k_pages, cache.v_pages), ctx.page_table(cache.group), ctx.tok_seq, ctx.tok_pos, owner)
+                             (cache.k_pages, cache.v_pages), ctx.page_table(cache.group), ctx.tok_seq, ctx.tok_pos, owner,
+                             ctx.prompt_rows_pay(a.nh, a.nkv, a.hd))
 
     def forward(self, resid, pending, ctx, cache, owner=True):
         if ctx.act_dtype == torch.float32:

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from synaptix_amd.cache import SequenceCache, CacheError
-from synaptix_amd.engine.batch import StepLayout, fill_host_buffer
+from synaptix_amd.engine.batch import StepContext, StepLayout, fill_host_buffer
 from synaptix_amd.kernels import runtime as rt
 from synaptix_amd.parts.base import KvNeed
 
@@ -136,3 +136,23 @@ def test_host_side_rules_of_the_kernels_stay_within_their_kernels_limits():
                 assert (s - 1) * step < K, "no slice may be empty"
                 assert K % 8 == 0 and (M <= 64 or K % 128 == 0)
             assert ops.gemm_slices(M, N, K, torch.float32) == 1
+
+
+def test_32_bit_prompts_share_workgroups_only_where_that_was_measured_to_pay():
+    """Steps timed with a wave a row and with 16 rows a workgroup: the latter walks a workgroup's sequences one after another, which single
+    tokens behind long contexts beside a prompt make up to six times slower than the former, and many short prompts half as slow again."""
+    from synaptix_amd.kernels import ops
+    pays = lambda past, new, *heads: ops.prompt_rows_pay(past, new, *heads)
+    for nh, nkv, hd in ((32, 8, 128), (32, 32, 128), (12, 12, 96), (32, 32, 64)):
+        assert pays([0] * 3, [120, 137, 233], nh, nkv, hd) and pays([0], [600], nh, nkv, hd) and pays([700] * 2, [260] * 2, nh, nkv, hd)
+    for nh, nkv, hd in ((32, 32, 128), (12, 12, 96), (8, 8, 64), (32, 32, 64)):
+        assert not pays([0] + [1500] * 20, [400] + [1] * 20, nh, nkv, hd)
+        assert not pays([0] * 6 + [2000] * 10, [64] * 6 + [1] * 10, nh, nkv, hd)
+    assert not pays([0] + [2000] * 3, [100] + [1] * 3, 32, 8, 128) and not pays([2000] * 3 + [0], [1] * 3 + [100], 40, 8, 80)
+    for n, each in ((2, 33), (8, 17), (8, 33), (16, 17)):
+        assert not pays([0] * n, [each] * n, 32, 8, 128)
+    assert pays([0] * 4, [64] * 4, 32, 8, 128) and pays([100] * 8, [17] * 8, 32, 8, 128) and pays([300] * 64, [16] * 64, 32, 8, 128)
+    assert not pays([0], [60], 32, 8, 128) and not pays([5000] * 70, [1] * 70, 32, 8, 128)
+    layout = StepLayout(57 + 60, 2, 0, [1])
+    ctx = StepContext(layout, torch.zeros(layout.total, dtype=torch.int32), torch.float32, [0, 1], [700, 0], [57, 60], None)
+    assert ctx.prompt_rows_pay(32, 8, 128) and not ctx.prompt_rows_pay(4, 4, 16)
