@@ -1579,9 +1579,11 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     // Few rows take the tiles from where their W makes tiles for most of the chip: up to 16 rows from 64 rows of W a compute unit on
     // (few-row kernel, tiles, at 1 row: 12,288 x 1,024 16.6, 19.6 us; 19,456 x 2,560 59, 56; 151,936 x 2,560 425, 274), up to 64 from
     // 24 on (17 rows: 4,096 x 4,096 28, 54; 6,144 x 2,560 37, 36; 19,456 x 2,560 91, 58; 33 rows: 4,096 x 4,096 45, 55; 6,144 x 2,560
-    // 63, 42; 64 rows: 2,560 x 9,728 132, 124; 4,096 x 4,096 56, 55).
+    // 63, 42; 64 rows: 2,560 x 9,728 132, 124; 4,096 x 4,096 56, 55).  17 and 18 rows from 32 on where K is a multiple of 1,024: all
+    // turns of the few-row kernel's loads are full then (17 rows: 6,144 x 4,096 48, 52; 8,192 x 4,096 50, 53; 6,144 x 8,192 96, 101;
+    // 9,728 x 4,096 69, 64; 22 rows: 6,144 x 4,096 53, 52).
     const long cus = syn_compute_units(), across = (N + 31) / 32, down = (M + 31) / 32;
-    if (loads16 && (M <= 16 ? N < 64 * cus : M <= 64 && N < 24 * cus)) {
+    if (loads16 && (M <= 16 ? N < 64 * cus : M <= 64 && N < (M <= 18 && K % 1024 == 0 ? 32 * cus + 1 : 24 * cus))) {
       const int groups = (N + 15) / 16;
       if (M <= 16) gemm_f32_few_kernel<1, 8><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
       else if (M <= 32) gemm_f32_few_kernel<2, 4><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);

@@ -232,6 +232,17 @@ def test_gemm_f32_tiles_cover_the_product(ops, M, N, K):
     close(out, (x.double() @ w.double().T).float(), 2 ** -24 * K * 4, 1e-6, f"gemm f32 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 6144, 1024), (18, 8192, 1024), (18, 8196, 1024), (19, 6144, 1024), (17, 8192, 1020)])
+def test_gemm_f32_of_few_rows_has_the_same_bits_on_both_sides_of_the_rule(ops, M, N, K):
+    """Around the sizes from which the tiles take 17 rows and more: row by row the bits that the kernel for few rows gives one row alone."""
+    x, w = rnd((M, K), 14).to(DEV), rnd((N, K), 15).to(DEV)
+    out, one = torch.full((M, N), float("nan"), device=DEV), torch.empty((1, N), device=DEV)
+    ops.gemm(x, w, out)
+    for m in (0, 15, 16, M - 1):
+        ops.gemm(x[m:m + 1].contiguous(), w, one)
+        assert torch.equal(out[m:m + 1], one), m
+
+
 @pytest.mark.parametrize("N,K", [(48, 4), (33, 68), (100, 260), (2560, 1000), (1000, 2052), (8200, 544), (9000, 612)])
 def test_gemm_f32_rows_do_not_depend_on_the_batch(ops, N, K):
     """Every split of the 32-bit products adds in the same order: a row has the same bits alone, among few and among many rows."""
