@@ -3,7 +3,7 @@
 //   gemm_simt      any shape and type; plain FMA: what the MFMA kernels refuse (K not a multiple of 8, or of 4 in 32 bits;
 //                  unaligned rows).
 //   gemm_f32_few   32-bit, up to 64 rows of a W that is not wide: v_mfma_f32_16x16x4_f32 over W streamed once, K over the waves.
-//   gemm_f32_tiles 32-bit, more rows or a wide W: tiles of 64 x 32, 32 x 64 or 32 x 32 through LDS.
+//   gemm_f32_tiles 32-bit, more rows or a wide W: tiles of 64 x 64, 64 x 32, 32 x 64 or 32 x 32 through LDS.
 //   gemm_skinny    bf16, M == 1: the weight matrix is streamed once from HBM through
 //                  v_mfma_f32_16x16x32_bf16; the waves of a workgroup split K and sum in LDS
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
@@ -549,8 +549,8 @@ static int share_grid(int M, int N, int BM, int BN) { return (((M + BM - 1) / BM
 // More rows, or a wide W: tiles of BM x BN, 4 waves of BM / 2 x BN / 2, k-tiles of 32 in a ring of three LDS buffers that loads
 // fill without passing through registers; a row's eight 16-byte chunks are swizzled as in gemm_direct.  Bound by the matrix units
 // (1,000 rows of 19,456 x 2,560: 121 TFLOP/s of some 150), alone on a compute unit by a k-tile's chain from load to sum (0.5 us a k-tile of
-// 64 x 32, 0.4 of 32 x 32), and with few rows by W (151,936 x 2,560, 1 row: 5.7 TB/s).  Four to six workgroups share a compute
-// unit; 64 x 64 was as fast at best, 128 x 64 and larger slower.  A k-tile is a chunk of the order above, and they come class by class.
+// 64 x 32, 0.4 of 32 x 32), and with few rows by W (151,936 x 2,560, 1 row: 5.7 TB/s).  Three to six workgroups share a compute
+// unit; 128 x 64 and larger were slower.  A k-tile is a chunk of the order above, and they come class by class.
 // D[n = 4 (lane / 16) + e][m = lane % 16].
 template <int BM, int BN>
 __global__ void __launch_bounds__(256)
@@ -1592,13 +1592,20 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
       return 0;
     }
     if (loads16) {
-      // 32 x 32 where each has a compute unit to itself, so that a tile's time is the product's (65 rows, 2,560 x 9,728: 124 us,
-      // 149 in 32 x 64, 147 in 64 x 32); otherwise 64 x 32 in up to four rounds of an even number of 32 rows (384 rows: 181, 184),
-      // and 32 x 64, which asks L2 for less of W's share and pads to 32 rows only (65 rows, 19,456 x 2,560: 97, 64 x 32 133; 256
-      // rows 227, 234; 1,000 rows 841, 843)
-      if (down * across <= cus)
+      // 64 x 64, the fastest for its size, where it goes round at least three times and no rounds of the halves are fewer by more than
+      // the 2.5 % that it is faster by; three workgroups share a compute unit, so a fourth round runs alone (64 x 64, the halves: 3
+      // rounds 6,144 x 2,560 with 490 rows 138 us, 141, 4,096 x 12,288 with 768 642, 669; 4 rounds 4,096 x 12,288 with 1,024 854, 839; 48
+      // rounds 24,576 x 4,096 with 2,000 3,240, 3,346).  32 x 32 where each has a compute unit to itself, so that a tile's time is the
+      // product's (65 rows, 2,560 x 9,728: 124 us, 149 in 32 x 64, 147 in 64 x 32).  64 x 32 in up to four rounds of an even number of 32
+      // rows (384 rows: 181, 184) and for two of them, whose W is read once so (151,936 x 2,560 with 33 rows: 455, 465).  Else 32 x 64,
+      // which asks L2 for less of W's share and pads to 32 rows only (65 rows, 19,456 x 2,560: 97, 64 x 32 133; 256 rows 227, 234).
+      const long square = ((M + 63) / 64 * ((N + 63) / 64) + cus - 1) / cus;
+      const long slim = ((M + 63) / 64 * across + cus - 1) / cus, flat = (down * ((N + 63) / 64) + cus - 1) / cus;
+      if (square >= 3 && square != 4 && 39 * square <= 20 * (slim < flat ? slim : flat))
+        gemm_f32_tiles_kernel<64, 64><<<share_grid(M, N, 64, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
+      else if (down * across <= cus)
         gemm_f32_tiles_kernel<32, 32><<<share_grid(M, N, 32, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else if (down % 2 == 0 && down / 2 * across <= 4 * cus)
+      else if (down == 2 || (down % 2 == 0 && down / 2 * across <= 4 * cus))
         gemm_f32_tiles_kernel<64, 32><<<share_grid(M, N, 64, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
       else
         gemm_f32_tiles_kernel<32, 64><<<share_grid(M, N, 32, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);

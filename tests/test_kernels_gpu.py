@@ -232,6 +232,18 @@ def test_gemm_f32_tiles_cover_the_product(ops, M, N, K):
     close(out, (x.double() @ w.double().T).float(), 2 ** -24 * K * 4, 1e-6, f"gemm f32 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(250, 12250, 36), (490, 6144, 64), (320, 16380, 100), (577, 13000, 40), (640, 16384, 32), (256, 16384, 36)])
+def test_gemm_f32_squares_have_the_bits_of_single_rows(ops, M, N, K):
+    """Tiles of 64 x 64 at 3, 5, 8 and 10 rounds and ragged ends, and of the halves at 4 rounds: every row as the kernel for few rows has it."""
+    x, w = rnd((M, K), 16).to(DEV), rnd((N, K), 17).to(DEV)
+    out, one = torch.full((M, N), float("nan"), device=DEV), torch.empty((1, N), device=DEV)
+    ops.gemm(x, w, out)
+    assert not bool(torch.isnan(out).any())
+    for m in sorted({0, 31, 32, 63, 64, M // 2, M - 2, M - 1}):
+        ops.gemm(x[m:m + 1].contiguous(), w, one)
+        assert torch.equal(out[m:m + 1], one), m
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 6144, 1024), (18, 8192, 1024), (18, 8196, 1024), (19, 6144, 1024), (17, 8192, 1020)])
 def test_gemm_f32_of_few_rows_has_the_same_bits_on_both_sides_of_the_rule(ops, M, N, K):
     """Around the sizes from which the tiles take 17 rows and more: row by row the bits that the kernel for few rows gives one row alone."""
