@@ -233,6 +233,20 @@ def test_a_top_k_that_leaves_nothing_out_is_off_for_long_rows_too(monkeypatch, t
     assert seen == [[0, 0]] and tokens[1] == 8191
 
 
+def test_rows_spread_over_workgroups_only_where_that_was_measured_to_pay():
+    """Rows drawn from, rows that are not, few and many of them: (rows, entries, top-k) on both sides of each line."""
+    from synaptix_amd.sampling.sampler import _shared_top_k
+    def takes(rows, V, k, greedy):
+        return _shared_top_k([SequenceSampler(GenerationConfig(top_k=k, temperature=0.0 if greedy else 0.7), []) for _ in range(rows)], greedy, rows, V)
+    for rows in (1, 24, 25, 64):
+        assert takes(rows, 8192, 64, False) == 64 and not takes(rows, 8192, 65, False) and not takes(rows, 8191, 1, False)
+        assert takes(rows, 65536, 512, False) == 512 and not takes(rows, 151936, 513, False) and not takes(rows, 151936, 0, False)
+    for rows in (1, 24):
+        assert takes(rows, 32768, 128, True) == 128 and not takes(rows, 32768, 129, True) and not takes(rows, 32767, 1, True)
+    for rows in (25, 64):
+        assert takes(rows, 65536, 192, True) == 192 and not takes(rows, 65536, 256, True) and not takes(rows, 40000, 1, True)
+
+
 def test_every_call_counts_the_penalties_tokens_in_memory_of_its_own(monkeypatch):
     """Calls on other streams or threads may be under way: no two of them may share counters."""
     import cpu_kernels
