@@ -159,7 +159,9 @@ SYN_EXPORT int syn_latent_intake(const float* proj, int width, const float* down
   SYN_CHECK(!v_fragments || rank % 16 == 0, "latent_intake: value pages in fragment order need a latent that is a multiple of 16, not %d", rank);
   SYN_CHECK(n_pairs == 0 || (cos_t && sin_t && max_position < capacity),
             "latent_intake: position %d is beyond the rotation's table of %d", max_position, capacity);
-  const bool fours = dim % 4 == 0 && rot % 4 == 0 && rank % 4 == 0 && rank <= 1024 && rot <= 1024 && width % 4 == 0 && down_stride % 4 == 0 &&
+  // (rows of few queries give most of a workgroup's threads nothing to do either way: 1,500 tokens with 4 heads of 32 + 16 6.2 us a value a
+  // thread, 6.7 in fours, 8 of 64 + 32 7.7 and 8.2, 16 of 128 + 64 14.9 and 13.1)
+  const bool fours = heads * (dim + rot) >= 1024 && dim % 4 == 0 && rot % 4 == 0 && rank % 4 == 0 && rank <= 1024 && rot <= 1024 && width % 4 == 0 && down_stride % 4 == 0 &&
                      ((uintptr_t)proj | (uintptr_t)down | (uintptr_t)q_nope | (uintptr_t)q_full | (uintptr_t)k_pages) % 16 == 0;
 #define SYN_INTAKE4(T)                                                                                                            \
   latent_intake4_kernel<T><<<n_tokens, 256, 0, stream>>>(proj, width, down, down_stride, gain, gain_is_f32, eps, cos_t, sin_t, n_pairs, \

@@ -404,6 +404,55 @@ def test_latent_intake_norms_turns_and_writes_the_pages(H, D, B, C, pairs, dtype
         assert torch.equal(vf, ops.latent_v_pages_to_kernel_order(vp))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D,B,C,pairs,spare", [(32, 128, 64, 512, 32, 0), (6, 128, 64, 1024, 20, 4), (16, 64, 8, 36, 4, 8), (24, 48, 0, 128, 0, 0),
+                                                 (40, 4, 1024, 16, 512, 4)])
+def test_latent_intake_of_wide_rows_four_values_at_a_time(H, D, B, C, pairs, spare, dtype):
+    """Sizes that the kernel for pieces of four values takes (a latent over one wave, over all of them, threads that hold latent and rotated
+    values both) against 64 bits and against the general kernel, which rows with one more column go to; the latent in the queries'
+    rows and in rows of its own; without cache writes the pages stay as they are.  The bounds: 32-bit sums of C squares, then a
+    dozen roundings of 2^-24; half a unit of the eighth bit, 2^-8, where the result is rounded to bf16."""
+    from synaptix_amd.kernels import ops
+    from synaptix_amd.parts import RotaryInterleaved
+    g = torch.Generator().manual_seed(H * C)
+    N, R, nq = 9, C + B, H * (D + B)
+    proj = torch.randn(N, nq + R + spare, generator=g, dtype=P.F64).float().double()
+    gain = torch.randn(C, generator=g, dtype=P.F64).to(dtype).double()
+    seqs, pos = [0, 0, 1, 0, 1, 1, 1, 0, 1], [63, 64, 0, 65, 1, 2, 3, 127, 70]
+    table = torch.tensor([[2, 1], [3, 0]], dtype=torch.int32, device=DEV)
+    cos, sin = RotaryInterleaved(70.0, 2 * pairs, 128).tables(DEV) if pairs else (None, None)
+    seq_d, pos_d = (torch.tensor(t, dtype=torch.int32, device=DEV) for t in (seqs, pos))
+
+    def run(rows, down=None, write=True, fragments=False):
+        out = [torch.full((N, H * D), 5.0, dtype=dtype, device=DEV), torch.full((N, H * R), 9.0, dtype=dtype, device=DEV),
+               torch.zeros((4, 1, 64, R), dtype=dtype, device=DEV), torch.zeros((4, 1, C, 64), dtype=dtype, device=DEV)]
+        ops.latent_intake(rows, gain.to(dtype).to(DEV), 1e-5, cos, sin, *out, table, seq_d, pos_d, H, D, B, C, max(pos), write_kv=write,
+                          v_fragments=fragments, down=down)
+        return out
+    whole = proj.float().to(DEV)
+    got = run(whole)
+    general = run(torch.cat([whole, torch.zeros(N, 1, device=DEV)], 1))
+    assert (nq + R + spare) % 4 == 0 and H * (D + B) >= 1024
+    eps = 2 ** -8 if dtype == torch.bfloat16 else 0.0
+    P_t, q, down = torch.tensor(pos), proj[:, :nq].view(N, H, D + B), proj[:, nq:nq + R]
+    near = lambda a, want: bool(((a.cpu().double() - want).abs() <= (eps + 2 ** -20) * want.abs() + 2 ** -20).all())
+    want_q = P.turn_pairs(q[..., D:], P_t, 70.0, 2 * pairs) if B else q[..., D:]
+    want_row = torch.cat([P.rms_norm(down[:, :C], gain, 1e-5), P.turn_pairs(down[:, C:], P_t, 70.0, 2 * pairs) if B else down[:, C:]], -1)
+    for qn, qf, kp, vp in (got, general):
+        assert near(qn.view(N, H, D), q[..., :D]) and near(qf.view(N, H, R)[..., C:], want_q) and bool((qf.view(N, H, R)[..., :C] == 9).all())
+        rows = [(int(table[seqs[n], pos[n] // 64]), pos[n] % 64) for n in range(N)]
+        assert near(torch.stack([kp[p, 0, s] for p, s in rows]), want_row)
+        assert near(torch.stack([vp[p, 0, :, s] for p, s in rows]), want_row[:, :C])
+        assert int((kp.float().abs().sum(-1) > 0).sum()) == N
+    assert torch.equal(got[0], general[0])
+    split = run(whole[:, :nq].contiguous(), down=torch.cat([whole[:, nq:], torch.zeros(N, -(R + spare) % 4 + 4, device=DEV)], 1)[:, :R + spare])
+    assert all(torch.equal(a, b) for a, b in zip(split, got))
+    left = run(whole, write=False)
+    assert torch.equal(left[0], got[0]) and torch.equal(left[1], got[1]) and not bool(left[2].any()) and not bool(left[3].any())
+    if C % 16 == 0:
+        assert torch.equal(run(whole, fragments=True)[3], ops.latent_v_pages_to_kernel_order(got[3]))
+
+
 # ----------------------------------------------------------------------------- whole models
 
 def lengths(name):
