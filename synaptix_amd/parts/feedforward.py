@@ -103,6 +103,15 @@ class UngatedMlp(FeedForward):
         return deferred_product(linear(h, self.w_up, h.dtype, point=self.activation), self.w_down)
 
 
+def router_slices_pay(n_rows, n_experts) -> bool:
+    """Whether a router's product runs in slices of K whose sums the choice adds itself: with few rows of W that fills the chip, with many
+    it is the choice, which reads a token's row of every slice one piece after another, that takes longer.  Product and choice, us, in one
+    and in slices: 1,500 tokens with 48 experts of 4,096 30 and 16, 128 31 and 21, 256 33 and 23, 1,024 41 and 45; 40 tokens with 256 23 and
+    19, 1,024 30 and 50; 16 with 48 23 and 14, 128 15 and 14, 256 16 and 19, 1,024 23 and 49; 8 with 8 experts of 2,048 16 and 12, 128 of 4,096
+    12.5 and 11.4; 1 with 8 of 2,048 8.9 and 10.4, 256 of 7,168 13 and 15."""
+    return n_rows >= 8 if n_experts <= 128 else n_experts <= 256 and n_rows > 32
+
+
 class RoutedExperts(FeedForward):
     """A mixture of small experts: each token goes through `top` of them, chosen by a router, and gets the weighted sum
     of their results.
@@ -235,9 +244,8 @@ class RoutedExperts(FeedForward):
         N, dev = h.shape[0], h.device
         ids = torch.empty((N, self.top), dtype=torch.int32, device=dev)
         weights = torch.empty((N, self.top), dtype=torch.float32, device=dev)
-        # (few rows of W: the choice adds the sums over slices of K itself; 1,500 tokens, 48 experts of 4,096: 25 -> 8.2 us, the
-        # choice 9 -> 11)
-        takes_parts = self.router == "top_logits" and self.shared_gate is None and h.dtype == self.w_router.dtype
+        takes_parts = (self.router == "top_logits" and self.shared_gate is None and h.dtype == self.w_router.dtype
+                       and router_slices_pay(N, self.w_router.shape[0]))
         logits = (linear_for_sum if takes_parts else linear)(h, self.w_router, *(() if takes_parts else (torch.float32,)))
         shared_gate = None
         if self.shared_gate is not None:

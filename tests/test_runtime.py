@@ -156,3 +156,11 @@ def test_32_bit_prompts_share_workgroups_only_where_that_was_measured_to_pay():
     layout = StepLayout(57 + 60, 2, 0, [1])
     ctx = StepContext(layout, torch.zeros(layout.total, dtype=torch.int32), torch.float32, [0, 1], [700, 0], [57, 60], None)
     assert ctx.prompt_rows_pay(32, 8, 128) and not ctx.prompt_rows_pay(4, 4, 16)
+
+
+def test_a_routers_product_runs_in_slices_only_where_that_was_measured_to_pay():
+    from synaptix_amd.parts.feedforward import router_slices_pay
+    for tokens, experts in ((1500, 48), (1500, 128), (1500, 256), (40, 256), (16, 48), (16, 128), (8, 8), (8, 128)):
+        assert router_slices_pay(tokens, experts), (tokens, experts)
+    for tokens, experts in ((1, 8), (1, 256), (8, 256), (16, 256), (17, 256), (16, 1024), (100, 1024), (1500, 1024), (4000, 1024)):
+        assert not router_slices_pay(tokens, experts), (tokens, experts)
