@@ -8,6 +8,7 @@
 //   q_nope[h] = q[h][0 .. dim)                                     -> q_nope [N][heads][dim]
 //   q_rot[h]  = rotate(q[h][dim .. dim + rot_dim), p)              -> q_full [N][heads][rank + rot_dim], behind the
 //                                                                    rank places that the absorbed query fills later
+//                                                                    (q_rank = 0: [N][heads][rot_dim], without them)
 // The cache row of the token is [c | k_rot] (k_pages[page][0][token][rank + rot_dim]); c is also written transposed
 // as the row's value (v_pages[page][0][rank][token]; with v_fragments in the order of the bf16 attention kernel's
 // fragments instead).  The rotation turns the pairs (2i, 2i + 1), i < n_pairs, by
@@ -29,7 +30,8 @@ latent_intake_kernel(const float* __restrict__ proj, int width, const float* __r
                      const float* __restrict__ cos_t, const float* __restrict__ sin_t, int n_pairs,
                      T* __restrict__ q_nope, T* __restrict__ q_full, T* __restrict__ k_pages, T* __restrict__ v_pages,
                      const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
-                     const int* __restrict__ tok_pos, int heads, int dim, int rot, int rank, int write_kv, int v_fragments) {
+                     const int* __restrict__ tok_pos, int heads, int dim, int rot, int rank, int q_rank, int write_kv,
+                     int v_fragments) {
   __shared__ float red[16];
   const int tok = blockIdx.x, pos = tok_pos[tok];
   const float* row = proj + (size_t)tok * width;
@@ -49,7 +51,7 @@ latent_intake_kernel(const float* __restrict__ proj, int width, const float* __r
       const float c = cs[e / 2], s = sn[e / 2];
       v = (e & 1) ? src[e] * c + src[e - 1] * s : src[e] * c - src[e + 1] * s;
     }
-    q_full[((size_t)tok * heads + h) * R + rank + e] = from_f32<T>(v);
+    q_full[((size_t)tok * heads + h) * (q_rank + rot) + q_rank + e] = from_f32<T>(v);
   }
   if (!write_kv) return;            // (uniform: no barrier has been reached)
   const float* down = down_rows + (size_t)tok * down_stride;
@@ -86,7 +88,8 @@ latent_intake4_kernel(const float* __restrict__ proj, int width, const float* __
                       const float* __restrict__ cos_t, const float* __restrict__ sin_t, int n_pairs,
                       T* __restrict__ q_nope, T* __restrict__ q_full, T* __restrict__ k_pages, T* __restrict__ v_pages,
                       const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
-                      const int* __restrict__ tok_pos, int heads, int dim, int rot, int rank, int write_kv, int v_fragments) {
+                      const int* __restrict__ tok_pos, int heads, int dim, int rot, int rank, int q_rank, int write_kv,
+                      int v_fragments) {
   typedef T out4 __attribute__((ext_vector_type(4)));
   __shared__ float red[16];
   const int tok = blockIdx.x, tid = threadIdx.x, pos = tok_pos[tok];
@@ -123,7 +126,7 @@ latent_intake4_kernel(const float* __restrict__ proj, int width, const float* __
 #pragma unroll 2
   for (int i = tid; i < heads * rot4; i += 256) {
     const int h = i / rot4, e = (i - h * rot4) * 4;
-    *(out4*)(q_full + ((size_t)tok * heads + h) * R + rank + e) = rounded(turned(*(const f32x4*)(row + h * qd + dim + e), e));
+    *(out4*)(q_full + ((size_t)tok * heads + h) * (q_rank + rot) + q_rank + e) = rounded(turned(*(const f32x4*)(row + h * qd + dim + e), e));
   }
   if (!write_kv) return;            // (uniform: no barrier has been reached)
   T* krow = k_pages + ((size_t)page * SYN_PAGE + slot) * R;
@@ -150,11 +153,12 @@ SYN_EXPORT int syn_latent_intake(const float* proj, int width, const float* down
                                  const float* cos_t, const float* sin_t, int n_pairs, int capacity, int max_position,
                                  void* q_nope, void* q_full, void* k_pages, void* v_pages, int is_f32,
                                  const int* page_table, int table_stride, const int* tok_seq, const int* tok_pos,
-                                 int n_tokens, int heads, int dim, int rot, int rank, int write_kv, int v_fragments,
+                                 int n_tokens, int heads, int dim, int rot, int rank, int q_rank, int write_kv, int v_fragments,
                                  hipStream_t stream) {
   SYN_CHECK(n_tokens > 0 && heads > 0 && dim > 0 && rot >= 0 && rank > 0, "latent_intake: empty input");
   SYN_CHECK(width >= heads * (dim + rot) && down_stride >= rank + rot,
             "latent_intake: rows of %d and %d values do not hold the queries and the latent", width, down_stride);
+  SYN_CHECK(q_rank == rank || q_rank == 0, "latent_intake: %d places in front of the queries' rotated parts", q_rank);
   SYN_CHECK(n_pairs >= 0 && 2 * n_pairs <= rot, "latent_intake: %d rotated pairs in %d values", n_pairs, rot);
   SYN_CHECK(!v_fragments || rank % 16 == 0, "latent_intake: value pages in fragment order need a latent that is a multiple of 16, not %d", rank);
   SYN_CHECK(n_pairs == 0 || (cos_t && sin_t && max_position < capacity),
@@ -166,7 +170,7 @@ SYN_EXPORT int syn_latent_intake(const float* proj, int width, const float* down
 #define SYN_INTAKE4(T)                                                                                                            \
   latent_intake4_kernel<T><<<n_tokens, 256, 0, stream>>>(proj, width, down, down_stride, gain, gain_is_f32, eps, cos_t, sin_t, n_pairs, \
                                                          (T*)q_nope, (T*)q_full, (T*)k_pages, (T*)v_pages, page_table, table_stride,   \
-                                                         tok_seq, tok_pos, heads, dim, rot, rank, write_kv, v_fragments)
+                                                         tok_seq, tok_pos, heads, dim, rot, rank, q_rank, write_kv, v_fragments)
   if (fours && is_f32) SYN_INTAKE4(float);
   else if (fours) SYN_INTAKE4(bf16);
 #undef SYN_INTAKE4
@@ -174,12 +178,12 @@ SYN_EXPORT int syn_latent_intake(const float* proj, int width, const float* down
     latent_intake_kernel<float><<<n_tokens, 256, 0, stream>>>(proj, width, down, down_stride, gain, gain_is_f32, eps, cos_t, sin_t, n_pairs,
                                                               (float*)q_nope, (float*)q_full, (float*)k_pages,
                                                               (float*)v_pages, page_table, table_stride, tok_seq, tok_pos,
-                                                              heads, dim, rot, rank, write_kv, v_fragments);
+                                                              heads, dim, rot, rank, q_rank, write_kv, v_fragments);
   else
     latent_intake_kernel<bf16><<<n_tokens, 256, 0, stream>>>(proj, width, down, down_stride, gain, gain_is_f32, eps, cos_t, sin_t, n_pairs,
                                                              (bf16*)q_nope, (bf16*)q_full, (bf16*)k_pages, (bf16*)v_pages,
                                                              page_table, table_stride, tok_seq, tok_pos, heads, dim, rot,
-                                                             rank, write_kv, v_fragments);
+                                                             rank, q_rank, write_kv, v_fragments);
   SYN_LAUNCH_CHECK("latent_intake");
   return 0;
 }

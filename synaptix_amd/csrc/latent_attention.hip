@@ -631,7 +631,8 @@ __global__ void __launch_bounds__(256, 2)
 latent_expanded_kernel(const bf16* __restrict__ q_nope, const bf16* __restrict__ q_rot, int q_rot_stride, const bf16* __restrict__ keys,
                        const bf16* __restrict__ rotated, const bf16* __restrict__ values, int n_rows,
                        const int* __restrict__ seq_start, const int* __restrict__ seq_past, int n_seqs, bf16* __restrict__ out,
-                       float scale, int nh, int window, const float* __restrict__ gate, int gate_stride, int gate_per_value) {
+                       float scale, int nh, int first_head, int all_heads, int window, const float* __restrict__ gate, int gate_stride,
+                       int gate_per_value) {
   constexpr int KS = (LX_DIM + LX_ROT) / 16, NOPE = SYN_PAGE * LX_DIM * 2, ROT = SYN_PAGE * LX_ROT * 2, BUF = 2 * NOPE + ROT;
   constexpr int DT = LX_DIM / 16, D32 = LX_DIM / 32, NLOAD = BUF / 1024 / 4, AHEAD = 6;
   extern __shared__ __attribute__((aligned(16))) char lds[];      // [2][unrotated keys | rotated keys | values]
@@ -663,7 +664,7 @@ latent_expanded_kernel(const bf16* __restrict__ q_nope, const bf16* __restrict__
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int d = 16 * ks + 8 * hh;
-    const size_t at = (size_t)(tok0 + row) * nh + head;
+    const size_t at = (size_t)(tok0 + row) * all_heads + first_head + head;
     qf[ks] = !valid ? zero8 : ks < LX_DIM / 16 ? *(const bf16x8*)(q_nope + at * LX_DIM + d) : *(const bf16x8*)(q_rot + at * q_rot_stride + d - LX_DIM);
   }
   f32x16 o[D32];
@@ -812,8 +813,8 @@ latent_expanded_kernel(const bf16* __restrict__ q_nope, const bf16* __restrict__
   const float l = l_run + __shfl_xor(l_run, 32, SYN_WAVE);
   if (!valid) return;
   const float inv = 1.f / l;
-  const size_t at = (size_t)(tok0 + row) * nh + head;
-  const float* grow = gate ? gate + (size_t)(tok0 + row) * gate_stride + (gate_per_value ? head * LX_DIM : head) : nullptr;
+  const size_t at = (size_t)(tok0 + row) * all_heads + first_head + head;
+  const float* grow = gate ? gate + (size_t)(tok0 + row) * gate_stride + (first_head + head) * (gate_per_value ? LX_DIM : 1) : nullptr;
   auto sigmoid = [](float z) { return 1.f / (1.f + expf(-z)); };
   const float of_head = gate && !gate_per_value ? sigmoid(grow[0]) : 1.f;
   bf16* orow = out + at * LX_DIM + 4 * hh;
@@ -845,16 +846,17 @@ SYN_EXPORT int syn_latent_rows(const void* k_pages, const int* page_table, int t
   return 0;
 }
 
-// q_nope [N][nh][128]; q_rot: the rotated parts, 64 values every q_rot_stride; keys [n_rows][nh][128], rotated [n_rows][64], values
-// [nh][128][n_rows] (rows as syn_latent_rows leaves them); out [N][nh][128] times sigmoid(gate), gate float rows every gate_stride: one
-// number a head or (gate_per_value) a value, or null.
+// The nh heads from first_head on of all_heads: q_nope [N][all_heads][128]; q_rot: the rotated parts, 64 values every q_rot_stride; keys
+// [n_rows][nh][128], rotated [n_rows][64], values [nh][128][n_rows] (rows as syn_latent_rows leaves them); out [N][all_heads][128] times
+// sigmoid(gate), gate float rows every gate_stride: one number a head or (gate_per_value) a value, or null.
 SYN_EXPORT int syn_latent_expanded(const void* q_nope, const void* q_rot, int q_rot_stride, const void* keys, const void* rotated,
                                    const void* values, int n_rows, const int* seq_start, const int* seq_past, int n_seqs, int n_tokens,
-                                   void* out, float scale, int nh, int dim, int rot, int window, const float* gate, int gate_stride,
-                                   int gate_per_value, hipStream_t stream) {
+                                   void* out, float scale, int nh, int first_head, int all_heads, int dim, int rot, int window,
+                                   const float* gate, int gate_stride, int gate_per_value, hipStream_t stream) {
   SYN_CHECK(dim == LX_DIM && rot == LX_ROT, "latent_expanded: heads of %d + %d values (%d + %d)", dim, rot, LX_DIM, LX_ROT);
   SYN_CHECK(n_seqs > 0 && n_tokens >= n_seqs && nh > 0 && n_rows > 0 && n_rows % SYN_PAGE == 0 && window >= 0 && scale > 0.f,
             "latent_expanded: %d tokens, %d rows, scale %g", n_tokens, n_rows, (double)scale);
+  SYN_CHECK(first_head >= 0 && first_head + nh <= all_heads, "latent_expanded: heads %d to %d of %d", first_head, first_head + nh, all_heads);
   SYN_CHECK(q_rot_stride % 8 == 0 && ((uintptr_t)q_nope | (uintptr_t)q_rot | (uintptr_t)keys | (uintptr_t)rotated | (uintptr_t)values | (uintptr_t)out) % 16 == 0,
             "latent_expanded: operands must be 16-byte aligned");
   SYN_CHECK((size_t)n_rows * LX_DIM * 2 < 0x7fffffffull && (size_t)nh * LX_DIM * 2 * SYN_PAGE < 0x7fffffffull, "latent_expanded: %d rows of %d heads", n_rows, nh);
@@ -868,7 +870,8 @@ SYN_EXPORT int syn_latent_expanded(const void* q_nope, const void* q_rot, int q_
   SYN_CHECK(tiles <= 65535, "latent_expanded: %d tiles", tiles);
   latent_expanded_kernel<<<dim3(nh, tiles), 256, LDS, stream>>>((const bf16*)q_nope, (const bf16*)q_rot, q_rot_stride, (const bf16*)keys,
                                                                 (const bf16*)rotated, (const bf16*)values, n_rows, seq_start, seq_past,
-                                                                n_seqs, (bf16*)out, scale, nh, window, gate, gate_stride, gate_per_value);
+                                                                n_seqs, (bf16*)out, scale, nh, first_head, all_heads, window, gate, gate_stride,
+                                                                gate_per_value);
   SYN_LAUNCH_CHECK("latent_expanded");
   return 0;
 }

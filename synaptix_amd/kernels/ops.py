@@ -1855,8 +1855,8 @@ def latent_v_pages_to_kernel_order(v):
 def latent_intake(proj, gain, eps, cos, sin, q_nope, q_full, k_pages, v_pages, page_table, tok_seq, tok_pos,
                   n_heads, dim, rot_dim, rank, max_position, write_kv=True, v_fragments=False, down=None):
     """From the fused projection proj [N, >= heads * (dim + rot_dim) + rank + rot_dim] float: q_nope [N, heads * dim];
-    the rotated query parts into q_full [N, heads * (rank + rot_dim)] behind each head's first `rank` places; the
-    token's cache row [RMSNorm(latent) * gain | rotated key part] into k_pages [pages, 1, 64, rank + rot_dim] and the
+    the rotated query parts into q_full [N, heads * (rank + rot_dim)] behind each head's first `rank` places (or [N, heads *
+    rot_dim] without them); the token's cache row [RMSNorm(latent) * gain | rotated key part] into k_pages [pages, 1, 64, rank + rot_dim] and the
     normed latent as its value into v_pages [pages, 1, rank, 64].  cos, sin [capacity, pairs]: pairs (2i, 2i + 1) of
     the rotated parts are turned, what lies behind 2 * pairs passes.  v_fragments: the value pages are kept in the order
     of the bf16 attention kernel's fragments (what latent_attention reads when it runs in tiles).
@@ -1881,7 +1881,8 @@ def latent_intake(proj, gain, eps, cos, sin, q_nope, q_full, k_pages, v_pages, p
         if 2 * n_pairs > rot_dim or max_position >= capacity:
             raise KernelError(f"latent_intake: {n_pairs} pairs in {rot_dim} values, position {max_position} of {capacity}")
     _need(q_nope, "latent_intake.q_nope", (_BF16, _F32), (N, n_heads * dim))
-    _need(q_full, "latent_intake.q_full", q_nope.dtype, (N, n_heads * R))
+    q_rank = 0 if isinstance(q_full, torch.Tensor) and q_full.dim() == 2 and q_full.shape[1] == n_heads * rot_dim else rank
+    _need(q_full, "latent_intake.q_full", q_nope.dtype, (N, n_heads * (q_rank + rot_dim)))
     _need(k_pages, "latent_intake.k_pages", q_nope.dtype, (None, 1, PAGE_TOKENS, R))
     _need(v_pages, "latent_intake.v_pages", q_nope.dtype, (k_pages.shape[0], 1, rank, PAGE_TOKENS))
     _need(page_table, "latent_intake.page_table", _I32, (None, None))
@@ -1890,7 +1891,7 @@ def latent_intake(proj, gain, eps, cos, sin, q_nope, q_full, k_pages, v_pages, p
     _call(load_library("core"), "syn_latent_intake", _ptr(proj), width, _ptr(down), down_stride, _ptr(gain), _is_f32(gain), ctypes.c_float(eps),
           _ptr(cos), _ptr(sin), n_pairs, capacity, int(max_position), _ptr(q_nope), _ptr(q_full), _ptr(k_pages),
           _ptr(v_pages), _is_f32(q_nope), _ptr(page_table), page_table.shape[1], _ptr(tok_seq), _ptr(tok_pos), N, n_heads,
-          dim, rot_dim, rank, int(bool(write_kv)), int(bool(v_fragments)), _stream())
+          dim, rot_dim, rank, q_rank, int(bool(write_kv)), int(bool(v_fragments)), _stream())
 
 
 # ----------------------------------------------------------------------------- latent attention
@@ -1904,6 +1905,20 @@ def latent_expanded_rows(past, new, window=0) -> int:
     """Rows of latent_rows for sequences of past[b] cached and new[b] new tokens: whole pages, from the first that some new token sees."""
     return PAGE_TOKENS * sum((p + n + PAGE_TOKENS - 1) // PAGE_TOKENS - (max(0, p - window + 1) // PAGE_TOKENS if window else 0)
                              for p, n in zip(past, new))
+
+
+LATENT_EXPANDED_BYTES = 256 << 20
+
+
+def latent_expanded_heads(rows, n_tokens, n_heads, rank, rot_dim) -> int:
+    """Of how many heads keys and values of so many rows are made at a time: with the rows themselves they take no more memory than the
+    queries and the results in the latent's space, which a step that makes them does without, or than LATENT_EXPANDED_BYTES.  Steps of
+    one layer (4,096 wide, 32 heads, a latent of 512), us and MB at their peak: 1,500 tokens behind 6,000 in one piece 1,190, in the 98 MB
+    that those queries and results take 1,340, absorbed 2,320 (260 MB each); 8,000 tokens, 1,000 each behind 7,000, in one piece 4,900 and
+    1,621 MB, 11 heads at a time 5,190 and 1,257, absorbed 11,160 and 1,257."""
+    budget = max(LATENT_EXPANDED_BYTES, 2 * (2 * n_tokens * n_heads * rank)) - 2 * rows * (rank + rot_dim)
+    groups = -(-n_heads // max(1, budget // (2 * rows * (128 + 128))))
+    return -(-n_heads // groups)
 
 
 def latent_rows(k_pages, page_table, seqs, rank, rot_dim, n_rows, window=0):
@@ -1925,19 +1940,22 @@ def latent_rows(k_pages, page_table, seqs, rank, rot_dim, n_rows, window=0):
     return latent, rotated
 
 
-def latent_expanded_attention(q_nope, q_full, rank, keys, rotated, values, seqs, out, scale, window=0, gate=None, gate_per_value=True):
+def latent_expanded_attention(q_nope, q_full, rank, keys, rotated, values, seqs, out, scale, window=0, gate=None, gate_per_value=True,
+                              first_head=0):
     """Attention of prompts with keys and values of every head's own: q_nope [N, heads, 128] and the rotated parts q_full [N, heads,
-    rank + 64] behind each row's first `rank` places, keys [rows, heads, 128], rotated [rows, 64] (shared by the heads), values
-    [heads, 128, rows], all bf16, rows as latent_rows leaves them; out [N, heads, 128] = sum_j softmax_j(scale (q_nope . k_j + q_rot . r_j))
+    rank + 64] behind each row's first `rank` places (which may be none), keys [rows, k, 128], rotated [rows, 64] (shared by the heads), values
+    [k, 128, rows] of the k heads from first_head on, which are the ones computed, all bf16, rows as latent_rows leaves them; out [N, heads, 128] = sum_j softmax_j(scale (q_nope . k_j + q_rot . r_j))
     v_j  [* sigmoid(gate)] over the keys at or before the query's position (window > 0: the last `window` of them).  gate as in
     heads_product."""
     _need(q_nope, "latent_expanded.q_nope", _BF16, (None, None, 128))
     N, Hn, D = q_nope.shape
     _need(q_full, "latent_expanded.q_full", _BF16, (N, Hn, rank + 64))
-    _need(keys, "latent_expanded.keys", _BF16, (None, Hn, D))
-    n_rows = keys.shape[0]
+    _need(keys, "latent_expanded.keys", _BF16, (None, None, D))
+    n_rows, k = keys.shape[:2]
+    if not (0 <= first_head and 0 < k <= Hn - first_head):
+        raise KernelError(f"latent_expanded: heads {first_head} to {first_head + k} of {Hn}")
     _need(rotated, "latent_expanded.rotated", _BF16, (n_rows, 64))
-    _need(values, "latent_expanded.values", _BF16, (Hn, D, n_rows))
+    _need(values, "latent_expanded.values", _BF16, (k, D, n_rows))
     seq_start, seq_past = seqs
     _need(seq_past, "latent_expanded.seq_past", _I32, (None,))
     B = seq_past.shape[0]
@@ -1948,7 +1966,7 @@ def latent_expanded_attention(q_nope, q_full, rank, keys, rotated, values, seqs,
         ld = _float_rows_view(gate, "latent_expanded.gate", N, Hn * D if gate_per_value else Hn)
     rot_parts = ctypes.c_void_p(q_full.data_ptr() + rank * q_full.element_size())
     _call(load_library("core"), "syn_latent_expanded", _ptr(q_nope), rot_parts, rank + 64, _ptr(keys), _ptr(rotated), _ptr(values), n_rows,
-          _ptr(seq_start), _ptr(seq_past), B, N, _ptr(out), ctypes.c_float(scale), Hn, D, 64, int(window or 0), _ptr(gate), ld,
+          _ptr(seq_start), _ptr(seq_past), B, N, _ptr(out), ctypes.c_float(scale), k, first_head, Hn, D, 64, int(window or 0), _ptr(gate), ld,
           int(bool(gate_per_value)), _stream())
 
 

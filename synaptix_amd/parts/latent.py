@@ -94,10 +94,11 @@ class LatentAttention(Mixer):
         self.w_o = _projection(get(self._n("o")))
         self.gain = get(self._n("down_norm"))
         # W_uk[h] as [rank, dim]: the query's product with it runs along dim
-        self.w_uk_t = get(self._n("up_k")).view(self.nh, self.dim, self.rank).transpose(1, 2).contiguous()
+        up_k = get(self._n("up_k"))
+        self.w_uk_t = up_k.view(self.nh, self.dim, self.rank).transpose(1, 2).contiguous()
         self.w_uv = get(self._n("up_v")).view(self.nh, self.vdim, self.rank).contiguous()
         # ... and for prompts as it is: the latents' product with it runs along the rank
-        self.w_uk = (_projection(get(self._n("up_k")))
+        self.w_uk = (_projection(up_k)
                      if self.w_uv.dtype == torch.bfloat16 and ops.latent_expanded_takes(self.dim, self.rot, self.vdim, self.rank) else None)
 
     def cache_need(self):
@@ -124,16 +125,16 @@ class LatentAttention(Mixer):
             ops.rmsnorm_rows(proj[:, :self.q_rank], self.q_gain, self.norm_eps, c_q)
             queries = linear(c_q, self.w_q_up, torch.float32)
         q_nope = torch.empty((N, nh * dim), dtype=act, device=dev)
-        q_full = torch.empty((N, nh * R), dtype=act, device=dev)
         cos, sin = self.position.tables(dev)
         table = ctx.page_table(cache.group)
         # (bf16 whose sizes the tiles on the matrix cores take: the value pages lie in that kernel's order)
         tiled = act == torch.bfloat16 and ops.latent_attention_tiled(rank, rot)
+        rows = self._expanded_rows(ctx) if tiled else 0
+        q_full = torch.empty((N, nh * (rot if rows else R)), dtype=act, device=dev)
         ops.latent_intake(queries, self.gain, self.norm_eps, cos, sin, q_nope, q_full, cache.k_pages, cache.v_pages, table,
                           ctx.tok_seq, ctx.tok_pos, nh, dim, rot, rank, ctx.max_position, write_kv=owner, v_fragments=tiled,
                           down=proj[:, at:])
         gate = proj[:, at + R:] if self.gate else None
-        rows = self._expanded_rows(ctx) if tiled else 0
         if rows:
             return deferred_product(self._expanded(q_nope, q_full, cache, table, ctx, rows, gate), self.w_o)
         # the query in the latent's space, into the first `rank` places of each head's row
@@ -161,13 +162,18 @@ class LatentAttention(Mixer):
         rows = ops.latent_expanded_rows(ctx.past, ctx.new_counts, self.window or 0)
         return rows if rows <= 8 * ctx.n_tokens else 0
 
-    def _expanded(self, q_nope, q_full, cache, table, ctx, rows, gate):
+    def _expanded(self, q_nope, q_rot, cache, table, ctx, rows, gate):
         N, nh, dim, vdim, seqs = q_nope.shape[0], self.nh, self.dim, self.vdim, (ctx.seq_start, ctx.seq_past)
         latent, rotated = ops.latent_rows(cache.k_pages, table, seqs, self.rank, self.rot, rows, self.window or 0)
-        keys = linear(latent, self.w_uk, latent.dtype)
-        values = torch.empty((nh * vdim, rows), dtype=latent.dtype, device=latent.device)
-        ops.gemm(self.w_uv.view(nh * vdim, self.rank), latent, values)      # (along the keys, as the second product reads them)
         o = torch.empty((N, nh, vdim), dtype=latent.dtype, device=latent.device)
-        ops.latent_expanded_attention(q_nope.view(N, nh, dim), q_full.view(N, nh, -1), self.rank, keys.view(rows, nh, dim), rotated,
-                                      values.view(nh, vdim, rows), seqs, o, self.scale, self.window or 0, gate, self.gate == "value")
+        at_once = ops.latent_expanded_heads(rows, N, nh, self.rank, self.rot)
+        memory = torch.empty((2, rows * at_once * dim), dtype=latent.dtype, device=latent.device)      # (dim and vdim are equal)
+        w_uk, per_head = self.w_uk.data, self.w_uk.data.shape[0] // nh
+        for h in range(0, nh, at_once):
+            k = min(at_once, nh - h)
+            keys, values = memory[0, :rows * k * dim].view(rows, k * dim), memory[1, :rows * k * vdim].view(k * vdim, rows)
+            ops.gemm(latent, w_uk[h * per_head:(h + k) * per_head], keys)
+            ops.gemm(self.w_uv[h:h + k].view(k * vdim, self.rank), latent, values)      # (along the keys, as the second product reads them)
+            ops.latent_expanded_attention(q_nope.view(N, nh, dim), q_rot.view(N, nh, -1), 0, keys.view(rows, k, dim), rotated,
+                                          values.view(k, vdim, rows), seqs, o, self.scale, self.window or 0, gate, self.gate == "value", h)
         return o.view(N, nh * vdim)

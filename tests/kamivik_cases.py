@@ -39,6 +39,8 @@ A1, A2 = "latent_attention", "latent_attention_2"
 # T: no rotated part at all in one layer, nothing turned in the other.
 # U: one expert of four for each token: a choice that the rounding of bfloat16 activations can turn at a near tie of
 #    two logits changes that token's result altogether, so this one is run in 32-bit only.
+# V: heads of 128 + 64 over 128 values and a latent of 128: the sizes at which steps of many tokens make keys and values of every
+#    head; a gate a head on the layer that sees everything, a gate a value on the one with a window of 70.
 CONFIGS = {
     "P": config(300, 64, [layer(A2, 4, 16, 8, 24, 32, window=20, ff=48, experts=6, top=2, dims=4),
                           layer(A1, 2, 32, 16, 16, 48, ff=None, base=500.0),
@@ -54,8 +56,10 @@ CONFIGS = {
                           layer(A2, 2, 8, 8, 8, 16, window=33, ff=32, experts=4, top=3, dims=0)]),
     "U": config(150, 56, [layer(A1, 2, 8, 8, 12, 16, ff=24, experts=4, top=1),
                           layer(A2, 2, 12, 4, 8, 20, window=7, ff=40, experts=6, top=1)], mult=0.9),
+    "V": config(260, 96, [layer(A1, 3, 128, 64, 128, 128, ff=None, scale=2.0 * 192 ** -0.5),
+                          layer(A2, 2, 128, 64, 128, 128, window=70, ff=None, dims=20, scale=2.0 * 192 ** -0.5)]),
 }
-SEEDS = {"P": 21, "Q": 22, "R": 23, "S": 24, "T": 25, "U": 26}
+SEEDS = {"P": 21, "Q": 22, "R": 23, "S": 24, "T": 25, "U": 26, "V": 27}
 
 
 def dtypes_of(name: str) -> list:

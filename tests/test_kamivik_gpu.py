@@ -423,8 +423,8 @@ def test_latent_intake_of_wide_rows_four_values_at_a_time(H, D, B, C, pairs, spa
     cos, sin = RotaryInterleaved(70.0, 2 * pairs, 128).tables(DEV) if pairs else (None, None)
     seq_d, pos_d = (torch.tensor(t, dtype=torch.int32, device=DEV) for t in (seqs, pos))
 
-    def run(rows, down=None, write=True, fragments=False):
-        out = [torch.full((N, H * D), 5.0, dtype=dtype, device=DEV), torch.full((N, H * R), 9.0, dtype=dtype, device=DEV),
+    def run(rows, down=None, write=True, fragments=False, parts=False):
+        out = [torch.full((N, H * D), 5.0, dtype=dtype, device=DEV), torch.full((N, H * (B if parts else R)), 9.0, dtype=dtype, device=DEV),
                torch.zeros((4, 1, 64, R), dtype=dtype, device=DEV), torch.zeros((4, 1, C, 64), dtype=dtype, device=DEV)]
         ops.latent_intake(rows, gain.to(dtype).to(DEV), 1e-5, cos, sin, *out, table, seq_d, pos_d, H, D, B, C, max(pos), write_kv=write,
                           v_fragments=fragments, down=down)
@@ -449,6 +449,9 @@ def test_latent_intake_of_wide_rows_four_values_at_a_time(H, D, B, C, pairs, spa
     assert all(torch.equal(a, b) for a, b in zip(split, got))
     left = run(whole, write=False)
     assert torch.equal(left[0], got[0]) and torch.equal(left[1], got[1]) and not bool(left[2].any()) and not bool(left[3].any())
+    if B:         # the queries' rotated parts without the places for the absorbed ones
+        assert all(torch.equal(run(r, parts=True)[1].view(N, H, B), full[1].view(N, H, R)[..., C:])
+                   for r, full in ((whole, got), (torch.cat([whole, torch.zeros(N, 1, device=DEV)], 1), general)))
     if C % 16 == 0:
         assert torch.equal(run(whole, fragments=True)[3], ops.latent_v_pages_to_kernel_order(got[3]))
 
@@ -509,6 +512,56 @@ def test_portions_of_several_sizes(name, dtype):
         at += n
     assert at == len(toks)
     assert_logits_close(torch.cat(got), want, dtype, f"{name} {dtype} in portions", sharp=True)
+
+
+# steps of (slot, tokens) over four requests, and how many of the model's two layers make keys and values of every head in each: whole
+# prompts together, one of a single token; a portion behind cached tokens, past the window, with single tokens beside it; more cached
+# rows than eight a new token; fewer than 129 tokens
+EXPANDED_STEPS = [([(0, 300)], 2), ([(1, 70), (2, 64), (3, 1)], 2), ([(0, 1), (1, 150), (2, 1), (3, 20)], 2), ([(0, 1), (1, 140), (3, 129)], 2),
+                  ([(0, 100), (2, 28)], 0), ([(1, 1), (2, 129)], 2), ([(0, 500)], 2), ([(0, 130), (1, 1)], 1)]
+
+
+@pytest.mark.parametrize("limit", [None, 0])
+def test_keys_and_values_of_every_head_against_the_plain_model_and_the_absorbed_layers(limit, monkeypatch):
+    """Layers of 128 + 64 over 128 in steps that take either form: against the plain model with the bounds of bf16, and against the same
+    steps with the up-projections absorbed in every layer, which round other numbers the same way: the two may differ by as much as
+    either does from the plain model.  limit 0: as few heads at a time as the absorbed layers' memory holds."""
+    from synaptix_amd.kernels import ops
+    from synaptix_amd.parts import LatentAttention
+    if limit is not None:
+        monkeypatch.setattr(ops, "LATENT_EXPANDED_BYTES", limit)
+    expanded, calls, heads = LatentAttention._expanded, [], []
+    monkeypatch.setattr(LatentAttention, "_expanded", lambda *a: (calls.append(1), expanded(*a))[1])
+    one = ops.latent_expanded_attention
+    monkeypatch.setattr(ops, "latent_expanded_attention", lambda *a: (heads.append(a[3].shape[1]), one(*a))[1])
+
+    def run():
+        eng = engine("V", "bfloat16", max_tokens=4096)
+        eng.prompt_graphs = False
+        slots, fed, got, took = [eng.acquire() for _ in range(4)], [0] * 4, [[] for _ in range(4)], []
+        for step, _ in EXPANDED_STEPS:
+            calls.clear()
+            out = eng.step([(slots[r], toks[r][fed[r]:fed[r] + n]) for r, n in step], want="all")
+            took.append(len(calls))
+            for (r, n), rows in zip(step, out.split([n for _, n in step])):
+                got[r].append(rows.float().cpu())
+                fed[r] += n
+        eng.cache.check()
+        return [torch.cat(g) for g in got], took
+    totals = [sum(n for step, _ in EXPANDED_STEPS for r, n in step if r == i) for i in range(4)]
+    toks = [tokens_for("V", n, 40 + i) for i, n in enumerate(totals)]
+    got, took = run()
+    assert took == [n for _, n in EXPANDED_STEPS]
+    assert (max(heads) < 3 and 1 in heads) if limit == 0 else set(heads) == {2, 3}
+    monkeypatch.setattr(LatentAttention, "_expanded_rows", lambda self, ctx: 0)
+    absorbed, took = run()
+    assert not any(took)
+    for i in range(4):
+        want = plain_logits("V", toks[i]).float()
+        assert_logits_close(got[i], want, "bfloat16", f"request {i}")
+        rms = lambda t: float(t.pow(2).mean().sqrt())
+        far, other, apart = rms(got[i] - want), rms(absorbed[i] - want), rms(got[i] - absorbed[i])
+        assert apart <= 1.5 * (far + other) and far <= 1.25 * other, (i, far, other, apart)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

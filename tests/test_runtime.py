@@ -164,3 +164,20 @@ def test_a_routers_product_runs_in_slices_only_where_that_was_measured_to_pay():
         assert router_slices_pay(tokens, experts), (tokens, experts)
     for tokens, experts in ((1, 8), (1, 256), (8, 256), (16, 256), (17, 256), (16, 1024), (100, 1024), (1500, 1024), (4000, 1024)):
         assert not router_slices_pay(tokens, experts), (tokens, experts)
+
+
+def test_keys_and_values_of_latent_prompts_stay_within_their_memory():
+    """Whatever the step: what the heads' keys and values take at a time, with the rows that they are made from, is no more than the limit
+    or the queries and results in the latent's space that the step does without, down to one head; every head is computed; steps below the limit go in one piece."""
+    from synaptix_amd.kernels import ops
+    for heads in (1, 2, 3, 8, 32, 128):
+        for rank in (128, 512):
+            for tokens in (129, 1500, 8000, 16000, 60000):
+                for ratio in (1, 3, 8):
+                    rows = tokens * ratio // 64 * 64
+                    k = ops.latent_expanded_heads(rows, tokens, heads, rank, 64)
+                    assert 1 <= k <= heads
+                    taken = 512 * rows * k + 2 * rows * (rank + 64)
+                    assert k == 1 or taken <= max(ops.LATENT_EXPANDED_BYTES, 4 * tokens * heads * rank), (heads, rank, tokens, ratio, k)
+                    assert k == heads or 512 * rows * heads + 2 * rows * (rank + 64) > ops.LATENT_EXPANDED_BYTES
+    assert ops.latent_expanded_heads(128000, 16000, 32, 512, 64) == 11 and ops.latent_expanded_heads(15232, 7000, 32, 512, 64) == 32
