@@ -996,8 +996,9 @@ static int launch_direct(const bf16* x, Weight w, void* out, Epilogue ep, int M,
 }
 
 // ------------------------------------------------------------------ 17 to 128 rows, W in fragment order: operands straight to registers
-// What bounds it: the stream of W, of which a compute unit has to keep some 64 KB under way.  Through a ring of LDS buffers W shares
-// the room with x (36 KB of it under way beside 96 rows of x), and every k-tile ends in a barrier.  Here the four waves of a workgroup
+// What bounds it: what a compute unit brings in, W and x together (13 to 15 bytes a clock), and W's stream from memory, of which a unit
+// has to keep some 64 KB under way.  Through a ring of LDS buffers W shares the room with x (36 KB of it under way beside 96 rows
+// of x), and every k-tile ends in a barrier.  Here the four waves of a workgroup
 // (one a SIMD, all 512 registers) split K, and each takes all rows of x and all 16 NF rows of W of the workgroup: a fragment of
 // either is loaded once a workgroup, straight into the registers of the one wave that multiplies it, S steps of 32 k-values ahead;
 // no barrier and no LDS until the waves' sums are added at the end, in the order of the waves.  x comes from the L2s, as many
@@ -1010,9 +1011,12 @@ __global__ void __launch_bounds__(256, 1)
 gemm_rows_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void* __restrict__ out, Epilogue ep, int M, int N, int K,
                  int k_slice) {
   static_assert(NF % 2 == 0 && S % 2 == 0, "fragments of W in pairs (gate and up), steps in pairs (a line of x)");
-  constexpr int FRAGS = NF * FM, CHUNK = FRAGS <= 36 ? FRAGS : FRAGS / 2;      // fragments of sums that pass through LDS at a time
-  static_assert(FRAGS % CHUNK == 0 && CHUNK % 2 == 0 && CHUNK <= 36, "the waves' sums in LDS");
-  extern __shared__ f32x4 part[];      // [4][CHUNK][64]
+  constexpr int FRAGS = NF * FM;
+  static_assert(4 * FRAGS * SYN_WAVE * 16 <= 160 * 1024, "the waves' sums in LDS");
+  // (256 vector registers beside the 256 of the sums.  With more, operands move between the two files next to the matrix
+  // instructions, which the compiler does not know for what they are: 288 gave wrong results)
+  static_assert(S * (NF + FM) * 4 <= 224 && FRAGS * 4 <= 256, "operands and sums in the registers of one wave a SIMD");
+  extern __shared__ f32x4 part[];      // [4][FRAGS][64]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE), lane = threadIdx.x % SYN_WAVE, r16 = lane % 16, g = lane / 16;
   const int n0 = (int)blockIdx.x * 16 * NF, k_begin = (int)blockIdx.y * k_slice;
   const int pairs = max(0, min(K - k_begin, k_slice)) / 64, steps = 2 * max(0, (pairs - wave + 3) / 4);
@@ -1067,44 +1071,40 @@ gemm_rows_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void* 
   for (int i = 0; i < NF; ++i)
 #pragma unroll
     for (int j = 0; j < FM; ++j) asm volatile("" : "+a"(acc[i][j]));
+  // fragment f: rows 2 (f / 2 / FM) + f % 2 of W (gate and up side by side), rows f / 2 % FM of x
 #pragma unroll
-  for (int c = 0; c < FRAGS / CHUNK; ++c) {
-    // fragment f: rows 2 (f / 2 / FM) + f % 2 of W (gate and up side by side), rows f / 2 % FM of x
-    if (c) __syncthreads();
+  for (int f = 0; f < FRAGS; ++f) {
+    const int q = f / 2;
+    part[(wave * FRAGS + f) * SYN_WAVE + lane] = acc[2 * (q / FM) + f % 2][q % FM];
+  }
+  __syncthreads();
+  for (int q = wave; q < FRAGS / 2; q += 4) {
+    f32x4 v[2];
 #pragma unroll
-    for (int f = 0; f < CHUNK; ++f) {
-      const int q = (c * CHUNK + f) / 2;
-      part[(wave * CHUNK + f) * SYN_WAVE + lane] = acc[2 * (q / FM) + f % 2][q % FM];
+    for (int h = 0; h < 2; ++h) {
+      v[h] = part[(2 * q + h) * SYN_WAVE + lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) v[h] += part[(w * FRAGS + 2 * q + h) * SYN_WAVE + lane];
     }
-    __syncthreads();
-    for (int q = wave; q < CHUNK / 2; q += 4) {
-      f32x4 v[2];
+    const int m = 16 * (q % FM) + r16, n = n0 + 32 * (q / FM) + 4 * g;
+    if (m >= M) continue;
+    if constexpr (PAIRED) {
+      bf16x4 r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = (bf16)gated(ep.act, v[0][e], v[1][e], ep.limit);
+      const int col = n0 / 2 + 16 * (q / FM) + 4 * g;
+      if (n < N) *(bf16x4*)((bf16*)out + (size_t)m * (N / 2) + col) = r;
+    } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        v[h] = part[(2 * q + h) * SYN_WAVE + lane];
-#pragma unroll
-        for (int w = 1; w < 4; ++w) v[h] += part[(w * CHUNK + 2 * q + h) * SYN_WAVE + lane];
-      }
-      const int pair = c * CHUNK / 2 + q, m = 16 * (pair % FM) + r16, n = n0 + 32 * (pair / FM) + 4 * g;
-      if (m >= M) continue;
-      if constexpr (PAIRED) {
+        if (n + 16 * h >= N) continue;
+        const size_t at = ((size_t)blockIdx.y * M + m) * N + n + 16 * h;
+        f32x4 o;
         bf16x4 r;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = (bf16)gated(ep.act, v[0][e], v[1][e], ep.limit);
-        const int col = n0 / 2 + 16 * (pair / FM) + 4 * g;
-        if (n < N) *(bf16x4*)((bf16*)out + (size_t)m * (N / 2) + col) = r;
-      } else {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (n + 16 * h >= N) continue;
-          const size_t at = ((size_t)blockIdx.y * M + m) * N + n + 16 * h;
-          f32x4 o;
-          bf16x4 r;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = point_activation(ep.point, v[h][e]), r[e] = (bf16)o[e];
-          if (ep.out_is_f32) *(f32x4*)((float*)out + at) = o;
-          else *(bf16x4*)((bf16*)out + at) = r;
-        }
+        for (int e = 0; e < 4; ++e) o[e] = point_activation(ep.point, v[h][e]), r[e] = (bf16)o[e];
+        if (ep.out_is_f32) *(f32x4*)((float*)out + at) = o;
+        else *(bf16x4*)((bf16*)out + at) = r;
       }
     }
   }
@@ -1112,7 +1112,7 @@ gemm_rows_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void* 
 
 template <int NF, int FM, int S, bool PAIRED>
 static int launch_rows_tile(const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K, int slices, hipStream_t stream) {
-  constexpr int CHUNK = NF * FM <= 36 ? NF * FM : NF * FM / 2, LDS = 4 * CHUNK * SYN_WAVE * 16;
+  constexpr int LDS = 4 * NF * FM * SYN_WAVE * 16;
   static OncePerDevice raised;
   const hipError_t e = once_per_device(raised, [&] {
     return hipFuncSetAttribute((const void*)gemm_rows_kernel<NF, FM, S, PAIRED>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);

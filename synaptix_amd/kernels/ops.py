@@ -340,11 +340,14 @@ def _bytes_a_unit(M, tile, K, slices, tiles, units, shared):
     return rounds * (tile + M) * (-(-K // (64 * slices)) * 64) * 2 + (8 * slices * M * tile * tiles / units if slices > 1 else 0)
 
 
-def _rows_choice(M, N, K, slices, gated):
+def _rows_choice(M, N, K, slices):
     """(bytes a compute unit, groups of 16 rows of W a workgroup, slices of K) of gemm_rows_kernel for a product in `slices` slices (None:
     the best), its workgroups going round once; None where it does not."""
     units, best = compute_units(), None
-    if N * K < 1 << 19:      # (less than 1 MB of W: a launch's time whatever the tiles)
+    # Less than 1 MB of W keeps the other tiles, and with them the order of its sums: small models with routers decide near ties by it, for
+    # a gain of a few microseconds (us here and there: 17 rows, 512 x 512 gated 4.5 and 6.2, 1,024 x 256 plain with its norm 6.8 and 7.3;
+    # 128 rows, 512 x 512 gated 9.1 and 13.4, plain 10.9 and 10.2).
+    if N * K < 1 << 19:
         return None
     for nf in (2, 4, 6):
         if M > {2: 128, 4: 96, 6: 48}[nf]:
@@ -364,12 +367,15 @@ def _tiles_bytes(M, N, K, slices, gated):
 
 
 def _rows_pay(new, old, M, gated):
-    """Both are bound by the bytes that a compute unit brings in, W's stream and x from the L2s; through a ring of LDS buffers they come
-    in a little faster from 33 rows of x on, where the registers hold fewer steps.  Measured, us (this kernel, tiles, ratio of the
-    bytes): gated 24,576 x 4,096 with 24 rows 39.2, 43.7, 0.91, with 48 42.4, 43.0, 0.82, with 64 46.3, 45.7; 16,384 x 2,048 with 64 20.5,
-    22.7, 0.67, with 128 28.7, 27.5, 0.86; 8,192 x 1,024 with 128 14.3, 17.8, 0.71; plain 2,560 x 9,728 with 24 11.9, 15.1, 0.68, with
-    64 17.0, 16.3, 0.85; 6,144 x 2,560 with 32 9.7, 10.2, 0.9; 4,096 x 12,288 with 32 20.5, 19.6, 1.0; 2,048 x 2,048 with 48 5.8, 7.5, 0.45, with
-    128 9.2, 10.6, 0.63; 1,024 x 4,096 with 96 7.8, 10.2, 0.57; 6,144 x 2,048 with 48 10.1, 9.5, 0.82."""
+    """Both bring W and x in at 13 to 16 bytes a clock a compute unit, x from the L2s or not (24,576 x 4,096 with two groups of W a workgroup,
+    16 to 128 rows of x: 35 to 113 us, 14.0 to 14.6 bytes; the tiles with 48 to 128 rows 41 to 47 us, 14 to 16), and W alone from memory at
+    5.7 TB/s.  Where the bytes of one come near the time of the other they hide each other in part only (six groups, a workgroup a unit,
+    16 to 48 rows: 36 to 40 us, 10.5 to 12.4 bytes a clock), through registers less than through a ring of LDS buffers, which keeps
+    more of W under way beside many rows of x.  So this kernel has to bring in fewer bytes, the fewer the more rows.  Measured, us (this
+    kernel, tiles, ratio of the bytes): gated 24,576 x 4,096 with 24 rows 39.2, 43.7, 0.91, with 48 42.4, 43.0, 0.82, with 64 46.3, 45.7;
+    16,384 x 2,048 with 64 20.5, 22.7, 0.67, with 128 28.7, 27.5, 0.86; 8,192 x 1,024 with 128 14.3, 17.8, 0.71; plain 2,560 x 9,728 with 24
+    11.9, 15.1, 0.68, with 64 17.0, 16.3, 0.85; 6,144 x 2,560 with 32 9.7, 10.2, 0.9; 4,096 x 12,288 with 32 20.5, 19.6, 1.0; 2,048 x 2,048 with 48
+    5.8, 7.5, 0.45, with 128 9.2, 10.6, 0.63; 1,024 x 4,096 with 96 7.8, 10.2, 0.57; 6,144 x 2,048 with 48 10.1, 9.5, 0.82."""
     return new <= (0.95 if M <= 32 and gated else 0.9 if M <= 32 else 0.75 if gated else 0.65) * old
 
 
@@ -378,7 +384,7 @@ def rows_tile(M, N, K, slices, gated=False) -> int:
     """Groups of 16 rows of W that a workgroup of gemm_rows_kernel takes for this product in so many slices, 0: it takes other tiles."""
     if M > ROWS_MAX or M <= (PACKED_MAX_ROWS_GATED if gated else PACKED_MAX_ROWS) or K % 128 or N % 16:
         return 0
-    new = _rows_choice(M, N, K, slices, gated)
+    new = _rows_choice(M, N, K, slices)
     if new is None or slices > 1 and slices != rows_slices(M, N, K):
         return 0
     return new[1] if slices > 1 or _rows_pay(new[0], _tiles_bytes(M, N, K, 1, gated), M, gated) else 0
@@ -390,7 +396,7 @@ def rows_slices(M, N, K) -> int:
     the slices of gemm_slices)."""
     if M > ROWS_MAX or M <= PACKED_MAX_ROWS or K % 128 or N % 16:
         return 0
-    new = _rows_choice(M, N, K, None, False)
+    new = _rows_choice(M, N, K, None)
     return new[2] if new is not None and _rows_pay(new[0], _tiles_bytes(M, N, K, gemm_slices(M, N, K, _BF16), False), M, False) else 0
 
 

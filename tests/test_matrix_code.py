@@ -42,7 +42,7 @@ def kernels_of(source, kernel, folder):
 STREAMED = [("gemm.hip", "gemm_stream_kernel"), ("grouped.hip", "grouped_stream_kernel")]
 
 
-@pytest.mark.parametrize("source,kernel", STREAMED)
+@pytest.mark.parametrize("source,kernel", STREAMED + [("gemm.hip", "gemm_rows_kernel")])
 def test_no_sum_moves_between_matrix_instructions(source, kernel, folder):
     for name, body in kernels_of(source, kernel, folder):
         matrix = [i for i, l in enumerate(body) if "v_mfma" in l]
