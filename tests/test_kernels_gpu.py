@@ -1729,6 +1729,70 @@ def test_filter_rows_counts_in_memory_of_any_content(ops):
     assert got == want
 
 
+def _sampled(monkeypatch, ops, rows, configs, either):
+    """The tokens of sample_batch over `rows` (a list of batches of logits, a step each) for samplers of these configurations, on the
+    route that its rule picks (either: on the two kernels whatever it picks), and how often ops.draw_top_k ran."""
+    from synaptix_amd.sampling import SequenceSampler, sample_batch, sampler
+    calls, draw = [], ops.draw_top_k
+    with monkeypatch.context() as m:
+        m.setattr(ops, "draw_top_k", lambda *a: (calls.append(1), draw(*a))[1])
+        if either:
+            m.setattr(sampler, "_shared_top_k", lambda *a: 0)
+        samplers = [SequenceSampler(c, list(range(30 * i, 30 * i + 40)) * 3, 11 * i) for i, c in enumerate(configs)]
+        return [sample_batch(x, samplers) for x in rows], len(calls)
+
+
+_MIXED = [dict(temperature=0.7, top_p=0.9, repetition_penalty=1.3), dict(temperature=1.4, min_p=0.05, presence_penalty=0.7),
+          dict(temperature=0.0, frequency_penalty=0.4), dict(temperature=0.9, top_p=0.6, min_p=0.02, frequency_penalty=-0.3, repeat_last_n=25),
+          dict(temperature=1.0), dict(temperature=0.0, top_p=0.3, repetition_penalty=1.2, presence_penalty=-0.5, repeat_last_n=7),
+          dict(temperature=1.0, top_p=0.0), dict(temperature=0.8, top_p=1.5, min_p=1.0), dict(temperature=1e-30, top_p=0.9),
+          dict(temperature=50.0, top_p=0.97, min_p=-1.0, repetition_penalty=0.5), dict(temperature=0.0, repetition_penalty=1e-3, presence_penalty=1e30)]
+
+
+@pytest.mark.parametrize("V", [32768, 33001, 151936])
+def test_sample_batch_gives_the_same_tokens_over_slices_and_by_whole_rows(ops, monkeypatch, V):
+    """Rows that differ in every option (a column handed over as another would show), with tokens that are penalised again in later steps;
+    no row drawn from; a row without top-k or with one too large, which takes the batch to whole rows; sixty rows."""
+    from synaptix_amd.sampling import GenerationConfig
+    ks = [50, 1, 7, 128, 3, 64, 20, 5, 2, 100, 9]
+    mixed = [GenerationConfig(top_k=k, **o) for k, o in zip(ks, _MIXED)]
+    greedy = [GenerationConfig(top_k=k, **dict(o, temperature=0.0)) for k, o in zip(ks, _MIXED)]
+    for n, (configs, routed) in enumerate([(mixed, True), (greedy, True), (mixed * 6, True),
+                                           (mixed[:3] + [GenerationConfig(temperature=0.9, top_p=0.8)], False),
+                                           ([GenerationConfig(top_k=min(V // 128, 512), **o) for o in _MIXED], True),
+                                           ([GenerationConfig(top_k=min(V // 128, 512) + 1, **o) for o in _MIXED], False),
+                                           ([GenerationConfig(top_k=V // 256, **dict(o, temperature=0.0)) for o in _MIXED], V // 256 <= 512),
+                                           ([GenerationConfig(top_k=V // 256 + 1, **dict(o, temperature=0.0)) for o in _MIXED], False)]):
+        rows = [rnd((len(configs), V), 170 + 10 * n + i, scale=2.5).to(DEV) for i in range(4)]
+        rows[1] = rows[1].round()
+        got, calls = _sampled(monkeypatch, ops, rows, configs, False)
+        want, none = _sampled(monkeypatch, ops, rows, configs, True)
+        assert got == want and calls == (len(rows) if routed else 0) and none == 0, n
+
+
+@pytest.mark.parametrize("route", ["slices", "whole rows"])
+def test_sample_batch_from_two_threads_on_two_streams(ops, monkeypatch, route):
+    """Calls that may be under way at once, on each route, give what the two kernels give one call after another."""
+    import threading
+    from synaptix_amd.sampling import GenerationConfig, sampler
+    cfg = GenerationConfig(temperature=0.8, top_k=40, top_p=0.9, repetition_penalty=1.3, frequency_penalty=0.2)
+    rows = [[rnd((8, 33000), 180 + i, scale=3.0).to(DEV)] * 20 for i in range(2)]
+    want = [_sampled(monkeypatch, ops, r, [cfg] * 8, True)[0] for r in rows]
+    if route == "whole rows":
+        monkeypatch.setattr(sampler, "_shared_top_k", lambda *a: 0)
+    from synaptix_amd.sampling import SequenceSampler, sample_batch
+    side = [[SequenceSampler(cfg, list(range(30 * i, 30 * i + 40)) * 3, 11 * i) for i in range(8)] for _ in range(2)]
+    got = [None, None]
+    torch.cuda.synchronize()
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got[i] = [sample_batch(x, side[i]) for x in rows[i]]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads], [t.join() for t in threads]
+    assert got == want
+
+
 def test_filter_rows_with_equal_values(ops):
     """Equal values at the k-th place and at the boundary of the probability mass: of equal entries the first in
     index order stay, so that top-k keeps exactly k; rows of one value only; rows that are -inf but for a few."""
