@@ -763,3 +763,33 @@ def test_a_plain_32_bit_layer_in_one_call_gives_what_its_parts_give(kw, monkeypa
     eng.model.blocks[1].feed_forward.__class__ = GatedMlp
     eng.model.blocks[1].feed_forward.forward = lambda h, ctx: 2 * GatedMlp.forward(eng.model.blocks[1].feed_forward, h, ctx)
     assert all(torch.equal(a, b) for a, b in zip(run(), other))
+
+
+def test_captured_32_bit_steps_take_the_layers_one_call_with_the_bits_of_their_parts(monkeypatch):
+    """A captured decode step records the layers' one call like an eager one: every replay has the bits of the eager step whose layers run
+    part by part, with eager work and synchronisations between the replays and rows of padding beside the sequences."""
+    from synaptix_amd import Engine, Qwen3Config
+    from synaptix_amd.parts import PreNormBlock
+    cfg = Qwen3Config(vocab_size=300, hidden_size=64, intermediate_size=176, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                      head_dim=16, max_position_embeddings=256, rope_theta=1e4, rms_norm_eps=1e-6, tie_word_embeddings=False, eos_token_id=None)
+    g = torch.Generator().manual_seed(6)
+    prompts = [torch.randint(0, 300, (n,), generator=g).tolist() for n in (5, 61, 100)]
+    tokens = [torch.randint(0, 300, (3,), generator=g).tolist() for _ in range(8)]
+    one, calls = PreNormBlock._whole_layer, []
+    counted = lambda *a: (calls.append(one(*a)), calls[-1])[1]
+    monkeypatch.setattr(PreNormBlock, "_whole_layer", counted)
+    graph, parts = (Engine.from_config(cfg, seed=3, dtype="float32", max_tokens=1024) for _ in range(2))
+    slots = [[e.acquire() for _ in prompts] for e in (graph, parts)]
+    graph.step(list(zip(slots[0], prompts)), want=None)
+    calls.clear()
+    runner = graph.decode_runner(3, 200)
+    got = []
+    for row in tokens:
+        got.append(runner.step(slots[0], row)[1].clone())
+        torch.cuda.synchronize()
+    assert calls and all(c is not None for c in calls)
+    monkeypatch.setattr(PreNormBlock, "_whole_layer", lambda *a: None)
+    parts.step(list(zip(slots[1], prompts)), want=None)
+    for row, replay in zip(tokens, got):
+        eager = parts.step([(s, [t]) for s, t in zip(slots[1], row)], want="last")
+        assert torch.equal(replay[:3], eager)
