@@ -96,7 +96,7 @@ class StepContext:
         """ops.prompt_rows_pay of the step's lengths and a layer's (heads, kv heads, head size), looked at once a step."""
         known = self._prompt_rows.get(heads)
         if known is None:
-            known = not self.one_token_each and ops.prompt_rows_pay(self.past, self.new_counts, *heads)
+            known = ops.prompt_rows_pay(self.past, self.new_counts, *heads)
             self._prompt_rows[heads] = known
         return known
 

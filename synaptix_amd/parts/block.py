@@ -114,7 +114,7 @@ class PreNormBlock(Block):
                               a.window or 0, terms["softcap"], terms["slopes"], a.nh, a.nkv, a.hd),
                              (n2.gain, n2.eps, n2.gain_offset), (f.w_gate_up.plain, f.w_down.plain, f.intermediate, f.activation),
                              (cache.k_pages, cache.v_pages), ctx.page_table(cache.group), ctx.tok_seq, ctx.tok_pos, owner,
-                             ctx.prompt_rows_pay(a.nh, a.nkv, a.hd))
+                             not ctx.one_token_each and ctx.prompt_rows_pay(a.nh, a.nkv, a.hd))
 
     def forward(self, resid, pending, ctx, cache, owner=True):
         if ctx.act_dtype == torch.float32:

@@ -159,7 +159,7 @@ class GqaAttention(Mixer):
                                   write_kv=owner, gain_offset=self.qk_gain_offset)
         if act == torch.float32:
             if h.is_cuda:
-                terms["prompts"] = ctx.prompt_rows_pay(nh, nkv, hd)
+                terms["prompts"] = not ctx.one_token_each and ctx.prompt_rows_pay(nh, nkv, hd)
             ops.attention_f32(q, cache.k_pages, cache.v_pages, table, ctx.tok_seq, ctx.tok_pos, o, self.scale, window,
                               nh, nkv, hd, **terms)
         elif ctx.one_token_each:
