@@ -1729,7 +1729,7 @@ def test_filter_rows_counts_in_memory_of_any_content(ops):
     assert got == want
 
 
-def _sampled(monkeypatch, ops, rows, configs, either):
+def _sampled_tokens(monkeypatch, ops, rows, configs, either):
     """The tokens of sample_batch over `rows` (a list of batches of logits, a step each) for samplers of these configurations, on the
     route that its rule picks (either: on the two kernels whatever it picks), and how often ops.draw_top_k ran."""
     from synaptix_amd.sampling import SequenceSampler, sample_batch, sampler
@@ -1765,8 +1765,8 @@ def test_sample_batch_gives_the_same_tokens_over_slices_and_by_whole_rows(ops, m
                                            ([GenerationConfig(top_k=V // 256 + 1, **dict(o, temperature=0.0)) for o in _MIXED], False)]):
         rows = [rnd((len(configs), V), 170 + 10 * n + i, scale=2.5).to(DEV) for i in range(4)]
         rows[1] = rows[1].round()
-        got, calls = _sampled(monkeypatch, ops, rows, configs, False)
-        want, none = _sampled(monkeypatch, ops, rows, configs, True)
+        got, calls = _sampled_tokens(monkeypatch, ops, rows, configs, False)
+        want, none = _sampled_tokens(monkeypatch, ops, rows, configs, True)
         assert got == want and calls == (len(rows) if routed else 0) and none == 0, n
 
 
@@ -1777,7 +1777,7 @@ def test_sample_batch_from_two_threads_on_two_streams(ops, monkeypatch, route):
     from synaptix_amd.sampling import GenerationConfig, sampler
     cfg = GenerationConfig(temperature=0.8, top_k=40, top_p=0.9, repetition_penalty=1.3, frequency_penalty=0.2)
     rows = [[rnd((8, 33000), 180 + i, scale=3.0).to(DEV)] * 20 for i in range(2)]
-    want = [_sampled(monkeypatch, ops, r, [cfg] * 8, True)[0] for r in rows]
+    want = [_sampled_tokens(monkeypatch, ops, r, [cfg] * 8, True)[0] for r in rows]
     if route == "whole rows":
         monkeypatch.setattr(sampler, "_shared_top_k", lambda *a: 0)
     from synaptix_amd.sampling import SequenceSampler, sample_batch
