@@ -732,8 +732,8 @@ def _mostly_prompts(n_tokens, page_table) -> bool:
 
 def prompt_rows_pay(past, new, n_heads, n_kv_heads, head_dim) -> bool:
     """Whether 32-bit attention of sequences with past[b] cached and new[b] new tokens is faster 16 (token, head) rows a workgroup than a
-    wave a row, which it is where it looks a seventh faster in estimates that are wrong by a tenth at the median and by a quarter in one
-    case of ten.  A wave a row: so many blocks of 64 keys a microsecond for all rows, and the longest row's own.  16 rows: a block is
+    wave a row, by estimates of both.  Of 500 drawn steps (1 to 24 sequences, prompts, portions and single tokens among them, 14 shapes) they
+    send 349 there, of which nine take 2 to 21 % longer than a wave a row would, and keep 20 that would take 8 to 29 % less.  A wave a row: so many blocks of 64 keys a microsecond for all rows, and the longest row's own.  16 rows: a block is
     read once for all of them that see it, but a workgroup walks its rows' sequences one after another, four blocks at a time, and
     one with fewer than four leaves waves without work.  Measured, us (a wave a row, 16 rows): 400 new tokens beside 20 single ones
     behind 1,500, 12 heads of 96 232 and 1,474, 32 of 128 over 8 kv heads 700 and 550; 100 beside 3 behind 2,000, 32 of 128 over 8
@@ -760,9 +760,9 @@ def prompt_rows_pay(past, new, n_heads, n_kv_heads, head_dim) -> bool:
             shared, walk = last, turns
             longest = max(longest, walk)
     size, idle = head_dim / 128, 1 - min(seen / n, 4) / 4
-    a_row = 4.5 + size * (seen * n_heads * (7.3e-3 - 1.9e-3 * size) + 6 * most)
-    sixteen = 5.7 + size * (10.6 * longest + visits * n_kv_heads * (15e-3 + 1.7e-3 * size) * (1 + 2.7 * idle))
-    return sixteen < 0.86 * a_row
+    a_row = 5.2 + size * (seen * n_heads * (7.0e-3 - 2.5e-3 * size) + 5.5 * most)
+    sixteen = 5.6 + size * (10.6 * longest + visits * n_kv_heads * (17.2e-3 + 1.85e-3 * size) * (1 + 2.1 * idle))
+    return sixteen < 0.97 * a_row
 
 
 def _fits(t, dtype, shape) -> bool:
