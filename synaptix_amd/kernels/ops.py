@@ -731,14 +731,15 @@ def _mostly_prompts(n_tokens, page_table) -> bool:
 
 
 def prompt_rows_pay(past, new, n_heads, n_kv_heads, head_dim) -> bool:
-    """Whether 32-bit attention of sequences with past[b] cached and new[b] new tokens is faster 16 (token, head) rows a workgroup than a
-    wave a row, by estimates of both.  Of 500 drawn steps (1 to 24 sequences, prompts, portions and single tokens among them, 14 shapes) they
-    send 349 there, of which nine take 2 to 21 % longer than a wave a row would, and keep 20 that would take 8 to 29 % less.  A wave a row: so many blocks of 64 keys a microsecond for all rows, and the longest row's own.  16 rows: a block is
-    read once for all of them that see it, but a workgroup walks its rows' sequences one after another, four blocks at a time, and
-    one with fewer than four leaves waves without work.  Measured, us (a wave a row, 16 rows): 400 new tokens beside 20 single ones
-    behind 1,500, 12 heads of 96 232 and 1,474, 32 of 128 over 8 kv heads 700 and 550; 100 beside 3 behind 2,000, 32 of 128 over 8
-    250 and 389, 64 over 8 378 and 277; up to 64 keys, 32 of 128 over 8: 2 times 33 tokens 22 and 35, 8 times 33 53 and 68, 16 times 17 51 and 70,
-    4 times 64 61 and 37; behind 100, 8 times 17 74 and 51; 120, 137 and 233 tokens 228 and 87."""
+    """Whether 32-bit attention of sequences with past[b] cached and new[b] new tokens is faster 16 (token, head) rows a workgroup
+    than a wave a row, by estimates of both. Of 500 drawn steps (1 to 24 sequences, prompts, portions and single tokens among them, 14
+    shapes) they send 349 there, of which nine take 2 to 21 % longer than a wave a row would, and keep 20 that would take 8 to 29 %
+    less. A wave a row: so many blocks of 64 keys a microsecond for all rows, and the longest row's own. 16 rows: a block is read once
+    for all of them that see it, but a workgroup walks its rows' sequences one after another, four blocks at a time, and one with
+    fewer than four leaves waves without work. Measured, us (a wave a row, 16 rows): 400 new tokens beside 20 single ones behind
+    1,500, 12 heads of 96 232 and 1,474, 32 of 128 over 8 kv heads 700 and 550; 100 beside 3 behind 2,000, 32 of 128 over 8 250 and
+    389, 64 over 8 378 and 277; up to 64 keys, 32 of 128 over 8: 2 times 33 tokens 22 and 35, 8 times 33 53 and 68, 16 times 17 51 and
+    70, 4 times 64 61 and 37; behind 100, 8 times 17 74 and 51; 120, 137 and 233 tokens 228 and 87."""
     group, n = n_heads // n_kv_heads, sum(new)
     if n * n_heads <= 8 * compute_units():
         return False
