@@ -1193,7 +1193,9 @@ static hipError_t raise_decode_lds() {
 // counters (may be null): n_seqs * kv heads * ceil(group / 16) ints, zero.  With them the splits are merged inside the
 // one launch where the grid is at most two workgroups a compute unit; where it is larger, and without them, a second
 // kernel merges (a workgroup that waits for its stores and counts itself in holds its place that much longer, which a
-// grid of several rounds pays in every round: 8 sequences of 32,000 tokens 9.3 ms a step against 9.1).
+// grid of several rounds pays in every round: 8 sequences of 32,000 tokens 9.3 ms a step against 9.1).  Inside it stays with a
+// work list of more sequences than fill the chip, which cuts only the longest of them (40 of 64 to 4,096 tokens: 65 us, 68 with the
+// second kernel).
 // items (may be null: every sequence in n_splits splits): n_items x {sequence, split | splits of the sequence << 16,
 // first, length}, `first` + split < n_seqs * n_splits being the place of the split's partial results and length
 // what seq_len holds for the sequence; behind them n_seqs x {first, splits}, the same by sequence.
@@ -1227,7 +1229,8 @@ static int launch_decode(const void* q, const QkvIntake* in, void* k_pages, void
   const hipError_t raised = raise_decode_lds();
   SYN_CHECK(raised == hipSuccess, "attention_decode: %zu bytes of LDS refused: %s", LDS_MAX, hipGetErrorString(raised));
   const dim3 grid = items ? dim3(nkv * chunks, n_items, 1) : dim3(n_seqs, nkv * chunks, n_splits);
-  const bool merge_inside = counters != nullptr && (long)n_seqs * nkv * chunks * n_splits <= 2L * syn_compute_units();
+  const long groups = (long)n_seqs * nkv * chunks, cus = syn_compute_units();
+  const bool merge_inside = counters != nullptr && (groups * n_splits <= 2 * cus || (items != nullptr && groups > cus));
   const DecodeWork work{workspace, merge_inside ? counters : nullptr, (const int4*)items};
   if (in)
     attn_decode_split_kernel<true><<<grid, waves * SYN_WAVE, lds, stream>>>(

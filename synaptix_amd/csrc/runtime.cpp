@@ -578,6 +578,98 @@ RT_API int syn_decode_items(const int* seq_len, int rows, int n_splits, long win
   return OK;
 }
 
+// The work list of a decode step whose sequences x kv heads alone are more workgroups than there are compute units: the same
+// items and the same table behind them, but what counts is which workgroups meet on a compute unit.  Workgroups go round
+// robin over the XCDs and in each round robin over its compute units, whatever these still have to do, and the kv heads of
+// an item follow one another in the grid: item p of the list and items p + places, p + 2 places, ... share their compute units
+// (`places`: compute units / kv heads).  A list in the order of the sequences lets chance decide which long ones meet: 64
+// sequences of 64 to 4,096 tokens (8 kv heads of 128) took 114 us a layer, 96 with equal sums on every compute unit; 64 of one
+// length take 93.5 either way.  Pieces are handed out longest first, each to the bin (a place of every round) with the
+// smallest sum.  Only sequences longer than an even share of all bins are cut, since a cut costs a prologue and a merge (64 equal ones
+// cut in two: 98 us).  Compute units share the memory's rate evenly and one alone gets at most 5/3 of an even share, so a few bins
+// of one length can beat all bins of several (33 sequences of 2,048 over 32 bins 68 us, in pairs over 17 bins 57): the number
+// of bins is the one that an estimate on these terms prefers, of all, and one for every live piece, every two and every three.
+RT_API int syn_decode_bins(const int* seq_len, int rows, int n_splits, long window, int places, int* items) {
+  if (rows <= 0 || n_splits <= 0 || places <= 0 || (long)rows * n_splits / places * places < rows)
+    return fail(MISUSE, "a work list for %d rows x %d splits over %d places", rows, n_splits, places);
+  constexpr long UNIT = 32, MIN_UNITS = 8;
+  constexpr int MAX_SPLITS = 64;
+  constexpr double PROLOGUE = 4, MERGE = 2, ALONE = 5.0 / 3.0;     // in units of keys; of an even share of the memory's rate
+  const long T = (long)rows * n_splits, rounds = T / places;
+  std::vector<long> units(rows), splits(rows), first(rows);
+  long total = 0;
+  for (int i = 0; i < rows; ++i) {
+    long keys = std::max(1, seq_len[i]);
+    if (window > 0) keys = std::min(keys, window);
+    units[i] = (keys + UNIT - 1) / UNIT;
+    if (units[i] > 1) total += units[i];
+  }
+  long pieces = 0;
+  for (long cap = std::max(MIN_UNITS, (total + places - 1) / places); ; cap += cap / 4 + 1) {
+    pieces = 0;
+    for (int i = 0; i < rows; ++i) {
+      splits[i] = std::min<long>(MAX_SPLITS, (units[i] + cap - 1) / cap);
+      pieces += splits[i];
+    }
+    if (pieces <= rounds * places) break;
+  }
+  struct Piece {
+    long units;
+    int seq, split;
+  };
+  std::vector<Piece> list, idle;       // idle: single units, padding rows mostly
+  long at = 0;
+  for (int i = 0; i < rows; ++i) {
+    first[i] = at;
+    at += splits[i];
+    for (int sp = 0; sp < splits[i]; ++sp)
+      (units[i] > 1 ? list : idle).push_back({(units[i] + splits[i] - 1) / splits[i], i, sp});
+  }
+  std::stable_sort(list.begin(), list.end(), [](const Piece& a, const Piece& b) { return a.units > b.units; });
+  const int live = (int)list.size();
+  std::vector<int> bin_of(live), best_bin(live);
+  std::vector<double> load(places);
+  double best = -1;
+  for (int k = 0; k <= 3; ++k) {
+    const int bins = k == 0 ? places : std::min(places, std::max(1, (live + k - 1) / k));
+    if ((k > 0 && bins == places) || (long)bins * rounds < live) continue;
+    std::fill(load.begin(), load.end(), 0.0);
+    std::vector<int> held(bins, 0);
+    typedef std::pair<double, int> Bin;
+    std::priority_queue<Bin, std::vector<Bin>, std::greater<Bin>> least;
+    for (int b = 0; b < bins; ++b) least.push({0.0, b});
+    for (int p = 0; p < live; ++p) {
+      const int b = least.top().second;
+      least.pop();
+      bin_of[p] = b;
+      load[b] += (double)list[p].units + PROLOGUE + (splits[list[p].seq] > 1 ? MERGE : 0.0);
+      if (++held[b] < rounds) least.push({load[b], b});
+    }
+    std::vector<double> sorted(load.begin(), load.begin() + bins);
+    std::sort(sorted.begin(), sorted.end());
+    double time = 0, done = 0;
+    for (int b = 0; b < bins; ++b) {     // the bins that are still at work share the memory's rate
+      time += (sorted[b] - done) / std::min(ALONE, (double)places / (bins - b));
+      done = sorted[b];
+    }
+    if (best < 0 || time < 0.999 * best) best = time, best_bin = bin_of;
+  }
+  for (long t = 0; t < T; ++t) items[4 * t] = -1, items[4 * t + 1] = items[4 * t + 2] = items[4 * t + 3] = 0;
+  auto put = [&](long t, const Piece& p) {
+    int* it = items + 4 * t;
+    it[0] = p.seq, it[1] = p.split | ((int)splits[p.seq] << 16), it[2] = (int)first[p.seq], it[3] = seq_len[p.seq];
+  };
+  std::vector<int> filled(places, 0);
+  for (int p = 0; p < live; ++p) put((long)filled[best_bin[p]]++ * places + best_bin[p], list[p]);
+  at = 0;
+  for (const Piece& p : idle) {
+    while (items[4 * at] >= 0) ++at;
+    put(at, p);
+  }
+  for (int i = 0; i < rows; ++i) items[4 * T + 2 * i] = (int)first[i], items[4 * T + 2 * i + 1] = (int)splits[i];
+  return OK;
+}
+
 // A decode step of `rows` rows of which the first B are sequences (one token each) and the rest
 // padding: token 0 at position 0 against a spare page that no sequence owns.  After the integer
 // tables lie 2 * rows floats: temperatures and uniform numbers (0 where none are given); after

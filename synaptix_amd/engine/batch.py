@@ -90,6 +90,9 @@ class StepContext:
         return self._tables[group]
 
     def decode_splits(self, n_kv_heads: int, group: int) -> int:
+        items = self.decode_items(group)
+        if items is not None:                 # the list has room for that many splits a sequence
+            return (items.numel() // self.n_seqs - 2) // 4
         return ops.decode_splits(self.n_seqs, n_kv_heads, self.layout.widths[group])
 
     def prompt_rows_pay(self, *heads) -> bool:

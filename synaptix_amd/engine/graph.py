@@ -90,8 +90,12 @@ class DecodeRunner:
         self.item_splits = [ops.decode_splits(rows, g.need.kv_heads, w) if engine.dtype == torch.bfloat16 else 0
                             for g, w in zip(groups, self.widths)]
         self.item_splits = [s if s > 1 else 0 for s in self.item_splits]
+        # where the rows alone are more workgroups than compute units: lists that give each of these the same share
+        self.item_bins = [ops.decode_bins(rows, g.need.kv_heads) if engine.dtype == torch.bfloat16 and s == 0 else 0
+                          for g, s in zip(groups, self.item_splits)]
         n_items = [4 * rows * s + 2 * rows if s else 0 for s in self.item_splits]       # ints of each list
-        self.total = n_int + 2 * rows + sum(n_items)           # + temperatures and uniforms as float bits + work lists
+        n_bins = [(4 * ops.DECODE_BIN_SPLITS + 2) * rows if b else 0 for b in self.item_bins]
+        self.total = n_int + 2 * rows + sum(n_items) + sum(n_bins)     # + temperatures and uniforms as float bits + work lists
         dev = engine.device
         self.dev = torch.zeros(self.total, dtype=torch.int32, device=dev)
         self.host = [torch.zeros(self.total, dtype=torch.int32, pin_memory=True) for _ in range(2)]
@@ -103,6 +107,12 @@ class DecodeRunner:
         for n in n_items:
             self.items.append(self.dev[at:at + n] if n else None)
             at += n
+        self.bins_at = []
+        for i, n in enumerate(n_bins):
+            if n:
+                self.bins_at.append((i, at))
+                self.items[i] = self.dev[at:at + n]
+                at += n
         self.out_tokens = torch.zeros(rows, dtype=torch.int32, device=dev)
         self.logits = None
         self.graph = None
@@ -122,6 +132,11 @@ class DecodeRunner:
         rt.check(rt.lib().syn_decode_fill(self.engine.cache._h, self.rows, B, rt.ints([int(s) for s in slots]),
                                           rt.ints([int(x) for x in tokens]), len(self.widths), rt.ints(self.widths),
                                           rt.ints(self.spare), t, u, rt.ints(self.item_splits), host.ctypes.data))
+        lens = host.ctypes.data + 4 * self.layout.off["seq_len"][0]
+        for i, at in self.bins_at:
+            window = self.engine.cache.groups[i].need.window
+            rt.check(rt.lib().syn_decode_bins(lens, self.rows, ops.DECODE_BIN_SPLITS, -1 if window is None else window,
+                                              self.item_bins[i], host.ctypes.data + 4 * at))
 
     def _forward(self, ctx):
         eng = self.engine

@@ -44,6 +44,7 @@ _SIGNATURES = {
     "syn_step_fill_padded": (_I, [_P, _I, _IP, _LP, _P, _L, _P, _I, _IP, _IP, _L, _I, _L, _P]),
     "syn_decode_fill": (_I, [_P, _I, _I, _IP, _IP, _I, _IP, _IP, _FP, _FP, _IP, _P]),
     "syn_decode_items": (_I, [_IP, _I, _I, _L, _IP]),
+    "syn_decode_bins": (_I, [_P, _I, _I, _L, _I, _P]),
     "syn_philox_block": (None, [_UP, _UP, _UP]),
     "syn_philox_new": (_P, [C.c_uint64]),
     "syn_philox_delete": (None, [_P]),
@@ -96,4 +97,13 @@ def decode_items(seq_len, n_splits: int, window=None) -> list:
     out = (C.c_int * (4 * rows * n_splits + 2 * rows))()
     check(lib().syn_decode_items(ints([int(x) for x in seq_len]), rows, int(n_splits),
                                  -1 if window is None else int(window), out))
+    return list(out)
+
+
+def decode_bins(seq_len, n_splits: int, places: int, window=None) -> list:
+    """The same for more sequences x kv heads than compute units (syn_decode_bins): items p, p + places, p + 2 places, ...
+    meet on the same compute units and get about the same sum of keys."""
+    rows = len(seq_len)
+    lens, out = ints([int(x) for x in seq_len]), (C.c_int * (4 * rows * n_splits + 2 * rows))()
+    check(lib().syn_decode_bins(lens, rows, int(n_splits), -1 if window is None else int(window), int(places), out))
     return list(out)

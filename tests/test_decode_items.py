@@ -97,3 +97,54 @@ def test_padding_rows_and_random_batches_keep_the_list_whole():
 def test_refuses_an_empty_list():
     with pytest.raises(rt.CacheError):
         rt.decode_items([], 4)
+
+
+def _binned(lengths, places, window=None):
+    """The list of bins: every sequence's splits once each with places of their own for the partial results, the table
+    behind the items, and the sum of units that every place gets."""
+    T, rows = 2 * len(lengths), len(lengths)
+    flat = rt.decode_bins(lengths, 2, places, window)
+    assert len(flat) == 4 * T + 2 * rows
+    seen, taken, load = {}, set(), [0] * places
+    for at in range(T):
+        seq, split_and_n, first, length = flat[4 * at:4 * at + 4]
+        split, n = split_and_n & 0xFFFF, split_and_n >> 16
+        if seq < 0:
+            continue
+        assert length == lengths[seq] and 0 <= split < n and flat[4 * T + 2 * seq:4 * T + 2 * seq + 2] == [first, n]
+        assert (seq, split) not in seen and first + split not in taken and 0 <= first + split < T
+        seen[(seq, split)] = n
+        taken.add(first + split)
+        units = -(-(lengths[seq] if window is None else min(lengths[seq], window)) // UNIT)
+        load[at % places] += -(-units // n)
+    n_of = {s: n for (s, _), n in seen.items()}
+    assert sorted(n_of) == list(range(rows)) and len(seen) == sum(n_of.values())
+    return load, n_of
+
+
+@pytest.mark.parametrize("rows,places", [(33, 32), (64, 32), (65, 64), (96, 32), (128, 8), (257, 256)])
+def test_bins_hold_every_piece_once_and_even_sums(rows, places):
+    rnd = random.Random(rows)
+    for window in (None, 500):
+        for hi in (1, 40, 4000, 40000):
+            lengths = [rnd.choice([1, rnd.randint(1, hi)]) for _ in range(rows)]
+            load, n_of = _binned(lengths, places, window)
+            units = [-(-(x if window is None else min(x, window)) // UNIT) for x in lengths]
+            share = max(UNIT // 4, -(-sum(u for u in units if u > 1) // places))
+            assert all(n == 1 for s, n in n_of.items() if units[s] <= share)       # only what is longer than a share is cut
+
+
+def test_bins_pair_long_sequences_with_short_ones():
+    lengths = [UNIT * (i + 1) for i in range(64)]                                  # 1 to 64 units
+    load, n_of = _binned(lengths, 32)
+    assert set(n_of.values()) == {1} and max(load) <= 1.05 * sum(load) / 32
+    load, n_of = _binned([8000] + [500] * 63, 32)                                  # one alone is longer than five shares
+    assert n_of[0] > 5 and max(load) <= 1.5 * sum(load) / 32
+    load, _ = _binned([2048] * 33 + [1] * 31, 32)                                  # pairs in half of the places, not one pair among singles
+    assert sum(u > 66 for u in load) == 16 and sum(64 <= u <= 66 for u in load) == 1
+
+
+def test_bins_refuse_what_does_not_fit():
+    for args in (([], 2, 8), ([5, 6], 2, 0), ([5] * 5, 1, 8)):
+        with pytest.raises(rt.CacheError):
+            rt.decode_bins(*args)

@@ -1209,6 +1209,48 @@ def test_attention_decode_bf16(ops, nh, nkv, hd, lens, window, splits):
         out, want, lens, splits, window, nh, nkv, work)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,rows,hi,window", [
+    (32, 8, 128, 33, 3000, 0),                  # one workgroup more than a compute unit
+    (32, 8, 128, 64, 300, 0),
+    (4, 4, 16, 65, 700, 0),
+    (8, 8, 64, 48, 900, 200),                   # a window
+    (64, 16, 128, 17, 4000, 0),                 # two sequences a place
+])
+def test_attention_decode_over_bins(ops, nh, nkv, hd, rows, hi, window):
+    """More sequences x kv heads than compute units, one much longer than the rest and some of a single token: the list that
+    gives every compute unit the same share of the keys, long sequences cut and merged inside the launch."""
+    gen = torch.Generator().manual_seed(rows)
+    lens = torch.randint(1, hi, (rows,), generator=gen).tolist()
+    lens[0], lens[1], lens[-1] = 3 * hi, hi, 1
+    width = (max(lens) + 63) // 64 + 1
+    pages = [(n + 63) // 64 for n in lens]
+    table = torch.zeros((rows, width), dtype=I32)
+    ids, at = torch.randperm(sum(pages), generator=gen).to(I32), 0
+    for b, p in enumerate(pages):
+        table[b, :p] = ids[at:at + p]
+        at += p
+    k, v = make_cache(sum(pages), nkv, hd, BF16, 80)
+    fill_sequences(k, v, table, lens, nkv, hd, BF16, 82)
+    q = rnd((rows, nh * hd), 81, BF16)
+    want = torch.empty((rows, nh * hd), dtype=F32)
+    lens_t, scale = torch.tensor(lens, dtype=I32), 1 / math.sqrt(hd)
+    ref.attention_f32(q.float(), k.float(), v.float(), table, torch.arange(rows, dtype=I32), lens_t - 1,
+                      want, scale, window, nh, nkv, hd)
+    places, d = ops.decode_bins(rows, nkv), lambda t: t.to(DEV)
+    assert places == 256 // nkv
+    items = rt.decode_bins(lens, ops.DECODE_BIN_SPLITS, places, window or None)
+    T = ops.DECODE_BIN_SPLITS * rows
+    assert window or max(items[4 * i + 1] >> 16 for i in range(T)) > 1
+    counters = torch.zeros(rows * nkv, dtype=I32, device=DEV)
+    work = torch.full((rows * nh * ops.DECODE_BIN_SPLITS * (hd + 2),), float("nan"), dtype=F32, device=DEV)
+    for kw in (dict(counters=counters), {}):                # merged in the launch, and by the second kernel
+        out = torch.full((rows, nh * hd), float("nan"), dtype=BF16, device=DEV)
+        ops.attention_decode_bf16(d(q), d(k), dv(v), d(table), d(lens_t), out, work, ops.DECODE_BIN_SPLITS, scale, window, nh, nkv,
+                                  hd, items=torch.tensor(items, dtype=I32, device=DEV), **kw)
+        close(out, want, 2e-2, 1e-2, what="decode attention over bins")
+    assert int(counters.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("lens,splits", [([2061] * 8, 4), ([2061], 16), ([3908, 457, 1200, 2500], 8)])
 def test_merge_inside_the_launch_reads_what_this_launch_wrote(ops, lens, splits):
     """The workgroup that merges the splits reads partial results that workgroups on other XCDs, each with a
