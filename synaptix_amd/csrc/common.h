@@ -285,7 +285,10 @@ __device__ __forceinline__ float gated_quick(float g, float u, float limit) {
 }
 
 // ---- the ring of k-tiles of the kernels that stream k-steps (gemm.hip, grouped.hip) ----
-// k-tiles in the ring: as many as 160 KB of LDS hold, at most eight (the two largest tiles gain nothing from a fifth)
+// k-tiles of W in the ring: as many pairs as 160 KB of LDS hold beside x's ring, at most eight.  k-tiles of x come in pairs, whole lines
+// of 128 bytes of a row, and a pair's loads are spread over two steps: x's ring holds one pair more than W's has pairs.
 constexpr int stream_stages(int bm, int bn) {
-  return bm == 256 && bn >= 192 ? 4 : 163840 / ((bm + bn) * 64) > 8 ? 8 : 163840 / ((bm + bn) * 64);
+  return (163840 - bm * 128) / ((bm + bn) * 64) >= 8 ? 8 : (163840 - bm * 128) / ((bm + bn) * 64) / 2 * 2;
 }
+constexpr int stream_pairs(int bm, int bn) { return stream_stages(bm, bn) / 2 + 1; }
+constexpr int stream_lds(int bm, int bn) { return stream_pairs(bm, bn) * bm * 128 + stream_stages(bm, bn) * bn * 64; }

@@ -1162,6 +1162,12 @@ static int launch_rows(int nf, const bf16* x, const bf16* wp, void* out, Epilogu
 //     from memory).  While the MFMAs of a k-step run (operands in registers), the fragments of the next one are read and the
 //     loads of the k-tile a ring ahead are issued, evenly between the MFMAs: a burst of loads holds up the wave that
 //     issues it (the texture addresser takes about 25 cycles for each);
+//   * x comes in whole lines: a load takes 128 bytes of each of 8 rows, two k-tiles at once, into a ring of its own.  Pieces of 64
+//     bytes, one k-tile of 16 rows, cost the caches a request each as well and every line twice (2,048 x 24,576 x 4,096, zeros:
+//     270 us, in whole lines 231; random numbers 298 -> 291; 1,024 rows 187 -> 169, 512 98 -> 84; 512 x 4,096 x 12,288 65 -> 53;
+//     40,960 x 2,560 x 9,728 1,655 -> 1,600; a prompt of 2,048 tokens at the 8B shape 26.75 -> 25.2 ms);
+//   * where the loads have got to is kept from step to step: 24 scalar instructions of two steps instead of 39 (of 512 x 6,144 x 4,096
+//     in tiles of 64 x 128, whose steps have eight MFMAs, 50.8 -> 40.1 us; 45.2 with x in pieces);
 //   * a workgroup goes through several tiles and its loads run ahead into the next one: no tile but the first waits for
 //     its first operands, and a tile's stores drain behind the next one's MFMAs;
 //   * W's fragment is the first operand, so that a lane's four results are neighbours in a row; two groups of them are joined
@@ -1172,8 +1178,9 @@ static int launch_rows(int nf, const bf16* x, const bf16* wp, void* out, Epilogu
 // Against the kernel before it (eight waves of 128 x 64, k-tiles of 64 in two buffers, a tile a workgroup), random operands,
 // W in fragment order, with the gated activation: 2,048 x 24,576 x 4,096 335 -> 278 us (1.48 PFLOP/s), 35,901 x 19,456 x
 // 2,560 3,056 -> 2,476 us (1.44); without: 8,192 x 24,576 x 4,096 1,313 -> 1,128 us, 35,901 x 2,560 x 9,728 1,533 -> 1,402.
-// Operands: W in fragment order (WP: pack_weight) or in plain rows, x in plain rows.  In LDS a row of 32 k-values is
-// four chunks of 16 bytes, slot s of row r holding chunk s ^ (r / 4 % 4), so that 16 lanes with the same chunk of 16 rows
+// Operands: W in fragment order (WP: pack_weight) or in plain rows, x in plain rows.  In LDS a row of 32 k-values of W in plain
+// rows is four chunks of 16 bytes, slot s of row r holding chunk s ^ (r / 4 % 4), a row of 64 of x eight chunks, slot s holding
+// chunk s ^ (r / 2 % 8), so that 16 lanes with the same chunk of 16 rows
 // touch every bank once; fragments of W lie as they come.  Rows beyond M or N lie behind the descriptors' ends: they are
 // read as zeros without traffic, and their results are dropped by the output's descriptor.
 
@@ -1197,14 +1204,14 @@ template <int BM, int BN, int OUT, bool WP>
 __global__ void __launch_bounds__(256, 1)
 gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void* __restrict__ out, Epilogue ep,
                    int M, int N, int K, int k_slice, int tiles, int whole, int streamed) {
-  constexpr int BK = 32, STAGES = stream_stages(BM, BN), WAVES = 4, ROWS = BM + BN;
-  constexpr int RPI = 16, PASSES = ROWS / (RPI * WAVES);      // rows of 64 bytes that a load of a wave fills; loads a k-tile
+  constexpr int BK = 32, STAGES = stream_stages(BM, BN), PAIRS = stream_pairs(BM, BN), WAVES = 4;
+  constexpr int XL = BM / 32, WL = BN / 64, PASSES = XL / 2 + WL;   // loads of a wave: of a pair of k-tiles of x, of a k-tile of W, a step
   constexpr int FM = BM / 32, FN = BN / 32;                   // fragments of 16 rows that a wave holds of x and of W
   constexpr int NM = FM * FN, NR = FM + FN;                   // MFMAs and fragment reads of a wave in a k-step
   constexpr int READ_EVERY = NM / NR > 3 ? 3 : NM / NR, LOAD_EVERY = NM / PASSES;
-  static_assert(ROWS % (RPI * WAVES) == 0 && BM % (RPI * WAVES) == 0 && BM % 32 == 0 && BN % 32 == 0, "tile shape");
+  static_assert(BM % 64 == 0 && BN % 64 == 0 && STAGES % 2 == 0 && stream_lds(BM, BN) <= 163840, "tile shape");
   static_assert(READ_EVERY >= 1 && LOAD_EVERY >= 1 && FN % 2 == 0, "reads, loads and stores find their places");
-  extern __shared__ __attribute__((aligned(16))) bf16 smem[];   // [STAGES][ROWS][32]
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];   // x [PAIRS][BM][64], W [STAGES][BN][32]
   const int tid = threadIdx.x, lane = tid % SYN_WAVE, grid = (int)gridDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / SYN_WAVE);   // scalar: LDS addresses of the loads stay scalar
   const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * (BN / 2);
@@ -1213,13 +1220,16 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
   int at = ((int)blockIdx.x % 8) * (grid / 8) + (int)blockIdx.x / 8;   // workgroup b runs on XCD b % 8
   if (at >= tiles) return;
 
-  // load p fills tile rows (p * WAVES + wave) * 16 .. + 16 (x first, then W): a fragment of W as it lies, or four rows at a time
-  unsigned src[PASSES];
+  // Load p of x fills tile rows (p * WAVES + wave) * 8 .. + 8, 128 bytes of each; of W rows (p * WAVES + wave) * 16 .. + 16, a fragment as
+  // it lies or four rows of 64 bytes at a time
+  unsigned src_x[XL], src_w[WL];
 #pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-    const int row0 = (p * WAVES + wave) * RPI, in = row0 < BM ? row0 : row0 - BM;
-    src[p] = WP && row0 >= BM ? (unsigned)((size_t)in * row_bytes + lane * 16)
-                              : (unsigned)((size_t)(in + lane / 4) * row_bytes + ((lane % 4) ^ (lane / 16)) * 16);
+  for (int p = 0; p < XL; ++p) src_x[p] = (unsigned)((size_t)((p * WAVES + wave) * 8 + lane / 8) * row_bytes + ((lane % 8) ^ (wave % 2 * 4 + lane / 16)) * 16);
+#pragma unroll
+  for (int p = 0; p < WL; ++p) {
+    const int row0 = (p * WAVES + wave) * 16;
+    src_w[p] = WP ? (unsigned)((size_t)row0 * row_bytes + lane * 16)
+                  : (unsigned)((size_t)(row0 + lane / 4) * row_bytes + ((lane % 4) ^ (lane / 16)) * 16);
   }
   struct Source {      // of a tile: the rows of x and W from its first k-value on, and its k-steps
     BufferView x, w;
@@ -1233,29 +1243,45 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     s.steps = (min(K, k0 + k_slice) - k0) / BK;
     return s;
   };
-  auto fetch = [&](const Source& s, int kt, int buf, int p) {
-    bf16* dst = smem + (size_t)buf * ROWS * BK + (size_t)(p * WAVES + wave) * RPI * BK;
-    const bool of_x = p * WAVES * RPI < BM;
-    buffer_to_lds16(of_x ? s.x : s.w, dst, src[p], kt * (BK * (int)sizeof(bf16)) * (WP && !of_x ? 16 : 1));
+  // Where the loads have got to, x's in pairs of k-tiles: the way from here on through this tile and into the next one.  (Kept from step
+  // to step, all in bytes: with one wave a SIMD, scalar instructions of a step stand beside its MFMAs, of which the smallest tile has
+  // eight.)
+  constexpr int W_TILE = BK * (int)sizeof(bf16) * (WP ? 16 : 1), X_PAIR = 2 * BK * (int)sizeof(bf16);
+  constexpr int W_BUF = BN * BK * (int)sizeof(bf16), X_BUF = BM * X_PAIR;
+  struct Way {
+    BufferView v;
+    int at, end;
+  };
+  auto onward = [&](Way& y, int by, const BufferView& then, int then_end) {
+    y.at += by;
+    if (__builtin_expect(y.at == y.end, 0)) y.v = then, y.at = 0, y.end = then_end;
+  };
+  const int x_to = wave * 8 * X_PAIR, w_to = PAIRS * X_BUF + wave * 16 * BK * (int)sizeof(bf16);
+  auto fetch_x = [&](const Way& y, int xbuf, int p) {
+    buffer_to_lds16(y.v, (char*)smem + xbuf + x_to + p * (WAVES * 8 * X_PAIR), src_x[p], y.at);
+  };
+  auto fetch_w = [&](const Way& y, int buf, int p) {
+    buffer_to_lds16(y.v, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], y.at);
   };
   f32x4 acc[FM][FN];
   const int r16 = lane % 16, q4 = lane / 16;
-  const int x_at = (wm + r16) * BK + (q4 ^ (r16 / 4)) * 8;
-  const int w_at = WP ? (BM + wn) * BK + lane * 8 : (BM + wn + r16) * BK + (q4 ^ (r16 / 4)) * 8;
+  // in bytes; the second k-tile of a pair: chunks 4 to 7, bit 2 of the slot
+  const int x_at = ((wm + r16) * 2 * BK + (q4 ^ (r16 / 2)) * 8) * 2, x_at2 = x_at ^ 64;
+  const int w_at = PAIRS * X_BUF + (WP ? wn * BK + lane * 8 : (wn + r16) * BK + (q4 ^ (r16 / 4)) * 8) * 2;
   bf16x8 a[2][FM], b[2][FN];      // two sets of fragments: one is multiplied while the other is read
-  auto read_one = [&](int buf, int set, int idx) {
-    const bf16* base = smem + (size_t)buf * ROWS * BK;
-    if (idx < FM) a[set][idx] = *(const bf16x8*)(base + x_at + idx * 16 * BK);
-    else b[set][idx - FM] = *(const bf16x8*)(base + w_at + (idx - FM) * 16 * BK);
+  auto read_one = [&](int xbuf, int half, int buf, int set, int idx) {
+    if (idx < FM) a[set][idx] = *(const bf16x8*)((const char*)smem + xbuf + (half ? x_at2 : x_at) + idx * 16 * X_PAIR);
+    else b[set][idx - FM] = *(const bf16x8*)((const char*)smem + buf + w_at + (idx - FM) * 16 * BK * 2);
   };
-  // k-step kt of a tile over fragment set SET (FRESH: its first one): reads the fragments of the next step and asks for the
-  // k-tile a ring ahead, which near a tile's end belongs to the workgroup's next tile
-  auto step = [&](const Source& now, const Source& then, int kt, int buf, auto set, auto fresh) {
+  Way way_x, way_w;
+  int buf = 0, xbuf = 0, xbuf_before = 0;
+  // A k-step over fragment set SET, the step's parity (FRESH: a tile's first): reads the fragments of the next step and asks for W's
+  // k-tile a ring ahead and half a pair of x, the second half of the pair begun in the step before or the first one of the pair
+  // that takes this pair's buffer, whose fragments are all in registers; near a tile's end they belong to the workgroup's next tile
+  auto step = [&](const Source& then, auto set, auto fresh) {
     constexpr int SET = decltype(set)::value;
-    const int next = buf + 1 == STAGES ? 0 : buf + 1;
-    const bool over = kt + STAGES >= now.steps;
-    const Source s = over ? then : now;
-    const int ahead = over ? kt + STAGES - now.steps : kt + STAGES;
+    const int next = buf + W_BUF == STAGES * W_BUF ? 0 : buf + W_BUF;
+    const int xnext = SET ? (xbuf + X_BUF == PAIRS * X_BUF ? 0 : xbuf + X_BUF) : xbuf;
 #pragma unroll
     for (int q = 0; q < NM; ++q) {
       const int j = q / FM, i = q % FM;
@@ -1263,10 +1289,18 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[i][j]) : "v"(b[SET][j]), "v"(a[SET][i]));
       else
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b[SET][j]), "v"(a[SET][i]));
-      if (q % LOAD_EVERY == 0 && q / LOAD_EVERY < PASSES) fetch(s, ahead, buf, q / LOAD_EVERY);
-      if (q % READ_EVERY == READ_EVERY - 1 && q / READ_EVERY < NR) read_one(next, SET ^ 1, q / READ_EVERY);
+      if (q % LOAD_EVERY == 0 && q / LOAD_EVERY < PASSES) {
+        const int p = q / LOAD_EVERY;
+        if (p < XL / 2) fetch_x(way_x, SET ? xbuf : xbuf_before, SET ? p : p + XL / 2);
+        else fetch_w(way_w, buf, p - XL / 2);
+      }
+      if (q % READ_EVERY == READ_EVERY - 1 && q / READ_EVERY < NR) read_one(xnext, SET ^ 1, next, SET ^ 1, q / READ_EVERY);
       __builtin_amdgcn_sched_barrier(0);
     }
+    onward(way_w, W_TILE, then.w, then.steps * W_TILE);
+    if constexpr (SET == 0) onward(way_x, X_PAIR, then.x, then.steps * (X_PAIR / 2));
+    else xbuf_before = xbuf, xbuf = xnext;
+    buf = next;
   };
   // Before the barrier that ends a step a wave waits until its reads have returned and all but its youngest loads, those of
   // the last STAGES - 2 steps, have landed: behind it the k-tile after the next is whole, and the buffer of this step's tile free.
@@ -1278,30 +1312,41 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     __builtin_amdgcn_sched_barrier(0);
   };
   TileAt t = stream_tile(at, tiles_m, tiles_n);
-  Source now = source(t);
+  bool more = at + grid < tiles;
+  TileAt t_next = stream_tile(more ? at + grid : at, tiles_m, tiles_n);   // (behind the last tile: loads that nobody reads)
+  Source then = source(t_next);
+  {
+    const Source now = source(t);
+    way_x = {now.x, 0, now.steps * (X_PAIR / 2)}, way_w = {now.w, 0, now.steps * W_TILE};
+  }
+  // what the steps before the first would have asked for
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s)
+  for (int p = 0; p < XL / 2; ++p) fetch_x(way_x, 0, p);
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) fetch(now, s, s, p);
+  for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+    for (int p = 0; p < XL / 2; ++p) fetch_x(way_x, (s + 1) / 2 * X_BUF, s % 2 ? p : p + XL / 2);
+#pragma unroll
+    for (int p = 0; p < WL; ++p) fetch_w(way_w, s * W_BUF, p);
+    onward(way_w, W_TILE, then.w, then.steps * W_TILE);
+    if (s % 2 == 0) onward(way_x, X_PAIR, then.x, then.steps * (X_PAIR / 2));
+  }
+  xbuf_before = STAGES / 2 * X_BUF;
+  int steps = source(t).steps;
   landed();
 #pragma unroll
-  for (int i = 0; i < NR; ++i) read_one(0, 0, i);
+  for (int i = 0; i < NR; ++i) read_one(0, 0, 0, 0, i);
   __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the first fragments are in registers,
   __builtin_amdgcn_s_barrier();         // everywhere
   __builtin_amdgcn_sched_barrier(0);
   using Even = std::integral_constant<int, 0>;
   using Odd = std::integral_constant<int, 1>;
-  int buf = 0;
   for (;;) {
-    const bool more = at + grid < tiles;
-    const TileAt t_next = stream_tile(more ? at + grid : at, tiles_m, tiles_n);   // (behind the last tile: loads that nobody reads)
-    const Source then = source(t_next);
-    auto turn = [&] { buf = buf + 1 == STAGES ? 0 : buf + 1; };
-    step(now, then, 0, buf, Even{}, std::true_type{}), landed(), turn();
-    step(now, then, 1, buf, Odd{}, std::false_type{}), landed(), turn();
-    for (int kt = 2; kt < now.steps; kt += 2) {
-      step(now, then, kt, buf, Even{}, std::false_type{}), landed(), turn();
-      step(now, then, kt + 1, buf, Odd{}, std::false_type{}), landed(), turn();
+    step(then, Even{}, std::true_type{}), landed();
+    step(then, Odd{}, std::false_type{}), landed();
+    for (int kt = 2; kt < steps; kt += 2) {
+      step(then, Even{}, std::false_type{}), landed();
+      step(then, Odd{}, std::false_type{}), landed();
     }
     // (the compiler does not know that the statements above are matrix instructions: their results may be read 18 states later)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -1373,7 +1418,10 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     }
     __builtin_amdgcn_sched_barrier(0);
     if (!more) break;
-    at += grid, t = t_next, now = then;
+    at += grid, t = t_next, steps = then.steps;
+    more = at + grid < tiles;
+    t_next = stream_tile(more ? at + grid : at, tiles_m, tiles_n);
+    then = source(t_next);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);   // nothing may be on its way into LDS when the workgroup ends
 }
@@ -1433,7 +1481,7 @@ template <int BM, int BN, int OUT, bool PLAIN>
 static int launch_stream(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices) {
   SYN_CHECK(K % 64 == 0 && stream_last_slice(K, slices) >= 32 * stream_stages(BM, BN) && (PLAIN || w.packed),
             "gemm: %d slices of K = %d do not fit tiles of %d x %d", slices, K, BM, BN);
-  const size_t lds = (size_t)stream_stages(BM, BN) * (BM + BN) * 32 * sizeof(bf16);
+  const size_t lds = stream_lds(BM, BN);
   static OncePerDevice raised;
   if (lds > 65536) {
     const hipError_t e = once_per_device(raised, [&] {
@@ -1449,7 +1497,9 @@ static int launch_stream(const bf16* x, Weight w, void* out, Epilogue ep, int M,
   SYN_CHECK(tiles < (1L << 30), "gemm: M = %d, N = %d make too many tiles", M, N);
   // every workgroup the same number of tiles, or one fewer: the fewest workgroups that need no further round
   const long cus = syn_compute_units(), rounds = (tiles + cus - 1) / cus;
-  const int grid = (int)(8 * ((tiles + 8 * rounds - 1) / (8 * rounds)));
+  // (where a tile has fewer steps than the loads of x run ahead each workgroup has one tile: what its loads reach behind it nobody reads)
+  const bool ahead = stream_last_slice(K, slices) >= 32 * (stream_stages(BM, BN) + 2);
+  const int grid = (int)(8 * (ahead ? (tiles + 8 * rounds - 1) / (8 * rounds) : (tiles + 7) / 8));
   const int whole = N % 16 == 0 && (uintptr_t)out % 16 == 0;      // stores of 16 bytes
   const size_t bytes = (size_t)slices * M * N * (OUT == SYN_OUT_F32 ? 4 : OUT == SYN_OUT_BF16 ? 2 : 1);
   const int streamed = bytes > (48u << 20);      // (of the 256 MB that the memory-side cache holds, beside x and W)
