@@ -362,12 +362,19 @@ __global__ void __launch_bounds__(256) grouped_product_tiled_kernel(GroupedArgs 
 
 // ---------------------------------------------------------------- bf16, many rows a group, W in fragment order: streamed
 // The scheme of the products of many rows (gemm_stream_kernel in gemm.hip: four waves with a quarter of the tile each,
-// accumulators in place, k-tiles of 32 in a ring of LDS buffers, one stream of k-steps over all tiles of a workgroup) for rows
-// sorted into segments: which tiles there are stands in seg_start, on the device, so every workgroup counts the segments'
-// tiles into LDS first and looks its tiles up there.  Rows of x are gathered by their loads (each lane asks for a piece of its
-// own row), rows of the output and their weights looked up by the stores.  Bound by the matrix units; what is left to the
-// tiles above is that they stage both operands through registers and wait for each k-tile.  1,500 tokens with 6 of 48 experts,
-// 2,048 x 4,096 with GELU and back, 32-bit results: 549 + 469 us -> 244 + 219.
+// accumulators in place, k-tiles in rings of LDS buffers, x in whole lines of 128 bytes of a row, one stream of k-steps over all
+// tiles of a workgroup) for rows sorted into segments: which tiles there are stands in seg_start, on the device, so every wave counts
+// the segments' tiles into registers first and looks its tiles up there.  Rows of x are gathered by their loads (each lane asks for a
+// piece of its own row), rows of the output and their weights looked up for the stores.
+// What bounds it: what a compute unit takes in, since all of W comes from memory and x from L2 (a k-step of 256 x 256 takes 0.55 to 0.7
+// us for 0.43 of MFMAs, with zeros as operands too), and the stores of a tile, which the next tile's first loads wait behind.  So
+//   * a segment's tiles get the same number of rows, and a k-step leaves out the 32 rows at a time that a tile does not have;
+//   * what the stores look up, and the next tile's row list, are asked for before the first store: behind stores they would wait
+//     for these, once for every 32 rows;
+//   * a last round of tiles for up to half of the workgroups is cut into halves of tiles for all.
+// 1,500 tokens with 6 of 48 experts (188 rows each), 2,048 x 4,096 with GELU and back, 32-bit results: 251 + 225 us -> 220 + 217 (x
+// in pieces of 64 bytes, tiles of up to 256 rows and lookups between the stores before); 310 rows each 353 + 383 -> 290 + 316, 120
+// rows 229 + 199 -> 187 + 190, 50 rows 185 + 168 -> 162 + 168, 32 experts with 256 rows 159 -> 162, 16 with 187 127 + 84 -> 101 + 85.
 // Tile order: the column tiles of a row tile follow each other, 32 in a row on one XCD.
 #define GS_MAX_GROUPS 512
 __device__ __forceinline__ float gelu_quick(float z) {
@@ -383,112 +390,184 @@ __device__ __forceinline__ float gelu_quick(float z) {
   return z * (z < 0.f ? q : 1.f - q);
 }
 
-constexpr int grouped_stages(int bm, int bn) {      // (beside the table of tiles)
-  const int most = (163840 - 4 * (GS_MAX_GROUPS + 64)) / ((bm + bn) * 64);
-  return stream_stages(bm, bn) < most ? stream_stages(bm, bn) : most;
-}
 template <int BM, int BN, bool F32, bool PAIR>
 __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, long a_bytes, long o_bytes) {
-  constexpr int BK = 32, STAGES = grouped_stages(BM, BN), WAVES = 4, ROWS = BM + BN, RPI = 16;
-  constexpr int XL = BM / (RPI * WAVES), WL = BN / (RPI * WAVES), PASSES = XL + WL;      // loads of a wave for a k-tile: x, W
-  constexpr int FM = BM / 32, FN = BN / 32, NM = FM * FN, NR = FM + FN;
-  constexpr int READ_EVERY = NM / NR > 3 ? 3 : NM / NR, LOAD_EVERY = NM / PASSES;
+  constexpr int BK = 32, STAGES = stream_stages(BM, BN), PAIRS = stream_pairs(BM, BN), WAVES = 4;
+  constexpr int XL = BM / 32, WL = BN / 64, PASSES = XL / 2 + WL;      // loads of a wave: of a pair of k-tiles of x, of a k-tile of W, a step
+  constexpr int FM = BM / 32, FN = BN / 32;
+  // A k-step of a wave goes row group by row group: 2 i + (its row of waves) is row group i's fragment of x, so that the waves share
+  // what rows a tile has.  The first FMU groups always run, the others where the tile has rows for them, and in each the right
+  // half of the columns where the tile has them; the loads lie in what always runs, since their number is what the waits count.
+  constexpr int FMU = FM > 2 ? FM / 2 : FM, H = FN / 2, LOAD_EVERY = FMU * H / PASSES;
   constexpr unsigned FAR = 0x80000000u;            // beyond every view of x and W: read as zeros without traffic
-  extern __shared__ __attribute__((aligned(16))) bf16 smem[];      // [STAGES][ROWS][32]
-  __shared__ int tiles_before[GS_MAX_GROUPS + 1];
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];      // x [PAIRS][BM][64], W [STAGES][BN][32]
   const int tid = threadIdx.x, lane = tid % SYN_WAVE, grid = (int)gridDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / SYN_WAVE);
-  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * (BN / 2);
+  const int wr = wave / 2, wc = wave % 2;
   const int col_tiles = (g.N + BN - 1) / BN;
-  if (wave == 0) {                                 // tiles of the segments before each: a prefix sum, 64 segments at a time
-    int before = 0;
-    for (int e0 = 0; e0 < g.groups; e0 += SYN_WAVE) {
-      const int e = e0 + lane;
-      int n = e < g.groups ? (g.seg_start[e + 1] - g.seg_start[e] + BM - 1) / BM : 0;
+  // lane l of tiles_up_to[i]: the tiles of all segments up to 64 i + l (a prefix sum in every wave's registers, 64 segments at a time)
+  constexpr int GROUP_PARTS = GS_MAX_GROUPS / SYN_WAVE;
+  int tiles_up_to[GROUP_PARTS], all_rows = 0;
 #pragma unroll
-      for (int off = 1; off < SYN_WAVE; off <<= 1) {
-        const int o = __shfl_up(n, off, SYN_WAVE);
-        if (lane >= off) n += o;
-      }
-      if (e < g.groups) tiles_before[e + 1] = before + n;
-      before += __shfl(n, SYN_WAVE - 1, SYN_WAVE);
+  for (int i = 0; i < GROUP_PARTS; ++i) {
+    if (i * SYN_WAVE >= g.groups) {
+      tiles_up_to[i] = all_rows;
+      continue;
     }
-    if (lane == 0) tiles_before[0] = 0;
+    const int e = i * SYN_WAVE + lane;
+    int n = e < g.groups ? (g.seg_start[e + 1] - g.seg_start[e] + BM - 1) / BM : 0;
+#pragma unroll
+    for (int off = 1; off < SYN_WAVE; off <<= 1) {
+      const int o = __shfl_up(n, off, SYN_WAVE);
+      if (lane >= off) n += o;
+    }
+    tiles_up_to[i] = all_rows + n;
+    all_rows = __builtin_amdgcn_readlane(tiles_up_to[i], SYN_WAVE - 1);
   }
-  __syncthreads();
-  const int tiles = __builtin_amdgcn_readfirstlane(tiles_before[g.groups]) * col_tiles;
+  // A last round that half of the workgroups could go round in is cut: each of its tiles becomes two of half the columns.
+  const int all = all_rows * col_tiles;
+  const int whole = all % grid * 2 <= grid ? all / grid * grid : all, tiles = 2 * all - whole;
   int at = ((int)blockIdx.x % 8) * (grid / 8) + (int)blockIdx.x / 8;
   if (at >= tiles) return;
   struct Tile {
-    int e, row0, row_end, n0;
+    int e, row0, row_end, n0, columns, active;      // columns: BN or half of them; active: row groups that hold rows
   };
   auto tile_of = [&](int i) {
+    const bool cut = i >= whole;
+    const int half = cut ? (i - whole) % 2 : 0;
+    if (cut) i = whole + (i - whole) / 2;
     const int rt = i / col_tiles;
-    int lo = 0, hi = g.groups;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) / 2;
-      if (tiles_before[mid] <= rt) lo = mid; else hi = mid;
+    int lo = 0, first = 0;      // the segment and the tiles before it: those up to `lo` segments are no more than rt
+#pragma unroll
+    for (int p = 0; p < GROUP_PARTS; ++p) {
+      const int n = p * SYN_WAVE < g.groups ? __builtin_popcountll(__ballot(tiles_up_to[p] <= rt)) : 0;
+      if (n > 0) first = __builtin_amdgcn_readlane(tiles_up_to[p], n - 1);
+      lo += n;
     }
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    const int first = __builtin_amdgcn_readfirstlane(tiles_before[lo]);
-    const int s0 = g.seg_start[lo], s1 = g.seg_start[lo + 1];
-    return Tile{lo, s0 + (rt - first) * BM, s1, (i % col_tiles) * BN};
+    const int s0 = __builtin_amdgcn_readfirstlane(g.seg_start[lo]), s1 = __builtin_amdgcn_readfirstlane(g.seg_start[lo + 1]);
+    // (the segment's tiles get the same number of rows, in steps of 32)
+    const int n = (s1 - s0 + BM - 1) / BM, rows = ((s1 - s0 + n - 1) / n + 31) / 32 * 32;
+    const int row0 = s0 + (rt - first) * rows, row_end = min(s1, row0 + rows), n0 = (i % col_tiles) * BN + half * (BN / 2);
+    return Tile{lo, row0, row_end, n0, cut || g.N - n0 <= BN / 2 ? BN / 2 : BN, (row_end - row0 + 31) / 32};
   };
   const BufferView vx = buffer_view(g.a, (size_t)a_bytes);
-  struct Source {
-    BufferView w;
-    unsigned x[XL];      // offsets of the lane's pieces of rows
-  };
   const size_t w_row = (size_t)g.K * sizeof(bf16);
-  auto source = [&](const Tile& t) {
-    Source s;
-    s.w = buffer_view((const bf16*)g.w + (size_t)t.e * g.w_group + (size_t)t.n0 * g.K, (size_t)(g.N - t.n0) * w_row);
+  struct Rows {
+    unsigned at[XL];      // offsets of the lane's pieces of rows: load p of x takes 128 bytes of tile rows (p * WAVES + wave) * 8 .. + 8
+  };
+  auto rows_of = [&](const Tile& t) {
+    Rows x;
+    const int r0 = t.row0 + wave * 8 + lane / 8;
+    int row[XL];
 #pragma unroll
-    for (int p = 0; p < XL; ++p) {
-      const int r = t.row0 + (p * WAVES + wave) * RPI + lane / 4;
-      const int row = r < t.row_end ? (g.a_rows ? g.a_rows[r] : r) : -1;
-      s.x[p] = row < 0 ? FAR : (unsigned)((size_t)row * g.lda * sizeof(bf16)) + ((lane % 4) ^ (lane / 16)) * 16;
+    for (int p = 0; p < XL; ++p) row[p] = min(r0 + p * WAVES * 8, t.row_end - 1);
+    if (g.a_rows) {      // (asked for together)
+#pragma unroll
+      for (int p = 0; p < XL; ++p) row[p] = g.a_rows[row[p]];
     }
-    return s;
+#pragma unroll
+    for (int p = 0; p < XL; ++p)
+      x.at[p] = r0 + p * WAVES * 8 < t.row_end ? (unsigned)((size_t)row[p] * g.lda * sizeof(bf16)) + ((lane % 8) ^ (wave % 2 * 4 + lane / 16)) * 16 : FAR;
+    return x;
+  };
+  auto weights_of = [&](const Tile& t) {
+    return buffer_view((const bf16*)g.w + (size_t)t.e * g.w_group + (size_t)t.n0 * g.K, (size_t)max(0, min(t.columns, g.N - t.n0)) * w_row);
   };
   unsigned src_w[WL];
 #pragma unroll
-  for (int p = 0; p < WL; ++p) src_w[p] = (unsigned)((size_t)(p * WAVES + wave) * RPI * w_row + lane * 16);
-  auto fetch = [&](const Source& s, int kt, int buf, int p) {
-    bf16* dst = smem + (size_t)buf * ROWS * BK + (size_t)(p * WAVES + wave) * RPI * BK;
-    if (p < XL) buffer_to_lds16(vx, dst, s.x[p < XL ? p : 0], kt * BK * (int)sizeof(bf16));
-    else buffer_to_lds16(s.w, dst, src_w[p < XL ? 0 : p - XL], kt * BK * (int)sizeof(bf16) * 16);
+  for (int p = 0; p < WL; ++p) src_w[p] = (unsigned)((size_t)(p * WAVES + wave) * 16 * w_row + lane * 16);
+  // where the loads have got to, as in gemm_stream_kernel
+  constexpr int W_TILE = BK * (int)sizeof(bf16) * 16, X_PAIR = 2 * BK * (int)sizeof(bf16);
+  constexpr int W_BUF = BN * BK * (int)sizeof(bf16), X_BUF = BM * X_PAIR;
+  const int steps = g.K / BK, w_end = steps * W_TILE, x_end = steps * (X_PAIR / 2);
+  const int x_to = wave * 8 * X_PAIR, w_to = PAIRS * X_BUF + wave * 16 * BK * (int)sizeof(bf16);
+  int x_way = 0, w_way = 0;
+  Rows x_rows, x_rows_then;
+  BufferView w_view, w_then;
+  auto onward_w = [&] {
+    w_way += W_TILE;
+    if (__builtin_expect(w_way == w_end, 0)) w_way = 0, w_view = w_then;
+  };
+  auto onward_x = [&] {
+    x_way += X_PAIR;
+    if (__builtin_expect(x_way == x_end, 0)) x_way = 0, x_rows = x_rows_then;
+  };
+  auto fetch_x = [&](int xbuf, int p) {
+    buffer_to_lds16(vx, (char*)smem + xbuf + x_to + p % XL * (WAVES * 8 * X_PAIR), x_rows.at[p % XL], x_way);
+  };
+  auto fetch_w = [&](int buf, int p) {
+    buffer_to_lds16(w_view, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], w_way);
   };
   f32x4 acc[FM][FN];
   const int r16 = lane % 16, q4 = lane / 16;
-  const int x_at = (wm + r16) * BK + (q4 ^ (r16 / 4)) * 8, w_at = (BM + wn) * BK + lane * 8;
+  // in bytes; the second k-tile of a pair: chunks 4 to 7, bit 2 of the slot
+  const int x_at = ((16 * wr + r16) * 2 * BK + (q4 ^ (r16 / 2)) * 8) * 2, x_at2 = x_at ^ 64;
   bf16x8 a[2][FM], b[2][FN];
-  auto read_one = [&](int buf, int set, int idx) {
-    const bf16* base = smem + (size_t)buf * ROWS * BK;
-    if (idx < FM) a[set][idx] = *(const bf16x8*)(base + x_at + idx * 16 * BK);
-    else b[set][idx - FM] = *(const bf16x8*)(base + w_at + (idx - FM) * 16 * BK);
-  };
-  const int steps = g.K / BK;
-  auto step = [&](const Source& now, const Source& then, int kt, int buf, auto set, auto fresh) {
+  auto read_x = [&](int xbuf, int half, int set, int i) { a[set][i] = *(const bf16x8*)((const char*)smem + xbuf + (half ? x_at2 : x_at) + i * 32 * X_PAIR); };
+  auto read_w = [&](int buf, int set, int j, int w_at) { b[set][j] = *(const bf16x8*)((const char*)smem + buf + w_at + j * 16 * BK * 2); };
+  int buf = 0, xbuf = 0, xbuf_before = STAGES / 2 * X_BUF;
+  auto step = [&](int parts, int w_at, auto set, auto fresh) {
     constexpr int SET = decltype(set)::value;
-    const int next = buf + 1 == STAGES ? 0 : buf + 1;
-    const bool over = kt + STAGES >= steps;
-    Source s;
-    s.w = over ? then.w : now.w;
-#pragma unroll
-    for (int p = 0; p < XL; ++p) s.x[p] = over ? then.x[p] : now.x[p];
-    const int ahead = over ? kt + STAGES - steps : kt + STAGES;
-#pragma unroll
-    for (int q = 0; q < NM; ++q) {
-      const int j = q / FM, i = q % FM;
+    const int next = buf + W_BUF == STAGES * W_BUF ? 0 : buf + W_BUF;
+    const int xnext = SET ? (xbuf + X_BUF == PAIRS * X_BUF ? 0 : xbuf + X_BUF) : xbuf;
+    // four matrix instructions of row group I from column J on, passed over as a whole where bit 2 I + J / H of `parts` is clear: the
+    // branch stands inside the statement, so that the sums stay where they are (around statements the compiler moved them)
+    auto four = [&](auto group, auto column) {
+      constexpr int I = decltype(group)::value, J = decltype(column)::value, BIT = 2 * I + J / H;
       if constexpr (decltype(fresh)::value)
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[i][j]) : "v"(b[SET][j]), "v"(a[SET][i]));
+        asm volatile("s_bitcmp1_b32 %9, %10\n\ts_cbranch_scc0 .Lpast%=\n\t"
+                     "v_mfma_f32_16x16x32_bf16 %0, %4, %8, 0\n\tv_mfma_f32_16x16x32_bf16 %1, %5, %8, 0\n\t"
+                     "v_mfma_f32_16x16x32_bf16 %2, %6, %8, 0\n\tv_mfma_f32_16x16x32_bf16 %3, %7, %8, 0\n.Lpast%=:"
+                     : "=a"(acc[I][J]), "=a"(acc[I][J + 1]), "=a"(acc[I][J + 2]), "=a"(acc[I][J + 3])
+                     : "v"(b[SET][J]), "v"(b[SET][J + 1]), "v"(b[SET][J + 2]), "v"(b[SET][J + 3]), "v"(a[SET][I]), "s"(parts), "n"(BIT) : "scc");
       else
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b[SET][j]), "v"(a[SET][i]));
-      if (q % LOAD_EVERY == 0 && q / LOAD_EVERY < PASSES) fetch(s, ahead, buf, q / LOAD_EVERY);
-      if (q % READ_EVERY == READ_EVERY - 1 && q / READ_EVERY < NR) read_one(next, SET ^ 1, q / READ_EVERY);
+        asm volatile("s_bitcmp1_b32 %9, %10\n\ts_cbranch_scc0 .Lpast%=\n\t"
+                     "v_mfma_f32_16x16x32_bf16 %0, %4, %8, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %5, %8, %1\n\t"
+                     "v_mfma_f32_16x16x32_bf16 %2, %6, %8, %2\n\tv_mfma_f32_16x16x32_bf16 %3, %7, %8, %3\n.Lpast%=:"
+                     : "+a"(acc[I][J]), "+a"(acc[I][J + 1]), "+a"(acc[I][J + 2]), "+a"(acc[I][J + 3])
+                     : "v"(b[SET][J]), "v"(b[SET][J + 1]), "v"(b[SET][J + 2]), "v"(b[SET][J + 3]), "v"(a[SET][I]), "s"(parts), "n"(BIT) : "scc");
       __builtin_amdgcn_sched_barrier(0);
+    };
+    auto row_group = [&](auto group) {
+      constexpr int I = decltype(group)::value;
+      if constexpr (I < FMU) {
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+          if constexpr (decltype(fresh)::value)
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[I][j]) : "v"(b[SET][j]), "v"(a[SET][I]));
+          else
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[I][j]) : "v"(b[SET][j]), "v"(a[SET][I]));
+          const int q = I * H + j;
+          if (q % LOAD_EVERY == 0 && q / LOAD_EVERY < PASSES) {
+            const int p = q / LOAD_EVERY;
+            if (p < XL / 2) fetch_x(SET ? xbuf : xbuf_before, SET ? p : p + XL / 2);
+            else fetch_w(buf, p - XL / 2);
+          }
+          if (q % FMU == FMU - 1) read_w(next, SET ^ 1, q / FMU, w_at);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        four(group, std::integral_constant<int, 0>{});
+      }
+      read_x(xnext, SET ^ 1, SET ^ 1, I);
+      __builtin_amdgcn_sched_barrier(0);
+      four(group, std::integral_constant<int, H>{});
+      if constexpr (I < FMU) {
+#pragma unroll
+        for (int j = H + I * H / FMU; j < H + (I + 1) * H / FMU; ++j) read_w(next, SET ^ 1, j, w_at);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    row_group(std::integral_constant<int, 0>{}), row_group(std::integral_constant<int, 1>{});
+    if constexpr (FM > 2) row_group(std::integral_constant<int, 2>{}), row_group(std::integral_constant<int, 3>{});
+    if constexpr (FM > 4) {
+      row_group(std::integral_constant<int, 4>{}), row_group(std::integral_constant<int, 5>{});
+      row_group(std::integral_constant<int, 6>{}), row_group(std::integral_constant<int, 7>{});
     }
+    onward_w();
+    if constexpr (SET == 0) onward_x();
+    else xbuf_before = xbuf, xbuf = xnext;
+    buf = next;
   };
   constexpr int YOUNGER = (STAGES - 2) * PASSES;
   auto landed = [&] {
@@ -497,54 +576,86 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
     __builtin_amdgcn_sched_barrier(0);
   };
   Tile t = tile_of(at);
-  Source now = source(t);
-  __builtin_amdgcn_s_waitcnt(0x0070);        // (the row lists' own loads: the counts below are those of the ring alone)
+  bool more = at + grid < tiles;
+  Tile t_next = more ? tile_of(at + grid) : t;       // (behind the last tile: loads that nobody reads)
+  x_rows = rows_of(t), w_view = weights_of(t);
+  x_rows_then = rows_of(t_next), w_then = weights_of(t_next);
+  __builtin_amdgcn_s_waitcnt(0x0070);        // (the row lists' own loads: the counts below are those of the rings alone)
   __builtin_amdgcn_sched_barrier(0);
+  // what the steps before the first would have asked for
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s)
+  for (int p = 0; p < XL / 2; ++p) fetch_x(0, p);
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) fetch(now, s, s, p);
+  for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+    for (int p = 0; p < XL / 2; ++p) fetch_x((s + 1) / 2 * X_BUF, s % 2 ? p : p + XL / 2);
+#pragma unroll
+    for (int p = 0; p < WL; ++p) fetch_w(s * W_BUF, p);
+    onward_w();
+    if (s % 2 == 0) onward_x();
+  }
   landed();
-#pragma unroll
-  for (int i = 0; i < NR; ++i) read_one(0, 0, i);
-  __builtin_amdgcn_s_waitcnt(0xc07f);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
   using Even = std::integral_constant<int, 0>;
   using Odd = std::integral_constant<int, 1>;
   const BufferView vo = buffer_view(g.out, (size_t)o_bytes);
-  int buf = 0;
   for (;;) {
-    const bool more = at + grid < tiles;
-    const Tile t_next = more ? tile_of(at + grid) : t;
-    const Source then = source(t_next);
-    auto turn = [&] { buf = buf + 1 == STAGES ? 0 : buf + 1; };
-    step(now, then, 0, buf, Even{}, std::true_type{}), landed(), turn();
-    step(now, then, 1, buf, Odd{}, std::false_type{}), landed(), turn();
+    const int active = t.active, wn = wc * (t.columns / 2), w_at = PAIRS * X_BUF + (wn * BK + lane * 8) * 2;
+    const bool wide = t.columns == BN;
+    // bit 2 i: row group i holds rows, bit 2 i + 1: and the tile its right half of columns
+    const int parts = ((1 << 2 * active) - 1) & (wide ? 0xffff : 0x5555);
+    // the first fragments: all of them, the tile before may have had fewer rows or columns
+#pragma unroll
+    for (int i = 0; i < FM; ++i) read_x(xbuf, 0, 0, i);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) read_w(buf, 0, j, w_at);
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): they are in registers,
+    __builtin_amdgcn_s_barrier();         // everywhere
+    __builtin_amdgcn_sched_barrier(0);
+    step(parts, w_at, Even{}, std::true_type{}), landed();
+    step(parts, w_at, Odd{}, std::false_type{}), landed();
     // (entered always, K >= 256: with a way round the loop the compiler carried some sums of the 256-row tile through vector
     // registers there, read right behind matrix instructions that it does not know for such)
     int kt = 2;
     do {
-      step(now, then, kt, buf, Even{}, std::false_type{}), landed(), turn();
-      step(now, then, kt + 1, buf, Odd{}, std::false_type{}), landed(), turn();
+      step(parts, w_at, Even{}, std::false_type{}), landed();
+      step(parts, w_at, Odd{}, std::false_type{}), landed();
       kt += 2;
     } while (kt < steps);
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // (see gemm_stream_kernel)
     __builtin_amdgcn_sched_barrier(0);
-    // lane: row t.row0 + wm + 16 i + r16, columns t.n0 + wn + 16 j + 4 q4 .. + 4
+    // What the stores look up, and the rows of the tile after the next: all of it before the first store, since whatever is loaded
+    // behind stores is waited for behind them too.
+    const int r0 = t.row0 + 16 * wr + r16;
+    int o_row[FM];
+    float weight_of[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) o_row[i] = min(r0 + 32 * i, t.row_end - 1), weight_of[i] = 1.f;
+    if (g.row_weight) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) weight_of[i] = g.row_weight[o_row[i]];
+    }
+    if (g.o_rows) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) o_row[i] = g.o_rows[o_row[i]];
+    }
+    const bool more_then = more && at + 2 * grid < tiles;
+    const Tile t_then = more_then ? tile_of(at + 2 * grid) : t_next;
+    const Rows rows_then = rows_of(t_then);
+    __builtin_amdgcn_sched_barrier(0);
+    // lane: row t.row0 + 32 i + 16 wr + r16, columns t.n0 + wn + 16 j + 4 q4 .. + 4
     auto store_all = [&](auto of) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
-        const int r = t.row0 + wm + 16 * i + r16;
-        const bool in = r < t.row_end;
-        const unsigned row = in ? (unsigned)((size_t)(g.o_rows ? g.o_rows[r] : r) * g.ldo * (F32 ? 4 : 2)) : 0u;
-        const float weight = in && g.row_weight ? g.row_weight[r] : 1.f;
+        if (i >= FMU && i >= active) break;
+        const unsigned row = (unsigned)((size_t)o_row[i] * g.ldo * (F32 ? 4 : 2));
+        const bool in = r0 + 32 * i < t.row_end;
+        const float weight = weight_of[i];
 #pragma unroll
         for (int j = 0; j < FN; ++j) asm volatile("" : "+a"(acc[i][j]));
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const int n = t.n0 + wn + 16 * j + 4 * q4;
-          const bool ok = in && n < g.N;
+          const bool ok = in && n < g.N && (j < H || wide);
           if constexpr (PAIR) {
             const float v0 = of(acc[i][j][0], acc[i][j][1]) * weight, v1 = of(acc[i][j][2], acc[i][j][3]) * weight;
             if constexpr (F32) {
@@ -571,9 +682,13 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
       }
     };
     if constexpr (PAIR) {
-      if (g.pair - 1 == SYN_ACT_SILU) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SILU, F32>(gt, up, 0.f); });
-      else if (g.pair - 1 == SYN_ACT_SWIGLU_LIMIT) store_all([&](float gt, float up) { return gated_quick<SYN_ACT_SWIGLU_LIMIT, F32>(gt, up, g.limit); });
-      else store_all([&](float gt, float up) { return gated_quick<SYN_ACT_GELU_TANH, F32>(gt, up, 0.f); });
+      // (one loop with a branch that all lanes share in it: with a loop for each activation the compiler moved sums around in the k-steps)
+      const int act = g.pair - 1;
+      store_all([&](float gt, float up) {
+        if (act == SYN_ACT_SILU) return gated_quick<SYN_ACT_SILU, F32>(gt, up, 0.f);
+        if (act == SYN_ACT_SWIGLU_LIMIT) return gated_quick<SYN_ACT_SWIGLU_LIMIT, F32>(gt, up, g.limit);
+        return gated_quick<SYN_ACT_GELU_TANH, F32>(gt, up, 0.f);
+      });
     } else {
       if (g.act == 0) store_all([&](float v, float) { return v; });
       else if (g.act == 2) store_all([&](float v, float) { return point_activation(SYN_POINT_RELU_SQUARED, v); });
@@ -581,14 +696,15 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
     }
     __builtin_amdgcn_sched_barrier(0);
     if (!more) break;
-    at += grid, t = t_next, now = then;
+    at += grid, t = t_next, t_next = t_then, more = more_then;
+    x_rows_then = rows_then, w_then = weights_of(t_next);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);
 }
 
 template <int BM, int BN, bool F32, bool PAIR>
 static int launch_grouped_stream(const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
-  const size_t lds = (size_t)grouped_stages(BM, BN) * (BM + BN) * 32 * sizeof(bf16);
+  const size_t lds = stream_lds(BM, BN);
   static OncePerDevice raised;
   const hipError_t e = once_per_device(raised, [&] {
     return hipFuncSetAttribute((const void*)grouped_stream_kernel<BM, BN, F32, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

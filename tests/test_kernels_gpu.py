@@ -798,12 +798,12 @@ def test_gated_epilogue_of_streamed_tiles_is_no_less_exact(ops, act, out_dtype):
 
 
 @pytest.mark.parametrize("counts,J,K", [([0, 1, 63, 64, 129, 300, 0, 43], 544, 320), ([48], 32, 256), ([600, 0, 5], 256, 512),
-                                        ([130] * 70, 288, 256)])
+                                        ([130] * 70, 288, 256), ([257, 225, 31, 256], 544, 320), ([50] * 300, 288, 256)])
 @pytest.mark.parametrize("act,gated,out_dtype", [(None, None, F32), ("gelu", None, BF16), ("gelu", None, F32), ("relu_squared", None, BF16),
                                                  (None, "silu", BF16), (None, ("swiglu_limit", 7.0), F32), (None, "gelu_tanh", BF16)])
 def test_streamed_experts(ops, counts, J, K, act, gated, out_dtype):
     """Rows of many experts through the streamed tiles: experts without rows, with one, at the edges of a tile and over several
-    tiles; gathered rows, scattered results with weights, every epilogue; places of out that no row names stay as they were."""
+    tiles, a last round in halves of tiles; gathered rows, scattered results with weights, every epilogue; places of out that no row names stay as they were."""
     E, P = len(counts), sum(counts)
     g = torch.Generator().manual_seed(J + K)
     x, w = rnd((P + 9, K), 90, BF16), rnd((E, J, K), 91, BF16, 0.3)
