@@ -262,7 +262,32 @@ __device__ __forceinline__ float packed_point(const Epilogue& ep, float v) {
 // memory for every wave (x stays in the caches); that costs as many requests as W from 16 rows on,
 // so the callers use this kernel up to 8 rows.  Wave kw of a group takes the k-steps kw * U .. + U,
 // then those KWAVES * U further on.
-template <int TILES, int KWAVES, int U, bool PAIRED>
+//
+// The rows of x as these kernels load them: lane r16 + 16 q has k-values 8 q .. + 8 of row r16.  EIGHT: of up to eight rows, lanes
+// r16 < 8 those of one k-step and lanes r16 >= 8 those of the next, so that a load asks for whole lines of 128 bytes.  A product with
+// W's fragment of the first k-step then leaves its sums in rows 0 to 7 and one with that of the next in rows 8 to 15; what stands
+// in the other rows mixes the two and is never read.  For plain products of 5 to 8 rows: 8 rows through 12,288 x 4,096 17.8 -> 16.8 us,
+// 10,304 x 4,096 16.9 -> 15.9, 5,120 x 25,600 62.8 -> 58.1, 4,096 x 12,288 18.7 -> 18.2, 4,096 x 4,096 7.55, 7.52; 5 rows 16.7, 16.5,
+// 16.0, 15.1, 57.7, 56.1, 17.8, 17.9, 7.5, 7.5.  Fewer rows cost few requests either way and lost up to 1.5 us; gated products,
+// whose x serves two groups of rows of W, gained nothing (33.2, 33.5).
+template <bool EIGHT>
+struct XRows {
+  const bf16* row;
+  bool ok;
+  int behind;
+  __device__ __forceinline__ XRows(const bf16* x, int M, int K, int r16, int kq) {
+    const int r = EIGHT ? r16 % 8 : r16;
+    behind = EIGHT ? r16 / 8 : 0;
+    ok = r < M;
+    row = x + (size_t)min(r, M - 1) * K + behind * 32 + kq;
+  }
+  __device__ __forceinline__ bf16x8 load(int ks, int ks_end) const {
+    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    return ok && ks + behind < ks_end ? *(const bf16x8*)(row + ks * 32) : zero;
+  }
+};
+
+template <int TILES, int KWAVES, int U, bool PAIRED, bool EIGHT>
 __global__ void __launch_bounds__(TILES * KWAVES * SYN_WAVE)
 gemm_packed_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void* __restrict__ out, Epilogue ep,
                    int M, int N, int K, int ks_slice, RowNorm rn) {
@@ -278,9 +303,8 @@ gemm_packed_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void
   const int nks = K / 32;
   const bool tile_in = nt < n_tiles;   // the last workgroup may hold a group beyond the end
   const bf16* wt = wp + ((size_t)min(nt, n_tiles - 1) * nks * 64 + lane) * 8;
-  const bool xok = r16 < M;
-  const bf16* xrow = x + (size_t)min(r16, M - 1) * K + kq;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const XRows<EIGHT> xr(x, M, K, r16, kq);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc_odd = {0.f, 0.f, 0.f, 0.f};
   // what the epilogue needs of a norm's halves is asked for now, not behind the loop
   RowStat stat;
   if (rn.ss) row_stat_load(rn, M, wave, WAVES, lane, stat);
@@ -305,20 +329,23 @@ gemm_packed_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void
       for (int u = 0; u < U; ++u) {
         const bool in = ks0 + u < ks_end;
         bw[u] = in ? __builtin_nontemporal_load((const bf16x8*)(wt + (size_t)(ks0 + u) * 512)) : zero;
-        ax[u] = (in && xok) ? *(const bf16x8*)(xrow + (ks0 + u) * 32) : zero;
+        if (!EIGHT || u % 2 == 0) ax[u] = xr.load(ks0 + u, ks_end);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[u], bw[u], acc, 0, 0, 0);
+      for (int u = 0; u < U; ++u) {
+        if (EIGHT && u % 2) acc_odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[u - 1], bw[u], acc_odd, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[u], bw[u], acc, 0, 0, 0);
+      }
     }
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) part[wave][j][lane] = acc[j];
+  for (int j = 0; j < 4; ++j) part[wave][j][lane] = EIGHT && lane >= 32 ? acc_odd[j] : acc[j];
   if (rn.ss) row_stat_finish(rn, M, wave, WAVES, lane, stat, inv);
   __syncthreads();
   auto summed = [&](int t, int j, int ln) {
     float s = 0.f;
 #pragma unroll
-    for (int q = 0; q < KWAVES; ++q) s += part[t * KWAVES + q][j][ln];
+    for (int q = 0; q < KWAVES; ++q) s += EIGHT ? part[t * KWAVES + q][j][ln % 32] + part[t * KWAVES + q][j][ln % 32 + 32] : part[t * KWAVES + q][j][ln];
     return s;
   };
   if constexpr (PAIRED) {
@@ -351,13 +378,21 @@ gemm_packed_kernel(const bf16* __restrict__ x, const bf16* __restrict__ wp, void
   }
 }
 
-template <int TILES, int KWAVES, int U, bool PAIRED = false>
-static void launch_packed(const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K,
+template <int TILES, int KWAVES, int U, bool PAIRED, bool EIGHT>
+static void launch_packed_as(const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K,
                           hipStream_t stream, int slices, const RowNorm& rn) {
   const int rows = TILES * 16;
   const int ks_slice = (K / 32 + slices - 1) / slices;
-  gemm_packed_kernel<TILES, KWAVES, U, PAIRED>
+  gemm_packed_kernel<TILES, KWAVES, U, PAIRED, EIGHT>
       <<<dim3((N + rows - 1) / rows, slices), TILES * KWAVES * SYN_WAVE, 0, stream>>>(x, wp, out, ep, M, N, K, ks_slice, rn);
+}
+template <int TILES, int KWAVES, int U, bool PAIRED = false>
+static void launch_packed(const bf16* x, const bf16* wp, void* out, Epilogue ep, int M, int N, int K,
+                          hipStream_t stream, int slices, const RowNorm& rn) {
+  if constexpr (!PAIRED) {
+    if (M >= 5 && M <= 8) return launch_packed_as<TILES, KWAVES, U, PAIRED, true>(x, wp, out, ep, M, N, K, stream, slices, rn);
+  }
+  launch_packed_as<TILES, KWAVES, U, PAIRED, false>(x, wp, out, ep, M, N, K, stream, slices, rn);
 }
 
 
