@@ -9,9 +9,9 @@
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
 //   gemm_packed    bf16, M <= 16 (used up to 8): the same over a copy of W kept in the order of the MFMA
 //                  fragments, so that every load of a wave is 1 KB of consecutive bytes.
-//   gemm_stream    bf16, M > 64, K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
+//   gemm_stream    bf16, M > 56 (gated 16), K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
 //                  stream of k-steps over all tiles of a workgroup.
-//   gemm_direct    bf16, up to 64 rows, and up to 256 where its tiles go round once or their reader adds partial sums: 32 to 256
+//   gemm_direct    bf16, up to 56 or 64 rows, uncut products of large weights up to 256 where its tiles go round once: 32 to 128
 //                  rows of x, 64 to 128 rows of W, 64 to 256 deep, straight into LDS: the rows of W arrive as whole
 //                  256-byte pieces, which streams them faster than loading MFMA fragments (64 bytes a row) straight
 //                  from memory.
@@ -1235,7 +1235,11 @@ __device__ __forceinline__ TileAt stream_tile(int i, int tiles_m, int tiles_n) {
 #define SYN_OUT_BF16 0
 #define SYN_OUT_F32 1
 #define SYN_OUT_GATED 2     // W: gate and up rows in turns of 16; bf16, half as wide
-template <int BM, int BN, int OUT, bool WP>
+// ONCE: the rows fit one tile, so that W is read once: its loads are marked non-temporal.  (A stream of weights through the L2s pushes
+// everything else out of them: a decode step of 64 sequences at the 8B shape 7.53 -> 7.25 ms, a prompt of 96 tokens 5.10 -> 4.78.  Where
+// several rows of tiles read W it lost: 41,000 tokens at the 4B shape 299 -> 317 ms, 1,733 28.97 -> 29.13, and in two rows of tiles 160
+// tokens at the 8B shape 176 -> 181 us a layer, 96 at the 4B shape 118 -> 125.)
+template <int BM, int BN, int OUT, bool WP, bool ONCE>
 __global__ void __launch_bounds__(256, 1)
 gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void* __restrict__ out, Epilogue ep,
                    int M, int N, int K, int k_slice, int tiles, int whole, int streamed) {
@@ -1296,7 +1300,7 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     buffer_to_lds16(y.v, (char*)smem + xbuf + x_to + p * (WAVES * 8 * X_PAIR), src_x[p], y.at);
   };
   auto fetch_w = [&](const Way& y, int buf, int p) {
-    buffer_to_lds16(y.v, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], y.at);
+    buffer_to_lds16<ONCE>(y.v, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], y.at);
   };
   f32x4 acc[FM][FN];
   const int r16 = lane % 16, q4 = lane / 16;
@@ -1463,27 +1467,27 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
 
 // The tiles that the kernel comes in, and the estimate of a product's time that picks one of them and the slices of K.  Three
 // things run side by side, and the longest counts most (a norm of order 2): rounds of tiles over the chip at `round` us for 4,096
-// of K, a quarter of them whatever stands in the tiles; the matrix units' power, at `power` us for 4,096 of K with a tile on every
+// of K, 45 % of them whatever stands in the tiles; the matrix units' power, at `power` us for 4,096 of K with a tile on every
 // compute unit; and the way of W from memory, which is longer where fewer compute units ask for it.  Rows and columns beyond M
 // and N are zeros, which draw next to no power: with 129 rows 19,456 x 2,560 takes 34 us, with 256, the same tiles, 48.  So
-// both count by the share of a tile that is filled.  The stores of the output come on top.
-// The figures are fitted to 9,200 products measured with weights that no cache held: 72 to 3,000 rows, multiples of the tiles and
-// others, through N x K = 6144 x 4096, 4096 x 4096, 4096 x 12288, 2560 x 9728, 10240 x 5120, 32768 x 4096, 12288 x 4096, 8192 x 2048,
-// 5120 x 17408, 2048 x 8192, 6144 x 2560 (32-bit sums in 1, 2 and 4 slices of K) and, gated, 24576 x 4096, 19456 x 2560, 51200 x
-// 5120, 16384 x 2048, 28672 x 4096, 32768 x 4096, 20480 x 8192, 22016 x 4096, 17408 x 5120, 8192 x 1024, every tile.  What
-// the estimate picks takes 0.6 % longer than the fastest on average; 4 % of the sizes lose more than 5 %, 2 % more than 10 %.
+// both count by the share of a tile that is filled.  The stores of the output come on top, and where W is read by more than one
+// row of tiles, so that it passes through the caches (ONCE above), what it pushes out of them: in a step of 96 rows gate+up of 24,576 x
+// 4,096 in tiles of 64 x 192 made a layer take 6 to 8 us longer than in tiles of 128 x 128, though by itself it is 5 us faster.
+// The figures are fitted to 744 sizes, every tile and number of slices, with weights that no cache held: 17 to 3,300 rows, multiples of
+// the tiles and others, through N x K = 6144 x 4096, 10240 x 5120, 12288 x 4096, 3072 x 1024, 4096 x 2048, 8192 x 2048, 6144 x 2560 (rounded to
+// bf16), 4096 x 4096, 4096 x 12288, 2560 x 4096, 2560 x 9728, 5120 x 8192, 5120 x 25600, 1024 x 4096, 2048 x 8192, 6144 x 2560 (32-bit sums
+// in 1 to 8 slices of K and the norm that adds them) and, gated, 24576 x 4096, 19456 x 2560, 51200 x 5120, 8192 x 1024.  What the
+// estimate picks takes 0.5 % longer than the fastest on average; 3 % of the sizes lose more than 5 %, 2 of them more than 10 %
+// (with x in pieces of 64 bytes and the figures and rules fitted to that, on the same products: 3.8 %, 25 %, 11 %).
 struct StreamTile {
   int bm, bn;
   double round, power;
   bool plain;       // also over W in plain rows (the others are compiled for fragment order alone)
 };
 static const StreamTile STREAM_TILES[] = {
-    {256, 256, 82.9, 33.2, true},  {256, 192, 74.7, 20.6, true},  {128, 128, 38.0, 14.4, true},  {192, 256, 67.0, 24.9, false},
-    {128, 256, 56.0, 25.9, false}, {256, 128, 66.6, 22.0, false}, {192, 192, 59.0, 26.9, false}, {128, 192, 45.3, 16.3, false},
-    {64, 128, 23.5, 12.2, true},   {64, 192, 38.1, 5.3, false},
-    // of gemm_direct, for gated products of one tile of rows that go round once (W arrives in longer pieces; 28,672 x 4,096 with 224
-    // rows 69.5 us through the best streamed tile, 65.7 so; 32,768 x 4,096 75.9, 69.5)
-    {192, 128, 49.5, 0.0, true},   {256, 128, 46.2, 20.7, true}};
+    {256, 256, 86.0, 24.8, true}, {256, 192, 64.6, 26.1, true}, {128, 128, 36.4, 0.0, true}, {192, 256, 69.0, 25.3, false},
+    {128, 256, 53.6, 0.0, false}, {256, 128, 49.8, 19.7, false}, {192, 192, 54.7, 22.7, false}, {128, 192, 46.5, 0.0, false},
+    {64, 128, 20.5, 13.0, true}, {64, 192, 31.6, 13.7, false}};
 constexpr int STREAMED_TILES = 10;
 static int stream_slice(int K, int slices) { return ((K + slices - 1) / slices + 127) / 128 * 128; }
 static int stream_last_slice(int K, int slices) { return K - (slices - 1) * stream_slice(K, slices); }
@@ -1491,22 +1495,21 @@ struct StreamPlan {
   int tile;        // -1: none takes this K (k-steps come in pairs, and a slice holds a ring of them at least)
   double us;
 };
-static StreamPlan plan_stream(int M, int N, int K, int slices, bool packed, int out_bytes, bool gated) {
+static StreamPlan plan_stream(int M, int N, int K, int slices, bool packed, int out_bytes) {
   StreamPlan best = {-1, 1e30};
   if (K % 64) return best;
   const long cus = syn_compute_units();
   const double k = stream_slice(K, slices) / 4096.0;
-  for (int i = 0; i < (int)(sizeof(STREAM_TILES) / sizeof(STREAM_TILES[0])); ++i) {
+  for (int i = 0; i < STREAMED_TILES; ++i) {
     const StreamTile& s = STREAM_TILES[i];
-    if (i < STREAMED_TILES ? (!packed && !s.plain) || stream_last_slice(K, slices) < 32 * stream_stages(s.bm, s.bn)
-                           : !gated || M > s.bm || M <= s.bm - 64 || tile_grid(M, N, s.bm, s.bn) > cus)
-      continue;
+    if ((!packed && !s.plain) || stream_last_slice(K, slices) < 32 * stream_stages(s.bm, s.bn)) continue;
     const long down = (M + s.bm - 1) / s.bm, across = (N + s.bn - 1) / s.bn, tiles = down * across * slices;
     const double filled = (double)M / (double)(down * s.bm) * (double)N / (double)(across * s.bn);
-    const double work = (double)((tiles + cus - 1) / cus) * s.round * k * (0.255 + 0.745 * filled) + 4.5;
+    const double work = (double)((tiles + cus - 1) / cus) * s.round * k * (0.453 + 0.547 * filled) + 0.7;
     const double power = (double)tiles / cus * s.power * k * filled;
-    const double ask = tiles < cus ? cbrt((double)cus / (double)tiles) : 1.0, way = 0.146e-6 * 2.0 * N * K * ask * ask;
-    const double us = sqrt(work * work + way * way + power * power) + 0.229e-6 * M * N * slices * out_bytes;
+    const double ask = tiles < cus ? cbrt((double)cus / (double)tiles) : 1.0, way = 0.124e-6 * 2.0 * N * K * ask * ask;
+    const double pushed = M > s.bm ? 0.06e-6 * fmax(0.0, 2.0 * N * K - 1e8) : 0.0;
+    const double us = sqrt(work * work + way * way + power * power) + 0.208e-6 * M * N * slices * out_bytes + pushed;
     if (us < best.us) best = {i, us};
   }
   return best;
@@ -1520,10 +1523,12 @@ static int launch_stream(const bf16* x, Weight w, void* out, Epilogue ep, int M,
   static OncePerDevice raised;
   if (lds > 65536) {
     const hipError_t e = once_per_device(raised, [&] {
-      hipError_t r = hipFuncSetAttribute((const void*)gemm_stream_kernel<BM, BN, OUT, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipError_t r = hipSuccess;
+      for (const void* k : {(const void*)gemm_stream_kernel<BM, BN, OUT, true, false>, (const void*)gemm_stream_kernel<BM, BN, OUT, true, true>})
+        if (r == hipSuccess) r = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if constexpr (PLAIN)
         if (r == hipSuccess)
-          r = hipFuncSetAttribute((const void*)gemm_stream_kernel<BM, BN, OUT, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+          r = hipFuncSetAttribute((const void*)gemm_stream_kernel<BM, BN, OUT, false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       return r;
     });
     SYN_CHECK(e == hipSuccess, "gemm: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
@@ -1539,10 +1544,14 @@ static int launch_stream(const bf16* x, Weight w, void* out, Epilogue ep, int M,
   const size_t bytes = (size_t)slices * M * N * (OUT == SYN_OUT_F32 ? 4 : OUT == SYN_OUT_BF16 ? 2 : 1);
   const int streamed = bytes > (48u << 20);      // (of the 256 MB that the memory-side cache holds, beside x and W)
   const int k_slice = stream_slice(K, slices);
-  if (w.packed)
-    gemm_stream_kernel<BM, BN, OUT, true><<<grid, 256, lds, stream>>>(x, w.p, out, ep, M, N, K, k_slice, (int)tiles, whole, streamed);
-  else if constexpr (PLAIN)
-    gemm_stream_kernel<BM, BN, OUT, false><<<grid, 256, lds, stream>>>(x, w.p, out, ep, M, N, K, k_slice, (int)tiles, whole, streamed);
+  auto launch = [&](auto kernel) { kernel<<<grid, 256, lds, stream>>>(x, w.p, out, ep, M, N, K, k_slice, (int)tiles, whole, streamed); };
+  if (!w.packed) {
+    if constexpr (PLAIN) launch(gemm_stream_kernel<BM, BN, OUT, false, false>);
+  } else if (M <= BM) {
+    launch(gemm_stream_kernel<BM, BN, OUT, true, true>);
+  } else {
+    launch(gemm_stream_kernel<BM, BN, OUT, true, false>);
+  }
   return 0;
 }
 
@@ -1577,15 +1586,11 @@ static int pick_register_tile(int M, int N) {
   return best;
 }
 
-// M > 64.  A K that the kernel above does not take goes through the tiles that pass through registers (any K that is a multiple
+// M > 56, gated M > 16.  A K that the kernel above does not take goes through the tiles that pass through registers (any K that is a multiple
 // of 8, one slice) or, in slices, through the smallest of those that load straight into LDS.
 template <bool PAIRED>
 static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1, int tile = -1) {
-  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2, PAIRED).tile;
-  if constexpr (PAIRED) {
-    if (tile == STREAMED_TILES) return launch_direct<192, 128, 64, 2, 2, true, 3>(x, w, out, ep, M, N, K, stream);
-    if (tile == STREAMED_TILES + 1) return launch_direct<256, 128, 64, 4, 2, true, 3>(x, w, out, ep, M, N, K, stream);
-  }
+  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
   if (tile >= 0) {
     if (PAIRED) return launch_stream_as<SYN_OUT_GATED>(tile, x, w, out, ep, M, N, K, stream, slices);
     if (ep.out_is_f32) return launch_stream_as<SYN_OUT_F32>(tile, x, w, out, ep, M, N, K, stream, slices);
@@ -1599,38 +1604,25 @@ static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, 
   return launch_tiled<128, 128, 64, 2, 2, PAIRED>(x, w.p, out, ep, M, N, K, stream);
 }
 
-// Whether an uncut product of 65 to 256 rows goes through the 64 x 128 tiles with k-tiles of 128 (gemm_direct): where they go round once
-// (tile_grid, which counts what each XCD gets), W arrives in longer pieces than the streamed tiles ask for.  Weights that no cache
-// holds, direct against streamed: 4096 x 4096 96 rows 26.6 us against 28.8, 128 rows 29.1, 35.4, 256 rows 29.2, 35.2; 10,240 x 5,120
-// 128 rows 39.6, 48.4; 4096 x 12288 192 rows 80.5, 101.2.  Not where the last 64 rows are few (4096 x 12288: 65 rows 71.5, 66.4; 81
-// rows 69.2, 71.3; 193 rows 76.9, 66.3; 208 rows 71.7, 71.2), and not in two rounds (10,240 x 4,096 129 rows 50.1, 27.7).
-static bool direct_one_round(int M, int N) {
-  return M <= 256 && (M - 1) % 64 >= 16 && tile_grid(M, N, 64, 128) <= syn_compute_units();
+// Whether an uncut product of 65 to 256 rows goes through the 64 x 128 tiles with k-tiles of 128 (gemm_direct): large weights whose tiles
+// go round once (tile_grid, which counts what each XCD gets) and whose last 64 rows are at least half full, where W arrives in longer
+// pieces than the streamed tiles ask for.  Direct against the best streamed tile, us: 12,288 x 4,096 with 96 rows 30.4, 32.1, 128 rows
+// 32.9, 35.2, 84 rows 34.7, 30.9; 6,144 x 4,096 with 96 rows 27.9, 28.6, 256 rows 30.4, 31.3; 10,240 x 5,120 with 128 rows 40.2, 41.9, 84
+// rows 38.1, 36.3; 4,096 x 2,048 with 128 rows 17.1, 13.1; 8,192 x 2,048 17.8, 16.0; 6,144 x 2,560 21.9, 15.9.
+static bool direct_one_round(int M, int N, int K) {
+  return M <= 256 && (M - 1) % 64 >= 31 && K >= 4096 && (long)N * K >= 24L << 20 && tile_grid(M, N, 64, 128) <= syn_compute_units();
 }
 
-// Whether a product of 177 to 256 rows whose reader adds partial sums takes the tiles of 128 x 128 that hold k-tiles of 64
-// (gemm_direct) in two slices: where they go round once and leave few compute units without work, since what they take hardly
-// depends on N.  Against the streamed tiles in the slices of the estimate, what the reader pays for further slices included, weights
-// that no cache holds: 6144 x 2560 177 rows 18.1 us against 19.7, 256 rows 18.6, 21.9; 6144 x 4096 177 rows 24.0, 23.5, 256 rows 24.4,
-// 26.9; 7168 x 8192 200 rows 43.1, 46.1; 8192 x 5120 256 rows 32.6, 36.3.  Not with three quarters of the compute units and longer
-// sums (6144 x 6144 192 rows 34.3, 32.2), nor with fewer (5120 x 4096 192 rows 23.7, 21.1), nor in short ones (8192 x 2048 192 rows
-// 17.1, 16.8; 200 rows 17.2, 15.8).
-static bool direct_two_slices(int M, int N, int K) {
-  const long tiles = 4L * ((N + 127) / 128), cus = syn_compute_units();
-  return M > 176 && M <= 256 && K % 128 == 0 && K >= 2560 && tiles <= cus && 4 * tiles >= 3 * cus && (K <= 4096 || 20 * tiles >= 17 * cus);
-}
-
-// Into how many slices of K a product of more than 64 rows is cut when its reader adds partial sums: the smallest estimate of
+// Into how many slices of K a product of more than 56 rows is cut when its reader adds partial sums: the smallest estimate of
 // the product's time and of what its reader pays for the slices beyond the first (M x N floats each, half of them from caches).
 SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
   int best = 1;
   double least = 1e30;
   if (M <= 0 || N <= 0 || K <= 0) return 1;
-  if (direct_two_slices(M, N, K)) return 2;
   for (int s : {1, 2, 3, 4, 6, 8}) {
-    const StreamPlan p = plan_stream(M, N, K, s, true, 4, false);
+    const StreamPlan p = plan_stream(M, N, K, s, true, 4);
     if (p.tile < 0) break;
-    const double us = p.us + (s - 1) * 0.12e-6 * 4.0 * M * N;
+    const double us = p.us + (s - 1) * 0.14e-6 * 4.0 * M * N;
     if (us < least) least = us, best = s;
   }
   return best;
@@ -1717,8 +1709,6 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   const bf16* xb = (const bf16*)x;
   const bf16* wb = (const bf16*)w;
   const Weight wt = {wb, w_packed != 0};
-  const bool few_row_tiles = (M > 176 && M <= 256 && slices >= 4 && 2L * ((N + 127) / 128) * slices <= syn_compute_units()) ||
-                             (slices == 2 && direct_two_slices(M, N, K));
   // (from sweeps at the shapes of an 8B model, N = 4096 .. 151936, K = 4096 and 12288, where no other are named)
   int rc = 0;
   if (tile >= 0) {
@@ -1736,25 +1726,16 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     else if (N >= 65536 && !w_packed) rc = launch_tiled<32, 32, 256, 1, 1>(xb, wb, out, ep, M, N, K, stream, slices);
     else if (K % 128 == 0) rc = launch_direct<32, 64, 128, 1, 2>(xb, wt, out, ep, M, N, K, stream, slices);
     else rc = launch_tiled<32, 64, 128, 1, 2>(xb, wb, out, ep, M, N, K, stream, slices);
-  } else if (M <= 64 && K % 128 == 0) {
+  } else if (M <= 64 && K % 128 == 0 && !(M > 56 && slices > 1)) {
     // 33 to 64 rows: 128 rows of W a workgroup, so that the rows of x are fetched half as often (every
-    // workgroup reads all of x), three k-tiles in a ring, one workgroup a compute unit.  A decode step of 64
-    // sequences: 7.70 -> 7.51 ms with this tile for q/k/v, o_proj and down_proj, 7.26 with it for gate+up
-    // as well (though that product then has only 192 workgroups); 64 x 64 tiles in a ring of four: 8.08.
+    // workgroup reads all of x), three k-tiles in a ring, one workgroup a compute unit.  57 rows and more in slices go to the
+    // streamed tiles, in the slices of their estimate (these tiles in the slices that fill the compute units, and streamed, the
+    // norm behind it included, us with 64 rows: 4,096 x 4,096 18.2, 16.1; 4,096 x 12,288 28.6, 29.0; 6,144 x 4,096 20.6, 20.8; 2,560 x 4,096
+    // 15.3, 13.9; 5,120 x 25,600 63.9, 58.6; with 48: 17.0, 15.5; 26.7, 28.4; 19.3, 19.7; 14.0, 13.4; 60.8, 57.7).
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
-  } else if (M > 64 && K % 128 == 0 && (M <= 128 ? slices > 1 : few_row_tiles)) {
-    // 65 to 128 rows of a narrow product whose reader adds partial sums, still bound by reading W: k-tiles of 64 in a ring
-    // of three, all of x beside 128 rows of W, and as many slices of K as fill the compute units (ops.gemm_slices).  128
-    // rows: q/k/v of an 8B layer in 4 slices 17 us, down_proj in 8 slices 26; in a prompt step o_proj and down_proj together
-    // take 42 us with 128 rows, and 43 with 96 over the streamed tiles.  177 to 256 rows where the two rows of tiles
-    // go round once in four slices and more, or in two (direct_two_slices).  In four slices, against the streamed tile of the estimate: 4096 x 12288 160 rows
-    // 34.3 us, 32.0; 192 rows 34.2, 36.5; 256 rows 37.0, 42.9; 4096 x 4096 160 rows 15.3, 14.9; 192 rows 15.6, 16.3; 256 rows
-    // 17.0, 18.6; 2560 x 9728 160 rows 26.1, 21.6; 192 rows 27.1, 25.8; 256 rows 28.9, 31.3.
-    rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
-  } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N)) {
-    // the same of up to 256 rows whose reader takes the finished product
+  } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N, K)) {
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream);
-  } else if (M <= 64) {
+  } else if (M <= 64 && K % 128 != 0) {
     rc = launch_tiled<64, 64, 128, 2, 2>(xb, wb, out, ep, M, N, K, stream, slices);
   } else {
     rc = launch_large<false>(xb, wt, out, ep, M, N, K, stream, slices);
@@ -1786,6 +1767,11 @@ SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, i
     rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream, 1, tile);
   } else if (rows && w_packed) {
     rc = launch_rows<true>(rows, xb, wb, out, ep, M, N, K, 1, stream);
+  } else if (M > 64 || (M > 16 && K >= 256 && K % 64 == 0)) {
+    // the streamed tiles from 17 rows on (W in fragment order, us against the tiles below: 19,456 x 2,560 with 24 rows 26.8 -> 23.3, 64 27.3 ->
+    // 26.7, 128 34.9 -> 32.9; 24,576 x 4,096 with 64 45.1 -> 43.6, 96 48.2, 47.9; 51,200 x 5,120 with 32 99 -> 94, 128 166 -> 111; 8,192 x 1,024 with
+    // 128 18.6 -> 9.4)
+    rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream);
   } else if (M == 1 && !w_packed) {
     // one row: fragments of W straight from memory; eight waves on the gate rows, eight on the up rows
     launch_skinny<2, 8, 4, true>(xb, wb, out, ep, M, N, K, stream);
@@ -1793,16 +1779,10 @@ SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, i
     if (N >= 65536 && !w_packed) rc = launch_tiled<32, 32, 256, 1, 1, true>(xb, wb, out, ep, M, N, K, stream);
     else if (K % 128 == 0) rc = launch_direct<32, 64, 128, 1, 2, true>(xb, wt, out, ep, M, N, K, stream);
     else rc = launch_tiled<32, 64, 128, 1, 2, true>(xb, wb, out, ep, M, N, K, stream);
-  } else if (M <= 64) {
-    if (K % 128 == 0) rc = launch_direct<64, 128, 128, 2, 2, true, 3>(xb, wt, out, ep, M, N, K, stream);
-    else rc = launch_tiled<64, 64, 128, 2, 2, true>(xb, wb, out, ep, M, N, K, stream);
-  } else if (M <= 128 && K % 64 == 0) {
-    // 65 to 128 rows: still bound by reading W.  All of x in one tile beside 96 rows of W, so that W is read once (by as many
-    // workgroups as there are compute units at N = 24576); k-tiles of 64 in a ring of four.  In a prompt step of 128 rows
-    // 50 us where the tiles for more rows take 51 for 96 (24,576 x 4,096); the smallest 128 x 128 tile took 66.
-    rc = launch_direct<128, 96, 64, 4, 1, true, 4>(xb, wt, out, ep, M, N, K, stream);
+  } else if (K % 128 == 0) {
+    rc = launch_direct<64, 128, 128, 2, 2, true, 3>(xb, wt, out, ep, M, N, K, stream);
   } else {
-    rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream);
+    rc = launch_tiled<64, 64, 128, 2, 2, true>(xb, wb, out, ep, M, N, K, stream);
   }
   if (rc) return rc;
   SYN_LAUNCH_CHECK("gemm_swiglu");

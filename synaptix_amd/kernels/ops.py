@@ -328,8 +328,9 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
 
 
 # Products of up to this many rows over a weight in fragment order may take the kernel whose operands go straight to registers
-# (gemm_rows_kernel in csrc/gemm.hip).
-ROWS_MAX = 128
+# (gemm_rows_kernel in csrc/gemm.hip); more go faster through the streamed tiles (72 rows: 4,096 x 2,048 15.5 us, 13.0; 8,192 x 2,048 16.2,
+# 13.8; 128 rows 21.8, 13.2; gated 8,192 x 1,024 with 48 rows 9.1, 9.1, with 64 10.4, 9.2; 24,576 x 4,096 with 48 42.4, 43.3, with 56 61.8, 43.7).
+ROWS_MAX, ROWS_MAX_GATED = 64, 48
 
 
 def _bytes_a_unit(M, tile, K, slices, tiles, units, shared):
@@ -382,7 +383,7 @@ def _rows_pay(new, old, M, gated):
 @functools.lru_cache(maxsize=4096)
 def rows_tile(M, N, K, slices, gated=False) -> int:
     """Groups of 16 rows of W that a workgroup of gemm_rows_kernel takes for this product in so many slices, 0: it takes other tiles."""
-    if M > ROWS_MAX or M <= (PACKED_MAX_ROWS_GATED if gated else PACKED_MAX_ROWS) or K % 128 or N % 16:
+    if M > (ROWS_MAX_GATED if gated else ROWS_MAX) or M <= (PACKED_MAX_ROWS_GATED if gated else PACKED_MAX_ROWS) or K % 128 or N % 16:
         return 0
     new = _rows_choice(M, N, K, slices)
     if new is None or slices > 1 and slices != rows_slices(M, N, K):
@@ -583,19 +584,11 @@ def gemm_slices(M, N, K, dtype):
     if dtype != _BF16 or K % 8 != 0 or N > 16384 or K < 2048:
         return 1
     units = compute_units()
-    if M > 64:
-        if K % 128:
-            return 1
-        if M <= 128 or 176 < M <= 256:
-            # still bound by reading W: tiles of 128 x 128, cut until they fill the compute units (from 177 rows on here
-            # only where that takes four slices; where it takes two, csrc/gemm.hip knows)
-            most, slices = min(8, units // (-(-M // 128) * -(-N // 128)), K // 512), 1
-            while slices * 2 <= most:
-                slices *= 2
-            if slices > (1 if M <= 128 else 2):
-                return slices
-        # more: what the tiles take on so many rows, and what the reader of partial sums pays for them (csrc/gemm.hip)
+    if M > 56 and K % 128 == 0:
+        # what the streamed tiles take on so many rows, and what the reader of partial sums pays for the slices (csrc/gemm.hip)
         return _stream_slices(M, N, K)
+    if M > 64:
+        return 1
     if M <= 32:
         # 64 rows of W a workgroup, up to three workgroups a compute unit
         most = min(4, 3 * units // -(-N // 64), K // 512)

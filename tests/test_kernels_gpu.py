@@ -2,6 +2,7 @@
 (tests/cpu_kernels.py), at sizes other than the engine's test models use, with sizes that are
 no multiple of any tile.  Tolerances follow the reference's ladder for its CUDA kernels
 (crates/synaptix-kernels-cuda/tests/*: float32 1e-5 .. 1e-4, bf16 around 1e-2 on O(1) data)."""
+import itertools
 import math
 
 import pytest
@@ -719,6 +720,34 @@ def test_gated_products_of_129_to_256_rows(ops, M, N, K, packed):
     # the sums are off by at most 1e-4 sqrt(K) (products exact, 32-bit sums of K terms of size one), and both factors carry that; one rounding
     off = (out.double() - want).abs() - 2 ** -8 * want.abs() - 1e-4 * math.sqrt(K) * (g.abs() + u.abs() + 1)
     assert torch.isfinite(out).all() and float(off.max()) <= 0, float(off.max())
+
+
+@pytest.mark.parametrize("kind", ["gated", "slices"])
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("K", [128, 192, 256, 512, 1152])
+def test_products_where_the_streamed_tiles_begin(ops, K, packed, kind):
+    """On both sides of the row counts and widths from which the streamed tiles are taken, and of a tile of rows (up to which W's loads
+    are marked non-temporal), every value against 64 bits; nothing is left unwritten."""
+    if packed and K % 128:
+        pytest.skip("in fragment order K is a multiple of 128")
+    for M, S in itertools.product((16, 17, 49, 64, 65, 129), (1,)) if kind == "gated" else itertools.product((56, 57, 64, 65, 128, 129), (1, 2, 4)):
+        N = 800
+        if S > 1 and K % (S * 128):
+            continue
+        x, w = rnd((M, K), 94, BF16).to(DEV), rnd((N, K), 95, BF16).to(DEV)
+        weight = ops.pack_weight(w) if packed else w
+        if kind == "gated":
+            out = torch.full((M, N // 2), float("nan"), dtype=BF16, device=DEV)
+            ops.gemm_swiglu(x, weight, out)
+            z = (x.double() @ w.double().T).view(M, N // 32, 2, 16)
+            g, u = z[:, :, 0].reshape(M, -1), z[:, :, 1].reshape(M, -1)
+            want, room = g * torch.sigmoid(g) * u, 1e-4 * math.sqrt(K) * (g.abs() + u.abs() + 1)      # as above
+            off = (out.double() - want).abs() - 2 ** -8 * want.abs() - room
+        else:
+            out = torch.full((S, M, N), float("nan"), dtype=F32, device=DEV)
+            ops.gemm(x, weight, out if S > 1 else out[0])
+            off = (out.double().sum(0) - x.double() @ w.double().T).abs() - 1e-4 * math.sqrt(K)
+        assert torch.isfinite(out).all() and float(off.max()) <= 0, (M, S, float(off.max()))
 
 
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
