@@ -471,12 +471,13 @@ __global__ void qk_norm_rope_kv_write_kernel(const TIn* __restrict__ qkv, int n_
 // The same for the q and k heads of bf16 rows whose head size is 8 * LPH with LPH = 2, 4, .. 32 lanes
 // a head and whose rotation covers the whole head (or is absent): a lane holds 8 values of a head
 // (16-byte load and store), the sum of squares is reduced over the LPH lanes of the head, and the
-// partner of a rotated pair sits LPH / 2 lanes away.  A block takes 256 / LPH heads of one token.
+// partner of a rotated pair sits LPH / 2 lanes away.  A block takes 256 / LPH heads of four tokens each, counted on through the
+// heads and then the tokens, so that only the last block may hold idle lanes.
 // PARTS: the rows come as n_parts float partial sums [n_parts][tokens][heads * HD] of a product cut
 // along K (part_stride elements apart), which are added first, in their order.
 template <int LPH, bool PARTS>
 __device__ __forceinline__ void
-qk_heads_part(int block_x, int block_y, const void* __restrict__ qkv_in, int n_parts, size_t part_stride,
+qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t part_stride,
               bf16* __restrict__ q_out, bf16* __restrict__ k_pages,
                 const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
                 const int* __restrict__ tok_pos, const void* __restrict__ q_gain, const void* __restrict__ k_gain,
@@ -484,8 +485,10 @@ qk_heads_part(int block_x, int block_y, const void* __restrict__ qkv_in, int n_p
                 const float* __restrict__ sin_t, int n_tokens, int nh, int nkv, int n_active) {
   constexpr int HD = LPH * 8, HPB = 256 / LPH, half = HD / 2;
   constexpr int TPB = 4;  // tokens a block takes, their loads in flight together
-  const int head_raw = block_y * HPB + threadIdx.x / LPH;  // q heads, then k heads
-  const int head = min(head_raw, n_active - 1);                // idle lanes repeat the last head: shuffles need them
+  const uint32_t item = (uint32_t)block * HPB + threadIdx.x / LPH;
+  const bool idle = item >= (uint32_t)((n_tokens + TPB - 1) / TPB) * (uint32_t)n_active;
+  const int block_x = idle ? 0 : item / (uint32_t)n_active;    // idle lanes repeat the first head: shuffles need them
+  const int head = idle ? 0 : item % (uint32_t)n_active;       // q heads, then k heads
   const int c = threadIdx.x % LPH;                             // which 8 values of the head
   const bool is_q = head < nh, low = c < LPH / 2;
   const void* gain = is_q ? q_gain : k_gain;
@@ -574,7 +577,7 @@ qk_heads_part(int block_x, int block_y, const void* __restrict__ qkv_in, int n_p
         v[e] = low ? v[e] * cc[e] - partner * sc[e] : v[e] * cc[e] + partner * sc[e];
       }
     }
-    if (head_raw >= n_active || tok >= n_tokens) continue;
+    if (idle || tok >= n_tokens) continue;
     bf16x8 o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = (bf16)v[e];
@@ -587,70 +590,116 @@ qk_heads_part(int block_x, int block_y, const void* __restrict__ qkv_in, int n_p
   }
 }
 
-// The v heads of the same rows: 64 tokens x 32 dims a block go through LDS and are written in the
-// order of v_page_offset, in which 8 consecutive positions of one dim are one 16-byte piece and the
-// 16 dims of a fragment follow each other at 16 bytes.
-#define V_DIMS 32
+// The v heads of the same rows, in the order of v_page_offset: 8 consecutive positions of one dim are one 16-byte piece, and the 16
+// dims of a fragment follow each other at 16 bytes.  A wave takes 8 tokens and 128 of their nkv * hd values, a lane two of these:
+// whole lines of the rows, all tokens' loads in flight together.  Eight tokens that follow each other in one sequence from a
+// position that is a multiple of 8 are stored as pieces; such eight rarely are the wave's own, so it takes the eight that begin
+// among its own (at most one such run does) and, value by value, what of its own lies in no run: the ends of sequences.
+// Bound by memory.  (64 tokens x 32 dims through LDS, 64 bytes of a row a load and 2 bytes a lane a store, before: 41,028 tokens of 32 +
+// 8 + 8 heads of 128 in 16 sequences, q and k with their norm included, 320 -> 248 us or 4.1 TB/s, 2,048 tokens of 64 + 8 + 8 28.0 -> 24.2,
+// of 32 + 8 + 8 19.1 -> 18.0; the q heads alone 149 and 20 us.)
 template <bool PARTS>   // as for qk_heads_part
 __device__ __forceinline__ void
-v_block_write_part(int block_x, int block_y, int block_z, const void* __restrict__ qkv_in, int n_parts,
-                   size_t part_stride, bf16* __restrict__ v_pages, const int* __restrict__ page_table,
-                     int table_stride, const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int n_tokens,
-                     int nh, int nkv, int hd) {
-  constexpr int LD = V_DIMS + 2, PAIRS = V_DIMS / 2;
-  __shared__ __attribute__((aligned(16))) bf16 vtile[64 * LD];
-  __shared__ size_t dst_base[SYN_PAGE];
-  __shared__ int dst_slot[SYN_PAGE];
-  const int tid = threadIdx.x, t0 = block_x * 64, kvh = block_y, d0 = block_z * V_DIMS;
-  const int heads = nh + 2 * nkv;
-  for (int idx = tid; idx < 64 * PAIRS; idx += 256) {
-    const int j = idx / PAIRS, pr = idx % PAIRS;
-    if (t0 + j < n_tokens && d0 + 2 * pr < hd) {   // head sizes are even
-      const size_t at = ((size_t)(t0 + j) * heads + nh + nkv + kvh) * hd + d0 + 2 * pr;
-      if constexpr (PARTS) {
-        float2 sum = make_float2(0.f, 0.f);
-        for (int p = 0; p < n_parts; ++p) {
-          const float2 v = *(const float2*)((const float*)qkv_in + (size_t)p * part_stride + at);
-          sum.x += v.x, sum.y += v.y;
-        }
-        vtile[j * LD + 2 * pr] = (bf16)sum.x, vtile[j * LD + 2 * pr + 1] = (bf16)sum.y;
-      } else {
-        *(uint32_t*)(vtile + j * LD + 2 * pr) = *(const uint32_t*)((const bf16*)qkv_in + at);
+v_octets_write_part(int group, int chunk, const void* __restrict__ qkv_in, int n_parts, size_t part_stride,
+                    bf16* __restrict__ v_pages, const int* __restrict__ page_table, int table_stride,
+                    const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int n_tokens, int nh, int nkv, int hd) {
+  const int lane = threadIdx.x % SYN_WAVE, t0 = group * 8;
+  // a lane a token: the wave's own are lanes 7 to 14, behind what a run that reaches into them may begin with, before where theirs may end
+  const int t = t0 - 7 + lane;
+  const bool there = lane < 22 && t >= 0 && t < n_tokens;
+  const int seq = there ? tok_seq[t] : -1, pos = there ? tok_pos[t] : 0;
+  const bool was = __shfl_up((int)there, 1, SYN_WAVE) != 0;
+  const int seq_before = __shfl_up(seq, 1, SYN_WAVE), pos_before = __shfl_up(pos, 1, SYN_WAVE);
+  const uint64_t follows = __ballot(lane > 0 && there && was && seq == seq_before && pos == pos_before + 1);
+  uint64_t runs = (uintptr_t)v_pages % 16 == 0 ? __ballot(there && pos % 8 == 0) : 0;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) runs &= follows >> i;
+  uint64_t covered = runs;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) covered |= runs << i;
+  constexpr uint64_t OWN = 0xffull << 7;
+  const int run = (runs & OWN) ? __ffsll((unsigned long long)(runs & OWN)) - 1 : -1;
+  const uint32_t rest = (uint32_t)((__ballot(there) & OWN & ~covered) >> 7);
+  int page = 0;
+  if (there && ((OWN >> lane) & 1)) page = page_table[(size_t)seq * table_stride + pos / SYN_PAGE];
+
+  const int e = chunk * 128 + 2 * lane, width = nkv * hd, heads = nh + 2 * nkv;
+  const bool active = e < width;
+  const int kvh = active ? e / hd : 0, d = active ? e % hd : 0;
+  const size_t column = (size_t)(nh + nkv) * hd + (active ? e : 0), row = (size_t)heads * hd;
+  // eight tokens from `first` on, those of `which`; each as two bf16 values
+  auto load = [&](uint32_t (&v)[8], int first, uint32_t which) {
+    if constexpr (PARTS) {
+      float2 sum[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum[i] = make_float2(0.f, 0.f);
+      for (int p = 0; p < n_parts; ++p) {
+        float2 part[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          part[i] = (which >> i & 1) ? *(const float2*)((const float*)qkv_in + (size_t)p * part_stride + (first + i) * row + column) : make_float2(0.f, 0.f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[i].x += part[i].x, sum[i].y += part[i].y;
       }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const bf16 two[2] = {(bf16)sum[i].x, (bf16)sum[i].y};
+        __builtin_memcpy(&v[i], two, 4);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = (which >> i & 1) ? *(const uint32_t*)((const bf16*)qkv_in + (first + i) * row + column) : 0;
+    }
+  };
+  if (run >= 0) {
+    uint32_t v[8];
+    load(v, t0 - 7 + run, 0xff);
+    const int at_page = __shfl(page, run, SYN_WAVE), slot = __shfl(pos, run, SYN_WAVE) % SYN_PAGE;
+    if (active) {
+      bf16* dst = v_pages + ((size_t)at_page * nkv + kvh) * SYN_PAGE * hd + v_page_offset(hd, d, slot);
+      uint4 low, high;      // dims d and d + 1, which follow each other at 16 bytes
+      low.x = (v[0] & 0xffff) | v[1] << 16, low.y = (v[2] & 0xffff) | v[3] << 16;
+      low.z = (v[4] & 0xffff) | v[5] << 16, low.w = (v[6] & 0xffff) | v[7] << 16;
+      high.x = v[0] >> 16 | (v[1] & 0xffff0000u), high.y = v[2] >> 16 | (v[3] & 0xffff0000u);
+      high.z = v[4] >> 16 | (v[5] & 0xffff0000u), high.w = v[6] >> 16 | (v[7] & 0xffff0000u);
+      ((uint4*)dst)[0] = low, ((uint4*)dst)[1] = high;
     }
   }
-  if (tid < 64 && t0 + tid < n_tokens) {
-    const int tok = t0 + tid, pos = tok_pos[tok];
-    const int page = page_table[(size_t)tok_seq[tok] * table_stride + pos / SYN_PAGE];
-    dst_base[tid] = ((size_t)page * nkv + kvh) * SYN_PAGE * hd;
-    dst_slot[tid] = pos % SYN_PAGE;
+  if (rest) {
+    uint32_t v[8];
+    load(v, t0, rest);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at_page = __shfl(page, 7 + i, SYN_WAVE), slot = __shfl(pos, 7 + i, SYN_WAVE) % SYN_PAGE;
+      if (!(rest >> i & 1) || !active) continue;
+      bf16 two[2];
+      __builtin_memcpy(two, &v[i], 4);
+      bf16* dst = v_pages + ((size_t)at_page * nkv + kvh) * SYN_PAGE * hd + v_page_offset(hd, d, slot);
+      dst[0] = two[0], dst[8] = two[1];
+    }
   }
-  __syncthreads();
-  const int j = tid % 64;
-  if (t0 + j < n_tokens)
-    for (int d = tid / 64; d < V_DIMS && d0 + d < hd; d += 4)
-      v_pages[dst_base[j] + v_page_offset(hd, d0 + d, dst_slot[j])] = vtile[j * LD + d];
 }
 
-// Both in one launch: the first qk_x * qk_y workgroups take the q and k heads, the others the v tiles
-// (v_x * nkv * v_z of them, none where the layer writes no cache).
+// Both in one launch: the first n_qk workgroups take the q and k heads, the others the v heads, a wave 8 tokens and one of v_chunks
+// (none where the layer writes no cache).
 template <int LPH, bool PARTS>
 __global__ void __launch_bounds__(256)
-qkv_prompt_kernel(int qk_x, int qk_y, int v_x, const void* __restrict__ qkv, int n_parts, size_t part_stride,
+qkv_prompt_kernel(int n_qk, int v_chunks, const void* __restrict__ qkv, int n_parts, size_t part_stride,
                   bf16* __restrict__ q_out, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,
                   const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
                   const int* __restrict__ tok_pos, const void* __restrict__ q_gain, const void* __restrict__ k_gain,
                   int gain_is_f32, float gain_offset, float eps, const float* __restrict__ cos_t,
                   const float* __restrict__ sin_t, int n_tokens, int nh, int nkv, int n_active) {
-  const int b = blockIdx.x, n_qk = qk_x * qk_y;
+  const int b = blockIdx.x;
   if (b < n_qk) {
-    qk_heads_part<LPH, PARTS>(b % qk_x, b / qk_x, qkv, n_parts, part_stride, q_out, k_pages, page_table, table_stride,
-                              tok_seq, tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens,
-                              nh, nkv, n_active);
+    qk_heads_part<LPH, PARTS>(b, qkv, n_parts, part_stride, q_out, k_pages, page_table, table_stride, tok_seq, tok_pos, q_gain, k_gain,
+                              gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh, nkv, n_active);
   } else {
-    const int c = b - n_qk;
-    v_block_write_part<PARTS>(c % v_x, (c / v_x) % nkv, c / (v_x * nkv), qkv, n_parts, part_stride, v_pages, page_table,
-                              table_stride, tok_seq, tok_pos, n_tokens, nh, nkv, LPH * 8);
+    const long c = (long)(b - n_qk) * (256 / SYN_WAVE) + threadIdx.x / SYN_WAVE;
+    const int group = (int)(c / v_chunks), chunk = (int)(c % v_chunks);
+    if (group * 8L >= n_tokens) return;
+    v_octets_write_part<PARTS>(group, chunk, qkv, n_parts, part_stride, v_pages, page_table, table_stride, tok_seq, tok_pos,
+                               n_tokens, nh, nkv, LPH * 8);
   }
 }
 
@@ -675,20 +724,20 @@ SYN_EXPORT int syn_qk_norm_rope_kv_write(const void* qkv, int n_parts, void* q_o
   if (fast) {
     const int n_active = write_kv ? nh + nkv : nh;
     const int hpb = 256 / lph;
-    const int qk_x = (n_tokens + 3) / 4, qk_y = (n_active + hpb - 1) / hpb;
-    const int v_x = (n_tokens + 63) / 64, v_blocks = write_kv ? v_x * nkv * ((hd + V_DIMS - 1) / V_DIMS) : 0;
+    const long n_qk = (((long)n_tokens + 3) / 4 * n_active + hpb - 1) / hpb, v_chunks = (nkv * hd + 127) / 128;
+    const long v_blocks = write_kv ? (((long)n_tokens + 7) / 8 * v_chunks + 3) / 4 : 0;
     const size_t part_stride = (size_t)n_tokens * (nh + 2 * nkv) * hd;
-    const long grid = (long)qk_x * qk_y + v_blocks;
+    const long grid = n_qk + v_blocks;
     SYN_CHECK(grid <= 0x7fffffffL, "qk_norm_rope_kv_write: %d tokens are too many for one launch", n_tokens);
 #define SYN_QKV(L)                                                                                                  \
   if (n_parts > 0)                                                                                                  \
     qkv_prompt_kernel<L, true><<<(unsigned)grid, 256, 0, stream>>>(                                                 \
-        qk_x, qk_y, v_x, qkv, n_parts, part_stride, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table,       \
+        (int)n_qk, (int)v_chunks, qkv, n_parts, part_stride, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table,       \
         table_stride, tok_seq, tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh,  \
         nkv, n_active);                                                                                             \
   else                                                                                                              \
     qkv_prompt_kernel<L, false><<<(unsigned)grid, 256, 0, stream>>>(                                                \
-        qk_x, qk_y, v_x, qkv, 0, 0, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table, table_stride, tok_seq, \
+        (int)n_qk, (int)v_chunks, qkv, 0, 0, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table, table_stride, tok_seq, \
         tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh, nkv, n_active)
     switch (lph) {
       case 2: SYN_QKV(2); break;

@@ -1038,6 +1038,37 @@ def test_qk_norm_rope_kv_write(ops, dtype, nh, nkv, hd, rot, norm):
     close(qd, qw, what="q without cache write", **tol)
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 16), (5, 3, 64), (8, 2, 128), (2, 3, 256), (40, 8, 128)])
+@pytest.mark.parametrize("step", ["one", "eight", "ragged", "singles", "gaps", "long"])
+def test_values_of_a_prompt_step_in_pieces_of_eight(ops, step, nh, nkv, hd):
+    """Sequences that begin and end anywhere among the eight tokens of a wave and among the eight positions of a piece, single tokens
+    between them, positions that do not follow each other: the values are copied, in place, and nothing else is written; keys and
+    queries as by the twin."""
+    past, new = {"one": ([13], [1]), "eight": ([56], [8]), "ragged": ([8, 0, 61, 5, 17], [9, 8, 30, 3, 26]), "singles": ([7, 8, 0, 30], [1, 1, 1, 1]),
+                 "gaps": ([0, 3], [40, 30]), "long": ([1, 0], [70, 135])}[step]
+    tok_seq, tok_pos, _, _, _ = step_arrays(past, new)
+    if step == "gaps":      # every third place from the 12th on is left out, and the last tokens run backwards
+        tok_pos = torch.tensor([p if i < 12 else p + i // 3 for i, p in enumerate(tok_pos.tolist())], dtype=I32)
+        tok_pos[-9:] = tok_pos[-9:].flip(0)
+    N, table = len(tok_seq), shuffled_table(5, 3, 3)
+    qkv = rnd((N, (nh + 2 * nkv) * hd), 25, BF16)
+    qg, kg = ((1 + 0.1 * rnd((hd,), 26 + i)).to(BF16) for i in range(2))
+    ang = torch.arange(200, dtype=F32)[:, None] * (10000.0 ** (-torch.arange(hd // 2, dtype=F32) * 2 / hd))[None]
+    cos, sin = torch.cos(ang), torch.sin(ang)
+    k0, v0 = make_cache(15, nkv, hd, BF16, 28)
+    kw, vw, qw = k0.clone(), v0.clone(), torch.empty((N, nh * hd), dtype=BF16)
+    ref.qk_norm_rope_kv_write(qkv, qw, kw, vw, table, tok_seq, tok_pos, qg, kg, 1e-5, cos, sin, nh, nkv, hd)
+    d = lambda t: t.to(DEV)
+    # (as whole rows, and as partial sums of which all but one are zero: 65 tokens and more take the same kernel)
+    for rows in (qkv, torch.stack([torch.zeros_like(qkv.float()), qkv.float()])):
+        kd, vd, qd = d(k0), dv(v0), torch.empty((N, nh * hd), dtype=BF16, device=DEV)
+        ops.qk_norm_rope_kv_write(d(rows), qd, kd, vd, d(table), d(tok_seq), d(tok_pos), d(qg), d(kg), 1e-5, d(cos), d(sin), nh, nkv, hd)
+        assert torch.equal(hv(vd), vw), "v is a copy"
+        close(qd, qw, 3e-2, 1e-2, what="q")
+        close(kd, kw, 3e-2, 1e-2, what="k pages")
+        assert torch.equal(kd.cpu()[kw == k0], k0[kw == k0])
+
+
 def fill_sequences(k, v, table, lens, nkv, hd, dtype, seed):
     """Write O(1) keys and values for positions below each length; the rest stays garbage."""
     for b, T in enumerate(lens):
