@@ -361,9 +361,9 @@ def _rows_choice(M, N, K, slices):
     return best
 
 
-def _tiles_bytes(M, N, K, slices, gated):
-    """The same of the tiles that gemm_direct_kernel takes."""
-    tile = 64 if M <= 32 else 96 if gated and M > 64 else 128
+def _tiles_bytes(M, N, K, slices):
+    """The same of the tiles that are taken otherwise."""
+    tile = 64 if M <= 32 else 128
     return _bytes_a_unit(M, tile, K, slices, -(-N // tile), compute_units(), M <= 32)
 
 
@@ -388,7 +388,7 @@ def rows_tile(M, N, K, slices, gated=False) -> int:
     new = _rows_choice(M, N, K, slices)
     if new is None or slices > 1 and slices != rows_slices(M, N, K):
         return 0
-    return new[1] if slices > 1 or _rows_pay(new[0], _tiles_bytes(M, N, K, 1, gated), M, gated) else 0
+    return new[1] if slices > 1 or _rows_pay(new[0], _tiles_bytes(M, N, K, 1), M, gated) else 0
 
 
 @functools.lru_cache(maxsize=4096)
@@ -398,7 +398,7 @@ def rows_slices(M, N, K) -> int:
     if M > ROWS_MAX or M <= PACKED_MAX_ROWS or K % 128 or N % 16:
         return 0
     new = _rows_choice(M, N, K, None)
-    return new[2] if new is not None and _rows_pay(new[0], _tiles_bytes(M, N, K, gemm_slices(M, N, K, _BF16), False), M, False) else 0
+    return new[2] if new is not None and _rows_pay(new[0], _tiles_bytes(M, N, K, gemm_slices(M, N, K, _BF16)), M, False) else 0
 
 
 PAIR = 16   # rows of the gate and of the up projection alternate in turns of this many
