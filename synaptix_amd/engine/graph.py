@@ -176,10 +176,10 @@ class DecodeRunner:
 
 # ----------------------------------------------------------------------------- short prompts
 # Token counts for which prompt steps are captured.  Beyond them the GPU takes as long as the host: 256 rows replayed 7.1 ms,
-# launched one by one 7.3 ms.  Each costs a capture at its first use (some 70 ms) and scratch memory, so another stands between two
-# only where padding costs more than those: of two prompts at the 8B and 4B shapes 96 tokens take 5.17 and 4.28 ms padded to 128,
-# 4.82 and 4.03 in 96 rows (7 and 6 %); 48 tokens padded to 64 4.12 and 3.27 against 3.96 and 3.24, 112 to 128 5.17 and 4.14
-# against 5.01 and 3.99, 80 to 96 4.82 and 4.07 against 4.69 and 3.89, 24 to 32 3.98 and 3.15 against 3.85 and 2.96 (1 to 6 %).
+# launched one by one 7.3 ms.  Each costs a capture at its first use (some 70 ms, what 200 steps and more save) and scratch memory,
+# so few stand between two.  Of two prompts at the 8B and 4B shapes 96 tokens take 5.06 and 3.79 ms padded to 128, 4.66 and 3.62 in
+# 96 rows (8 and 4 %); without rows of their own 24 tokens padded to 32 take 3.86 and 2.80 against 3.76 and 2.66, 48 to 64 4.25 and
+# 3.41 against 3.93 and 3.10 (8 and 9 %), 80 to 96 4.81 and 3.63 against 4.55 and 3.47, 112 to 128 5.14 and 3.79 against 5.04 and 3.74.
 PROMPT_ROWS = (16, 32, 64, 96, 128)
 PROMPT_SEQS = (1, 2, 4, 8)             # sequences of the step (one more, for the padding tokens, is added)
 
