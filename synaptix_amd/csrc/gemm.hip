@@ -1484,32 +1484,46 @@ struct StreamTile {
   double round, power;
   bool plain;       // also over W in plain rows (the others are compiled for fragment order alone)
 };
-static const StreamTile STREAM_TILES[] = {
-    {256, 256, 86.0, 24.8, true}, {256, 192, 64.6, 26.1, true}, {128, 128, 36.4, 0.0, true}, {192, 256, 69.0, 25.3, false},
-    {128, 256, 53.6, 0.0, false}, {256, 128, 49.8, 19.7, false}, {192, 192, 54.7, 22.7, false}, {128, 192, 46.5, 0.0, false},
-    {64, 128, 20.5, 13.0, true}, {64, 192, 31.6, 13.7, false}};
 constexpr int STREAMED_TILES = 10;
+struct StreamFit {
+  StreamTile tiles[STREAMED_TILES];
+  // share of a round that an empty tile takes, us of any product, us a byte: of W, of the output, of W beyond 100 MB that several rows of
+  // tiles read, of partial sums beyond the first that their reader adds
+  double empty, fixed, weight, store, pushed, reader;
+};
+static const StreamFit STREAMED = {
+    {{256, 256, 86.0, 24.8, true}, {256, 192, 64.6, 26.1, true}, {128, 128, 36.4, 0.0, true}, {192, 256, 69.0, 25.3, false},
+     {128, 256, 53.6, 0.0, false}, {256, 128, 49.8, 19.7, false}, {192, 192, 54.7, 22.7, false}, {128, 192, 46.5, 0.0, false},
+     {64, 128, 20.5, 13.0, true}, {64, 192, 31.6, 13.7, false}},
+    0.453, 0.7, 0.124e-6, 0.208e-6, 0.06e-6, 0.14e-6};
+// An earlier fit, of the kernel when it read x in pieces of 64 bytes.  It picks nothing any more, but products that it cut hand on their
+// sums in 32 bits, and do so still (syn_gemm_sums_line).
+static const StreamFit SUMS_LINE = {
+    {{256, 256, 82.9, 33.2, true}, {256, 192, 74.7, 20.6, true}, {128, 128, 38.0, 14.4, true}, {192, 256, 67.0, 24.9, false},
+     {128, 256, 56.0, 25.9, false}, {256, 128, 66.6, 22.0, false}, {192, 192, 59.0, 26.9, false}, {128, 192, 45.3, 16.3, false},
+     {64, 128, 23.5, 12.2, true}, {64, 192, 38.1, 5.3, false}},
+    0.255, 4.5, 0.146e-6, 0.229e-6, 0.0, 0.12e-6};
 static int stream_slice(int K, int slices) { return ((K + slices - 1) / slices + 127) / 128 * 128; }
 static int stream_last_slice(int K, int slices) { return K - (slices - 1) * stream_slice(K, slices); }
 struct StreamPlan {
   int tile;        // -1: none takes this K (k-steps come in pairs, and a slice holds a ring of them at least)
   double us;
 };
-static StreamPlan plan_stream(int M, int N, int K, int slices, bool packed, int out_bytes) {
+static StreamPlan plan_stream(const StreamFit& fit, int M, int N, int K, int slices, bool packed, int out_bytes) {
   StreamPlan best = {-1, 1e30};
   if (K % 64) return best;
   const long cus = syn_compute_units();
   const double k = stream_slice(K, slices) / 4096.0;
   for (int i = 0; i < STREAMED_TILES; ++i) {
-    const StreamTile& s = STREAM_TILES[i];
+    const StreamTile& s = fit.tiles[i];
     if ((!packed && !s.plain) || stream_last_slice(K, slices) < 32 * stream_stages(s.bm, s.bn)) continue;
     const long down = (M + s.bm - 1) / s.bm, across = (N + s.bn - 1) / s.bn, tiles = down * across * slices;
     const double filled = (double)M / (double)(down * s.bm) * (double)N / (double)(across * s.bn);
-    const double work = (double)((tiles + cus - 1) / cus) * s.round * k * (0.453 + 0.547 * filled) + 0.7;
+    const double work = (double)((tiles + cus - 1) / cus) * s.round * k * (fit.empty + (1.0 - fit.empty) * filled) + fit.fixed;
     const double power = (double)tiles / cus * s.power * k * filled;
-    const double ask = tiles < cus ? cbrt((double)cus / (double)tiles) : 1.0, way = 0.124e-6 * 2.0 * N * K * ask * ask;
-    const double pushed = M > s.bm ? 0.06e-6 * fmax(0.0, 2.0 * N * K - 1e8) : 0.0;
-    const double us = sqrt(work * work + way * way + power * power) + 0.208e-6 * M * N * slices * out_bytes + pushed;
+    const double ask = tiles < cus ? cbrt((double)cus / (double)tiles) : 1.0, way = fit.weight * 2.0 * N * K * ask * ask;
+    const double pushed = M > s.bm ? fit.pushed * fmax(0.0, 2.0 * N * K - 1e8) : 0.0;
+    const double us = sqrt(work * work + way * way + power * power) + fit.store * M * N * slices * out_bytes + pushed;
     if (us < best.us) best = {i, us};
   }
   return best;
@@ -1590,7 +1604,7 @@ static int pick_register_tile(int M, int N) {
 // of 8, one slice) or, in slices, through the smallest of those that load straight into LDS.
 template <bool PAIRED>
 static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1, int tile = -1) {
-  if (tile < 0) tile = plan_stream(M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
+  if (tile < 0) tile = plan_stream(STREAMED, M, N, K, slices, w.packed, PAIRED ? 1 : ep.out_is_f32 ? 4 : 2).tile;
   if (tile >= 0) {
     if (PAIRED) return launch_stream_as<SYN_OUT_GATED>(tile, x, w, out, ep, M, N, K, stream, slices);
     if (ep.out_is_f32) return launch_stream_as<SYN_OUT_F32>(tile, x, w, out, ep, M, N, K, stream, slices);
@@ -1615,18 +1629,23 @@ static bool direct_one_round(int M, int N, int K) {
 
 // Into how many slices of K a product of more than 56 rows is cut when its reader adds partial sums: the smallest estimate of
 // the product's time and of what its reader pays for the slices beyond the first (M x N floats each, half of them from caches).
-SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
+static int plan_slices(const StreamFit& fit, int M, int N, int K) {
   int best = 1;
   double least = 1e30;
   if (M <= 0 || N <= 0 || K <= 0) return 1;
   for (int s : {1, 2, 3, 4, 6, 8}) {
-    const StreamPlan p = plan_stream(M, N, K, s, true, 4);
+    const StreamPlan p = plan_stream(fit, M, N, K, s, true, 4);
     if (p.tile < 0) break;
-    const double us = p.us + (s - 1) * 0.14e-6 * 4.0 * M * N;
+    const double us = p.us + (s - 1) * fit.reader * 4.0 * M * N;
     if (us < least) least = us, best = s;
   }
   return best;
 }
+SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) { return plan_slices(STREAMED, M, N, K); }
+
+// Whether a product that could be rounded to 16 bits hands on its 32-bit sums whatever number of slices is the fastest now: a line that a
+// fit of the tiles' times must not move, since it decides how precise a result is.  (Products that are cut hand them on in any case.)
+SYN_EXPORT int syn_gemm_sums_line(int M, int N, int K) { return plan_slices(SUMS_LINE, M, N, K) > 1; }
 
 // ------------------------------------------------------------------ entry point
 // dtype: 0 = float in, float out; 1 = bf16 in, bf16 out; 2 = bf16 in, float out.
@@ -1635,7 +1654,7 @@ SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) {
 // w_packed: w is the weight in fragment order (pack_weight; bf16, N a multiple of 16, K of 128): for the tiles that
 // load straight into LDS; the other kernels read plain rows only.
 // point: what the finished sums pass before they are stored (point_activation; one slice).
-// tile: -1, or for tests and measurements one of STREAM_TILES, whatever the rules below would take (bf16 operands).
+// tile: -1, or for tests and measurements one of STREAMED.tiles, whatever the rules below would take (bf16 operands).
 SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int M, int N, int K, int force_simt,
                         int slices, int w_packed, int point, int tile, int rows, hipStream_t stream) {
   SYN_CHECK(tile < 0 || (dtype != 0 && !force_simt && K % 64 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0),

@@ -331,6 +331,7 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
 # (gemm_rows_kernel in csrc/gemm.hip); more go faster through the streamed tiles (72 rows: 4,096 x 2,048 15.5 us, 13.0; 8,192 x 2,048 16.2,
 # 13.8; 128 rows 21.8, 13.2; gated 8,192 x 1,024 with 48 rows 9.1, 9.1, with 64 10.4, 9.2; 24,576 x 4,096 with 48 42.4, 43.3, with 56 61.8, 43.7).
 ROWS_MAX, ROWS_MAX_GATED = 64, 48
+ROWS_MIN_WEIGHT = 1 << 19
 
 
 def _bytes_a_unit(M, tile, K, slices, tiles, units, shared):
@@ -348,7 +349,7 @@ def _rows_choice(M, N, K, slices):
     # Less than 1 MB of W keeps the other tiles, and with them the order of its sums: small models with routers decide near ties by it, for
     # a gain of a few microseconds (us here and there: 17 rows, 512 x 512 gated 4.5 and 6.2, 1,024 x 256 plain with its norm 6.8 and 7.3;
     # 128 rows, 512 x 512 gated 9.1 and 13.4, plain 10.9 and 10.2).
-    if N * K < 1 << 19:
+    if N * K < ROWS_MIN_WEIGHT:
         return None
     for nf in (2, 4, 6):
         if M > {2: 128, 4: 96, 6: 48}[nf]:
@@ -601,14 +602,24 @@ def gemm_slices(M, N, K, dtype):
     return slices
 
 
+@functools.lru_cache(maxsize=4096)
+def _sums_line(M, N, K) -> bool:
+    return bool(load_library("core").syn_gemm_sums_line(M, N, K))
+
+
 def gemm_keeps_sums(M, N, K, dtype) -> bool:
     """Whether a bf16 product whose reader takes 32-bit sums (q, k and v in front of their norm and rotation) hands them on,
-    in as many slices as gemm_slices finds fastest, rather than round them to 16 bits.  Decided by the sizes alone, not by the
-    number of slices: the sums stay wherever 256 x 256 tiles fill at most half of the compute units.  Wider or longer products
+    in as many slices as gemm_slices finds fastest, rather than round them to 16 bits.  They stay wherever 256 x 256 tiles fill at
+    most half of the compute units, up to 128 rows whatever K is, and on a line of sizes beyond that which does not move with the
+    number of slices (csrc/gemm.hip: syn_gemm_sums_line); products that are cut hand them on in any case.  Wider or longer products
     would pay for the doubled bytes (2,048 rows, N = 6144: 25 MB more written and read a layer)."""
-    if dtype != _BF16 or K % 8 != 0 or N > 16384 or K < 2048:
+    if dtype != _BF16 or K % 8 != 0 or N > 16384:
         return False
-    if M > 64 and K % 128 == 0 and 2 * -(-M // 256) * -(-N // 256) <= compute_units():
+    if 64 < M <= 128 and K % 128 == 0 and N * K >= ROWS_MIN_WEIGHT:
+        return True
+    if K < 2048:
+        return False
+    if M > 64 and K % 128 == 0 and (2 * -(-M // 256) * -(-N // 256) <= compute_units() or _sums_line(M, N, K)):
         return True
     return gemm_slices(M, N, K, dtype) > 1
 

@@ -116,6 +116,26 @@ def test_sums_of_short_prompts_stay_in_32_bits_whatever_the_number_of_slices():
             assert ops.gemm_keeps_sums(M, N, K, torch.bfloat16) >= (ops.gemm_slices(M, N, K, torch.bfloat16) > 1)
 
 
+def test_sums_that_were_handed_on_in_32_bits_stay_so_whatever_the_fit_of_the_tiles_says():
+    """Rows of wider and longer products whose q, k and v have reached their norm as 32-bit sums, and 65 to 128 rows of short ones: what
+    picks tiles and slices may change, none of these may come to be rounded."""
+    import torch
+    from synaptix_amd.kernels import ops
+    kept = {(10240, 5120): [(1537, 1792)], (12288, 5120): [(1281, 1536)], (7168, 5120): [(2305, 2560)], (16384, 4096): [(1025, 1152)],
+            (10240, 8192): [(1537, 1920), (2049, 2112), (3649, 4096), (4865, 5376)],
+            (8192, 8192): [(1025, 1152), (2049, 2304), (2817, 2880), (4609, 5120), (6145, 6656)], (8192, 4096): [(2113, 2304)],
+            (5120, 5120): [(3073, 3648), (4801, 4864)], (4096, 4096): [(4417, 4608)], (16384, 8192): [(1281, 1344), (2305, 2560), (3073, 3264)],
+            (3072, 1024): [(65, 128)], (6144, 1536): [(65, 128)], (512, 1024): [(65, 128)]}
+    for (N, K), ranges in kept.items():
+        for lo, hi in ranges:
+            for M in (*range(lo, hi, 7), hi):
+                assert ops.gemm_keeps_sums(M, N, K, torch.bfloat16), (M, N, K)
+    # rounded as before: prompts of the 8B and 4B shapes beyond half of the compute units, short products of more rows, small ones
+    for M, N, K in ((1281, 6144, 4096), (2048, 6144, 4096), (2600, 6144, 4096), (1281, 6144, 2560), (4096, 6144, 2560), (129, 3072, 1024),
+                    (2048, 3072, 1024), (100, 256, 1024), (2048, 10240, 5120)):
+        assert not ops.gemm_keeps_sums(M, N, K, torch.bfloat16), (M, N, K)
+
+
 def test_host_side_rules_of_the_kernels_stay_within_their_kernels_limits():
     """The numbers of splits and slices that the host picks: pure functions, checked over a grid of sizes."""
     import torch
