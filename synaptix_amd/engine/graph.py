@@ -79,6 +79,12 @@ def _state_rewind(engine, slots):
     return lambda: engine.cache.put_states(saved)
 
 
+def bin_places(rows: int, needs, item_splits, dtype) -> list:
+    """ops.decode_bins of each group of layers: 0 where its sequences are split, and where none of its layers would read the list."""
+    return [ops.decode_bins(rows, n.kv_heads, n.listed_heads) if dtype == torch.bfloat16 and s == 0 else 0
+            for n, s in zip(needs, item_splits)]
+
+
 class DecodeRunner:
     def __init__(self, engine, rows: int, widths: list):
         self.engine, self.rows, self.widths = engine, rows, list(widths)
@@ -90,9 +96,8 @@ class DecodeRunner:
         self.item_splits = [ops.decode_splits(rows, g.need.kv_heads, w) if engine.dtype == torch.bfloat16 else 0
                             for g, w in zip(groups, self.widths)]
         self.item_splits = [s if s > 1 else 0 for s in self.item_splits]
-        # where the rows alone are more workgroups than compute units: lists that give each of these the same share
-        self.item_bins = [ops.decode_bins(rows, g.need.kv_heads) if engine.dtype == torch.bfloat16 and s == 0 else 0
-                          for g, s in zip(groups, self.item_splits)]
+        # where the rows alone are more workgroups than compute units: lists that share the keys out to these
+        self.item_bins = bin_places(rows, [g.need for g in groups], self.item_splits, engine.dtype)
         n_items = [4 * rows * s + 2 * rows if s else 0 for s in self.item_splits]       # ints of each list
         n_bins = [(4 * ops.DECODE_BIN_SPLITS + 2) * rows if b else 0 for b in self.item_bins]
         self.total = n_int + 2 * rows + sum(n_items) + sum(n_bins)     # + temperatures and uniforms as float bits + work lists

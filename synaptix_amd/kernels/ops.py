@@ -881,14 +881,15 @@ def decode_splits(n_seqs, n_kv_heads, max_pages):
 DECODE_BIN_SPLITS = 2    # room in a list of bins: twice as many items as rows (it cuts what is longer than an even share only)
 
 
-def decode_bins(n_seqs, n_kv_heads) -> int:
+def decode_bins(n_seqs, n_kv_heads, heads_a_group=1) -> int:
     """Over how many places decode attention's work list spreads its items so that every compute unit gets the same share
     (runtime.decode_bins), or 0 where it is not laid out so: with no more workgroups than compute units, where decode_splits
-    cuts every sequence, and where the kv heads do not divide the compute units.  Also with as many rows as places each
-    workgroup has eight waves and a compute unit to itself: 32 rows over 32 places gained 5 to 30 % on unequal lengths and lost 4 to
+    cuts every sequence, where the kv heads do not divide the compute units, where no kernel reads the list (heads_a_group 0) and
+    where it takes a kv head's queries in several workgroups (more than 16 of them), which the places do not count.  Also with as
+    many rows as places each workgroup has eight waves and a compute unit to itself: 32 rows over 32 places gained 5 to 30 % on unequal lengths and lost 4 to
     20 % on equal ones in workgroups of four."""
     cus = compute_units()
-    return cus // n_kv_heads if n_seqs * n_kv_heads > cus and cus % n_kv_heads == 0 else 0
+    return cus // n_kv_heads if 0 < heads_a_group <= 16 and n_seqs * n_kv_heads > cus and cus % n_kv_heads == 0 else 0
 
 
 def _decode_work(name, counters, items, B, n_splits, n_heads, n_kv_heads):

@@ -7,7 +7,7 @@ the layer: crates/synaptix-models/llm/common/src/model.rs:780).
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Optional
 
 import torch
@@ -45,6 +45,8 @@ class KvNeed:
     v_dim: Optional[int] = None       # size of a value where it differs from the keys' (None: head_dim)
     keep_first: int = 0               # with a window: the first keys of a sequence that stay visible for good
     v_heads: Optional[int] = None     # value heads where several kv heads read the values of one (None: kv_heads)
+    # query heads a kv head, where the decode kernel that reads a step's work lists takes them (0: no such kernel reads this cache)
+    listed_heads: int = field(default=0, compare=False)
 
 
 def flat_needs(need) -> tuple:

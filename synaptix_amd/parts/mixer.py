@@ -93,7 +93,7 @@ class GqaAttention(Mixer):
             self.k_gain = get(p + "k_norm.weight").to(self.q_gain.dtype)
 
     def cache_need(self):
-        return KvNeed(self.nkv, self.hd, self.window)
+        return KvNeed(self.nkv, self.hd, self.window, listed_heads=self.nh // self.nkv)
 
     def check(self, dtype):
         if self.hd % 2 or self.hd > ops.MAX_HEAD_DIM:

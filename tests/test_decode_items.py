@@ -148,3 +148,19 @@ def test_bins_refuse_what_does_not_fit():
     for args in (([], 2, 8), ([5, 6], 2, 0), ([5] * 5, 1, 8)):
         with pytest.raises(rt.CacheError):
             rt.decode_bins(*args)
+
+
+def test_bins_are_laid_out_for_layers_that_read_them():
+    """Only the attention over one set of pages of plain heads reads a list; latent and window layers do not, nor a kernel that takes a
+    kv head's queries in several workgroups, which the places do not count."""
+    import torch
+    from synaptix_amd.engine.graph import bin_places
+    from synaptix_amd.parts import GqaAttention, KvNeed, NoPosition
+    plain = lambda heads, kv, window=None: GqaAttention("a.", 64, heads, kv, 64, position=NoPosition(), window=window).cache_need()
+    assert plain(32, 8) == KvNeed(8, 64) and hash(plain(32, 8)) == hash(plain(8, 8))      # layers of other heads share its pages
+    needs = [plain(32, 8), plain(32, 8, 100), plain(128, 8), plain(256, 8), KvNeed(8, 64, 100, v_dim=64), KvNeed(1, 576, None, v_dim=512)]
+    assert bin_places(33, needs, [0] * 6, torch.bfloat16) == [32, 32, 32, 0, 0, 0]
+    assert bin_places(300, needs, [0] * 6, torch.bfloat16) == [32, 32, 32, 0, 0, 0]
+    assert bin_places(32, needs, [0] * 6, torch.bfloat16) == [0] * 6                      # a workgroup a compute unit
+    assert bin_places(33, needs, [2] + [0] * 5, torch.bfloat16)[0] == 0                   # every sequence is split
+    assert bin_places(33, needs, [0] * 6, torch.float32) == [0] * 6
