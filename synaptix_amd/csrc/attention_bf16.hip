@@ -1189,13 +1189,19 @@ static hipError_t raise_decode_lds() {
   });
 }
 
+// Whether the splits of a launch with counters are merged inside it: where the grid is at most two workgroups a compute unit; where it
+// is larger a second kernel merges (a workgroup that waits for its stores and counts itself in holds its place that much longer, which a
+// grid of several rounds pays in every round: 8 sequences of 32,000 tokens 9.3 ms a step against 9.1).  Inside it stays with a work list
+// of more sequences than fill the chip, which cuts only the longest of them (40 of 64 to 4,096 tokens: 65 us, 68 with the second
+// kernel).  The lists are told apart by sequences x kv heads, as they are laid out: with more of these than compute units none splits
+// every sequence.
+static bool decode_merges_inside(int n_seqs, int nkv, int chunks, int n_splits, bool items) {
+  const long rows = (long)n_seqs * nkv, cus = syn_compute_units();
+  return rows * chunks * n_splits <= 2 * cus || (items && rows > cus);
+}
+
 // workspace: n_seqs * nh * n_splits * (HD + 2) floats (unused with one split).
-// counters (may be null): n_seqs * kv heads * ceil(group / 16) ints, zero.  With them the splits are merged inside the
-// one launch where the grid is at most two workgroups a compute unit; where it is larger, and without them, a second
-// kernel merges (a workgroup that waits for its stores and counts itself in holds its place that much longer, which a
-// grid of several rounds pays in every round: 8 sequences of 32,000 tokens 9.3 ms a step against 9.1).  Inside it stays with a
-// work list of more sequences than fill the chip, which cuts only the longest of them (40 of 64 to 4,096 tokens: 65 us, 68 with the
-// second kernel).
+// counters (may be null, then a second kernel merges the splits): n_seqs * kv heads * ceil(group / 16) ints, zero.
 // items (may be null: every sequence in n_splits splits): n_items x {sequence, split | splits of the sequence << 16,
 // first, length}, `first` + split < n_seqs * n_splits being the place of the split's partial results and length
 // what seq_len holds for the sequence; behind them n_seqs x {first, splits}, the same by sequence.
@@ -1229,8 +1235,7 @@ static int launch_decode(const void* q, const QkvIntake* in, void* k_pages, void
   const hipError_t raised = raise_decode_lds();
   SYN_CHECK(raised == hipSuccess, "attention_decode: %zu bytes of LDS refused: %s", LDS_MAX, hipGetErrorString(raised));
   const dim3 grid = items ? dim3(nkv * chunks, n_items, 1) : dim3(n_seqs, nkv * chunks, n_splits);
-  const long groups = (long)n_seqs * nkv * chunks, cus = syn_compute_units();
-  const bool merge_inside = counters != nullptr && (groups * n_splits <= 2 * cus || (items != nullptr && groups > cus));
+  const bool merge_inside = counters != nullptr && decode_merges_inside(n_seqs, nkv, chunks, n_splits, items != nullptr);
   const DecodeWork work{workspace, merge_inside ? counters : nullptr, (const int4*)items};
   if (in)
     attn_decode_split_kernel<true><<<grid, waves * SYN_WAVE, lds, stream>>>(
@@ -1247,6 +1252,12 @@ static int launch_decode(const void* q, const QkvIntake* in, void* k_pages, void
     SYN_LAUNCH_CHECK("attention_decode_merge");
   }
   return 0;
+}
+
+// Which of the two a launch takes (1: inside it), for tests of the rule
+SYN_EXPORT int syn_attention_decode_merges_inside(int n_seqs, int nkv, int nh, int n_splits, int items) {
+  if (n_seqs <= 0 || nkv <= 0 || nh < nkv || n_splits <= 0) return 0;
+  return decode_merges_inside(n_seqs, nkv, (nh / nkv + 15) / 16, n_splits, items != 0);
 }
 
 SYN_EXPORT int syn_attention_decode_bf16(const void* q, const void* k_pages, const void* v_pages,

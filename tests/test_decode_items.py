@@ -164,3 +164,19 @@ def test_bins_are_laid_out_for_layers_that_read_them():
     assert bin_places(32, needs, [0] * 6, torch.bfloat16) == [0] * 6                      # a workgroup a compute unit
     assert bin_places(33, needs, [2] + [0] * 5, torch.bfloat16)[0] == 0                   # every sequence is split
     assert bin_places(33, needs, [0] * 6, torch.float32) == [0] * 6
+
+
+def test_only_lists_of_bins_are_merged_inside_large_launches():
+    """A list that splits every sequence goes by the size of the grid, as a launch without a list does, also where more than 16 heads a
+    kv head make it larger than sequences x kv heads."""
+    from synaptix_amd.kernels import ops
+    from synaptix_amd.kernels.build import load_library
+    inside = load_library("attn_hd128").syn_attention_decode_merges_inside
+    for rows, kv, heads in ((200, 1, 32), (100, 2, 64), (8, 8, 32), (32, 8, 32), (8, 8, 256), (30, 4, 128)):
+        splits = ops.decode_splits(rows, kv, 512)
+        assert splits > 1 or rows * kv >= 256
+        chunks = -(-heads // kv // 16)
+        assert bool(inside(rows, kv, heads, splits, 1)) == (rows * kv * chunks * splits <= 512) == bool(inside(rows, kv, heads, splits, 0))
+    for rows, kv, heads in ((33, 8, 32), (64, 8, 32), (257, 1, 16)):
+        assert ops.decode_splits(rows, kv, 512) == 1 and ops.decode_bins(rows, kv, heads // kv)
+        assert inside(rows, kv, heads, ops.DECODE_BIN_SPLITS, 1)
