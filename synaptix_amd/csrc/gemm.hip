@@ -23,6 +23,7 @@
 // Reference counterparts: crates/synaptix-kernels-cuda/src/best_cu/gemm/gemm_bf16.cu (TN family,
 // mma.sync m16n8k16), best_cu/gemv/mma_gemv.cu:19-133 (M == 1), best_cu/gemm/gemm_f32.cu (SIMT).
 // The tilings here are made for 64-lane waves and MFMA operand layouts, not translated.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -1627,8 +1628,40 @@ static bool direct_one_round(int M, int N, int K) {
   return M <= 256 && (M - 1) % 64 >= 31 && K >= 4096 && (long)N * K >= 24L << 20 && tile_grid(M, N, 64, 128) <= syn_compute_units();
 }
 
-// Into how many slices of K a product of more than 56 rows is cut when its reader adds partial sums: the smallest estimate of
-// the product's time and of what its reader pays for the slices beyond the first (M x N floats each, half of them from caches).
+// The slices of K in which the tiles of 64 or 128 rows by 128 of W that load straight into LDS (gemm_direct) fill the compute units.
+static long direct_groups(int M, int N) { return (long)((M + 127) / 128) * ((N + 127) / 128); }
+static int direct_slices(int M, int N, int K) {
+  const long most = std::min<long>({8, syn_compute_units() / direct_groups(M, N), K / 512});
+  int slices = 1;
+  while (slices * 2 <= most) slices *= 2;
+  return slices;
+}
+
+// Whether a cut product of 57 to 64 rows goes through the streamed tiles, in the slices of their estimate: a large W whose tiles of
+// gemm_direct leave three eighths of the compute units without work, which slices in other numbers than powers of two reach.  Kernel times
+// in a prompt step of 64 rows, us, these tiles and streamed: 5,120 x 25,600 cut in 4 and 6 56.1, 46.5, 10,240 x 5,120 in 2 and 3 26.1, 24.0,
+// 5,120 x 8,192 in 4 and 6 21.4, 19.5; smaller ones and those that fill them: 6,144 x 4,096 13.6, 14.7, 4,096 x 12,288 21.1, 21.7, 2,560 x
+// 9,728 15.9, 17.4, 8,192 x 28,672 in 4 and 8 6 less.  Steps with every product streamed, and so: 8B shape 4.07, 3.95 ms, 4B 3.21, 3.11.
+static bool few_rows_streamed(int N, int K) {
+  return (long)N * K >= 24L << 20 && 8 * direct_groups(64, N) * direct_slices(64, N, K) <= 5L * syn_compute_units();
+}
+
+// Whether a cut product of 65 to 128 or 177 to 256 rows goes through the tiles of 128 x 128 that hold k-tiles of 64 (gemm_direct): where
+// their workgroups, one or two rows of tiles in slices that are a power of two, fill three quarters of the compute units and more, and W
+// has 48 to 96 MB.  Less of it the streamed tiles bring in with fewer partial sums, more of it in longer runs.  What a layer of a prompt
+// step gains over the streamed tiles, us: 6,144 x 4,096 with 4,096 x 12,288 behind it 0.3 with 96 rows, 0.8 with 128 and 192, 4.2 with 256;
+// with 96 and 128 rows 6,144 x 4,096 alone 4.0, 3.8, 6,144 x 6,144 3.0, 2.7, 7,168 x 5,120 2.7, 0.8, 3,072 x 8,192 1.6, 0.6 (with 192 and 256
+// rows from 2.0 less to 2.7 more).  Beyond: 8,192 x 8,192 0.8, 1.2, 4,096 x 14,336 -2.7, -2.8, 6,144 x 16,384 -7.3, -7.5, 8,192 x 28,672 -1.8,
+// -3.5.  Below, or with fewer workgroups: 4,096 x 4,096 -1.5, -2.8, 6,144 x 2,560 -0.5, -2.3, 2,560 x 9,728 (160 of them) -1.4, -2.5.
+static bool direct_cut(int M, int N, int K) {
+  const long w = (long)N * K, groups = direct_groups(M, N), cus = syn_compute_units();
+  if (!(M > 64 && M <= 128) && !(M > 176 && M <= 256)) return false;
+  return K % 128 == 0 && w >= 24L << 20 && w <= 48L << 20 && groups <= cus && 4 * groups * direct_slices(M, N, K) >= 3 * cus;
+}
+
+// Into how many slices of K a product of more than 56 rows is cut when its reader adds partial sums: those of the tiles above or, for
+// the streamed ones, the smallest estimate of the product's time and of what its reader pays for the slices beyond the first (M x N
+// floats each, half of them from caches).
 static int plan_slices(const StreamFit& fit, int M, int N, int K) {
   int best = 1;
   double least = 1e30;
@@ -1641,7 +1674,11 @@ static int plan_slices(const StreamFit& fit, int M, int N, int K) {
   }
   return best;
 }
-SYN_EXPORT int syn_gemm_stream_slices(int M, int N, int K) { return plan_slices(STREAMED, M, N, K); }
+SYN_EXPORT int syn_gemm_cut_slices(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 1;
+  if (M <= 64 ? !few_rows_streamed(N, K) : direct_cut(M, N, K)) return direct_slices(M, N, K);
+  return plan_slices(STREAMED, M, N, K);
+}
 
 // Whether a product that could be rounded to 16 bits hands on its 32-bit sums whatever number of slices is the fastest now: a line that a
 // fit of the tiles' times must not move, since it decides how precise a result is.  (Products that are cut hand them on in any case.)
@@ -1745,13 +1782,12 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     else if (N >= 65536 && !w_packed) rc = launch_tiled<32, 32, 256, 1, 1>(xb, wb, out, ep, M, N, K, stream, slices);
     else if (K % 128 == 0) rc = launch_direct<32, 64, 128, 1, 2>(xb, wt, out, ep, M, N, K, stream, slices);
     else rc = launch_tiled<32, 64, 128, 1, 2>(xb, wb, out, ep, M, N, K, stream, slices);
-  } else if (M <= 64 && K % 128 == 0 && !(M > 56 && slices > 1)) {
+  } else if (M <= 64 && K % 128 == 0 && !(M > 56 && slices > 1 && few_rows_streamed(N, K))) {
     // 33 to 64 rows: 128 rows of W a workgroup, so that the rows of x are fetched half as often (every
-    // workgroup reads all of x), three k-tiles in a ring, one workgroup a compute unit.  57 rows and more in slices go to the
-    // streamed tiles, in the slices of their estimate (these tiles in the slices that fill the compute units, and streamed, the
-    // norm behind it included, us with 64 rows: 4,096 x 4,096 18.2, 16.1; 4,096 x 12,288 28.6, 29.0; 6,144 x 4,096 20.6, 20.8; 2,560 x 4,096
-    // 15.3, 13.9; 5,120 x 25,600 63.9, 58.6; with 48: 17.0, 15.5; 26.7, 28.4; 19.3, 19.7; 14.0, 13.4; 60.8, 57.7).
+    // workgroup reads all of x), three k-tiles in a ring, one workgroup a compute unit
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
+  } else if (slices > 1 && direct_cut(M, N, K) && slices == direct_slices(M, N, K)) {
+    rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
   } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N, K)) {
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream);
   } else if (M <= 64 && K % 128 != 0) {

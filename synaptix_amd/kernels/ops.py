@@ -571,8 +571,8 @@ def packed_slices(N, K):
 
 
 @functools.lru_cache(maxsize=4096)
-def _stream_slices(M, N, K):
-    return int(load_library("core").syn_gemm_stream_slices(M, N, K))
+def _cut_slices(M, N, K):
+    return int(load_library("core").syn_gemm_cut_slices(M, N, K))
 
 
 def gemm_slices(M, N, K, dtype):
@@ -586,8 +586,8 @@ def gemm_slices(M, N, K, dtype):
         return 1
     units = compute_units()
     if M > 56 and K % 128 == 0:
-        # what the streamed tiles take on so many rows, and what the reader of partial sums pays for the slices (csrc/gemm.hip)
-        return _stream_slices(M, N, K)
+        # with the tiles that take so many rows of this product (csrc/gemm.hip)
+        return _cut_slices(M, N, K)
     if M > 64:
         return 1
     if M <= 32:

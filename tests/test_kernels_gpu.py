@@ -750,6 +750,21 @@ def test_products_where_the_streamed_tiles_begin(ops, K, packed, kind):
         assert torch.isfinite(out).all() and float(off.max()) <= 0, (M, S, float(off.max()))
 
 
+@pytest.mark.parametrize("N,K", [(3072, 8192), (5120, 8192), (4096, 4096)])
+@pytest.mark.parametrize("M", [57, 64, 65, 97, 128, 129, 177, 256])
+def test_products_in_the_slices_of_their_tiles(ops, M, N, K):
+    """57 to 256 rows in the slices that the rules pick, through the tiles that load straight into LDS and through the streamed ones."""
+    x, w = rnd((M, K), 96, BF16).to(DEV), rnd((N, K), 97, BF16).to(DEV)
+    S = ops.gemm_slices(M, N, K, BF16)
+    assert S > 1
+    want = x.double() @ w.double().T
+    for weight in (w, ops.pack_weight(w)):
+        out = torch.full((S, M, N), float("nan"), dtype=F32, device=DEV)
+        ops.gemm(x, weight, out)
+        off = (out.double().sum(0) - want).abs() - 1e-4 * math.sqrt(K)
+        assert torch.isfinite(out).all() and float(off.max()) <= 0, float(off.max())
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
 @pytest.mark.parametrize("M,I,K", [(300, 1200, 256), (2100, 4112, 512)])
 def test_gated_activations_of_many_rows(ops, act, M, I, K):

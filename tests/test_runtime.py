@@ -158,6 +158,21 @@ def test_host_side_rules_of_the_kernels_stay_within_their_kernels_limits():
             assert ops.gemm_slices(M, N, K, torch.float32) == 1
 
 
+def test_cut_products_take_the_tiles_whose_slices_fill_the_compute_units():
+    """57 to 256 rows: slices of the tiles that load straight into LDS where these fill the compute units (a power of two), of the streamed
+    tiles elsewhere."""
+    import torch
+    from synaptix_amd.kernels import ops
+    cut = lambda M, N, K: ops.gemm_slices(M, N, K, torch.bfloat16)
+    for N, K, s in ((6144, 4096, 4), (4096, 4096, 8), (4096, 12288, 8), (6144, 2560, 4), (2560, 4096, 8), (2560, 9728, 8), (4096, 2048, 4), (2048, 2048, 4),
+                    (2048, 8192, 8), (8192, 28672, 4), (3072, 1024 * 3, 4)):
+        assert {cut(M, N, K) for M in (33, 48, 56, 57, 60, 64)} == {s}, (N, K)
+    for N, K, few, s in ((10240, 5120, 2, 3), (5120, 8192, 4, 6), (5120, 25600, 4, 6)):
+        assert cut(56, N, K) == few and {cut(M, N, K) for M in (57, 64)} == {s}, (N, K)
+    for N, K, s in ((6144, 4096, 4), (4096, 12288, 8), (6144, 6144, 4), (7168, 5120, 4), (3072, 8192, 8)):
+        assert {cut(M, N, K) for M in (65, 96, 128)} == {s} and {cut(M, N, K) for M in (177, 224, 256)} == {s // 2}, (N, K)
+
+
 def test_32_bit_prompts_share_workgroups_only_where_that_was_measured_to_pay():
     """Steps timed with a wave a row and with 16 rows a workgroup: the latter walks a workgroup's sequences one after another, which single
     tokens behind long contexts beside a prompt make up to six times slower than the former, and many short prompts half as slow again."""
