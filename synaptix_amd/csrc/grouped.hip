@@ -374,6 +374,9 @@ __global__ void __launch_bounds__(256) grouped_product_tiled_kernel(GroupedArgs 
 //   * a last round of tiles for up to half of the workgroups is cut into halves of tiles for all.
 // W's loads are marked non-temporal: a tile of W meets one or two tiles of rows, and x stays in the L2s for it (four layers scored at 1,500
 // places 3.48 -> 3.30 ms).
+// ACT: the gated activation is compiled in: as a branch inside the one loop over the sums it made the epilogue of 256 x 256 tiles
+// 13,000 instructions instead of 3,600, and the product 1 to 18 % slower (32 experts of 2,048 x 2,048 with 224 unequal rows 111 -> 91 us,
+// 8 of 8,192 x 4,096 with 2,048 987 -> 940).
 // 1,500 tokens with 6 of 48 experts (188 rows each), 2,048 x 4,096 with GELU and back, 32-bit results: 251 + 225 us -> 220 + 217 (x
 // in pieces of 64 bytes, tiles of up to 256 rows and lookups between the stores before); 310 rows each 353 + 383 -> 290 + 316, 120
 // rows 229 + 199 -> 187 + 190, 50 rows 185 + 168 -> 162 + 168, 32 experts with 256 rows 159 -> 162, 16 with 187 127 + 84 -> 101 + 85.
@@ -392,7 +395,8 @@ __device__ __forceinline__ float gelu_quick(float z) {
   return z * (z < 0.f ? q : 1.f - q);
 }
 
-template <int BM, int BN, bool F32, bool PAIR>
+constexpr int NO_PAIR = -1;
+template <int BM, int BN, bool F32, int ACT>
 __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, long a_bytes, long o_bytes) {
   constexpr int BK = 32, STAGES = stream_stages(BM, BN), PAIRS = stream_pairs(BM, BN), WAVES = 4;
   constexpr int XL = BM / 32, WL = BN / 64, PASSES = XL / 2 + WL;      // loads of a wave: of a pair of k-tiles of x, of a k-tile of W, a step
@@ -658,7 +662,7 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
         for (int j = 0; j < FN; ++j) {
           const int n = t.n0 + wn + 16 * j + 4 * q4;
           const bool ok = in && n < g.N && (j < H || wide);
-          if constexpr (PAIR) {
+          if constexpr (ACT != NO_PAIR) {
             const float v0 = of(acc[i][j][0], acc[i][j][1]) * weight, v1 = of(acc[i][j][2], acc[i][j][3]) * weight;
             if constexpr (F32) {
               buffer_store4(vo, v0, ok ? row + (n / 2) * 4 : SYN_NOWHERE);
@@ -683,14 +687,8 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
         }
       }
     };
-    if constexpr (PAIR) {
-      // (one loop with a branch that all lanes share in it: with a loop for each activation the compiler moved sums around in the k-steps)
-      const int act = g.pair - 1;
-      store_all([&](float gt, float up) {
-        if (act == SYN_ACT_SILU) return gated_quick<SYN_ACT_SILU, F32>(gt, up, 0.f);
-        if (act == SYN_ACT_SWIGLU_LIMIT) return gated_quick<SYN_ACT_SWIGLU_LIMIT, F32>(gt, up, g.limit);
-        return gated_quick<SYN_ACT_GELU_TANH, F32>(gt, up, 0.f);
-      });
+    if constexpr (ACT != NO_PAIR) {
+      store_all([&](float gt, float up) { return gated_quick<ACT, F32>(gt, up, g.limit); });
     } else {
       if (g.act == 0) store_all([&](float v, float) { return v; });
       else if (g.act == 2) store_all([&](float v, float) { return point_activation(SYN_POINT_RELU_SQUARED, v); });
@@ -704,22 +702,28 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
   __builtin_amdgcn_s_waitcnt(0x0070);
 }
 
-template <int BM, int BN, bool F32, bool PAIR>
+template <int BM, bool F32, int ACT>
 static int launch_grouped_stream(const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
+  constexpr int BN = 256;
   const size_t lds = stream_lds(BM, BN);
   static OncePerDevice raised;
   const hipError_t e = once_per_device(raised, [&] {
-    return hipFuncSetAttribute((const void*)grouped_stream_kernel<BM, BN, F32, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return hipFuncSetAttribute((const void*)grouped_stream_kernel<BM, BN, F32, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   });
   SYN_CHECK(e == hipSuccess, "grouped_product: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-  grouped_stream_kernel<BM, BN, F32, PAIR><<<syn_compute_units() / 8 * 8, 256, lds, stream>>>(g, a_bytes, o_bytes);
+  grouped_stream_kernel<BM, BN, F32, ACT><<<syn_compute_units() / 8 * 8, 256, lds, stream>>>(g, a_bytes, o_bytes);
   return 0;
 }
-template <bool F32, bool PAIR>
-static int launch_grouped_stream_as(int bm, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
-  if (bm == 64) return launch_grouped_stream<64, 256, F32, PAIR>(g, a_bytes, o_bytes, stream);
-  if (bm == 128) return launch_grouped_stream<128, 256, F32, PAIR>(g, a_bytes, o_bytes, stream);
-  return launch_grouped_stream<256, 256, F32, PAIR>(g, a_bytes, o_bytes, stream);
+template <bool F32, int ACT>
+static int launch_grouped_stream_as(int rows, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
+  if (rows == 64) return launch_grouped_stream<64, F32, ACT>(g, a_bytes, o_bytes, stream);
+  if (rows == 128) return launch_grouped_stream<128, F32, ACT>(g, a_bytes, o_bytes, stream);
+  return launch_grouped_stream<256, F32, ACT>(g, a_bytes, o_bytes, stream);
+}
+template <int ACT>
+static int launch_grouped_stream_for(int rows, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
+  return g.out_is_f32 ? launch_grouped_stream_as<true, ACT>(rows, g, a_bytes, o_bytes, stream)
+                      : launch_grouped_stream_as<false, ACT>(rows, g, a_bytes, o_bytes, stream);
 }
 
 // rows_bound: with segments, the number of rows in all segments together (what the index lists hold)
@@ -769,10 +773,11 @@ SYN_EXPORT int syn_grouped_product(const void* a, long lda, long a_group, const 
       const double us = tiles / syn_compute_units() * cost[i];
       if (us < least) least = us, bm = 64 << i;
     }
-    const int rc = pair ? (out_is_f32 ? launch_grouped_stream_as<true, true>(bm, g, a_bytes, o_bytes, stream)
-                                      : launch_grouped_stream_as<false, true>(bm, g, a_bytes, o_bytes, stream))
-                        : (out_is_f32 ? launch_grouped_stream_as<true, false>(bm, g, a_bytes, o_bytes, stream)
-                                      : launch_grouped_stream_as<false, false>(bm, g, a_bytes, o_bytes, stream));
+    int rc;
+    if (!pair) rc = launch_grouped_stream_for<NO_PAIR>(bm, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SILU) rc = launch_grouped_stream_for<SYN_ACT_SILU>(bm, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SWIGLU_LIMIT) rc = launch_grouped_stream_for<SYN_ACT_SWIGLU_LIMIT>(bm, g, a_bytes, o_bytes, stream);
+    else rc = launch_grouped_stream_for<SYN_ACT_GELU_TANH>(bm, g, a_bytes, o_bytes, stream);
     if (rc) return rc;
   } else if (!in_is_f32 && chunks && force_simt == 0 && rows_a_group >= 48) {
     const int row_tiles = seg_start ? (rows_bound + GT_BM - 1) / GT_BM + groups : (M + GT_BM - 1) / GT_BM;

@@ -883,6 +883,13 @@ def test_streamed_experts(ops, counts, J, K, act, gated, out_dtype):
     close(out, want.float(), 2e-4 * math.sqrt(K), 1e-4 if out_dtype == F32 else 2 ** -8 + 1e-4, f"{counts} {J} x {K} {act} {gated}")
 
 
+@pytest.mark.parametrize("counts", [[60, 70, 64], [300, 250]])       # the lower tile; plain loads of W
+@pytest.mark.parametrize("out_dtype", [BF16, F32])
+@pytest.mark.parametrize("gated", ["silu", ("swiglu_limit", 7.0), "gelu_tanh", None])
+def test_streamed_experts_of_every_gate(ops, counts, gated, out_dtype):
+    test_streamed_experts(ops, counts, 288, 320, None, gated, out_dtype)
+
+
 def test_slices_fill_the_compute_units(ops):
     """The host-side rule for the products over packed weights: one slice where the workgroups fill their
     rounds, more where they would leave the last round half empty."""
