@@ -372,8 +372,7 @@ __global__ void __launch_bounds__(256) grouped_product_tiled_kernel(GroupedArgs 
 //   * what the stores look up, and the next tile's row list, are asked for before the first store: behind stores they would wait
 //     for these, once for every 32 rows;
 //   * a last round of tiles for up to half of the workgroups is cut into halves of tiles for all.
-// W's loads are marked non-temporal: a tile of W meets one or two tiles of rows, and x stays in the L2s for it (four layers scored at 1,500
-// places 3.48 -> 3.30 ms).
+// ONCE: W's loads are marked non-temporal, where a tile of W meets one tile of rows, so that x stays in the L2s (stream_once).
 // ACT: the gated activation is compiled in: as a branch inside the one loop over the sums it made the epilogue of 256 x 256 tiles
 // 13,000 instructions instead of 3,600, and the product 1 to 18 % slower (32 experts of 2,048 x 2,048 with 224 unequal rows 111 -> 91 us,
 // 8 of 8,192 x 4,096 with 2,048 987 -> 940).
@@ -396,7 +395,7 @@ __device__ __forceinline__ float gelu_quick(float z) {
 }
 
 constexpr int NO_PAIR = -1;
-template <int BM, int BN, bool F32, int ACT>
+template <int BM, int BN, bool F32, int ACT, bool ONCE>
 __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, long a_bytes, long o_bytes) {
   constexpr int BK = 32, STAGES = stream_stages(BM, BN), PAIRS = stream_pairs(BM, BN), WAVES = 4;
   constexpr int XL = BM / 32, WL = BN / 64, PASSES = XL / 2 + WL;      // loads of a wave: of a pair of k-tiles of x, of a k-tile of W, a step
@@ -502,7 +501,7 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
     buffer_to_lds16(vx, (char*)smem + xbuf + x_to + p % XL * (WAVES * 8 * X_PAIR), x_rows.at[p % XL], x_way);
   };
   auto fetch_w = [&](int buf, int p) {
-    buffer_to_lds16<true>(w_view, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], w_way);
+    buffer_to_lds16<ONCE>(w_view, (char*)smem + buf + w_to + p * (WAVES * 16 * BK * (int)sizeof(bf16)), src_w[p], w_way);
   };
   f32x4 acc[FM][FN];
   const int r16 = lane % 16, q4 = lane / 16;
@@ -702,29 +701,37 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
   __builtin_amdgcn_s_waitcnt(0x0070);
 }
 
-template <int BM, bool F32, int ACT>
+template <int BM, bool F32, int ACT, bool ONCE>
 static int launch_grouped_stream(const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
   constexpr int BN = 256;
   const size_t lds = stream_lds(BM, BN);
   static OncePerDevice raised;
   const hipError_t e = once_per_device(raised, [&] {
-    return hipFuncSetAttribute((const void*)grouped_stream_kernel<BM, BN, F32, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return hipFuncSetAttribute((const void*)grouped_stream_kernel<BM, BN, F32, ACT, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   });
   SYN_CHECK(e == hipSuccess, "grouped_product: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-  grouped_stream_kernel<BM, BN, F32, ACT><<<syn_compute_units() / 8 * 8, 256, lds, stream>>>(g, a_bytes, o_bytes);
+  grouped_stream_kernel<BM, BN, F32, ACT, ONCE><<<syn_compute_units() / 8 * 8, 256, lds, stream>>>(g, a_bytes, o_bytes);
   return 0;
 }
 template <bool F32, int ACT>
-static int launch_grouped_stream_as(int rows, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
-  if (rows == 64) return launch_grouped_stream<64, F32, ACT>(g, a_bytes, o_bytes, stream);
-  if (rows == 128) return launch_grouped_stream<128, F32, ACT>(g, a_bytes, o_bytes, stream);
-  return launch_grouped_stream<256, F32, ACT>(g, a_bytes, o_bytes, stream);
+static int launch_grouped_stream_as(int rows, bool once, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
+  if (rows == 64) return launch_grouped_stream<64, F32, ACT, true>(g, a_bytes, o_bytes, stream);
+  if (rows == 128) return once ? launch_grouped_stream<128, F32, ACT, true>(g, a_bytes, o_bytes, stream) : launch_grouped_stream<128, F32, ACT, false>(g, a_bytes, o_bytes, stream);
+  return once ? launch_grouped_stream<256, F32, ACT, true>(g, a_bytes, o_bytes, stream) : launch_grouped_stream<256, F32, ACT, false>(g, a_bytes, o_bytes, stream);
 }
 template <int ACT>
-static int launch_grouped_stream_for(int rows, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
-  return g.out_is_f32 ? launch_grouped_stream_as<true, ACT>(rows, g, a_bytes, o_bytes, stream)
-                      : launch_grouped_stream_as<false, ACT>(rows, g, a_bytes, o_bytes, stream);
+static int launch_grouped_stream_for(int rows, bool once, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
+  return g.out_is_f32 ? launch_grouped_stream_as<true, ACT>(rows, once, g, a_bytes, o_bytes, stream)
+                      : launch_grouped_stream_as<false, ACT>(rows, once, g, a_bytes, o_bytes, stream);
 }
+
+// Whether W's loads are marked non-temporal, from what the host knows: the rows a segment has on average (most segments in one tile then).
+// Non-temporal loads against plain ones, gated products and the others: equal segments of 50 to 188 rows -7 and -6 %, 224 rows -5 and -7,
+// 310 and more +2 to 5 and +1 to 3; unequal ones (0.4 to 1.6 times the average) -4 to 7 and -3 to 5 %, with 224 rows +2 and 0, 256 +4 and 0, more
+// +4 and +5 (184 products of 8 to 128 experts, 768 to 28,672 wide, with 50 to 2,048 rows a segment, in tiles of 256 rows).
+static bool stream_once(long rows_a_group) { return rows_a_group <= 224; }
+// (for tests of the rule)
+SYN_EXPORT int syn_grouped_stream_once(int rows_a_group) { return stream_once(rows_a_group); }
 
 // rows_bound: with segments, the number of rows in all segments together (what the index lists hold)
 // a_total, o_total: rows that a and out hold
@@ -773,11 +780,12 @@ SYN_EXPORT int syn_grouped_product(const void* a, long lda, long a_group, const 
       const double us = tiles / syn_compute_units() * cost[i];
       if (us < least) least = us, bm = 64 << i;
     }
+    const bool once = stream_once(rows_a_group);
     int rc;
-    if (!pair) rc = launch_grouped_stream_for<NO_PAIR>(bm, g, a_bytes, o_bytes, stream);
-    else if (pair - 1 == SYN_ACT_SILU) rc = launch_grouped_stream_for<SYN_ACT_SILU>(bm, g, a_bytes, o_bytes, stream);
-    else if (pair - 1 == SYN_ACT_SWIGLU_LIMIT) rc = launch_grouped_stream_for<SYN_ACT_SWIGLU_LIMIT>(bm, g, a_bytes, o_bytes, stream);
-    else rc = launch_grouped_stream_for<SYN_ACT_GELU_TANH>(bm, g, a_bytes, o_bytes, stream);
+    if (!pair) rc = launch_grouped_stream_for<NO_PAIR>(bm, once, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SILU) rc = launch_grouped_stream_for<SYN_ACT_SILU>(bm, once, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SWIGLU_LIMIT) rc = launch_grouped_stream_for<SYN_ACT_SWIGLU_LIMIT>(bm, once, g, a_bytes, o_bytes, stream);
+    else rc = launch_grouped_stream_for<SYN_ACT_GELU_TANH>(bm, once, g, a_bytes, o_bytes, stream);
     if (rc) return rc;
   } else if (!in_is_f32 && chunks && force_simt == 0 && rows_a_group >= 48) {
     const int row_tiles = seg_start ? (rows_bound + GT_BM - 1) / GT_BM + groups : (M + GT_BM - 1) / GT_BM;

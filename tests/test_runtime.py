@@ -173,6 +173,13 @@ def test_cut_products_take_the_tiles_whose_slices_fill_the_compute_units():
         assert {cut(M, N, K) for M in (65, 96, 128)} == {s} and {cut(M, N, K) for M in (177, 224, 256)} == {s // 2}, (N, K)
 
 
+def test_experts_weights_are_loaded_past_the_caches_where_most_segments_are_one_tile():
+    """Non-temporal loads of W were faster for up to 224 rows an expert on average, and slower beyond, where several tiles of rows read it."""
+    from synaptix_amd.kernels.build import load_library
+    once = load_library("core").syn_grouped_stream_once
+    assert all(once(r) for r in (48, 100, 188, 224)) and not any(once(r) for r in (225, 256, 310, 750, 1024, 2048))
+
+
 def test_32_bit_prompts_share_workgroups_only_where_that_was_measured_to_pay():
     """Steps timed with a wave a row and with 16 rows a workgroup: the latter walks a workgroup's sequences one after another, which single
     tokens behind long contexts beside a prompt make up to six times slower than the former, and many short prompts half as slow again."""
