@@ -376,9 +376,10 @@ __global__ void __launch_bounds__(256) grouped_product_tiled_kernel(GroupedArgs 
 // ACT: the gated activation is compiled in: as a branch inside the one loop over the sums it made the epilogue of 256 x 256 tiles
 // 13,000 instructions instead of 3,600, and the product 1 to 18 % slower (32 experts of 2,048 x 2,048 with 224 unequal rows 111 -> 91 us,
 // 8 of 8,192 x 4,096 with 2,048 987 -> 940).
-// 1,500 tokens with 6 of 48 experts (188 rows each), 2,048 x 4,096 with GELU and back, 32-bit results: 251 + 225 us -> 220 + 217 (x
-// in pieces of 64 bytes, tiles of up to 256 rows and lookups between the stores before); 310 rows each 353 + 383 -> 290 + 316, 120
-// rows 229 + 199 -> 187 + 190, 50 rows 185 + 168 -> 162 + 168, 32 experts with 256 rows 159 -> 162, 16 with 187 127 + 84 -> 101 + 85.
+// 1,500 tokens with 6 of 48 experts (188 rows each), 2,048 x 4,096 with GELU and back, 32-bit results: 244 + 212 us -> 192 + 187 (x
+// in pieces of 64 bytes, tiles of up to 256 rows and lookups between the stores before); 310 rows each 335 + 378 -> 280 + 296, 128
+// rows 232 + 194 -> 169 + 166, 50 rows 182 + 158 -> 154 + 150, 750 rows 592 + 620 -> 560 + 584.  Gated, 8 experts of 4,096 x 4,096
+// and back: 80 rows 158 + 84 -> 94 + 57, 2,048 rows 881 + 473 -> 862 + 463; 32 of 1,024 x 2,048 with 256 rows 79 + 52 -> 77 + 46.
 // Tile order: the column tiles of a row tile follow each other, 32 in a row on one XCD.
 #define GS_MAX_GROUPS 512
 __device__ __forceinline__ float gelu_quick(float z) {
@@ -400,10 +401,11 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
   constexpr int BK = 32, STAGES = stream_stages(BM, BN), PAIRS = stream_pairs(BM, BN), WAVES = 4;
   constexpr int XL = BM / 32, WL = BN / 64, PASSES = XL / 2 + WL;      // loads of a wave: of a pair of k-tiles of x, of a k-tile of W, a step
   constexpr int FM = BM / 32, FN = BN / 32;
+  static_assert(FM == 4 || FM == 8, "row groups of a k-step");
   // A k-step of a wave goes row group by row group: 2 i + (its row of waves) is row group i's fragment of x, so that the waves share
   // what rows a tile has.  The first FMU groups always run, the others where the tile has rows for them, and in each the right
   // half of the columns where the tile has them; the loads lie in what always runs, since their number is what the waits count.
-  constexpr int FMU = FM > 2 ? FM / 2 : FM, H = FN / 2, LOAD_EVERY = FMU * H / PASSES;
+  constexpr int FMU = FM / 2, H = FN / 2, LOAD_EVERY = FMU * H / PASSES;
   constexpr unsigned FAR = 0x80000000u;            // beyond every view of x and W: read as zeros without traffic
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];      // x [PAIRS][BM][64], W [STAGES][BN][32]
   const int tid = threadIdx.x, lane = tid % SYN_WAVE, grid = (int)gridDim.x;
@@ -564,7 +566,7 @@ __global__ void __launch_bounds__(256, 1) grouped_stream_kernel(GroupedArgs g, l
       }
     };
     row_group(std::integral_constant<int, 0>{}), row_group(std::integral_constant<int, 1>{});
-    if constexpr (FM > 2) row_group(std::integral_constant<int, 2>{}), row_group(std::integral_constant<int, 3>{});
+    row_group(std::integral_constant<int, 2>{}), row_group(std::integral_constant<int, 3>{});
     if constexpr (FM > 4) {
       row_group(std::integral_constant<int, 4>{}), row_group(std::integral_constant<int, 5>{});
       row_group(std::integral_constant<int, 6>{}), row_group(std::integral_constant<int, 7>{});
@@ -715,9 +717,9 @@ static int launch_grouped_stream(const GroupedArgs& g, long a_bytes, long o_byte
 }
 template <bool F32, int ACT>
 static int launch_grouped_stream_as(int rows, bool once, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
-  if (rows == 64) return launch_grouped_stream<64, F32, ACT, true>(g, a_bytes, o_bytes, stream);
-  if (rows == 128) return once ? launch_grouped_stream<128, F32, ACT, true>(g, a_bytes, o_bytes, stream) : launch_grouped_stream<128, F32, ACT, false>(g, a_bytes, o_bytes, stream);
-  return once ? launch_grouped_stream<256, F32, ACT, true>(g, a_bytes, o_bytes, stream) : launch_grouped_stream<256, F32, ACT, false>(g, a_bytes, o_bytes, stream);
+  if (rows == 128) return launch_grouped_stream<128, F32, ACT, true>(g, a_bytes, o_bytes, stream);
+  if (once) return launch_grouped_stream<256, F32, ACT, true>(g, a_bytes, o_bytes, stream);
+  return launch_grouped_stream<256, F32, ACT, false>(g, a_bytes, o_bytes, stream);
 }
 template <int ACT>
 static int launch_grouped_stream_for(int rows, bool once, const GroupedArgs& g, long a_bytes, long o_bytes, hipStream_t stream) {
@@ -725,12 +727,21 @@ static int launch_grouped_stream_for(int rows, bool once, const GroupedArgs& g, 
                       : launch_grouped_stream_as<false, ACT>(rows, once, g, a_bytes, o_bytes, stream);
 }
 
-// Whether W's loads are marked non-temporal, from what the host knows: the rows a segment has on average (most segments in one tile then).
+// Rows of a streamed tile, and whether W's loads are marked non-temporal, from what the host knows: the rows a segment has on average.
+// A tile leaves out the rows that its segment does not have, so the higher one costs little where there are few, while a segment of two
+// tiles brings in W twice: against the best of 64, 128 and 256 with equal and unequal segments, 50 rows on average 1.01, 1.02 and 1.06
+// and 1.10, 1.02 and 1.07 times as long, 80 rows 1.52, 1.01, 1.04 and 1.44, 1.01, 1.04, 100 rows 1.42, 1.01, 1.04 and 1.63, 1.19, 1.01, 128 rows 1.37,
+// 1.01, 1.04 and 1.80, 1.31, 1.00.  Tiles of 64 rows won 6 % at most (8 experts with 50 rows each).
 // Non-temporal loads against plain ones, gated products and the others: equal segments of 50 to 188 rows -7 and -6 %, 224 rows -5 and -7,
 // 310 and more +2 to 5 and +1 to 3; unequal ones (0.4 to 1.6 times the average) -4 to 7 and -3 to 5 %, with 224 rows +2 and 0, 256 +4 and 0, more
-// +4 and +5 (184 products of 8 to 128 experts, 768 to 28,672 wide, with 50 to 2,048 rows a segment, in tiles of 256 rows).
+// +4 and +5.
+// All of it over 184 products of 8 to 128 experts, 768 to 28,672 wide, with 50 to 2,048 rows a segment: what this picks takes 1.6 % longer than
+// the best of the six on average, 4 % of them lose more than 10, 1.32 times as long at the worst (8 experts with 400 unequal rows, whose
+// tiles just exceed a round).
+static int stream_rows(long rows_a_group) { return rows_a_group <= 80 ? 128 : 256; }
 static bool stream_once(long rows_a_group) { return rows_a_group <= 224; }
-// (for tests of the rule)
+// (for tests of the rules)
+SYN_EXPORT int syn_grouped_stream_rows(int rows_a_group) { return stream_rows(rows_a_group); }
 SYN_EXPORT int syn_grouped_stream_once(int rows_a_group) { return stream_once(rows_a_group); }
 
 // rows_bound: with segments, the number of rows in all segments together (what the index lists hold)
@@ -767,25 +778,13 @@ SYN_EXPORT int syn_grouped_product(const void* a, long lda, long a_group, const 
                         a_total > 0 && o_total > 0 && a_bytes < (1L << 31) && o_bytes < (1L << 32) - 16 &&
                         (long)N * K * 2 < (1L << 31) && !(act == 1 && out_is_f32);
   if (streamed) {
-    // rows of a tile: tiles spread evenly over the compute units, at what a tile of 128 x 256 and 256 x 256 took of the products of
-    // many rows for 4,096 of K (for 64 x 256: one of 64 x 192), segments as if equally long and half a tile of each left empty.
-    // Coarse: it knows neither whole rounds nor the way of W.  Over 270 products (8 to 128 experts, 768 to 8,192 wide, 48 to 750
-    // rows a segment, equal and unequal ones) what it picks takes 8 % longer than the best of the three on average, and
-    // 1.77 times as long at the worst (8 experts, 100 rows each), where the tiles above took longer still.
-    const double cost[3] = {31.0, 52.1, 74.6};
-    int bm = 64;
-    double least = 1e30;
-    for (int i = 0; i < 3; ++i) {
-      const double tiles = ((double)rows_a_group / (64 << i) + 0.5) * groups * ((N + 255) / 256);
-      const double us = tiles / syn_compute_units() * cost[i];
-      if (us < least) least = us, bm = 64 << i;
-    }
+    const int rows = stream_rows(rows_a_group);
     const bool once = stream_once(rows_a_group);
     int rc;
-    if (!pair) rc = launch_grouped_stream_for<NO_PAIR>(bm, once, g, a_bytes, o_bytes, stream);
-    else if (pair - 1 == SYN_ACT_SILU) rc = launch_grouped_stream_for<SYN_ACT_SILU>(bm, once, g, a_bytes, o_bytes, stream);
-    else if (pair - 1 == SYN_ACT_SWIGLU_LIMIT) rc = launch_grouped_stream_for<SYN_ACT_SWIGLU_LIMIT>(bm, once, g, a_bytes, o_bytes, stream);
-    else rc = launch_grouped_stream_for<SYN_ACT_GELU_TANH>(bm, once, g, a_bytes, o_bytes, stream);
+    if (!pair) rc = launch_grouped_stream_for<NO_PAIR>(rows, once, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SILU) rc = launch_grouped_stream_for<SYN_ACT_SILU>(rows, once, g, a_bytes, o_bytes, stream);
+    else if (pair - 1 == SYN_ACT_SWIGLU_LIMIT) rc = launch_grouped_stream_for<SYN_ACT_SWIGLU_LIMIT>(rows, once, g, a_bytes, o_bytes, stream);
+    else rc = launch_grouped_stream_for<SYN_ACT_GELU_TANH>(rows, once, g, a_bytes, o_bytes, stream);
     if (rc) return rc;
   } else if (!in_is_f32 && chunks && force_simt == 0 && rows_a_group >= 48) {
     const int row_tiles = seg_start ? (rows_bound + GT_BM - 1) / GT_BM + groups : (M + GT_BM - 1) / GT_BM;

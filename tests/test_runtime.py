@@ -180,6 +180,13 @@ def test_experts_weights_are_loaded_past_the_caches_where_most_segments_are_one_
     assert all(once(r) for r in (48, 100, 188, 224)) and not any(once(r) for r in (225, 256, 310, 750, 1024, 2048))
 
 
+def test_experts_tiles_hold_the_rows_of_a_segment():
+    """Tiles of 64 rows took up to twice as long as the others with 80 and 100 rows an expert, tiles of 128 up to twice with 160 and more."""
+    from synaptix_amd.kernels.build import load_library
+    rows = load_library("core").syn_grouped_stream_rows
+    assert {rows(r) for r in (48, 64, 80)} == {128} and {rows(r) for r in (81, 128, 188, 310, 2048)} == {256}
+
+
 def test_32_bit_prompts_share_workgroups_only_where_that_was_measured_to_pay():
     """Steps timed with a wave a row and with 16 rows a workgroup: the latter walks a workgroup's sequences one after another, which single
     tokens behind long contexts beside a prompt make up to six times slower than the former, and many short prompts half as slow again."""
