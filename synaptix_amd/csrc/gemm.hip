@@ -688,7 +688,16 @@ gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, 
 // of the first kind take the first tile (their own gate, the partner's up), the others the second (the
 // partner's gate, their own up), so that a store covers 32 consecutive outputs of a row (64 bytes, not
 // twice 32).  A last tile without a neighbour is stored by the lanes of the first kind alone.
-template <int TM, int TN, bool PAIRED>
+// QUICK: the gated activation as the streamed tiles apply it, so that a product's bits do not depend on which of the two it takes
+// (W in plain rows or in fragment order).
+template <bool QUICK>
+__device__ __forceinline__ float gated_epilogue(const Epilogue& ep, float g, float up) {
+  if constexpr (!QUICK) return gated(ep.act, g, up, ep.limit);
+  if (ep.act == SYN_ACT_SILU) return gated_quick<SYN_ACT_SILU, false>(g, up, 0.f);
+  if (ep.act == SYN_ACT_SWIGLU_LIMIT) return gated_quick<SYN_ACT_SWIGLU_LIMIT, false>(g, up, ep.limit);
+  return gated_quick<SYN_ACT_GELU_TANH, false>(g, up, 0.f);
+}
+template <int TM, int TN, bool PAIRED, bool QUICK = false>
 __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TM][TN], void* __restrict__ out, Epilogue ep,
                                             size_t slice, int M, int N, int mw, int nw, int lane) {
   if constexpr (PAIRED) {
@@ -705,10 +714,10 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TM][TN], void* _
             const float own1 = acc[i][j + 1 < TN ? j + 1 : j][e], other1 = __shfl_xor(own1, 16, SYN_WAVE);
             const float g = first ? own0 : other1, up = first ? other0 : own1;
             if (m < M && nw + (j + (first ? 0 : 1)) * 32 < N)
-              ((bf16*)out)[(size_t)m * (N / 2) + (nw + j * 32) / 2 + lane % 32] = (bf16)gated(ep.act, g, up, ep.limit);
+              ((bf16*)out)[(size_t)m * (N / 2) + (nw + j * 32) / 2 + lane % 32] = (bf16)gated_epilogue<QUICK>(ep, g, up);
           } else {
             if (m < M && nw + j * 32 < N && first)
-              ((bf16*)out)[(size_t)m * (N / 2) + (nw + j * 32) / 2 + lane % 16] = (bf16)gated(ep.act, own0, other0, ep.limit);
+              ((bf16*)out)[(size_t)m * (N / 2) + (nw + j * 32) / 2 + lane % 16] = (bf16)gated_epilogue<QUICK>(ep, own0, other0);
           }
         }
   } else {
@@ -994,7 +1003,7 @@ gemm_direct_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
     next_landed(more);
     __builtin_amdgcn_s_barrier();
   }
-  store_tiles<TM, TN, PAIRED>(acc, out, ep, blockIdx.y, M, N, m0 + wm, n0 + wn, lane);
+  store_tiles<TM, TN, PAIRED, true>(acc, out, ep, blockIdx.y, M, N, m0 + wm, n0 + wn, lane);
 }
 
 // A weight [N, K] as a product is handed it: plain rows, or in fragment order (pack_weight)
@@ -1624,8 +1633,12 @@ static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, 
 // pieces than the streamed tiles ask for.  Direct against the best streamed tile, us: 12,288 x 4,096 with 96 rows 30.4, 32.1, 128 rows
 // 32.9, 35.2, 84 rows 34.7, 30.9; 6,144 x 4,096 with 96 rows 27.9, 28.6, 256 rows 30.4, 31.3; 10,240 x 5,120 with 128 rows 40.2, 41.9, 84
 // rows 38.1, 36.3; 4,096 x 2,048 with 128 rows 17.1, 13.1; 8,192 x 2,048 17.8, 16.0; 6,144 x 2,560 21.9, 15.9.
-static bool direct_one_round(int M, int N, int K) {
-  return M <= 256 && (M - 1) % 64 >= 31 && K >= 4096 && (long)N * K >= 24L << 20 && tile_grid(M, N, 64, 128) <= syn_compute_units();
+// W in plain rows, which the streamed tiles ask for in pieces of 64 bytes of a row, goes through them whatever its size and the rows that
+// the last 64 hold: 1,024 x 1,024 9, 11; 2,048 x 2,048 with 96 rows 14, 17, 4,096 x 4,096 27, 38, 128 rows 30, 41, 65 rows 25, 33, 2,560 x 9,728
+// with 96 rows 61, 88, 12,288 x 4,096 31, 42; not in two rounds (10,240 x 5,120 with 160 rows 70, 54).
+static bool direct_one_round(int M, int N, int K, bool packed) {
+  if (M > 256 || K % 128 != 0 || tile_grid(M, N, 64, 128) > syn_compute_units()) return false;
+  return !packed || ((M - 1) % 64 >= 31 && K >= 4096 && (long)N * K >= 24L << 20);
 }
 
 // The slices of K in which the tiles of 64 or 128 rows by 128 of W that load straight into LDS (gemm_direct) fill the compute units.
@@ -1640,10 +1653,10 @@ static int direct_slices(int M, int N, int K) {
 // Whether a cut product of 57 to 64 rows goes through the streamed tiles, in the slices of their estimate: a large W whose tiles of
 // gemm_direct leave three eighths of the compute units without work, which slices in other numbers than powers of two reach.  Kernel times
 // in a prompt step of 64 rows, us, these tiles and streamed: 5,120 x 25,600 cut in 4 and 6 56.1, 46.5, 10,240 x 5,120 in 2 and 3 26.1, 24.0,
-// 5,120 x 8,192 in 4 and 6 21.4, 19.5; smaller ones and those that fill them: 6,144 x 4,096 13.6, 14.7, 4,096 x 12,288 21.1, 21.7, 2,560 x
+// 5,120 x 8,192 in 4 and 6 21.4, 19.5 (W in fragment order); smaller ones and those that fill them: 6,144 x 4,096 13.6, 14.7, 4,096 x 12,288 21.1, 21.7, 2,560 x
 // 9,728 15.9, 17.4, 8,192 x 28,672 in 4 and 8 6 less.  Steps with every product streamed, and so: 8B shape 4.07, 3.95 ms, 4B 3.21, 3.11.
-static bool few_rows_streamed(int N, int K) {
-  return (long)N * K >= 24L << 20 && 8 * direct_groups(64, N) * direct_slices(64, N, K) <= 5L * syn_compute_units();
+static bool few_rows_streamed(int N, int K, bool packed) {
+  return packed && (long)N * K >= 24L << 20 && 8 * direct_groups(64, N) * direct_slices(64, N, K) <= 5L * syn_compute_units();
 }
 
 // Whether a cut product of 65 to 128 or 177 to 256 rows goes through the tiles of 128 x 128 that hold k-tiles of 64 (gemm_direct): where
@@ -1653,36 +1666,41 @@ static bool few_rows_streamed(int N, int K) {
 // with 96 and 128 rows 6,144 x 4,096 alone 4.0, 3.8, 6,144 x 6,144 3.0, 2.7, 7,168 x 5,120 2.7, 0.8, 3,072 x 8,192 1.6, 0.6 (with 192 and 256
 // rows from 2.0 less to 2.7 more).  Beyond: 8,192 x 8,192 0.8, 1.2, 4,096 x 14,336 -2.7, -2.8, 6,144 x 16,384 -7.3, -7.5, 8,192 x 28,672 -1.8,
 // -3.5.  Below, or with fewer workgroups: 4,096 x 4,096 -1.5, -2.8, 6,144 x 2,560 -0.5, -2.3, 2,560 x 9,728 (160 of them) -1.4, -2.5.
-static bool direct_cut(int M, int N, int K) {
+// W in plain rows: up to 128 rows whatever W (the product and the sum of its slices, these tiles and streamed: 6,144 x 2,560 with 128 rows 20,
+// 24, 2,560 x 9,728 with 96 26, 27, 4,608 x 3,584 22, 20), above it where they fill the compute units (4,096 x 4,096 with 256 rows 25, 29,
+// 8,192 x 4,096 37, 39; 5,120 x 5,120, 160 workgroups, 40, 36).
+static bool direct_cut(int M, int N, int K, bool packed) {
   const long w = (long)N * K, groups = direct_groups(M, N), cus = syn_compute_units();
   if (!(M > 64 && M <= 128) && !(M > 176 && M <= 256)) return false;
-  return K % 128 == 0 && w >= 24L << 20 && w <= 48L << 20 && groups <= cus && 4 * groups * direct_slices(M, N, K) >= 3 * cus;
+  if (K % 128 != 0 || groups > cus) return false;
+  if (packed ? w < 24L << 20 || w > 48L << 20 : M <= 128) return !packed;
+  return 4 * groups * direct_slices(M, N, K) >= 3 * cus;
 }
 
 // Into how many slices of K a product of more than 56 rows is cut when its reader adds partial sums: those of the tiles above or, for
 // the streamed ones, the smallest estimate of the product's time and of what its reader pays for the slices beyond the first (M x N
 // floats each, half of them from caches).
-static int plan_slices(const StreamFit& fit, int M, int N, int K) {
+static int plan_slices(const StreamFit& fit, int M, int N, int K, bool packed) {
   int best = 1;
   double least = 1e30;
   if (M <= 0 || N <= 0 || K <= 0) return 1;
   for (int s : {1, 2, 3, 4, 6, 8}) {
-    const StreamPlan p = plan_stream(fit, M, N, K, s, true, 4);
+    const StreamPlan p = plan_stream(fit, M, N, K, s, packed, 4);
     if (p.tile < 0) break;
     const double us = p.us + (s - 1) * fit.reader * 4.0 * M * N;
     if (us < least) least = us, best = s;
   }
   return best;
 }
-SYN_EXPORT int syn_gemm_cut_slices(int M, int N, int K) {
+SYN_EXPORT int syn_gemm_cut_slices(int M, int N, int K, int packed) {
   if (M <= 0 || N <= 0 || K <= 0) return 1;
-  if (M <= 64 ? !few_rows_streamed(N, K) : direct_cut(M, N, K)) return direct_slices(M, N, K);
-  return plan_slices(STREAMED, M, N, K);
+  if (M <= 64 ? !few_rows_streamed(N, K, packed) : direct_cut(M, N, K, packed)) return direct_slices(M, N, K);
+  return plan_slices(STREAMED, M, N, K, packed);
 }
 
 // Whether a product that could be rounded to 16 bits hands on its 32-bit sums whatever number of slices is the fastest now: a line that a
 // fit of the tiles' times must not move, since it decides how precise a result is.  (Products that are cut hand them on in any case.)
-SYN_EXPORT int syn_gemm_sums_line(int M, int N, int K) { return plan_slices(SUMS_LINE, M, N, K) > 1; }
+SYN_EXPORT int syn_gemm_sums_line(int M, int N, int K) { return plan_slices(SUMS_LINE, M, N, K, true) > 1; }
 
 // ------------------------------------------------------------------ entry point
 // dtype: 0 = float in, float out; 1 = bf16 in, bf16 out; 2 = bf16 in, float out.
@@ -1782,13 +1800,13 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
     else if (N >= 65536 && !w_packed) rc = launch_tiled<32, 32, 256, 1, 1>(xb, wb, out, ep, M, N, K, stream, slices);
     else if (K % 128 == 0) rc = launch_direct<32, 64, 128, 1, 2>(xb, wt, out, ep, M, N, K, stream, slices);
     else rc = launch_tiled<32, 64, 128, 1, 2>(xb, wb, out, ep, M, N, K, stream, slices);
-  } else if (M <= 64 && K % 128 == 0 && !(M > 56 && slices > 1 && few_rows_streamed(N, K))) {
+  } else if (M <= 64 && K % 128 == 0 && !(M > 56 && slices > 1 && few_rows_streamed(N, K, wt.packed))) {
     // 33 to 64 rows: 128 rows of W a workgroup, so that the rows of x are fetched half as often (every
     // workgroup reads all of x), three k-tiles in a ring, one workgroup a compute unit
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
-  } else if (slices > 1 && direct_cut(M, N, K) && slices == direct_slices(M, N, K)) {
+  } else if (slices > 1 && direct_cut(M, N, K, wt.packed) && slices == direct_slices(M, N, K)) {
     rc = launch_direct<128, 128, 64, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream, slices);
-  } else if (M > 64 && slices == 1 && K % 128 == 0 && direct_one_round(M, N, K)) {
+  } else if (M > 64 && slices == 1 && direct_one_round(M, N, K, wt.packed)) {
     rc = launch_direct<64, 128, 128, 2, 4, false, 3>(xb, wt, out, ep, M, N, K, stream);
   } else if (M <= 64 && K % 128 != 0) {
     rc = launch_tiled<64, 64, 128, 2, 2>(xb, wb, out, ep, M, N, K, stream, slices);
@@ -1798,6 +1816,18 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   if (rc) return rc;
   SYN_LAUNCH_CHECK("gemm");
   return 0;
+}
+
+// Rows of the tile of gemm_direct that a gated product of 65 to 256 rows over W in plain rows goes through, 0: the streamed tiles.  One tile
+// of rows beside 96 or 128 rows of W each, where these go round once and fill most of the compute units, us, these and streamed: 96 rows,
+// 24,576 x 4,096 46, 54, 22,016 x 4,160 45, 53, 20,480 x 5,120 54, 67, 18,944 x 3,584 41, 47, 19,456 x 2,560 35, 37, 16,384 x 2,048 (171 tiles) 28,
+// 25, 28,672 x 4,096 (299) 87, 59; 160 rows, 24,576 x 4,096 63, 74, 20,480 x 5,120 74, 102, 28,672 x 4,096 64, 77, 32,768 x 4,096 71, 80, 16,384
+// x 2,048 (128 tiles) 39, 26, 51,200 x 5,120 (400) 151, 146.
+static int direct_gated_tile(int M, int N, int K) {
+  const int cus = syn_compute_units(), by96 = (N + 95) / 96, by128 = (N + 127) / 128;
+  if (K % 64 != 0 || K < 2048) return 0;
+  if (M <= 128) return 4 * by96 >= 3 * cus && by96 <= cus ? 128 : 0;
+  return M <= 256 && 16 * by128 >= 9 * cus && by128 <= cus ? (M <= 192 ? 192 : 256) : 0;
 }
 
 // out[M, N/2] = silu(x . Wg^T) * (x . Wu^T), bf16, where w [N, K] holds the rows of Wg and of Wu in
@@ -1822,10 +1852,18 @@ SYN_EXPORT int syn_gemm_swiglu(const void* x, const void* w, void* out, int M, i
     rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream, 1, tile);
   } else if (rows && w_packed) {
     rc = launch_rows<true>(rows, xb, wb, out, ep, M, N, K, 1, stream);
-  } else if (M > 64 || (M > 16 && K >= 256 && K % 64 == 0)) {
+  } else if (!w_packed && M > 64 && direct_gated_tile(M, N, K)) {
+    const int tile = direct_gated_tile(M, N, K);
+    if (tile == 128) rc = launch_direct<128, 96, 64, 4, 1, true, 4>(xb, wt, out, ep, M, N, K, stream);
+    else if (tile == 192) rc = launch_direct<192, 128, 64, 2, 2, true, 3>(xb, wt, out, ep, M, N, K, stream);
+    else rc = launch_direct<256, 128, 64, 4, 2, true, 3>(xb, wt, out, ep, M, N, K, stream);
+  } else if (M > 64 || (M > 16 && K >= 256 && K % 64 == 0 && (w_packed || K % 128 != 0 || (M > 32 && (long)N * K < 12L << 20)))) {
     // the streamed tiles from 17 rows on (W in fragment order, us against the tiles below: 19,456 x 2,560 with 24 rows 26.8 -> 23.3, 64 27.3 ->
     // 26.7, 128 34.9 -> 32.9; 24,576 x 4,096 with 64 45.1 -> 43.6, 96 48.2, 47.9; 51,200 x 5,120 with 32 99 -> 94, 128 166 -> 111; 8,192 x 1,024 with
-    // 128 18.6 -> 9.4)
+    // 128 18.6 -> 9.4).  W in plain rows from 65 on, or where K keeps it from the tiles below that load straight into LDS, or where it is small
+    // (these tiles and those, 33 to 64 rows: 24,576 x 4,096 50, 38, 12,288 x 4,096 43, 34, 16,384 x 2,048 25, 22, 6,144 x 2,560 30, 25, 8,192 x 1,024
+    // 10, 13, 2,048 x 2,048 15, 18; 17 to 32: 24,576 x 4,096 49, 40, 2,560 x 9,728 88, 39, 8,192 x 1,024 10, 9; K = 4,160, 22,016 wide 47, 47,
+    // K = 1,088, 8,192 wide 10, 14).
     rc = launch_large<true>(xb, wt, out, ep, M, N, K, stream);
   } else if (M == 1 && !w_packed) {
     // one row: fragments of W straight from memory; eight waves on the gate rows, eight on the up rows

@@ -571,23 +571,23 @@ def packed_slices(N, K):
 
 
 @functools.lru_cache(maxsize=4096)
-def _cut_slices(M, N, K):
-    return int(load_library("core").syn_gemm_cut_slices(M, N, K))
+def _cut_slices(M, N, K, packed):
+    return int(load_library("core").syn_gemm_cut_slices(M, N, K, int(packed)))
 
 
-def gemm_slices(M, N, K, dtype):
+def gemm_slices(M, N, K, dtype, packed=True):
     """Into how many slices of K a product is cut when its reader can add partial sums.  A product
     with few rows of W has too few workgroups (one for every 64 rows) to pull the weights at speed.
     The cut aims at one round of workgroups over the 256 compute units; up to 32 rows of x, where the
     tiles keep three k-tiles in flight, four slices are enough (and leave the reader fewer partial
     sums to add); measured at the shapes of an 8B model (N = 4096 and 6144, K = 4096 and 12288) for
-    1, 8, 32 and 64 rows."""
+    1, 8, 32 and 64 rows.  packed: the weight is in fragment order, or else in plain rows."""
     if dtype != _BF16 or K % 8 != 0 or N > 16384 or K < 2048:
         return 1
     units = compute_units()
     if M > 56 and K % 128 == 0:
         # with the tiles that take so many rows of this product (csrc/gemm.hip)
-        return _cut_slices(M, N, K)
+        return _cut_slices(M, N, K, bool(packed))
     if M > 64:
         return 1
     if M <= 32:

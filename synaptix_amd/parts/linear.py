@@ -253,6 +253,8 @@ def product_slices(n_rows, w, dtype) -> int:
         slices = ops.rows_slices(n_rows, *w.shape)
         if slices:
             return slices
+    if w.packed is None and w.device.type == "cuda":
+        return ops.gemm_slices(n_rows, w.shape[0], w.shape[1], dtype, packed=False)
     return ops.gemm_slices(n_rows, w.shape[0], w.shape[1], dtype)
 
 

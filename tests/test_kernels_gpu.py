@@ -765,6 +765,29 @@ def test_products_in_the_slices_of_their_tiles(ops, M, N, K):
         assert torch.isfinite(out).all() and float(off.max()) <= 0, float(off.max())
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(18528, 2112), (18528, 2048), (4096, 2048), (768, 4096)])
+def test_gated_and_uncut_products_over_plain_rows(ops, M, N, K):
+    """17 to 256 rows over W in plain rows, through the tiles that load straight into LDS and through the streamed ones."""
+    x, w = rnd((M, K), 98, BF16).to(DEV), rnd((N, K), 99, BF16).to(DEV)
+    z = x.double() @ w.double().T
+    out, gated = torch.full((M, N), float("nan"), dtype=F32, device=DEV), torch.full((M, N // 2), float("nan"), dtype=BF16, device=DEV)
+    ops.gemm(x, w, out)
+    assert torch.isfinite(out).all() and float((out.double() - z).abs().max()) <= 1e-4 * math.sqrt(K)
+    ops.gemm_swiglu(x, w, gated)
+    z = z.view(M, N // 32, 2, 16)
+    g, u = z[:, :, 0].reshape(M, -1), z[:, :, 1].reshape(M, -1)
+    want, room = g * torch.sigmoid(g) * u, 1e-4 * math.sqrt(K) * (g.abs() + u.abs() + 1)
+    off = (gated.double() - want).abs() - 2 ** -8 * want.abs() - room
+    assert torch.isfinite(gated).all() and float(off.max()) <= 0, float(off.max())
+    if K % 128 == 0:          # the bits do not depend on how W lies
+        packed = ops.pack_weight(w)
+        again, gated2 = torch.empty_like(out), torch.empty_like(gated)
+        ops.gemm(x, packed, again)
+        ops.gemm_swiglu(x, packed, gated2)
+        assert torch.equal(again, out) and torch.equal(gated2, gated)
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", ("swiglu_limit", 7.0)])
 @pytest.mark.parametrize("M,I,K", [(300, 1200, 256), (2100, 4112, 512)])
 def test_gated_activations_of_many_rows(ops, act, M, I, K):

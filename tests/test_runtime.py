@@ -173,6 +173,17 @@ def test_cut_products_take_the_tiles_whose_slices_fill_the_compute_units():
         assert {cut(M, N, K) for M in (65, 96, 128)} == {s} and {cut(M, N, K) for M in (177, 224, 256)} == {s // 2}, (N, K)
 
 
+def test_cut_products_over_plain_rows_keep_the_slices_that_fill_the_compute_units():
+    """W in plain rows, which the streamed tiles read in short pieces: powers of two up to 128 rows whatever W, above where they fill."""
+    import torch
+    from synaptix_amd.kernels import ops
+    cut = lambda M, N, K: ops.gemm_slices(M, N, K, torch.bfloat16, packed=False)
+    for N, K, s in ((6144, 2560, 4), (4096, 4096, 8), (2560, 9728, 8), (10240, 5120, 2), (5120, 8192, 4), (4096, 12288, 8)):
+        assert {cut(M, N, K) for M in (48, 57, 64, 65, 96, 128)} == {s}, (N, K)
+    for N, K, s in ((4096, 4096, 4), (8192, 4096, 2), (6144, 4096, 2), (4096, 12288, 4)):
+        assert {cut(M, N, K) for M in (177, 256)} == {s}, (N, K)
+
+
 def test_experts_weights_are_loaded_past_the_caches_where_most_segments_are_one_tile():
     """Non-temporal loads of W were faster for up to 224 rows an expert on average, and slower beyond, where several tiles of rows read it."""
     from synaptix_amd.kernels.build import load_library
