@@ -132,6 +132,19 @@ def test_bins_hold_every_piece_once_and_even_sums(rows, places):
             units = [-(-(x if window is None else min(x, window)) // UNIT) for x in lengths]
             share = max(UNIT // 4, -(-sum(u for u in units if u > 1) // places))
             assert all(n == 1 for s, n in n_of.items() if units[s] <= share)       # only what is longer than a share is cut
+            # every piece goes to the smallest sum: no sum is above their mean and the longest piece, over as many places as there are
+            # pieces, or a half or a third as many
+            flat = rt.decode_bins(lengths, 2, places, window)
+            sums, longest, live = [0] * places, 0, 0
+            for at in range(2 * rows):
+                seq, split_and_n = flat[4 * at], flat[4 * at + 1] >> 16
+                if seq >= 0 and units[seq] > 1:
+                    piece = -(-units[seq] // split_and_n) + 4 + (2 if split_and_n > 1 else 0)      # what starting and merging it cost included
+                    sums[at % places] += piece
+                    longest, live = max(longest, piece), live + 1
+            used = sum(x > 0 for x in sums)
+            assert used >= min(places, -(-live // 3))
+            assert not used or max(sums) <= sum(sums) / used + longest
 
 
 def test_bins_pair_long_sequences_with_short_ones():

@@ -442,6 +442,39 @@ def test_a_captured_step_keeps_its_own_scratch_memory():
     eng.cache.check()
 
 
+def test_captured_decode_of_more_sequences_than_fill_the_chip():
+    """40 unequal sequences over 8 kv heads, one much longer than the rest, through a captured step of 64 rows, whose work list spreads the
+    keys over the compute units and cuts the longest: the logits of the same step launched kernel by kernel."""
+    from synaptix_amd import Engine, Qwen3Config
+    from synaptix_amd.config import resolve_architecture
+    from synaptix_amd.weights import load_weights
+    from synaptix_amd.weights.source import RandomSource
+    cfg = Qwen3Config.from_dict(dict(num_hidden_layers=2, hidden_size=256, num_attention_heads=16, num_key_value_heads=8, head_dim=32,
+                                     intermediate_size=512, vocab_size=700, tie_word_embeddings=False, rope_theta=1e6, rms_norm_eps=1e-6,
+                                     max_position_embeddings=4096, eos_token_id=None, bos_token_id=None))
+    model = resolve_architecture(cfg.to_dict()).build(cfg, max_positions=4096)
+    load_weights(model, RandomSource(model.tensor_specs(), 5, std=0.05), torch.bfloat16, "cuda:0")
+    eng = Engine(model, "bfloat16", max_tokens=64 * 140)
+    lens = [3000] + [1 + (97 * i) % 190 for i in range(39)]
+    slots = [eng.acquire() for _ in lens]
+    for i in range(0, 40, 8):
+        eng.step([(s, random_tokens(700, n, 300 + n)) for s, n in zip(slots[i:i + 8], lens[i:i + 8])], want=None)
+    runner = eng.decode_runner(40, 3100)
+    assert runner.item_bins == [32]
+    for step in range(3):
+        toks = random_tokens(700, 40, 900 + step)
+        _, got = runner.step(slots, toks)
+        got = got.clone()
+        i, at = runner.bins_at[0]
+        items = runner.dev[at:at + 8 * runner.rows].view(-1, 4).cpu()
+        assert int((items[:, 1] >> 16)[items[:, 0] == 0].max()) > 1 and set(range(40)) <= set(items[:, 0].tolist())
+        for s, n in zip(slots, lens):
+            eng.cache.truncate(s, n + step)
+        want = eng.step([(s, [t]) for s, t in zip(slots, toks)], want="last")
+        assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
+    eng.cache.check()
+
+
 def test_generation_with_and_without_graph_agree():
     from synaptix_amd.engine.generate import generate, GenerationConfig
     V = CONFIGS["A"]["vocab_size"]

@@ -1356,6 +1356,47 @@ def test_attention_decode_over_bins(ops, nh, nkv, hd, rows, hi, window):
     assert int(counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("nh,nkv,hd,rows,hi,window,parts", [(32, 8, 128, 33, 2000, 0, 4), (8, 8, 64, 48, 900, 200, 0), (16, 4, 32, 65, 500, 0, 2)])
+def test_fused_decode_over_bins(ops, nh, nkv, hd, rows, hi, window, parts):
+    """The same through the kernel that a decode step runs, which makes q, k and v of the new tokens itself and writes them to the cache."""
+    gen = torch.Generator().manual_seed(rows)
+    lens = torch.randint(1, hi, (rows,), generator=gen).tolist()
+    lens[0], lens[1], lens[-1] = 3 * hi, hi, 1
+    width = (max(lens) + 63) // 64 + 1
+    pages = [(n + 63) // 64 for n in lens]
+    table = torch.zeros((rows, width), dtype=I32)
+    ids, at = torch.randperm(sum(pages), generator=gen).to(I32), 0
+    for b, p in enumerate(pages):
+        table[b, :p] = ids[at:at + p]
+        at += p
+    k, v = make_cache(sum(pages), nkv, hd, BF16, 83)
+    fill_sequences(k, v, table, lens, nkv, hd, BF16, 84)
+    qkv = rnd((rows, (nh + 2 * nkv) * hd), 85, F32)
+    qkv = (qkv[None] * (torch.arange(1, parts + 1, dtype=F32)[:, None, None] / sum(range(parts + 1)))).contiguous() if parts else qkv.to(BF16)
+    qg, kg = ((1 + 0.2 * rnd((hd,), 86 + i)).to(BF16) for i in range(2))
+    ang = torch.arange(max(lens) + 1, dtype=F32)[:, None] * (0.3 / (1 + torch.arange(hd // 2, dtype=F32)))[None, :]
+    cos, sin = torch.cos(ang), torch.sin(ang)
+    seq_len, scale = torch.tensor(lens, dtype=I32), 1 / math.sqrt(hd)
+    k_ref, v_ref, q_ref = k.clone(), v.clone(), torch.empty((rows, nh * hd), dtype=BF16)
+    ref.qk_norm_rope_kv_write(qkv, q_ref, k_ref, v_ref, table, torch.arange(rows, dtype=I32), seq_len - 1, qg, kg, 1e-5, cos, sin, nh, nkv, hd)
+    want = torch.empty((rows, nh * hd), dtype=F32)
+    ref.attention_f32(q_ref.float(), k_ref.float(), v_ref.float(), table, torch.arange(rows, dtype=I32), seq_len - 1, want, scale, window, nh, nkv, hd)
+    S = ops.DECODE_BIN_SPLITS
+    items = rt.decode_bins(lens, S, ops.decode_bins(rows, nkv, nh // nkv), window or None)
+    assert window or max(items[4 * i + 1] >> 16 for i in range(S * rows)) > 1
+    d = lambda t: t.to(DEV)
+    counters = torch.zeros(rows * nkv, dtype=I32, device=DEV)
+    work = torch.full((rows * nh * S * (hd + 2),), float("nan"), dtype=F32, device=DEV)
+    for kw in (dict(counters=counters), {}):
+        kd, vd, out = d(k), dv(v), torch.full((rows, nh * hd), float("nan"), dtype=BF16, device=DEV)
+        ops.attention_decode_fused_bf16(d(qkv), kd, vd, d(table), d(seq_len), out, work, S, scale, window, nh, nkv, hd, d(qg), d(kg), 1e-5,
+                                        d(cos), d(sin), items=torch.tensor(items, dtype=I32, device=DEV), **kw)
+        close(out, want, 2e-2, 1e-2, what="fused decode attention over bins")
+        close(kd, k_ref.float(), 2e-2, 1e-2, what="k pages after the step")
+        close(hv(vd), v_ref.float(), 2e-2, 1e-2, what="v pages after the step")
+    assert int(counters.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("lens,splits", [([2061] * 8, 4), ([2061], 16), ([3908, 457, 1200, 2500], 8)])
 def test_merge_inside_the_launch_reads_what_this_launch_wrote(ops, lens, splits):
     """The workgroup that merges the splits reads partial results that workgroups on other XCDs, each with a
