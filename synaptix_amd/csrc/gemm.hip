@@ -9,10 +9,10 @@
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
 //   gemm_packed    bf16, M <= 16 (used up to 8): the same over a copy of W kept in the order of the MFMA
 //                  fragments, so that every load of a wave is 1 KB of consecutive bytes.
-//   gemm_stream    bf16, M > 56 (gated 16), K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
+//   gemm_stream    bf16, M > 64 (gated 16), K a multiple of 64: tiles of 256 x 256 down to 64 x 128, loads straight into LDS, one
 //                  stream of k-steps over all tiles of a workgroup.
-//   gemm_direct    bf16, up to 56 or 64 rows, uncut products of large weights up to 256 where its tiles go round once: 32 to 128
-//                  rows of x, 64 to 128 rows of W, 64 to 256 deep, straight into LDS: the rows of W arrive as whole
+//   gemm_direct    bf16, up to 64 rows, and up to 256 where its tiles fill the compute units and go round once (large weights, or W in
+//                  plain rows): 32 to 256 rows of x, 64 to 128 rows of W, 64 to 256 deep, straight into LDS: the rows of W arrive as whole
 //                  256-byte pieces, which streams them faster than loading MFMA fragments (64 bytes a row) straight
 //                  from memory.
 //   gemm_tiled     bf16, any K that is a multiple of 8: the tiles pass through registers on their way to LDS.
@@ -1040,7 +1040,8 @@ static int launch_direct(const bf16* x, Weight w, void* out, Epilogue ep, int M,
   return 0;
 }
 
-// ------------------------------------------------------------------ 17 to 128 rows, W in fragment order: operands straight to registers
+// ------------------------------------------------------------------ 9 to 128 rows, W in fragment order: operands straight to registers
+// (The rules take it up to 64 rows, gated 48; `rows` asks for it up to 128.)
 // What bounds it: what a compute unit brings in, W and x together (13 to 15 bytes a clock), and W's stream from memory, of which a unit
 // has to keep some 64 KB under way.  Through a ring of LDS buffers W shares the room with x (36 KB of it under way beside 96 rows
 // of x), and every k-tile ends in a barrier.  Here the four waves of a workgroup
@@ -1246,9 +1247,10 @@ __device__ __forceinline__ TileAt stream_tile(int i, int tiles_m, int tiles_n) {
 #define SYN_OUT_F32 1
 #define SYN_OUT_GATED 2     // W: gate and up rows in turns of 16; bf16, half as wide
 // ONCE: the rows fit one tile, so that W is read once: its loads are marked non-temporal.  (A stream of weights through the L2s pushes
-// everything else out of them: a decode step of 64 sequences at the 8B shape 7.53 -> 7.25 ms, a prompt of 96 tokens 5.10 -> 4.78.  Where
-// several rows of tiles read W it lost: 41,000 tokens at the 4B shape 299 -> 317 ms, 1,733 28.97 -> 29.13, and in two rows of tiles 160
-// tokens at the 8B shape 176 -> 181 us a layer, 96 at the 4B shape 118 -> 125.)
+// everything else out of them.  Steps with the hint taken from the gated product, ms: 8B shape 64 rows 4.07 -> 4.30, 96 4.70 -> 4.91, 128
+// 5.07 -> 5.26, eight layers of the 32B one 64 1.89 -> 2.00, 96 2.00 -> 2.18, 256 2.78 -> 3.10; from q/k/v, o_proj or down_proj of the latter 10 to
+// 60 us.  Where several rows of tiles read W it lost: 41,000 tokens at the 4B shape 299 -> 317 ms, 1,733 28.97 -> 29.13, and in two rows of tiles
+// 160 tokens at the 8B shape 176 -> 181 us a layer, 96 at the 4B shape 118 -> 125.)
 template <int BM, int BN, int OUT, bool WP, bool ONCE>
 __global__ void __launch_bounds__(256, 1)
 gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void* __restrict__ out, Epilogue ep,
@@ -1481,8 +1483,10 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
 // compute unit; and the way of W from memory, which is longer where fewer compute units ask for it.  Rows and columns beyond M
 // and N are zeros, which draw next to no power: with 129 rows 19,456 x 2,560 takes 34 us, with 256, the same tiles, 48.  So
 // both count by the share of a tile that is filled.  The stores of the output come on top, and where W is read by more than one
-// row of tiles, so that it passes through the caches (ONCE above), what it pushes out of them: in a step of 96 rows gate+up of 24,576 x
-// 4,096 in tiles of 64 x 192 made a layer take 6 to 8 us longer than in tiles of 128 x 128, though by itself it is 5 us faster.
+// row of tiles, so that it passes through the caches (ONCE above), what it pushes out of them: with 96 and 128 rows gate+up in tiles of 64 x
+// 192, by itself the faster one, made a layer take longer than in tiles of 128 x 128: 24,576 x 4,096 by 7.4 and 5.1 us, 23,552 x 4,096 10 and
+// 7.5, 22,528 x 5,120 7.3 and 3.5, 24,576 x 6,144 12 and 12; with 160 and 192 rows in tiles of 128 x 192 against 256 x 128 the last of them
+// 4 us, the others from 2 less to the same.
 // The figures are fitted to 744 sizes, every tile and number of slices, with weights that no cache held: 17 to 3,300 rows, multiples of
 // the tiles and others, through N x K = 6144 x 4096, 10240 x 5120, 12288 x 4096, 3072 x 1024, 4096 x 2048, 8192 x 2048, 6144 x 2560 (rounded to
 // bf16), 4096 x 4096, 4096 x 12288, 2560 x 4096, 2560 x 9728, 5120 x 8192, 5120 x 25600, 1024 x 4096, 2048 x 8192, 6144 x 2560 (32-bit sums
@@ -1610,7 +1614,7 @@ static int pick_register_tile(int M, int N) {
   return best;
 }
 
-// M > 56, gated M > 16.  A K that the kernel above does not take goes through the tiles that pass through registers (any K that is a multiple
+// M > 64, gated M > 16, and cut products of 57 rows and more.  A K that the kernel above does not take goes through the tiles that pass through registers (any K that is a multiple
 // of 8, one slice) or, in slices, through the smallest of those that load straight into LDS.
 template <bool PAIRED>
 static int launch_large(const bf16* x, Weight w, void* out, Epilogue ep, int M, int N, int K, hipStream_t stream, int slices = 1, int tile = -1) {

@@ -182,9 +182,10 @@ class DecodeRunner:
 # ----------------------------------------------------------------------------- short prompts
 # Token counts for which prompt steps are captured.  Beyond them the GPU takes as long as the host: 256 rows replayed 7.1 ms,
 # launched one by one 7.3 ms.  Each costs a capture at its first use (some 70 ms, what 200 steps and more save) and scratch memory,
-# so few stand between two.  Of two prompts at the 8B and 4B shapes 96 tokens take 5.06 and 3.79 ms padded to 128, 4.66 and 3.62 in
-# 96 rows (8 and 4 %); without rows of their own 24 tokens padded to 32 take 3.86 and 2.80 against 3.76 and 2.66, 48 to 64 4.25 and
-# 3.41 against 3.93 and 3.10 (8 and 9 %), 80 to 96 4.81 and 3.63 against 4.55 and 3.47, 112 to 128 5.14 and 3.79 against 5.04 and 3.74.
+# so one stands between two powers of two only where it gains 5 % and more on average over the 8B and 4B shapes and eight layers of the 32B
+# one.  Steps of two prompts, padded to the next power of two or count below and in rows of their own, ms: 96 tokens 5.13, 3.85, 2.18 and
+# 4.73, 3.70, 2.01 (6.5 %); 24 3.77, 2.76, 1.88 and 3.66, 2.62, 1.83 (3.7 %), 48 3.96, 3.12, 1.90 and 3.82, 2.95, 1.88 (3.2 %), 80 (to 96) 4.73,
+# 3.70, 2.00 and 4.52, 3.56, 1.92 (4.2 %), 112 5.13, 3.86, 2.18 and 4.92, 3.80, 2.10 (3.0 %).
 PROMPT_ROWS = (16, 32, 64, 96, 128)
 PROMPT_SEQS = (1, 2, 4, 8)             # sequences of the step (one more, for the padding tokens, is added)
 

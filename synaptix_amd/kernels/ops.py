@@ -352,7 +352,7 @@ def _rows_choice(M, N, K, slices):
     if N * K < ROWS_MIN_WEIGHT:
         return None
     for nf in (2, 4, 6):
-        if M > {2: 128, 4: 96, 6: 48}[nf]:
+        if nf == 6 and M > 48:
             continue
         tiles = -(-N // (16 * nf))
         for s in (range(1, 9) if slices is None else (slices,)):
@@ -363,7 +363,7 @@ def _rows_choice(M, N, K, slices):
 
 
 def _tiles_bytes(M, N, K, slices):
-    """The same of the tiles that are taken otherwise."""
+    """The same of the tiles that are taken otherwise (those that load straight into LDS)."""
     tile = 64 if M <= 32 else 128
     return _bytes_a_unit(M, tile, K, slices, -(-N // tile), compute_units(), M <= 32)
 
@@ -374,10 +374,11 @@ def _rows_pay(new, old, M, gated):
     5.7 TB/s.  Where the bytes of one come near the time of the other they hide each other in part only (six groups, a workgroup a unit,
     16 to 48 rows: 36 to 40 us, 10.5 to 12.4 bytes a clock), through registers less than through a ring of LDS buffers, which keeps
     more of W under way beside many rows of x.  So this kernel has to bring in fewer bytes, the fewer the more rows.  Measured, us (this
-    kernel, tiles, ratio of the bytes): gated 24,576 x 4,096 with 24 rows 39.2, 43.7, 0.91, with 48 42.4, 43.0, 0.82, with 64 46.3, 45.7;
-    16,384 x 2,048 with 64 20.5, 22.7, 0.67, with 128 28.7, 27.5, 0.86; 8,192 x 1,024 with 128 14.3, 17.8, 0.71; plain 2,560 x 9,728 with 24
-    11.9, 15.1, 0.68, with 64 17.0, 16.3, 0.85; 6,144 x 2,560 with 32 9.7, 10.2, 0.9; 4,096 x 12,288 with 32 20.5, 19.6, 1.0; 2,048 x 2,048 with 48
-    5.8, 7.5, 0.45, with 128 9.2, 10.6, 0.63; 1,024 x 4,096 with 96 7.8, 10.2, 0.57; 6,144 x 2,048 with 48 10.1, 9.5, 0.82."""
+    kernel, tiles that load straight into LDS, ratio of the bytes): gated 24,576 x 4,096 with 24 rows 39.2, 43.7, 0.91, with 48 42.4, 43.0, 0.82;
+    plain 2,560 x 9,728 with 24 11.9, 15.1, 0.68, with 64 17.0, 16.3, 0.85; 6,144 x 2,560 with 32 9.7, 10.2, 0.9; 4,096 x 12,288 with 32 20.5, 19.6,
+    1.0; 2,048 x 2,048 with 48 5.8, 7.5, 0.45; 6,144 x 2,048 with 48 10.1, 9.5, 0.82.  The bytes of those tiles stand for the streamed ones as
+    well, which gated products take from 17 rows on otherwise: over 78 of 13 gated shapes with 17 to 48 rows what this picks takes 1.9 %
+    longer than the best on average, 1.33 times at the worst (12,288 x 3,072 with 17 rows streamed 21.9, here 16.5)."""
     return new <= (0.95 if M <= 32 and gated else 0.9 if M <= 32 else 0.75 if gated else 0.65) * old
 
 
@@ -882,8 +883,8 @@ DECODE_BIN_SPLITS = 2    # room in a list of bins: twice as many items as rows (
 
 
 def decode_bins(n_seqs, n_kv_heads, heads_a_group=1) -> int:
-    """Over how many places decode attention's work list spreads its items so that every compute unit gets the same share
-    (runtime.decode_bins), or 0 where it is not laid out so: with no more workgroups than compute units, where decode_splits
+    """Over how many places decode attention's work list spreads its items so that compute units get about the same sum of keys, or
+    fewer of them several sequences each where that is estimated faster (runtime.decode_bins), or 0 where it is not laid out so: with no more workgroups than compute units, where decode_splits
     cuts every sequence, where the kv heads do not divide the compute units, where no kernel reads the list (heads_a_group 0) and
     where it takes a kv head's queries in several workgroups (more than 16 of them), which the places do not count.  Also with as
     many rows as places each workgroup has eight waves and a compute unit to itself: 32 rows over 32 places gained 5 to 30 % on unequal lengths and lost 4 to
@@ -896,7 +897,7 @@ def _decode_work(name, counters, items, B, n_splits, n_heads, n_kv_heads):
     """The optional arguments of the decode kernels.  counters: int32, at least B * kv heads * ceil(group / 16),
     zero (the kernel leaves them zero): with them the splits are merged inside the one launch where its grid is
     small enough for that to pay.  items: int32 [4 * B * n_splits + 2 * B], the work list that hands longer
-    sequences more splits (runtime.decode_items lays it out) or every compute unit the same share (runtime.decode_bins)."""
+    sequences more splits (runtime.decode_items lays it out) or compute units about the same sum of keys (runtime.decode_bins)."""
     n_items = 0
     if items is not None:
         _need(items, f"{name}.items", _I32, (4 * B * n_splits + 2 * B,))
