@@ -1663,21 +1663,20 @@ static bool few_rows_streamed(int N, int K, bool packed) {
   return packed && (long)N * K >= 24L << 20 && 8 * direct_groups(64, N) * direct_slices(64, N, K) <= 5L * syn_compute_units();
 }
 
-// Whether a cut product of 65 to 128 or 177 to 256 rows goes through the tiles of 128 x 128 that hold k-tiles of 64 (gemm_direct): where
-// their workgroups, one or two rows of tiles in slices that are a power of two, fill three quarters of the compute units and more, and W
-// has 48 to 96 MB.  Less of it the streamed tiles bring in with fewer partial sums, more of it in longer runs.  What a layer of a prompt
-// step gains over the streamed tiles, us: 6,144 x 4,096 with 4,096 x 12,288 behind it 0.3 with 96 rows, 0.8 with 128 and 192, 4.2 with 256;
-// with 96 and 128 rows 6,144 x 4,096 alone 4.0, 3.8, 6,144 x 6,144 3.0, 2.7, 7,168 x 5,120 2.7, 0.8, 3,072 x 8,192 1.6, 0.6 (with 192 and 256
-// rows from 2.0 less to 2.7 more).  Beyond: 8,192 x 8,192 0.8, 1.2, 4,096 x 14,336 -2.7, -2.8, 6,144 x 16,384 -7.3, -7.5, 8,192 x 28,672 -1.8,
-// -3.5.  Below, or with fewer workgroups: 4,096 x 4,096 -1.5, -2.8, 6,144 x 2,560 -0.5, -2.3, 2,560 x 9,728 (160 of them) -1.4, -2.5.
-// W in plain rows: up to 128 rows whatever W (the product and the sum of its slices, these tiles and streamed: 6,144 x 2,560 with 128 rows 20,
-// 24, 2,560 x 9,728 with 96 26, 27, 4,608 x 3,584 22, 20), above it where they fill the compute units (4,096 x 4,096 with 256 rows 25, 29,
+// Whether a cut product goes through the tiles of 128 x 128 that hold k-tiles of 64 (gemm_direct), in slices that are a power of two.  W in
+// fragment order: 177 to 256 rows, where their workgroups fill three quarters of the compute units and more and W has 48 to 96 MB (less of
+// it the streamed tiles bring in with fewer partial sums, more of it in longer runs).  What a layer of a prompt step gains over the streamed
+// tiles, us: 6,144 x 4,096 with 4,096 x 12,288 behind it 0.8 with 192 rows, 4.2 with 256, 6,144 x 6,144 -1.2, -2.0, 8,192 x 6,144 0.5, 2.2,
+// 7,168 x 5,120 -0.3, 2.7, 3,072 x 8,192 0.2, -0.9; beyond: 4,096 x 14,336 -3.7, -1.8, 6,144 x 16,384 -20, -20, 8,192 x 28,672 -46, -23; below:
+// 4,096 x 4,096 -1.4, -1.0.  (65 to 128 rows gained 1 % of the 8B shape's step on one card and lost 1 to 2 on another.)
+// W in plain rows: 65 to 128 rows whatever W (the product and the sum of its slices, these tiles and streamed: 6,144 x 2,560 with 128 rows 20,
+// 24, 2,560 x 9,728 with 96 26, 27, 4,608 x 3,584 22, 20), 177 to 256 where they fill the compute units (4,096 x 4,096 with 256 rows 25, 29,
 // 8,192 x 4,096 37, 39; 5,120 x 5,120, 160 workgroups, 40, 36).
 static bool direct_cut(int M, int N, int K, bool packed) {
   const long w = (long)N * K, groups = direct_groups(M, N), cus = syn_compute_units();
-  if (!(M > 64 && M <= 128) && !(M > 176 && M <= 256)) return false;
-  if (K % 128 != 0 || groups > cus) return false;
-  if (packed ? w < 24L << 20 || w > 48L << 20 : M <= 128) return !packed;
+  if (K % 128 != 0 || groups > cus || M <= 64 || M > 256) return false;
+  if (M <= 176) return !packed && M <= 128;
+  if (packed && (w < 24L << 20 || w > 48L << 20)) return false;
   return 4 * groups * direct_slices(M, N, K) >= 3 * cus;
 }
 
