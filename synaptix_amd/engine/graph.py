@@ -183,9 +183,9 @@ class DecodeRunner:
 # Token counts for which prompt steps are captured.  Beyond them the GPU takes as long as the host: 256 rows replayed 7.1 ms,
 # launched one by one 7.3 ms.  Each costs a capture at its first use (some 70 ms, what 200 steps and more save) and scratch memory,
 # so one stands between two powers of two only where it gains 5 % and more on average over the 8B and 4B shapes and eight layers of the 32B
-# one.  Steps of two prompts, padded to the next power of two or count below and in rows of their own, ms: 96 tokens 5.13, 3.85, 2.18 and
-# 4.73, 3.70, 2.01 (6.5 %); 24 3.77, 2.76, 1.88 and 3.66, 2.62, 1.83 (3.7 %), 48 3.96, 3.12, 1.90 and 3.82, 2.95, 1.88 (3.2 %), 80 (to 96) 4.73,
-# 3.70, 2.00 and 4.52, 3.56, 1.92 (4.2 %), 112 5.13, 3.86, 2.18 and 4.92, 3.80, 2.10 (3.0 %).
+# one.  Steps of two prompts, padded to the count above that stands and in rows of their own, ms: 96 tokens 5.12, 3.85, 2.18 and 4.72, 3.70,
+# 2.00 (6.6 %); 24 3.78, 2.76, 1.89 and 3.66, 2.62, 1.83 (3.7 %), 48 3.96, 3.12, 1.90 and 3.82, 2.95, 1.89 (3.2 %), 80 4.71, 3.70, 2.00 and 4.49,
+# 3.56, 1.92 (4.2 %), 112 5.13, 3.87, 2.18 and 4.93, 3.81, 2.10 (3.1 %).
 PROMPT_ROWS = (16, 32, 64, 96, 128)
 PROMPT_SEQS = (1, 2, 4, 8)             # sequences of the step (one more, for the padding tokens, is added)
 
