@@ -1702,7 +1702,8 @@ SYN_EXPORT int syn_gemm_cut_slices(int M, int N, int K, int packed) {
 }
 
 // Whether a product that could be rounded to 16 bits hands on its 32-bit sums whatever number of slices is the fastest now: a line that a
-// fit of the tiles' times must not move, since it decides how precise a result is.  (Products that are cut hand them on in any case.)
+// fit of the tiles' times must not move, since it decides how precise a result is.  (Products that are cut hand them on in any case.  Eight
+// layers of the 32B shape with 1,600 tokens, whose q, k and v this concerns: 11.2 ms rounded, 11.4 so, 12.3 when the line was drawn.)
 SYN_EXPORT int syn_gemm_sums_line(int M, int N, int K) { return plan_slices(SUMS_LINE, M, N, K, true) > 1; }
 
 // ------------------------------------------------------------------ entry point
