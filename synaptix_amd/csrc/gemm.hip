@@ -2,8 +2,7 @@
 //
 //   gemm_simt      any shape and type; plain FMA: what the MFMA kernels refuse (K not a multiple of 8, or of 4 in 32 bits;
 //                  unaligned rows).
-//   gemm_f32_few   32-bit, up to 64 rows of a W that is not wide: v_mfma_f32_16x16x4_f32 over W streamed once, K over the waves.
-//   gemm_f32_tiles 32-bit, more rows or a wide W: tiles of 64 x 64, 64 x 32, 32 x 64 or 32 x 32 through LDS.
+//   gemm_f32       32-bit, K a multiple of 4: gemm_f32.hip.
 //   gemm_skinny    bf16, M == 1: the weight matrix is streamed once from HBM through
 //                  v_mfma_f32_16x16x32_bf16; the waves of a workgroup split K and sum in LDS
 //                  (also over paired gate/up rows, with the gated activation as the epilogue).
@@ -498,187 +497,6 @@ static int tile_grid(int M, int N, int BM, int BN) {
   const int PM = tiles_m < 8 ? tiles_m : 8, PN = 4;
   const int panels = ((tiles_m + PM - 1) / PM) * ((tiles_n + PN - 1) / PN);
   return (panels + 7) / 8 * 8 * PM * PN;
-}
-
-// ------------------------------------------------------------------ 32-bit products on the matrix units
-// v_mfma_f32_16x16x4 multiplies and adds in 32 bits, as the plain kernel's fused multiply-adds do, at 256 of them a clock and
-// compute unit (a large library product reaches 149 TFLOP/s here; the plain kernel 20).  Which four k-values a step multiplies
-// is free as long as both operands agree: a lane loads four neighbouring ones (16 bytes) and gives them to four steps one
-// after another.
-// The order of the sums is the same whatever the number of rows, so a row's results do not depend on what else is in the
-// batch: K in chunks of 32, chunk c of class c % 16; the chunks of a class one after another in ascending order, each in eight steps
-// (16 values in four steps of every fourth one, twice); then the sixteen sums in the order of the classes.
-//
-// Up to 64 rows of x and a W that is not wide: bound by reading W, which no cache holds.  A workgroup owns 16 rows of W; its 16 waves take a class
-// each, eight loads of 16 k-values (four with many rows of x) at a time, so that the workgroup has up to 128 KB of W under way,
-// and their partial tiles are added in LDS in the order of the waves.  D[n = 4 (lane / 16) + j][m = lane % 16].
-// W of 2,560 x 9,728: 1 row 1,604 -> 38 us, 16 rows 1,655 -> 52 (plain kernel, this one).  The sums' error against 64 bits is a quarter of the plain kernel's (4.5e-7, 1.8e-6), since a class is a
-// sixteenth of K.
-template <int FM, int U>
-__global__ void __launch_bounds__(16 * SYN_WAVE)
-gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K, int point) {
-  constexpr int WAVES = 16;
-  __shared__ f32x4 part[WAVES][FM > 2 ? 2 : FM][SYN_WAVE];
-  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE, r16 = lane % 16, k4 = 4 * (lane / 16);
-  const int n0 = (int)blockIdx.x * 16;
-  // (rows of W beyond N and of x beyond M repeat the last one: their results are never stored)
-  const float* wr = w + (size_t)min(n0 + r16, N - 1) * K + k4;
-  const float* xr[FM];
-#pragma unroll
-  for (int i = 0; i < FM; ++i) xr[i] = x + (size_t)min(16 * i + r16, M - 1) * K + k4;
-  f32x4 acc[FM];
-#pragma unroll
-  for (int i = 0; i < FM; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = wave * 32; k0 < K; k0 += WAVES * 16 * U) {
-    f32x4 b[U], a[U][FM];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u / 2 * WAVES * 32 + u % 2 * 16;
-      const bool in = k + k4 < K;      // (K is a multiple of 4)
-      b[u] = in ? __builtin_nontemporal_load((const f32x4*)(wr + k)) : zero;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) a[u][i] = in ? *(const f32x4*)(xr[i] + k) : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < FM; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][e], a[u][i][e], acc[i], 0, 0, 0);
-  }
-#pragma unroll
-  for (int i0 = 0; i0 < FM; i0 += 2) {     // two groups of 16 rows of x at a time
-    __syncthreads();
-#pragma unroll
-    for (int i = i0; i < FM && i < i0 + 2; ++i) part[wave][i - i0][lane] = acc[i];
-    __syncthreads();
-    const int i = i0 + wave / 4, j = wave % 4;       // four waves a group, one value of a lane's four each
-    if (wave < 8 && i < FM) {
-      float v = 0.f;
-#pragma unroll
-      for (int q = 0; q < WAVES; ++q) v += part[q][(i - i0) % (FM > 2 ? 2 : FM)][lane][j];
-      const int m = 16 * i + r16, n = n0 + 4 * (lane / 16) + j;
-      if (m < M && n < N) out[(size_t)m * N + n] = point_activation(point, v);
-    }
-  }
-}
-
-// Which tile of a product that the matrix units bound: every XCD gets as many as every other (to one tile), a run of the tiles in
-// bands of at most eight rows of tiles, all bands alike, column after column of a band.  In panels of 8 x 4 (tile_of_workgroup) the
-// XCDs' shares differ by a panel, and all panels of a short last band can go to the same ones: 640 rows of 19,456 x 2,560 837 ->
-// 524 us, 384 rows of 2,560 x 9,728 263 -> 180, 192 rows 180 -> 147.
-__device__ __forceinline__ bool tile_of_share(int M, int N, int BM, int BN, int& tm, int& tn) {
-  const int tiles_n = (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM, tiles = tiles_m * tiles_n;
-  const int bands = (tiles_m + 7) / 8, high = (tiles_m + bands - 1) / bands;
-  const int xcd = (int)blockIdx.x % 8, local = (int)blockIdx.x / 8, more = tiles % 8;
-  if (local >= tiles / 8 + (xcd < more)) return false;
-  const int t = xcd * (tiles / 8) + min(xcd, more) + local, band = t / (high * tiles_n), in_band = t - band * high * tiles_n;
-  const int rows = min(high, tiles_m - band * high);
-  tm = band * high + in_band % rows;
-  tn = in_band / rows;
-  return true;
-}
-
-static int share_grid(int M, int N, int BM, int BN) { return (((M + BM - 1) / BM) * ((N + BN - 1) / BN) + 7) / 8 * 8; }
-
-// More rows, or a wide W: tiles of BM x BN, 4 waves of BM / 2 x BN / 2, k-tiles of 32 in a ring of three LDS buffers that loads
-// fill without passing through registers; a row's eight 16-byte chunks are swizzled as in gemm_direct.  Bound by the matrix units
-// (1,000 rows of 19,456 x 2,560: 121 TFLOP/s of some 150), alone on a compute unit by a k-tile's chain from load to sum (0.5 us a k-tile of
-// 64 x 32, 0.4 of 32 x 32), and with few rows by W (151,936 x 2,560, 1 row: 5.7 TB/s).  Three to six workgroups share a compute
-// unit; 128 x 64 and larger were slower.  A k-tile is a chunk of the order above, and they come class by class.
-// D[n = 4 (lane / 16) + e][m = lane % 16].
-template <int BM, int BN>
-__global__ void __launch_bounds__(256)
-gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K, int point) {
-  constexpr int BK = 32, STAGES = 3, ROWS = BM + BN, RPI = 8, WAVES = 4, PASSES = ROWS / (RPI * WAVES);
-  constexpr int CLASSES = 16, FM = BM / 32, FN = BN / 32;
-  static_assert((BM == 64 || BM == 32) && (BN == 64 || BN == 32), "tile shape");
-  __shared__ __attribute__((aligned(16))) float smem[STAGES * ROWS * BK];
-  const int lane = threadIdx.x % SYN_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE);
-  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * (BN / 2);
-  int tm, tn;
-  if (!tile_of_share(M, N, BM, BN, tm, tn)) return;
-  const int m0 = tm * BM, n0 = tn * BN, nk = (K + BK - 1) / BK;
-  const size_t row_bytes = (size_t)K * sizeof(float);
-  const BufferView vx = buffer_view(x + (size_t)m0 * K, (size_t)(M - m0) * row_bytes);
-  const BufferView vw = buffer_view(w + (size_t)n0 * K, (size_t)(N - n0) * row_bytes);
-  unsigned src[PASSES];
-#pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-    const int row0 = (p * WAVES + wave) * RPI, row = row0 + lane / 8, in = row0 < BM ? row : row - BM;
-    src[p] = (unsigned)((size_t)in * row_bytes + (((lane % 8) ^ (row >> 1)) & 7) * 16);
-  }
-  // (where K is no multiple of 32 the last k-tile also brings values of the next row, which no step below multiplies, and
-  // behind the last row nothing)
-  auto fetch = [&](int kt, int buf) {
-#pragma unroll
-    for (int p = 0; p < PASSES; ++p)
-      buffer_to_lds16(p * WAVES * RPI < BM ? vx : vw, smem + ((size_t)buf * ROWS + (p * WAVES + wave) * RPI) * BK, src[p], kt * BK * 4);
-  };
-  struct Place {      // in the order of the k-tiles
-    int kt, of_class;
-  };
-  auto next = [&](Place p) { return p.kt + CLASSES < nk ? Place{p.kt + CLASSES, p.of_class} : Place{p.of_class + 1, p.of_class + 1}; };
-  f32x4 acc[FM][FN] = {}, total[FM][FN] = {};
-  Place load = {0, 0}, at = {0, 0};
-#pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < nk) fetch(load.kt, t), load = next(load);
-  const int r16 = lane % 16, q = lane / 16;
-  for (int i = 0; i < nk; ++i) {
-    // this wave's loads of the i-th k-tile have landed (all but the youngest tile's), and behind the barrier everyone's
-    if (i + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f70 | PASSES);
-    else __builtin_amdgcn_s_waitcnt(0x0f70);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (i + STAGES - 1 < nk) fetch(load.kt, (i + STAGES - 1) % STAGES), load = next(load);   // that buffer was read before the barrier
-    const float* xs = smem + (size_t)(i % STAGES) * ROWS * BK;
-    const float* ws = xs + BM * BK;
-    const int steps = min(BK, K - at.kt * BK);
-    auto sixteen = [&](int c, bool in) {     // sixteen k-values: four chunks of 4, one for each quarter of the wave
-      f32x4 a[FM], b[FN];
-#pragma unroll
-      for (int j = 0; j < FM; ++j) a[j] = *(const f32x4*)(xs + (wm + 16 * j + r16) * BK + (((c + q) ^ ((wm + 16 * j + r16) >> 1)) & 7) * 4);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) b[j] = *(const f32x4*)(ws + (wn + 16 * j + r16) * BK + (((c + q) ^ ((BM + wn + 16 * j + r16) >> 1)) & 7) * 4);
-      if (!in) {
-#pragma unroll
-        for (int j = 0; j < FM; ++j) a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < FN; ++j) b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int ia = 0; ia < FM; ++ia)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[ia][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][e], a[ia][e], acc[ia][j], 0, 0, 0);
-    };
-    if (steps == BK) {
-      sixteen(0, true), sixteen(4, true);
-    } else {
-      for (int c = 0; 4 * c < steps; c += 4) sixteen(c, 4 * (c + q) < steps);
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this tile's reads are done when the next barrier is reached
-    const Place behind = next(at);
-    if (behind.of_class != at.of_class) {
-#pragma unroll
-      for (int ia = 0; ia < FM; ++ia)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) total[ia][j] += acc[ia][j], acc[ia][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    at = behind;
-  }
-#pragma unroll
-  for (int ia = 0; ia < FM; ++ia)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + wm + 16 * ia + r16, n = n0 + wn + 16 * j + 4 * q + e;
-        if (m < M && n < N) out[(size_t)m * N + n] = point_activation(point, total[ia][j][e]);
-      }
 }
 
 // The accumulators of a wave (TM x TN tiles of MFMA 32x32: D[m = 8*(e/4) + 4*(lane/32) + e%4][n = lane%32])
@@ -1714,8 +1532,10 @@ SYN_EXPORT int syn_gemm_sums_line(int M, int N, int K) { return plan_slices(SUMS
 // load straight into LDS; the other kernels read plain rows only.
 // point: what the finished sums pass before they are stored (point_activation; one slice).
 // tile: -1, or for tests and measurements one of STREAMED.tiles, whatever the rules below would take (bf16 operands).
+// scratch: working memory for 32-bit operands (syn_gemm_f32_scratch floats, or null where that is none).
+int launch_gemm_f32(const float* x, const float* w, float* out, int M, int N, int K, int point, float* scratch, int64_t scratch_floats, hipStream_t stream);   // gemm_f32.hip
 SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int M, int N, int K, int force_simt,
-                        int slices, int w_packed, int point, int tile, int rows, hipStream_t stream) {
+                        int slices, int w_packed, int point, int tile, int rows, float* scratch, int64_t scratch_floats, hipStream_t stream) {
   SYN_CHECK(tile < 0 || (dtype != 0 && !force_simt && K % 64 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0),
             "gemm: the streamed tiles take aligned bf16 operands and a K that is a multiple of 64 (K = %d)", K);
   SYN_CHECK(point >= 0 && point < SYN_POINT_COUNT && (point == SYN_POINT_NONE || slices == 1),
@@ -1730,43 +1550,8 @@ SYN_EXPORT int syn_gemm(const void* x, const void* w, void* out, int dtype, int 
   if (dtype == 0) {
     const float *xf = (const float*)x, *wf = (const float*)w;
     float* of = (float*)out;
-    const bool loads16 = !force_simt && K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
-    // Few rows take the tiles from where their W makes tiles for most of the chip: up to 16 rows from 64 rows of W a compute unit on
-    // (few-row kernel, tiles, at 1 row: 12,288 x 1,024 16.6, 19.6 us; 19,456 x 2,560 59, 56; 151,936 x 2,560 425, 274), up to 64 from
-    // 24 on (17 rows: 4,096 x 4,096 28, 54; 6,144 x 2,560 37, 36; 19,456 x 2,560 91, 58; 33 rows: 4,096 x 4,096 45, 55; 6,144 x 2,560
-    // 63, 42; 64 rows: 2,560 x 9,728 132, 124; 4,096 x 4,096 56, 55).  17 and 18 rows from 32 on where K is a multiple of 1,024: all
-    // turns of the few-row kernel's loads are full then (17 rows: 6,144 x 4,096 48, 52; 8,192 x 4,096 50, 53; 6,144 x 8,192 96, 101;
-    // 9,728 x 4,096 69, 64; 22 rows: 6,144 x 4,096 53, 52).
-    const long cus = syn_compute_units(), across = (N + 31) / 32, down = (M + 31) / 32;
-    if (loads16 && (M <= 16 ? N < 64 * cus : M <= 64 && N < (M <= 18 && K % 1024 == 0 ? 32 * cus + 1 : 24 * cus))) {
-      const int groups = (N + 15) / 16;
-      if (M <= 16) gemm_f32_few_kernel<1, 8><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else if (M <= 32) gemm_f32_few_kernel<2, 4><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else gemm_f32_few_kernel<4, 4><<<groups, 16 * SYN_WAVE, 0, stream>>>(xf, wf, of, M, N, K, point);
-      SYN_LAUNCH_CHECK("gemm_f32_few");
-      return 0;
-    }
-    if (loads16) {
-      // 64 x 64, the fastest for its size, where it goes round at least three times and no rounds of the halves are fewer by more than
-      // the 2.5 % that it is faster by; three workgroups share a compute unit, so a fourth round runs alone (64 x 64, the halves: 3
-      // rounds 6,144 x 2,560 with 490 rows 138 us, 141, 4,096 x 12,288 with 768 642, 669; 4 rounds 4,096 x 12,288 with 1,024 854, 839; 48
-      // rounds 24,576 x 4,096 with 2,000 3,240, 3,346).  32 x 32 where each has a compute unit to itself, so that a tile's time is the
-      // product's (65 rows, 2,560 x 9,728: 124 us, 149 in 32 x 64, 147 in 64 x 32).  64 x 32 in up to four rounds of an even number of 32
-      // rows (384 rows: 181, 184) and for two of them, whose W is read once so (151,936 x 2,560 with 33 rows: 455, 465).  Else 32 x 64,
-      // which asks L2 for less of W's share and pads to 32 rows only (65 rows, 19,456 x 2,560: 97, 64 x 32 133; 256 rows 227, 234).
-      const long square = ((M + 63) / 64 * ((N + 63) / 64) + cus - 1) / cus;
-      const long slim = ((M + 63) / 64 * across + cus - 1) / cus, flat = (down * ((N + 63) / 64) + cus - 1) / cus;
-      if (square >= 3 && square != 4 && 39 * square <= 20 * (slim < flat ? slim : flat))
-        gemm_f32_tiles_kernel<64, 64><<<share_grid(M, N, 64, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else if (down * across <= cus)
-        gemm_f32_tiles_kernel<32, 32><<<share_grid(M, N, 32, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else if (down == 2 || (down % 2 == 0 && down / 2 * across <= 4 * cus))
-        gemm_f32_tiles_kernel<64, 32><<<share_grid(M, N, 64, 32), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
-      else
-        gemm_f32_tiles_kernel<32, 64><<<share_grid(M, N, 32, 64), 256, 0, stream>>>(xf, wf, of, M, N, K, point);
-      SYN_LAUNCH_CHECK("gemm_f32_tiles");
-      return 0;
-    }
+    if (!force_simt && K % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0)
+      return launch_gemm_f32(xf, wf, of, M, N, K, point, scratch, scratch_floats, stream);
     gemm_simt_kernel<float, float><<<simt_grid, 256, 0, stream>>>(xf, wf, of, M, N, K, point);
     SYN_LAUNCH_CHECK("gemm_simt");
     return 0;

@@ -29,7 +29,7 @@ ARCH = "gfx950"
 FLAGS = ["-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden"]
-CORE_SOURCES = ["elementwise.hip", "sampling.hip", "gemm.hip", "attention_f32.hip", "probes.hip", "streams.hip",
+CORE_SOURCES = ["elementwise.hip", "sampling.hip", "gemm.hip", "gemm_f32.hip", "attention_f32.hip", "probes.hip", "streams.hip",
                 "attention_window.hip", "matrix_memory.hip", "grouped.hip", "latent.hip", "latent_attention.hip", "recurrent.hip", "block_f32.hip"]
 RUNTIME_SOURCES = ["runtime.cpp"]
 REF_SOURCES = ["ref/ref_kernels.cpp"]          # the kernels' plain C++ twins (host code)

@@ -323,8 +323,19 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
     else:
         _need(out, "gemm.out", (_BF16, _F32), (M, N))
         code = 2 if out.dtype == _F32 else 1
+    floats = _f32_floats(M, N, K) if code == 0 and not force_simt else 0
+    scratch = torch.empty(floats, dtype=_F32, device=x.device) if floats else None
     _call(load_library("core"), "syn_gemm", _ptr(x), _ptr(w), _ptr(out), code, M, N, K, 1 if force_simt else 0,
-          slices, 1 if packed else 0, point_of, tile, rows, _stream())
+          slices, 1 if packed else 0, point_of, tile, rows, _ptr(scratch), ctypes.c_int64(floats), _stream())
+
+
+@functools.lru_cache(maxsize=4096)
+def _f32_floats(M, N, K) -> int:
+    """Floats of working memory of a 32-bit product: parts of x, and sums over parts of K."""
+    fn = load_library("core").syn_gemm_f32_scratch
+    fn.restype = ctypes.c_int64
+    return fn(M, N, K)
+
 
 
 # Products of up to this many rows over a weight in fragment order may take the kernel whose operands go straight to registers

@@ -270,6 +270,57 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops, N, K):
             assert torch.equal(out, whole[lo:lo + m]), (m, lo)
 
 
+# which kernel these take: few rows whole and in blocks of 16; tiles of 16 x 64, 32 x 64, 32 x 128, 64 x 64 and 64 x 128, whole and with K cut;
+# more rows than the parts of x are kept for at a time; K that ends inside a chunk, a class and a group
+F32_EDGES = [(16, 1000, 4100), (64, 130, 1000), (33, 6148, 516), (16, 6144, 2560), (17, 2564, 4096), (31, 19460, 100), (96, 19456, 260),
+             (65, 2570, 1028), (128, 2560, 2048), (300, 2561, 36), (490, 2560, 516), (300, 19460, 68), (2049, 70, 132), (2300, 1100, 64)]
+
+
+@pytest.mark.parametrize("M,N,K", F32_EDGES)
+def test_gemm_f32_in_parts_is_as_exact_as_32_bit_steps(ops, M, N, K):
+    """Operands of mixed sizes through every kernel and rule of the 32-bit products: each result within what a chain of K / 32 + 40 rounded
+    steps of the sum of magnitudes allows, the whole no further from 64 bits than fused multiply-adds, and a row's bits those of the row alone."""
+    x, w = rnd((M, K), 31), rnd((N, K), 32)
+    x[:, ::3] *= 1e-4
+    w[::5] *= 300.0
+    out = torch.full((M, N), float("nan"), device=DEV)
+    xd, wd = x.to(DEV), w.to(DEV)
+    ops.gemm(xd, wd, out)
+    plain = torch.empty((M, N), device=DEV)
+    ops.gemm(xd, wd, plain, force_simt=True)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    diff = (out.cpu().double() - want).abs()
+    assert bool((diff <= 2.0 ** -23 * (K / 32 + 40) * size).all()), float((diff / size).max())
+    assert float(diff.norm()) <= float((plain.cpu().double() - want).norm()) + 1e-8 * float(want.norm())
+    one = torch.empty((1, N), device=DEV)
+    for m in (0, M // 2, M - 1):
+        ops.gemm(xd[m:m + 1].contiguous(), wd, one)
+        assert torch.equal(out[m:m + 1], one), m
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 100, 260), (17, 6144, 1024), (96, 2560, 2048), (300, 2561, 36), (490, 19460, 68)])
+def test_gemm_f32_keeps_what_is_no_number_and_what_is_large_or_small(ops, M, N, K):
+    """Infinities and NaN in x and W give what fused multiply-adds give, in their rows and columns only; the largest numbers, which round to
+    an infinity in 16 bits, and rows of numbers whose parts have no 16-bit form stay what they are."""
+    x, w = rnd((M, K), 33), rnd((N, K), 34)
+    x[0, 1], x[1, K - 1], x[2, 0] = float("inf"), float("nan"), float("-inf")
+    w[5, K // 2], w[7, :] = float("inf"), 0.0
+    big = torch.finfo(F32).max
+    x[M - 1], w[9] = 0.0, 0.0
+    x[M - 1, K - 4], w[9, K - 4] = big, 0.5
+    out, plain = torch.empty((M, N), device=DEV), torch.empty((M, N), device=DEV)
+    ops.gemm(x.to(DEV), w.to(DEV), out)
+    ops.gemm(x.to(DEV), w.to(DEV), plain, force_simt=True)
+    out, plain = out.cpu(), plain.cpu()
+    assert torch.equal(out.isnan(), plain.isnan()) and torch.equal(out.isposinf(), plain.isposinf()) and torch.equal(out.isneginf(), plain.isneginf())
+    assert float(out[M - 1, 9]) == 0.5 * big and bool(torch.isnan(out[0, 7])) and not bool(torch.isfinite(out[:3]).any() and torch.isfinite(out[1]).any())
+    small = rnd((M, K), 35) * 1e-36
+    ops.gemm(small.to(DEV), w[:5].contiguous().to(DEV), out := torch.empty((M, 5), device=DEV))
+    want = small.double() @ w[:5].double().T
+    # (a chain of K fused steps of 2^-24 each; the matrix units alone, which take parts below 2^-126 for zero, are off by 2.5e-5)
+    assert float((out.cpu().double() - want).norm() / want.norm()) < 2.0 ** -24 * K
+
+
 @pytest.mark.parametrize("nh,nkv,hd,window", [(8, 2, 64, 0), (8, 4, 32, 100), (4, 4, 6, 0), (8, 1, 128, 64)])
 def test_attention_f32_does_not_depend_on_the_batch(ops, nh, nkv, hd, window):
     """Many tokens (a wave a head) and few of the same (the keys over four waves): the same bits."""
