@@ -471,11 +471,13 @@ __global__ void qk_norm_rope_kv_write_kernel(const TIn* __restrict__ qkv, int n_
 // The same for the q and k heads of bf16 rows whose head size is 8 * LPH with LPH = 2, 4, .. 32 lanes
 // a head and whose rotation covers the whole head (or is absent): a lane holds 8 values of a head
 // (16-byte load and store), the sum of squares is reduced over the LPH lanes of the head, and the
-// partner of a rotated pair sits LPH / 2 lanes away.  A block takes 256 / LPH heads of four tokens each, counted on through the
+// partner of a rotated pair sits LPH / 2 lanes away.  A block takes 256 / LPH heads of TPB tokens each, counted on through the
 // heads and then the tokens, so that only the last block may hold idle lanes.
 // PARTS: the rows come as n_parts float partial sums [n_parts][tokens][heads * HD] of a product cut
 // along K (part_stride elements apart), which are added first, in their order.
-template <int LPH, bool PARTS>
+// TPB, the tokens a lane takes with their loads in flight together: 4 where they fill the chip, which bounds them by memory, else 1, with four
+// parts in flight, since a lane's trips to memory one after another are then what it takes (qkv_tokens_a_lane).
+template <int LPH, bool PARTS, int TPB>
 __device__ __forceinline__ void
 qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t part_stride,
               bf16* __restrict__ q_out, bf16* __restrict__ k_pages,
@@ -484,7 +486,7 @@ qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t pa
                 int gain_is_f32, float gain_offset, float eps, const float* __restrict__ cos_t,
                 const float* __restrict__ sin_t, int n_tokens, int nh, int nkv, int n_active) {
   constexpr int HD = LPH * 8, HPB = 256 / LPH, half = HD / 2;
-  constexpr int TPB = 4;  // tokens a block takes, their loads in flight together
+  constexpr int PB = TPB == 1 ? 4 : 1;      // parts whose loads are in flight together
   const uint32_t item = (uint32_t)block * HPB + threadIdx.x / LPH;
   const bool idle = item >= (uint32_t)((n_tokens + TPB - 1) / TPB) * (uint32_t)n_active;
   const int block_x = idle ? 0 : item / (uint32_t)n_active;    // idle lanes repeat the first head: shuffles need them
@@ -508,26 +510,33 @@ qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t pa
   float val[TPB][8];
   int pos[TPB];
   float4 cs[TPB][2], sn[TPB][2];
+  int seq[TPB];
   if constexpr (PARTS) {
 #pragma unroll
     for (int t = 0; t < TPB; ++t) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) val[t][e] = 0.f;
-      pos[t] = tok_pos[min(block_x * TPB + t, n_tokens - 1)];
+      pos[t] = tok_pos[min(block_x * TPB + t, n_tokens - 1)], seq[t] = tok_seq[min(block_x * TPB + t, n_tokens - 1)];
     }
-    for (int p = 0; p < n_parts; ++p) {
-      float4 lo4[TPB], hi4[TPB];     // the tokens' loads of one part in flight together
+    for (int p0 = 0; p0 < n_parts; p0 += PB) {
+      float4 lo4[PB][TPB], hi4[PB][TPB];
 #pragma unroll
-      for (int t = 0; t < TPB; ++t) {
-        const int tok = min(block_x * TPB + t, n_tokens - 1);
-        const float4* src = (const float4*)((const float*)qkv_in + (size_t)p * part_stride +
-                                            ((size_t)tok * (nh + 2 * nkv) + head) * HD + c * 8);
-        lo4[t] = src[0], hi4[t] = src[1];
-      }
+      for (int p = 0; p < PB; ++p)
 #pragma unroll
-      for (int t = 0; t < TPB; ++t) {
-        val[t][0] += lo4[t].x, val[t][1] += lo4[t].y, val[t][2] += lo4[t].z, val[t][3] += lo4[t].w;
-        val[t][4] += hi4[t].x, val[t][5] += hi4[t].y, val[t][6] += hi4[t].z, val[t][7] += hi4[t].w;
+        for (int t = 0; t < TPB; ++t) {
+          const int tok = min(block_x * TPB + t, n_tokens - 1);
+          const float4* src = (const float4*)((const float*)qkv_in + (size_t)min(p0 + p, n_parts - 1) * part_stride +
+                                              ((size_t)tok * (nh + 2 * nkv) + head) * HD + c * 8);
+          lo4[p][t] = src[0], hi4[p][t] = src[1];
+        }
+#pragma unroll
+      for (int p = 0; p < PB; ++p) {
+        if (p0 + p >= n_parts) break;      // (the same for all lanes)
+#pragma unroll
+        for (int t = 0; t < TPB; ++t) {
+          val[t][0] += lo4[p][t].x, val[t][1] += lo4[p][t].y, val[t][2] += lo4[p][t].z, val[t][3] += lo4[p][t].w;
+          val[t][4] += hi4[p][t].x, val[t][5] += hi4[p][t].y, val[t][6] += hi4[p][t].z, val[t][7] += hi4[p][t].w;
+        }
       }
     }
   } else {
@@ -536,12 +545,17 @@ qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t pa
     for (int t = 0; t < TPB; ++t) {
       const int tok = min(block_x * TPB + t, n_tokens - 1);
       raw[t] = *(const bf16x8*)((const bf16*)qkv_in + ((size_t)tok * (nh + 2 * nkv) + head) * HD + c * 8);
-      pos[t] = tok_pos[tok];
+      pos[t] = tok_pos[tok], seq[t] = tok_seq[tok];
     }
 #pragma unroll
     for (int t = 0; t < TPB; ++t)
 #pragma unroll
       for (int e = 0; e < 8; ++e) val[t][e] = (float)raw[t][e];
+  }
+  int page[TPB];      // (asked for beside the angles, not behind the norm)
+  if (!is_q) {
+#pragma unroll
+    for (int t = 0; t < TPB; ++t) page[t] = page_table[(size_t)seq[t] * table_stride + pos[t] / SYN_PAGE];
   }
   if (cos_t) {
 #pragma unroll
@@ -584,8 +598,7 @@ qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t pa
     if (is_q) {
       *(bf16x8*)(q_out + ((size_t)tok * nh + head) * HD + c * 8) = o;
     } else {
-      const int page = page_table[(size_t)tok_seq[tok] * table_stride + pos[t] / SYN_PAGE];
-      *(bf16x8*)(k_pages + (((size_t)page * nkv + (head - nh)) * SYN_PAGE + pos[t] % SYN_PAGE) * HD + c * 8) = o;
+      *(bf16x8*)(k_pages + (((size_t)page[t] * nkv + (head - nh)) * SYN_PAGE + pos[t] % SYN_PAGE) * HD + c * 8) = o;
     }
   }
 }
@@ -598,7 +611,7 @@ qk_heads_part(int block, const void* __restrict__ qkv_in, int n_parts, size_t pa
 // Bound by memory.  (64 tokens x 32 dims through LDS, 64 bytes of a row a load and 2 bytes a lane a store, before: 41,028 tokens of 32 +
 // 8 + 8 heads of 128 in 16 sequences, q and k with their norm included, 320 -> 248 us or 4.1 TB/s, 2,048 tokens of 64 + 8 + 8 28.0 -> 24.2,
 // of 32 + 8 + 8 19.1 -> 18.0; the q heads alone 149 and 20 us.)
-template <bool PARTS>   // as for qk_heads_part
+template <bool PARTS, int PB>   // PARTS as for qk_heads_part, PB of them in flight together
 __device__ __forceinline__ void
 v_octets_write_part(int group, int chunk, const void* __restrict__ qkv_in, int n_parts, size_t part_stride,
                     bf16* __restrict__ v_pages, const int* __restrict__ page_table, int table_stride,
@@ -633,13 +646,20 @@ v_octets_write_part(int group, int chunk, const void* __restrict__ qkv_in, int n
       float2 sum[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) sum[i] = make_float2(0.f, 0.f);
-      for (int p = 0; p < n_parts; ++p) {
-        float2 part[8];
+      for (int p0 = 0; p0 < n_parts; p0 += PB) {
+        float2 part[PB][8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          part[i] = (which >> i & 1) ? *(const float2*)((const float*)qkv_in + (size_t)p * part_stride + (first + i) * row + column) : make_float2(0.f, 0.f);
+        for (int p = 0; p < PB; ++p)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sum[i].x += part[i].x, sum[i].y += part[i].y;
+          for (int i = 0; i < 8; ++i)
+            part[p][i] = (which >> i & 1) ? *(const float2*)((const float*)qkv_in + (size_t)min(p0 + p, n_parts - 1) * part_stride + (first + i) * row + column)
+                                          : make_float2(0.f, 0.f);
+#pragma unroll
+        for (int p = 0; p < PB; ++p) {
+          if (p0 + p >= n_parts) break;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sum[i].x += part[p][i].x, sum[i].y += part[p][i].y;
+        }
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -682,7 +702,7 @@ v_octets_write_part(int group, int chunk, const void* __restrict__ qkv_in, int n
 
 // Both in one launch: the first n_qk workgroups take the q and k heads, the others the v heads, a wave 8 tokens and one of v_chunks
 // (none where the layer writes no cache).
-template <int LPH, bool PARTS>
+template <int LPH, bool PARTS, int TPB>
 __global__ void __launch_bounds__(256)
 qkv_prompt_kernel(int n_qk, int v_chunks, const void* __restrict__ qkv, int n_parts, size_t part_stride,
                   bf16* __restrict__ q_out, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,
@@ -692,15 +712,24 @@ qkv_prompt_kernel(int n_qk, int v_chunks, const void* __restrict__ qkv, int n_pa
                   const float* __restrict__ sin_t, int n_tokens, int nh, int nkv, int n_active) {
   const int b = blockIdx.x;
   if (b < n_qk) {
-    qk_heads_part<LPH, PARTS>(b, qkv, n_parts, part_stride, q_out, k_pages, page_table, table_stride, tok_seq, tok_pos, q_gain, k_gain,
+    qk_heads_part<LPH, PARTS, TPB>(b, qkv, n_parts, part_stride, q_out, k_pages, page_table, table_stride, tok_seq, tok_pos, q_gain, k_gain,
                               gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh, nkv, n_active);
   } else {
     const long c = (long)(b - n_qk) * (256 / SYN_WAVE) + threadIdx.x / SYN_WAVE;
     const int group = (int)(c / v_chunks), chunk = (int)(c % v_chunks);
     if (group * 8L >= n_tokens) return;
-    v_octets_write_part<PARTS>(group, chunk, qkv, n_parts, part_stride, v_pages, page_table, table_stride, tok_seq, tok_pos,
+    v_octets_write_part<PARTS, TPB == 1 ? 4 : 1>(group, chunk, qkv, n_parts, part_stride, v_pages, page_table, table_stride, tok_seq, tok_pos,
                                n_tokens, nh, nkv, LPH * 8);
   }
+}
+
+// Tokens a lane of qk_heads_part: one at a time (and, of partial sums, four parts) where what counts are a lane's trips to memory, four
+// where memory does.  Four and one, us, 32 + 8 + 8 heads of 128: of bf16 rows 96 tokens 4.6, 3.0, 2,048 13.3, 12.1, 4,096 21.7, 21.9, 8,192 44.9,
+// 47.9, 41,000 205, 230; of two parts 96 5.5, 3.5, 512 9.3, 8.2, 2,048 28.4, 28.0, 8,192 105, 99; of four 96 8.9, 4.9, 256 9.7, 6.9, 512 12.8, 11.4, 768
+// 18.6, 19.7; of eight 96 13.3, 6.8, 256 14.6, 10.5.  (Before, all four: 5.0, 6.0, 9.3 and 13.6 for 96 tokens of rows and of 2, 4 and 8 parts.)
+static int qkv_tokens_a_lane(int n_tokens, int n_active, int heads_a_block, int n_parts) {
+  const long blocks = (long)n_tokens * n_active / heads_a_block;
+  return (n_parts == 0 ? blocks <= 8192 : n_parts <= 2 || blocks * n_parts <= 5120) ? 1 : 4;
 }
 
 SYN_EXPORT int syn_qk_norm_rope_kv_write(const void* qkv, int n_parts, void* q_out, void* k_pages, void* v_pages,
@@ -716,29 +745,30 @@ SYN_EXPORT int syn_qk_norm_rope_kv_write(const void* qkv, int n_parts, void* q_o
   SYN_CHECK(n_parts >= 0 && n_parts <= 64, "qk_norm_rope_kv_write: %d partial sums", n_parts);
   // prompts in bf16: the kernels that move 16 bytes a lane, where the head size and the rotation allow them
   const int lph = hd / 8;
-  // (partial sums of up to 64 tokens stay with the kernel below, one wave a head: measured a little faster there)
-  const bool fast = !is_f32 && (n_parts == 0 || n_tokens > 64) && hd % 8 == 0 && lph >= 2 && lph <= 32 && (lph & (lph - 1)) == 0 &&
+  // (more than four partial sums of up to 64 tokens stay with the kernel below, one wave a head, which asks for all of them at once: 32 tokens of
+  // 32 + 8 + 8 heads of 128 in 8 parts 4.5 us, in the other one 5.3; in 4 parts 4.0 and 3.6, in 2 3.8 and 3.1)
+  const bool fast = !is_f32 && (n_parts <= 4 || n_tokens > 64) && hd % 8 == 0 && lph >= 2 && lph <= 32 && (lph & (lph - 1)) == 0 &&
                     (cos_t == nullptr || rot == hd) && (uintptr_t)qkv % 16 == 0 && (uintptr_t)q_out % 16 == 0 &&
                     (uintptr_t)k_pages % 16 == 0 && (uintptr_t)q_gain % 16 == 0 && (uintptr_t)k_gain % 16 == 0 &&
                     (uintptr_t)cos_t % 16 == 0 && (uintptr_t)sin_t % 16 == 0;
   if (fast) {
     const int n_active = write_kv ? nh + nkv : nh;
     const int hpb = 256 / lph;
-    const long n_qk = (((long)n_tokens + 3) / 4 * n_active + hpb - 1) / hpb, v_chunks = (nkv * hd + 127) / 128;
+    const int tpb = qkv_tokens_a_lane(n_tokens, n_active, hpb, n_parts);
+    const long n_qk = (((long)n_tokens + tpb - 1) / tpb * n_active + hpb - 1) / hpb, v_chunks = (nkv * hd + 127) / 128;
     const long v_blocks = write_kv ? (((long)n_tokens + 7) / 8 * v_chunks + 3) / 4 : 0;
     const size_t part_stride = (size_t)n_tokens * (nh + 2 * nkv) * hd;
     const long grid = n_qk + v_blocks;
     SYN_CHECK(grid <= 0x7fffffffL, "qk_norm_rope_kv_write: %d tokens are too many for one launch", n_tokens);
-#define SYN_QKV(L)                                                                                                  \
-  if (n_parts > 0)                                                                                                  \
-    qkv_prompt_kernel<L, true><<<(unsigned)grid, 256, 0, stream>>>(                                                 \
-        (int)n_qk, (int)v_chunks, qkv, n_parts, part_stride, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table,       \
-        table_stride, tok_seq, tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh,  \
-        nkv, n_active);                                                                                             \
-  else                                                                                                              \
-    qkv_prompt_kernel<L, false><<<(unsigned)grid, 256, 0, stream>>>(                                                \
-        (int)n_qk, (int)v_chunks, qkv, 0, 0, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table, table_stride, tok_seq, \
-        tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh, nkv, n_active)
+#define SYN_QKV_AS(L, P, T)                                                                                          \
+  qkv_prompt_kernel<L, P, T><<<(unsigned)grid, 256, 0, stream>>>(                                                   \
+      (int)n_qk, (int)v_chunks, qkv, n_parts, part_stride, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages, page_table, table_stride, \
+      tok_seq, tok_pos, q_gain, k_gain, gain_is_f32, gain_offset, eps, cos_t, sin_t, n_tokens, nh, nkv, n_active)
+#define SYN_QKV(L)                                  \
+  if (n_parts > 0 && tpb == 1) SYN_QKV_AS(L, true, 1);  \
+  else if (n_parts > 0) SYN_QKV_AS(L, true, 4);         \
+  else if (tpb == 1) SYN_QKV_AS(L, false, 1);           \
+  else SYN_QKV_AS(L, false, 4)
     switch (lph) {
       case 2: SYN_QKV(2); break;
       case 4: SYN_QKV(4); break;
@@ -747,6 +777,7 @@ SYN_EXPORT int syn_qk_norm_rope_kv_write(const void* qkv, int n_parts, void* q_o
       default: SYN_QKV(32); break;
     }
 #undef SYN_QKV
+#undef SYN_QKV_AS
     SYN_LAUNCH_CHECK("qkv_prompt");
     return 0;
   }

@@ -1134,6 +1134,41 @@ def test_qk_norm_rope_kv_write(ops, dtype, nh, nkv, hd, rot, norm):
     close(qd, qw, what="q without cache write", **tol)
 
 
+@pytest.mark.parametrize("parts", [0, 2, 3, 4, 5])
+def test_prompt_intake_has_the_same_bits_with_one_and_four_tokens_a_lane(ops, parts):
+    """2,801 tokens at once (four tokens a lane, but for two parts) and in pieces of 401, 100 and 37 (one a lane, or up to 64 tokens in more
+    than four parts a wave a head, which adds a head's squares in another order): the same q, keys and values."""
+    nh, nkv, hd, N = 40, 8, 128, 2801
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rows = torch.randn(((parts,) if parts else ()) + (N, (nh + 2 * nkv) * hd), generator=g, device=DEV)
+    rows = rows if parts else rows.to(BF16)
+    gain = (1 + 0.1 * rnd((hd,), 22)).to(BF16).to(DEV)
+    cos, sin = torch.randn(3000, hd // 2, generator=g, device=DEV), torch.randn(3000, hd // 2, generator=g, device=DEV)
+    pages = (N + 63) // 64
+    table = torch.randperm(pages, generator=torch.Generator().manual_seed(1)).to(I32)[None].to(DEV)
+    pos, seq = torch.arange(N, dtype=I32, device=DEV), torch.zeros(N, dtype=I32, device=DEV)
+
+    def run(piece):
+        q = torch.full((N, nh * hd), float("nan"), dtype=BF16, device=DEV)
+        k, v = torch.zeros((pages, nkv, 64, hd), dtype=BF16, device=DEV), torch.zeros((pages, nkv, hd, 64), dtype=BF16, device=DEV)
+        for a in range(0, N, piece):
+            ops.qk_norm_rope_kv_write(rows[..., a:a + piece, :].contiguous(), q[a:a + piece], k, v, table, seq[a:a + piece], pos[a:a + piece], gain, gain,
+                                      1e-5, cos, sin, nh, nkv, hd)
+        return q, k, v
+    whole = run(N)
+    assert not bool(torch.isnan(whole[0]).any())
+    for piece in (401, 100, 37):
+        got = run(piece)
+        assert torch.equal(got[2], whole[2]), piece
+        for a, b in zip(got[:2], whole[:2]):
+            if parts > 4 and piece <= 64:
+                # another order of 128 squares moves a head's factor by 2^-20 at most, so a value by that of the two products it is the
+                # difference of (below 16 each), and to the next number of 16 bits (2^-7 of it at most)
+                close(a, b, 2.0 ** -15, 2.0 ** -7, "q and k in more than four parts")
+            else:
+                assert torch.equal(a, b), piece
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 16), (5, 3, 64), (8, 2, 128), (2, 3, 256), (40, 8, 128)])
 @pytest.mark.parametrize("step", ["one", "eight", "ragged", "singles", "gaps", "long"])
 def test_values_of_a_prompt_step_in_pieces_of_eight(ops, step, nh, nkv, hd):
