@@ -1549,16 +1549,25 @@ def diff_heads(a, out, lam, eps, post, n_kv_heads, heads_per_kv, vdim):
 
 # ----------------------------------------------------------------------------- sampling
 
+def _need_tokens(out, name, n_rows):
+    """Token ids on the device, or in pinned host memory, which the kernels write to as well (there when the stream has been waited for)."""
+    if isinstance(out, torch.Tensor) and out.device.type == "cpu" and out.is_pinned():
+        if out.dtype is not _I32 or tuple(out.shape) != (n_rows,) or not out.is_contiguous():
+            raise KernelError(f"{name}: {list(out.shape)} of {out.dtype}, expected int32 [{n_rows}]")
+        return
+    _need(out, name, _I32, (n_rows,))
+
+
 def sample_rows(logits, temperature, uniform, out):
     """out[r] = argmax (last of equal maxima) where temperature[r] <= 0 or temperature is None,
     else a draw from softmax(logits[r] / temperature[r]) by inverse CDF with uniform[r] (-inf is never drawn where
-    anything else is left)."""
+    anything else is left).  out [R] int32 on the device or in pinned host memory."""
     _need(logits, "sample_rows.logits", _F32, (None, None))
     R, V = logits.shape
     if temperature is not None:
         _need(temperature, "sample_rows.temperature", _F32, (R,))
         _need(uniform, "sample_rows.uniform", _F32, (R,))
-    _need(out, "sample_rows.out", _I32, (R,))
+    _need_tokens(out, "sample_rows.out", R)
     _call(load_library("core"), "syn_sample_rows", _ptr(logits), _ptr(temperature),
           _ptr(uniform if temperature is not None else None), _ptr(out), R, V, _stream())
 
@@ -1606,13 +1615,14 @@ def draw_top_k(logits, out, max_k, temperature, top_k, top_p, min_p, repetition,
                id_start=None):
     """filter_rows and sample_rows(temperature=draw) in one for rows that all have a top-k (1 <= top_k <= max_k <= DRAW_TOP_K_MAX,
     max_k < V), spread over many workgroups a row; the options as in filter_rows.  draw [R]: 1 where the row is drawn from with
-    uniform[r], 0 where its largest is taken.  out [R] int32: the tokens that those two give."""
+    uniform[r], 0 where its largest is taken.  out [R] int32, as in sample_rows: the tokens that those two give."""
     _need(logits, "draw_top_k.logits", _F32, (None, None))
     R, V = logits.shape
     for name, t, dt in (("temperature", temperature, _F32), ("top_k", top_k, _I32), ("top_p", top_p, _F32),
                         ("min_p", min_p, _F32), ("repetition", repetition, _F32), ("presence", presence, _F32),
-                        ("frequency", frequency, _F32), ("draw", draw, _F32), ("uniform", uniform, _F32), ("out", out, _I32)):
+                        ("frequency", frequency, _F32), ("draw", draw, _F32), ("uniform", uniform, _F32)):
         _need(t, f"draw_top_k.{name}", dt, (R,))
+    _need_tokens(out, "draw_top_k.out", R)
     if (ids is None) != (id_start is None):
         raise KernelError("draw_top_k: ids and id_start come together")
     if ids is not None:

@@ -2160,3 +2160,27 @@ def test_stream_scope_holds_the_stream_that_is_current_when_it_opens(ops):
         ref.rmsnorm_rows(x.cpu(), gain.cpu(), 1e-6, want)
         close(out, want, 1e-5, what="launched under a nested scope")
     assert held() == main
+
+
+@pytest.mark.parametrize("rows", [1, 9])
+def test_tokens_reach_pinned_memory_as_they_reach_the_device(ops, rows):
+    """sample_rows into pinned host memory, launched and replayed from a graph with new logits: what the device gets; plain host memory is refused."""
+    x = rnd((rows, 3000), 61).to(DEV)
+    want, got = torch.empty(rows, dtype=I32, device=DEV), torch.full((rows,), -1, dtype=I32, pin_memory=True)
+    t, u = torch.full((rows,), 0.7, device=DEV), torch.rand(rows, generator=torch.Generator().manual_seed(2)).to(DEV)
+    ops.sample_rows(x, t, u, want)
+    ops.sample_rows(x, t, u, got)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want.cpu())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.sample_rows(x, t, u, got)
+    for i in range(4):
+        x.copy_(rnd((rows, 3000), 70 + i))
+        ops.sample_rows(x, t, u, want)
+        graph.replay()
+        torch.cuda.current_stream().synchronize()
+        assert torch.equal(got, want.cpu()), i
+    for bad in (torch.empty(rows, dtype=I32), torch.empty(rows + 1, dtype=I32, pin_memory=True), torch.empty(rows, dtype=torch.int64, pin_memory=True)):
+        with pytest.raises(ops.KernelError):
+            ops.sample_rows(x, t, u, bad)
