@@ -6,7 +6,8 @@
 //   state_space_scan   a scalar decay a head:   S <- exp(-exp(A) dt) S + dt B x^T,  y = S^T C + D x      (S: N x P)
 //   channel_delta_scan a decay for every key channel and the delta rule:
 //                      S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q                 (S: D x P)
-//   head_delta_scan    the same with one decay a head, S <- g S (prompts in chunks on the matrix cores)
+//   head_delta_scan    the same with one decay a head, S <- g S (prompts in chunks on the matrix cores), head_delta_step: single tokens, with
+//                      the convolution, the heads' norm and the gate
 //   gated_linear_scan  a decay for every key channel, no correction: S <- diag(g) S + k v^T,  o = S^T q   (S: D x P; prompts in
 //                      chunks on the matrix cores), gated_linear_step: single tokens, with the heads' norm and gate
 //   diff_heads         two softmax maps over the same values, o = rms_norm(a1 - lambda a2) (1 - c)
@@ -478,6 +479,164 @@ delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ beta,
     const int n = slice * R + i;
     if (col_ok && n < D) S[(size_t)n * E + p] = s[i];
   }
+}
+
+// ---------------------------------------------------------------- delta rule with one decay a head, single tokens in one launch
+// Of steps that bring one token a sequence: the convolution with its state's shift, the scan, the heads' norm and the gate, which as
+// three launches spend most of their time starting and waiting for one another (8 sequences, 32 heads of 128 x 128 over 8 key heads: 4.8 +
+// 11.6 + 4.7 us, so 11.8; a session of 24 steps of four layers, two of them such, 16.46 -> 15.92 ms).  What bounds it: the state's way in and out (64 KB a head), which is
+// asked for before anything else.  A workgroup takes a head of a sequence: 128 columns of the state times four slices of its rows, R a thread.
+// The channels of q and k belong to H / K heads, whose workgroups all read their convolution state: each counts itself in once it
+// has read, and the one that counts last writes the shifted state and leaves the counter at zero; no one waits for it.
+// The sums are those of short_conv_single_kernel, delta_scan_kernel and head_norm_gate_kernel in the same order (four slices of rows).
+#define DS_COLS 128
+template <int R, typename TOut>
+__global__ void __launch_bounds__(4 * DS_COLS)
+delta_step_kernel(const float* __restrict__ u, int u_stride, const float* __restrict__ w, int taps, float* __restrict__ conv, int conv_rows,
+                  const float* __restrict__ beta, int beta_stride, const float* __restrict__ a, int a_stride, const float* __restrict__ a_bias,
+                  const float* __restrict__ a_log, float q_scale, float unit_eps, float* __restrict__ state, int state_rows,
+                  const int* __restrict__ seq_start, const int* __restrict__ seq_slot, const float* __restrict__ gain, float norm_eps,
+                  const float* __restrict__ gate, int gate_stride, TOut* __restrict__ out, int* __restrict__ counters, int H, int K, int D, int E) {
+  constexpr int SL = 4, ROWS = SL * R;
+  __shared__ __attribute__((aligned(16))) float qs[ROWS], ks[ROWS], vs[DS_COLS], os[DS_COLS], red[2][SL][DS_COLS];
+  __shared__ int last;
+  const int head = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid % SYN_WAVE, slice = tid / DS_COLS, p = tid % DS_COLS;
+  const int share = H / K, kvh = head / share, n = seq_start[b], C = 2 * K * D + H * E, keep = taps - 1;
+  const int given = seq_slot[b];
+  const int slot = given < 0 || given >= state_rows ? state_rows - 1 : given, conv_slot = given < 0 || given >= conv_rows ? conv_rows - 1 : given;
+  float* S = state + ((size_t)slot * H + head) * D * E;
+  float s[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = slice * R + i;
+    s[i] = (p < E && r < D) ? S[(size_t)r * E + p] : 0.f;
+  }
+  // the convolution, a channel a thread: q, k, v of this head
+  const int part = tid < D ? 0 : tid < 2 * D ? 1 : tid < 2 * D + E ? 2 : 3;
+  const int c = part == 0 ? kvh * D + tid : part == 1 ? K * D + kvh * D + tid - D : 2 * K * D + head * E + tid - 2 * D;
+  float* st = conv + (size_t)conv_slot * keep * C + c;
+  float held[RC_MAX_TAPS], now = 0.f;
+  if (part < 3) {
+    now = u[(size_t)n * u_stride + c];
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < RC_MAX_TAPS; ++i)
+      if (i < keep) {
+        held[i] = st[(size_t)i * C];
+        acc = fmaf(w[(size_t)c * taps + i], held[i], acc);
+      }
+    acc = rc_silu(fmaf(w[(size_t)c * taps + keep], now, acc));
+    if (part == 0) qs[tid] = acc;
+    else if (part == 1) ks[tid - D] = acc;
+    else vs[tid - 2 * D] = acc;
+  }
+  for (int i = D + tid; i < ROWS; i += 4 * DS_COLS) qs[i] = ks[i] = 0.f;
+  auto shift = [&] {
+#pragma unroll
+    for (int i = 0; i < RC_MAX_TAPS; ++i)
+      if (i < keep) st[(size_t)i * C] = i + 1 < keep ? held[i + 1 < RC_MAX_TAPS ? i + 1 : i] : now;
+  };
+  if (part == 2) shift();      // (this head's alone)
+  float gated[DS_COLS / SYN_WAVE], gains[DS_COLS / SYN_WAVE];
+#pragma unroll
+  for (int i = 0; i < DS_COLS / SYN_WAVE; ++i) {
+    const int d = lane + i * SYN_WAVE;
+    gated[i] = tid < SYN_WAVE && d < E ? gate[(size_t)n * gate_stride + (size_t)head * E + d] : 0.f;
+    gains[i] = tid < SYN_WAVE && d < E ? gain[head * E + d] : 0.f;
+  }
+  const float step = a[(size_t)n * a_stride + head] + a_bias[head], A = -expf(a_log[head]), write = beta[(size_t)n * beta_stride + head];
+  __syncthreads();      // what this workgroup reads of the convolution's state has been read
+  const bool counted = share > 1 && keep > 0;
+  int before = share - 1;      // (its way back is waited for behind the sums)
+  if (counted && tid == 0) before = __hip_atomic_fetch_add(&counters[b * K + kvh], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float sq = 0.f, sk = 0.f, dot = 0.f;
+#pragma unroll
+  for (int i = 0; i < (ROWS + SYN_WAVE - 1) / SYN_WAVE; ++i) {
+    const int d = lane + i * SYN_WAVE;
+    const float qv = d < ROWS ? qs[d] : 0.f, kv = d < ROWS ? ks[d] : 0.f;
+    sq = fmaf(qv, qv, sq), sk = fmaf(kv, kv, sk), dot = fmaf(qv, kv, dot);
+  }
+  sq = wave_sum(sq), sk = wave_sum(sk), dot = wave_sum(dot);
+  const float iq = q_scale / sqrtf(sq + unit_eps), ik = 1.f / sqrtf(sk + unit_eps);
+  const float g = expf(A * rc_softplus(step)), bt = 1.f / (1.f + expf(-write));
+  const float4 *q4 = (const float4*)(qs + slice * R), *k4 = (const float4*)(ks + slice * R);
+  float rk[4] = {0.f, 0.f, 0.f, 0.f}, rq[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < R; i += 4) {
+    const float4 kv = k4[i / 4], qv = q4[i / 4];
+    rk[0] = fmaf(s[i], kv.x * ik, rk[0]), rq[0] = fmaf(s[i], qv.x * iq, rq[0]);
+    rk[1] = fmaf(s[i + 1], kv.y * ik, rk[1]), rq[1] = fmaf(s[i + 1], qv.y * iq, rq[1]);
+    rk[2] = fmaf(s[i + 2], kv.z * ik, rk[2]), rq[2] = fmaf(s[i + 2], qv.z * iq, rq[2]);
+    rk[3] = fmaf(s[i + 3], kv.w * ik, rk[3]), rq[3] = fmaf(s[i + 3], qv.w * iq, rq[3]);
+  }
+  red[0][slice][p] = (rk[0] + rk[1]) + (rk[2] + rk[3]);
+  red[1][slice][p] = (rq[0] + rq[1]) + (rq[2] + rq[3]);
+  if (tid == 0) {
+    last = before == share - 1;
+    if (counted && last) __hip_atomic_store(&counters[b * K + kvh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const float rks = ((red[0][0][p] + red[0][1][p]) + (red[0][2][p] + red[0][3][p])) * g;
+  const float rqs = ((red[1][0][p] + red[1][1][p]) + (red[1][2][p] + red[1][3][p])) * g;
+  const float up = p < E ? bt * (vs[p] - rks) : 0.f;
+  if (slice == 0) os[p] = p < E ? fmaf(up, dot * iq * ik, rqs) : 0.f;
+#pragma unroll
+  for (int i = 0; i < R; i += 4) {
+    const float4 kv = k4[i / 4];
+    s[i] = fmaf(kv.x * ik, up, g * s[i]), s[i + 1] = fmaf(kv.y * ik, up, g * s[i + 1]);
+    s[i + 2] = fmaf(kv.z * ik, up, g * s[i + 2]), s[i + 3] = fmaf(kv.w * ik, up, g * s[i + 3]);
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = slice * R + i;
+    if (p < E && r < D) S[(size_t)r * E + p] = s[i];
+  }
+  if (last && part < 2) shift();
+  __syncthreads();
+  if (tid >= SYN_WAVE) return;
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < DS_COLS / SYN_WAVE; ++i) {
+    const float v = os[lane + i * SYN_WAVE];      // (zeros beyond E)
+    ss += v * v;
+  }
+  const float inv = 1.f / sqrtf(wave_sum(ss) / (float)E + norm_eps);
+#pragma unroll
+  for (int i = 0; i < DS_COLS / SYN_WAVE; ++i) {
+    const int d = lane + i * SYN_WAVE;
+    if (d >= E) continue;
+    float v = os[d] * inv * gains[i];
+    v *= gated[i] / (1.f + expf(-gated[i]));
+    out[(size_t)n * H * E + (size_t)head * E + d] = from_f32<TOut>(v);
+  }
+}
+
+// Whether syn_head_delta_step takes heads of these sizes.
+SYN_EXPORT int syn_head_delta_step_takes(int D, int E, int taps) { return D >= 1 && D <= 128 && E >= 1 && E <= DS_COLS && taps >= 1 && taps <= RC_MAX_TAPS; }
+
+// counters: n_seqs * K of them, zero, and zero again when the launch is done.
+SYN_EXPORT int syn_head_delta_step(const float* u, int u_stride, const float* w, int taps, float* conv, int conv_rows, const float* beta,
+                                   int beta_stride, const float* a, int a_stride, const float* a_bias, const float* a_log, float q_scale,
+                                   float unit_eps, float* state, int state_rows, const int* seq_start, const int* seq_slot, int n_seqs,
+                                   const float* gain, float norm_eps, const float* gate, int gate_stride, void* out, int out_is_f32,
+                                   int* counters, int H, int K, int D, int E, hipStream_t stream) {
+  SYN_CHECK(n_seqs > 0 && n_seqs <= 65535 && H > 0 && K > 0 && H % K == 0, "head_delta_step: %d sequences, %d heads over %d", n_seqs, H, K);
+  SYN_CHECK(syn_head_delta_step_takes(D, E, taps), "head_delta_step: heads of %d x %d with %d taps", D, E, taps);
+  SYN_CHECK(u_stride >= 2 * K * D + H * E && beta_stride >= H && a_stride >= H && gate_stride >= H * E && conv_rows > 0 && state_rows > 0,
+            "head_delta_step: rows of %d, %d, %d and %d values", u_stride, beta_stride, a_stride, gate_stride);
+  const dim3 grid(H, n_seqs);
+#define SYN_DS(R, T)                                                                                                              \
+  delta_step_kernel<R, T><<<grid, 4 * DS_COLS, 0, stream>>>(u, u_stride, w, taps, conv, conv_rows, beta, beta_stride, a, a_stride, a_bias, a_log, \
+                                                            q_scale, unit_eps, state, state_rows, seq_start, seq_slot, gain, norm_eps, gate,      \
+                                                            gate_stride, (T*)out, counters, H, K, D, E)
+  if (out_is_f32) {
+    if (D <= 32) SYN_DS(8, float); else if (D <= 64) SYN_DS(16, float); else SYN_DS(32, float);
+  } else {
+    if (D <= 32) SYN_DS(8, bf16); else if (D <= 64) SYN_DS(16, bf16); else SYN_DS(32, bf16);
+  }
+#undef SYN_DS
+  SYN_LAUNCH_CHECK("head_delta_step");
+  return 0;
 }
 
 // ---------------------------------------------------------------- delta rule with one decay a head, prompts in chunks

@@ -1473,6 +1473,43 @@ def head_delta_scan(qkv, beta, a, a_bias, a_log, q_scale, unit_eps, state, seq_s
                 n_key_heads, dim, vdim, n_heads, not chunked, (qkv.shape[0], _ptr(work)))
 
 
+@functools.lru_cache(maxsize=None)
+def head_delta_step_takes(dim: int, vdim: int, taps: int) -> bool:
+    """Whether head_delta_step takes heads of dim x vdim behind a convolution of so many taps."""
+    return bool(load_library("core").syn_head_delta_step_takes(dim, vdim, taps))
+
+
+def head_delta_step(u, conv_weight, conv_state, beta, a, a_bias, a_log, q_scale, unit_eps, state, seq_start, seq_slot, gain, norm_eps, gate,
+                    out, counters, n_heads, n_key_heads, dim, vdim):
+    """short_conv (with silu), head_delta_scan and head_norm_gate (silu) in one launch for steps that bring one token a sequence:
+    u a float view [N, 2 K * dim + H * vdim] before the convolution, gate a float view [N, H * vdim]; gain float [H * vdim]; out bf16 or float
+    [N, H * vdim]; the others as there.  counters: int32 [at least sequences * K], zero, and zero again behind the launch."""
+    name, H, K = "head_delta_step", n_heads, n_key_heads
+    if K <= 0 or H % K:
+        raise KernelError(f"{name}: {H} heads do not divide into {K} key heads")
+    _need(conv_weight, name + ".conv_weight", _F32, (2 * K * dim + H * vdim, None))
+    C, taps = conv_weight.shape
+    if not head_delta_step_takes(dim, vdim, taps):
+        raise KernelError(f"{name}: heads of {dim} x {vdim} with {taps} taps")
+    _need(out, name + ".out", (_BF16, _F32), (None, H * vdim))
+    N = out.shape[0]
+    u_stride = _float_rows_view(u, name + ".u", N, C)
+    _need(conv_state, name + ".conv_state", _F32, (None, taps - 1, C))
+    stride, a_stride, gate_stride = (_float_rows_view(t, f"{name}.{n}", N, w)
+                                     for t, n, w in ((beta, "beta", H), (a, "a", H), (gate, "gate", H * vdim)))
+    for n, t, w in (("a_bias", a_bias, H), ("a_log", a_log, H), ("gain", gain, H * vdim)):
+        _need(t, f"{name}.{n}", _F32, (w,))
+    _need(state, name + ".state", _F32, (None, H, dim, vdim))
+    B = _step_seqs(name, seq_start, seq_slot)
+    _need(counters, name + ".counters", _I32)
+    if B != N or counters.numel() < B * K:
+        raise KernelError(f"{name}: {N} tokens of {B} sequences with {counters.numel()} counters")
+    _call(load_library("core"), "syn_head_delta_step", _ptr(u), u_stride, _ptr(conv_weight), taps, _ptr(conv_state), conv_state.shape[0],
+          _ptr(beta), stride, _ptr(a), a_stride, _ptr(a_bias), _ptr(a_log), ctypes.c_float(q_scale), ctypes.c_float(unit_eps), _ptr(state),
+          state.shape[0], _ptr(seq_start), _ptr(seq_slot), B, _ptr(gain), ctypes.c_float(norm_eps), _ptr(gate), gate_stride, _ptr(out),
+          _is_f32(out), _ptr(counters), H, K, dim, vdim, _stream())
+
+
 GATED_LINEAR_MAX_VDIM = 512
 
 

@@ -257,6 +257,12 @@ class HeadDeltaMixer(Mixer):
         N, H, C, E = h.shape[0], self.nh, self.channels, self.nh * self.vdim
         conv_state, cell = cache
         proj = linear(h, self.w_in, torch.float32)          # [N, q | k | v | gate | step | decay] float
+        o = torch.empty((N, E), dtype=h.dtype, device=proj.device)
+        if ctx.one_token_each and ops.head_delta_step_takes(self.dim, self.vdim, self.taps):
+            ops.head_delta_step(proj[:, :C], self.conv, conv_state.state, proj[:, C + E:], proj[:, C + E + H:], self.a_bias, self.a_log,
+                                self.q_scale, self.UNIT_EPS, cell.state, ctx.seq_start, ctx.seq_slot, self.gain, self.norm_eps, proj[:, C:], o,
+                                ctx.counters("head_delta_step", N * self.nk), H, self.nk, self.dim, self.vdim)
+            return deferred_product(o, self.w_o)
         qkv = torch.empty((N, C), dtype=torch.float32, device=proj.device)
         ops.short_conv(proj[:, :C], self.conv, None, conv_state.state, ctx.tok_seq, ctx.tok_pos, ctx.seq_start,
                        ctx.seq_past, ctx.seq_slot, qkv, silu=True)
@@ -264,7 +270,6 @@ class HeadDeltaMixer(Mixer):
         ops.head_delta_scan(qkv, proj[:, C + E:], proj[:, C + E + H:], self.a_bias, self.a_log, self.q_scale, self.UNIT_EPS,
                             cell.state, ctx.seq_start, ctx.seq_slot, raw, H, self.nk, self.dim, self.vdim,
                             chunked=not ctx.one_token_each, scratch=ctx.scratch)
-        o = torch.empty((N, E), dtype=h.dtype, device=proj.device)
         ops.head_norm_gate(raw, self.gain, self.norm_eps, proj[:, C:], o, H, self.vdim, silu=True)
         return deferred_product(o, self.w_o)
 

@@ -127,6 +127,41 @@ def test_the_scan_in_portions_from_states_in_given_rows(H, K, D, E):
         assert float((state[rows[i]].cpu().double() - S).abs().max()) < 2e-5 * max(1.0, float(S.abs().max())), f"state of {i}"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,K,D,E,taps", [(8, 2, 32, 16, 4), (4, 4, 64, 64, 2), (32, 8, 128, 128, 4), (6, 3, 100, 72, 4), (5, 1, 8, 40, 1),
+                                          (12, 2, 128, 127, 16), (16, 1, 33, 128, 3)])
+def test_single_tokens_in_one_launch_are_those_of_three(H, K, D, E, taps, dtype):
+    """Convolution, scan, norm and gate in one launch against the three kernels, five steps one after another over seven sequences in rows of
+    their own (one of them padding, in the last row): results, both states and the counters, which are zero again."""
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + D + E)
+    C, B, rows = 2 * K * D + H * E, 7, 9
+    w, bias, a_log = dev(0.4 * randn(g, C, taps)), dev(0.1 * randn(g, H)), dev(0.5 * randn(g, H) - 1.0)
+    gain = dev((1 + 0.1 * randn(g, E)).repeat(H))
+    slots = torch.tensor([3, 0, 7, 1, 5, -1, 2], dtype=torch.int32, device=DEV)
+    start, seq = torch.arange(B + 1, dtype=torch.int32, device=DEV), torch.arange(B, dtype=torch.int32, device=DEV)
+    conv = [dev(randn(g, rows, taps - 1, C)) for _ in range(1)] * 2
+    state = [dev(0.2 * randn(g, rows, H, D, E)) for _ in range(1)] * 2
+    conv, state = [t.clone() for t in conv], [t.clone() for t in state]
+    counters = torch.zeros(B * K, dtype=torch.int32, device=DEV)
+    for i in range(5):
+        proj = dev(randn(g, B, C + H * E + 2 * H + 3))
+        cols = proj[:, :C], proj[:, C:], proj[:, C + H * E:], proj[:, C + H * E + H:]
+        qkv, raw = torch.empty((B, C), device=DEV), torch.empty((B, H * E), device=DEV)
+        want, got = torch.empty((B, H * E), dtype=dtype, device=DEV), torch.full((B, H * E), float("nan"), dtype=dtype, device=DEV)
+        ops.short_conv(cols[0], w, None, conv[0], seq, seq, start, torch.zeros_like(seq), slots, qkv, silu=True)
+        ops.head_delta_scan(qkv, cols[2], cols[3], bias, a_log, D ** -0.5, 1e-6, state[0], start, slots, raw, H, K, D, E)
+        ops.head_norm_gate(raw, gain, 1e-6, cols[1], want, H, E, silu=True)
+        ops.head_delta_step(cols[0], w, conv[1], cols[2], cols[3], bias, a_log, D ** -0.5, 1e-6, state[1], start, slots, gain, 1e-6, cols[1], got,
+                            counters, H, K, D, E)
+        assert not bool(counters.any()) and torch.equal(conv[1], conv[0]), i
+        # sums of up to D products in another number of slices: D * 2^-24 of their size, which a norm divides by; a rounding to 16 bits
+        tol = D * 2.0 ** -21 * float(want.float().abs().max())
+        close = lambda a, b, rel: bool(((a.float() - b.float()).abs() <= tol + rel * b.float().abs()).all())
+        assert close(got, want, 0.0 if dtype == torch.float32 else 2.0 ** -7), (i, float((got.float() - want.float()).abs().max()))
+        assert float((state[1] - state[0]).abs().max()) <= D * 2.0 ** -22 * float(state[0].abs().max()), i
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 def test_a_token_far_back_still_counts(chunked):
     """A value written 150 tokens ago, read with its key by the last token: most of the result is that value (the plain cell
