@@ -537,6 +537,64 @@ __global__ void head_norm_gate_kernel(const float* __restrict__ o, const float* 
   }
 }
 
+// Many heads of up to 1,024 values: four neighbouring values a lane, LP lanes a head (so several heads a wave), NV times; all of a
+// head is asked for at once and stays in registers.  What bounds it is memory, 10 bytes a value with bf16 results; one value a
+// lane, read twice, with a wave for a head of 128 leaves most of the loads' width unused.  3,270 tokens of 32 heads of 128: 50 -> 25 us (5.2 TB/s), 2,048 32 -> 17; 96 tokens, which stay with the kernel
+// above, 10 either way.
+template <typename TOut, int NV>
+__global__ void __launch_bounds__(256)
+head_norm_gate_vec_kernel(const float* __restrict__ o, const float* __restrict__ gain, float eps, const float* __restrict__ gate,
+                          int gate_stride, TOut* __restrict__ out, int out_stride, int n_items, int H, int vdim, int kind, int LP) {
+  const int item = blockIdx.x * (256 / LP) + threadIdx.x / LP, l = threadIdx.x % LP;
+  const bool on = item < n_items;
+  const int at_item = on ? item : n_items - 1, tok = at_item / H, h = at_item % H;
+  const f32x4* x = (const f32x4*)(o + ((size_t)tok * H + h) * vdim);
+  const f32x4* gp = gate ? (const f32x4*)(gate + (size_t)tok * gate_stride + (size_t)h * vdim) : nullptr;
+  const f32x4* wp = gain ? (const f32x4*)(gain + (size_t)h * vdim) : nullptr;
+  f32x4 v[NV], g[NV], w[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int d = l + i * LP;
+    const bool in = 4 * d < vdim;
+    v[i] = in ? x[d] : f32x4{0.f, 0.f, 0.f, 0.f};
+    if (gp && in) g[i] = gp[d];
+    if (wp && in) w[i] = wp[d];
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (4 * (l + i * LP) >= vdim) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (gp && kind == HNG_SILU_FIRST) v[i][e] *= g[i][e] / (1.f + expf(-g[i][e]));
+      ss = fmaf(v[i][e], v[i][e], ss);
+    }
+  }
+  for (int off = 1; off < LP; off <<= 1) ss += __shfl_xor(ss, off, SYN_WAVE);
+  const float inv = 1.f / sqrtf(ss / (float)vdim + eps);
+  TOut* to = out + (size_t)tok * out_stride + (size_t)h * vdim;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int d = l + i * LP;
+    if (!on || 4 * d >= vdim) continue;
+    f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[e] = v[i][e] * inv;
+      if (wp) r[e] *= w[i][e];
+      if (gp && kind != HNG_SILU_FIRST) r[e] *= (kind == HNG_SILU ? g[i][e] : 1.f) / (1.f + expf(-g[i][e]));
+    }
+    if constexpr (sizeof(TOut) == 4) {
+      ((f32x4*)to)[d] = r;
+    } else {
+      bf16x4 q;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q[e] = (bf16)r[e];
+      ((bf16x4*)to)[d] = q;
+    }
+  }
+}
+
 SYN_EXPORT int syn_head_norm_gate(const float* o, const float* gain, float eps, const float* gate, int gate_stride,
                                   void* out, int out_stride, int out_is_f32, int n_tokens, int H, int vdim, int kind,
                                   hipStream_t stream) {
@@ -546,6 +604,22 @@ SYN_EXPORT int syn_head_norm_gate(const float* o, const float* gain, float eps, 
   SYN_CHECK(kind >= HNG_SIGMOID && kind <= HNG_SILU, "head_norm_gate: unknown kind of gate %d", kind);
   const int wpb = 4, items = n_tokens * H;
   const int grid = (items + wpb - 1) / wpb;
+  // four values a lane need rows in pieces of 16 bytes (8 of bf16 results), and pay where there are enough heads to fill the compute units;
+  // for fewer a launch's start is what counts
+  const bool fours = vdim % 4 == 0 && vdim <= 1024 && gate_stride % 4 == 0 && out_stride % 4 == 0 &&
+                     ((uintptr_t)o | (uintptr_t)gain | (uintptr_t)gate) % 16 == 0 && (uintptr_t)out % (out_is_f32 ? 16 : 8) == 0;
+  if (fours && items >= 16 * syn_compute_units()) {
+    int LP = 1;
+    while (LP < 64 && 4 * LP < vdim) LP *= 2;
+    const int blocks = (int)(((long)items * LP + 255) / 256), nv = (vdim + 4 * LP - 1) / (4 * LP);
+#define SYN_HNG(T, NV)                                                                                                          \
+  head_norm_gate_vec_kernel<T, NV><<<blocks, 256, 0, stream>>>(o, gain, eps, gate, gate_stride, (T*)out, out_stride, items, H, vdim, kind, LP)
+    if (out_is_f32) { if (nv == 1) SYN_HNG(float, 1); else if (nv == 2) SYN_HNG(float, 2); else SYN_HNG(float, 4); }
+    else { if (nv == 1) SYN_HNG(bf16, 1); else if (nv == 2) SYN_HNG(bf16, 2); else SYN_HNG(bf16, 4); }
+#undef SYN_HNG
+    SYN_LAUNCH_CHECK("head_norm_gate_vec");
+    return 0;
+  }
   if (out_is_f32)
     head_norm_gate_kernel<float><<<grid, wpb * SYN_WAVE, 0, stream>>>(o, gain, eps, gate, gate_stride, (float*)out, out_stride, items,
                                                                       H, vdim, kind);

@@ -50,6 +50,52 @@ short_conv_kernel(const float* __restrict__ u, int u_stride, const float* __rest
   out[(size_t)n * C + c] = act ? rc_silu(acc) : acc;
 }
 
+// Steps of many tokens: a thread takes four channels of T tokens, whose T + TAPS - 1 rows of inputs it asks for together; an input
+// before the step's first token comes from the state.  The same sums in the same order.  What bounds it is memory, 8 bytes a
+// channel; one channel of one token a thread (above) spends its time on the way to four inputs of 4 bytes and four weights.
+// 3,270 tokens of 6,144 channels in eight sequences: 102 -> 37 us (4.3 TB/s), 2,048 in one 63 -> 27; 96 tokens 17.4 us of launches and
+// gaps either way.
+template <int TAPS, int T>
+__global__ void __launch_bounds__(256)
+short_conv_rows_kernel(const float* __restrict__ u, int u_stride, const float* __restrict__ w, const float* __restrict__ bias,
+                       int act, const float* __restrict__ state, int state_rows, const int* __restrict__ tok_seq,
+                       const int* __restrict__ tok_pos, const int* __restrict__ seq_past, const int* __restrict__ seq_slot,
+                       float* __restrict__ out, int N, int C) {
+  const int c = 4 * (blockIdx.y * blockDim.x + threadIdx.x), n0 = blockIdx.x * T;
+  if (c >= C) return;
+  f32x4 row[T + TAPS - 1];
+#pragma unroll
+  for (int i = 0; i < T + TAPS - 1; ++i)      // (tokens before the step's first and behind its last: loaded, not used)
+    row[i] = *(const f32x4*)(u + (size_t)min(max(n0 + i - (TAPS - 1), 0), N - 1) * u_stride + c);
+  float wv[4 * TAPS];
+#pragma unroll
+  for (int i = 0; i < TAPS; ++i) ((f32x4*)wv)[i] = ((const f32x4*)(w + (size_t)c * TAPS))[i];
+  const f32x4 first = bias ? *(const f32x4*)(bias + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int n = n0 + t;
+    if (n >= N) break;
+    const int seq = tok_seq[n], in_step = tok_pos[n] - seq_past[seq];
+    f32x4 acc = first;
+    int slot = seq_slot[seq];
+    if (slot < 0 || slot >= state_rows) slot = state_rows - 1;
+    const float* st = state + (size_t)slot * (TAPS - 1) * C + c;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      const int back = TAPS - 1 - j;
+      f32x4 v = row[t + j];
+      if (back > in_step) v = *(const f32x4*)(st + (size_t)(TAPS - 1 - (back - in_step)) * C);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(wv[e * TAPS + j], v[e], acc[e]);
+    }
+    if (act) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = rc_silu(acc[e]);
+    }
+    *(f32x4*)(out + (size_t)n * C + c) = acc;
+  }
+}
+
 // The state after the step: the last taps - 1 inputs of (old state, the step's inputs).  One thread a (sequence,
 // channel) reads what it keeps before it writes.
 __global__ void __launch_bounds__(256)
@@ -116,8 +162,23 @@ SYN_EXPORT int syn_short_conv(const float* u, int u_stride, const float* w, cons
     SYN_LAUNCH_CHECK("short_conv_single");
     return 0;
   }
-  short_conv_kernel<<<dim3(n_tokens, bx), 256, 0, stream>>>(u, u_stride, w, bias, act, state, state_rows, tok_seq, tok_pos,
-                                                           seq_past, seq_slot, out, n_tokens, C, taps);
+  // four channels a thread need rows, weights and states in pieces of 16 bytes; tokens a thread: as many as leave each compute
+  // unit two workgroups
+  const bool fours = C % 4 == 0 && u_stride % 4 == 0 && ((uintptr_t)u | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)state | (uintptr_t)out) % 16 == 0;
+  const int by = (C / 4 + 255) / 256;
+  const bool eight = (long)(n_tokens + 7) / 8 * by >= 2L * syn_compute_units();
+#define SYN_CONV(TAPS, T)                                                                                                        \
+  short_conv_rows_kernel<TAPS, T><<<dim3((n_tokens + T - 1) / T, by), 256, 0, stream>>>(u, u_stride, w, bias, act, state, state_rows, \
+                                                                                        tok_seq, tok_pos, seq_past, seq_slot, out, n_tokens, C)
+  if (fours && taps >= 2 && taps <= 4) {
+    if (taps == 4) { if (eight) SYN_CONV(4, 8); else SYN_CONV(4, 2); }
+    else if (taps == 3) { if (eight) SYN_CONV(3, 8); else SYN_CONV(3, 2); }
+    else { if (eight) SYN_CONV(2, 8); else SYN_CONV(2, 2); }
+  } else {
+    short_conv_kernel<<<dim3(n_tokens, bx), 256, 0, stream>>>(u, u_stride, w, bias, act, state, state_rows, tok_seq, tok_pos,
+                                                             seq_past, seq_slot, out, n_tokens, C, taps);
+  }
+#undef SYN_CONV
   SYN_LAUNCH_CHECK("short_conv");
   if (taps > 1) {
     short_conv_state_kernel<<<dim3(bx, n_seqs), 256, 0, stream>>>(u, u_stride, state, state_rows, seq_start, seq_slot, C, taps);

@@ -800,3 +800,85 @@ def test_command_line_and_trace_replay_as_a_user_starts_them(tmp_path):
         assert sorted(out) == sorted(want)
         for k, w in want.items():
             assert_logits_close(out[k], w, dtype, f"trace step {k} in {dtype}", sharp=True)
+
+
+def shifted(t):
+    """The same rows one value into longer ones: pieces of 16 bytes do not reach them, which leaves the general kernels."""
+    longer = torch.full((t.shape[0], t.shape[1] + 1), float("nan"), dtype=t.dtype, device=t.device)
+    longer[:, 1:] = t
+    return longer[:, 1:]
+
+
+def seq_tables(lens, past):
+    """(seq of every token, its position, the sequences' first tokens) of a step."""
+    seq = [b for b, n in enumerate(lens) for _ in range(n)]
+    pos = [past[b] + i for b, n in enumerate(lens) for i in range(n)]
+    start = [sum(lens[:b]) for b in range(len(lens) + 1)]
+    return ints(seq), ints(pos), ints(start)
+
+
+@pytest.mark.parametrize("lens", [[1, 2, 127], [3, 1, 1, 9, 5, 1], [2051], [700, 1, 2, 3, 1345]])
+@pytest.mark.parametrize("C,taps,bias", [(1028, 4, False), (2048, 3, True), (12, 2, True)])
+def test_convolution_of_four_channels_a_thread_is_that_of_one(lens, C, taps, bias):
+    """Sequences that begin and end anywhere within a thread's tokens, with and without earlier inputs: the same sums in the same order."""
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(C + len(lens))
+    past = [7 * (b % 2) for b in range(len(lens))]
+    seq, pos, start = seq_tables(lens, past)
+    slots = ints([(3 * b + 1) % 7 if b != 2 else -1 for b in range(len(lens))])
+    u, w, b = dev(randn(g, sum(lens), C)), dev(randn(g, C, taps)), dev(randn(g, C)) if bias else None
+    before = dev(randn(g, 8, taps - 1, C))
+    got, states = [], []
+    for rows in (u, shifted(u)):
+        out, state = torch.full_like(u, float("nan")), before.clone()
+        ops.short_conv(rows, w, b, state, seq, pos, start, ints(past), slots, out, silu=True)
+        got.append(out), states.append(state)
+    assert torch.equal(got[0], got[1]) and torch.equal(states[0], states[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("how", [dict(), dict(silu=True), dict(silu_first=True)])
+@pytest.mark.parametrize("N,H,E", [(1025, 4, 128), (4097, 1, 4), (700, 6, 100), (1400, 3, 260), (4100, 1, 1024), (2049, 2, 72)])
+def test_heads_normed_four_values_a_lane(N, H, E, how, dtype):
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(N + E)
+    o, gate, gain = dev(randn(g, N, H * E)), dev(randn(g, N, H * E + 4)), dev(1 + 0.1 * randn(g, H * E))
+    o[3] = 0.0
+    got = []
+    for rows in (gate[:, 4:], shifted(gate)[:, 4:]):
+        for given in (gain, None):
+            out = torch.full((N, H * E), float("nan"), dtype=dtype, device=DEV)
+            ops.head_norm_gate(o, given, 1e-6, rows, out, H, E, **how)
+            got.append(out.float())
+    for a, b in ((got[0], got[2]), (got[1], got[3])):
+        # one sum of E squares in another order on either side: E * 2^-24 of the result after the root; the root, the two quotients and the
+        # three products behind it round by 2^-24 each, on both sides; 16 bits round up or down
+        rel = (E + 12) * 2.0 ** -24 + (0.0 if dtype == torch.float32 else 2.0 ** -7)
+        assert bool(((a - b).abs() <= rel * b.abs()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N", [512, 1027, 2055])
+@pytest.mark.parametrize("nh,nk,D,write", [(32, 8, 128, True), (8, 8, 128, True), (5, 1, 12, True), (16, 4, 100, False), (56, 8, 128, True)])
+def test_intake_of_many_tokens_is_that_of_few(nh, nk, D, write, N, dtype):
+    """Prompts of three sequences that end anywhere, tokens behind earlier ones, one, two, four and eight tokens a workgroup."""
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(nh + N)
+    lens, past = [N // 3, 1, N - 1 - N // 3], [70, 0, 13]
+    seq, pos, _ = seq_tables(lens, past)
+    pages = (N + 90) // 64 + 1
+    table = torch.randperm(3 * pages, generator=g).to(torch.int32).view(3, pages).to(DEV)
+    rows, qg, kg = dev(randn(g, N, (nh + nk) * D + 4)), dev(1 + 0.3 * randn(g, nh * D)), dev(1 + 0.3 * randn(g, nk * D))
+    rows[5] = 0.0
+    got = []
+    for r in (rows, shifted(rows)):
+        qo = torch.full((N, nh * D), float("nan"), dtype=dtype, device=DEV)
+        kp, vp = torch.zeros((3 * pages, nk, 64, D), dtype=dtype, device=DEV), torch.zeros((3 * pages, nk, D, 64), dtype=dtype, device=DEV)
+        ops.window_intake(r, None, qo, kp, vp, table, seq, pos, qg, kg, 1e-5, nh, nk, D, D, write_kv=write, norm_whole=True,
+                          values_are_keys=True, q_temp=(0.3, 64))
+        got.append((qo.float(), kp.float(), vp.float()))
+    # sums of nh D squares in another order; two quotients, the root and three products on both sides; 16 bits round up or down
+    rel = (nh * D + 12) * 2.0 ** -24 + (0.0 if dtype == torch.float32 else 2.0 ** -7)
+    for a, b in zip(got[0][:2], got[1][:2]):
+        assert bool(((a - b).abs() <= rel * b.abs()).all())
+    assert torch.equal(got[0][2], got[1][2]) and bool(got[0][1].any()) == write
