@@ -35,6 +35,7 @@ struct Epilogue {
   int act;
   float limit;      // the bound of an activation that has one (gated, csrc/common.h)
   int point;        // SYN_POINT_NONE, or what a plain product's sums pass before they are stored
+  int add = 0;      // float results of the streamed tiles: added to what the output holds
 };
 
 // ------------------------------------------------------------------ SIMT, any type
@@ -1277,12 +1278,40 @@ gemm_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, void*
         }
       }
     };
+    // The sums added to what is there (the residual rows; syn_gemm_add): what the tile's rows hold is asked for up to four groups of 16 rows ahead, and
+    // always before the stores that would otherwise be waited for with it.  (Four groups beside 256 columns spilled: 8,000 rows of 4,096 x 4,096
+    // 283 us with the norm instead of 260.)
+    auto add_all = [&] {
+      constexpr int AHEAD = FM < 4 ? FM : FN > 6 ? 2 : 4;      // (what the registers hold beside the next tile's first fragments)
+      f32x4 have[AHEAD][FN];
+      auto place = [&](int i, int j) {
+        const int n = t.n * BN + wn + 16 * j + 4 * q4;
+        return n < N ? (unsigned)(16 * i + r16) * N * 4 + n * 4 : SYN_NOWHERE;
+      };
+      auto ask = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) have[i % AHEAD][j] = __builtin_bit_cast(f32x4, buffer_load16(vo, place(i, j)));
+      };
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) ask(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+        for (int j = 0; j < FN; ++j) buffer_store16(vo, __builtin_bit_cast(u32x4, have[i % AHEAD][j] + acc[i][j]), place(i, j), streamed);
+        if (i + AHEAD < FM) ask(i + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
     if constexpr (OUT == SYN_OUT_GATED) {
       if (ep.act == SYN_ACT_SILU) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SILU, false>(g, u, 0.f); });
       else if (ep.act == SYN_ACT_SWIGLU_LIMIT) store_all([&](float g, float u) { return gated_quick<SYN_ACT_SWIGLU_LIMIT, false>(g, u, ep.limit); });
       else store_all([&](float g, float u) { return gated_quick<SYN_ACT_GELU_TANH, false>(g, u, 0.f); });
     } else {
-      if (ep.point == SYN_POINT_NONE) store_all([&](float v, float) { return v; });
+      if (OUT == SYN_OUT_F32 && ep.add) add_all();
+      else if (ep.point == SYN_POINT_NONE) store_all([&](float v, float) { return v; });
       else store_all([&](float v, float) { return point_activation(SYN_POINT_RELU_SQUARED, v); });
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1617,6 +1646,25 @@ static int direct_gated_tile(int M, int N, int K) {
   if (K % 64 != 0 || K < 2048) return 0;
   if (M <= 128) return 4 * by96 >= 3 * cus && by96 <= cus ? 128 : 0;
   return M <= 256 && 16 * by128 >= 9 * cus && by128 <= cus ? (M <= 192 ? 192 : 256) : 0;
+}
+
+// resid[M, N] float += x . w^T (bf16, w in fragment order): a product whose reader adds it to the residual rows adds it itself, so that
+// the norm behind it reads 4 bytes a value and writes 2, instead of 8 and 6, and writes no rows of its own.  The same sums, added once, as
+// the norm would (float + float).  Product and norm, us, before and so: 41,028 rows, 2,560 x 4,096 1,044 -> 968, 2,560 x 9,728 1,942 ->
+// 1,855; 2,048 rows, 4,096 x 4,096 79 -> 73, 8,192 x 4,096 145 -> 137, 2,048 x 2,048 32.0 -> 30.3; 8,000 rows, 4,096 x 12,288 608 -> 592, 1,024 x
+// 4,096 74.5 -> 72.8; 512 rows, 5,120 x 512 18.2 -> 17.1.  Not where cutting K gains more: 1,024 rows, 4,096 x 12,288 in 4 slices 105, 121 so.
+// syn_gemm_adds: whether there are many rows and the streamed tiles take them (the caller sees to it that K would not be cut: partial sums
+// are the norm's to add).
+SYN_EXPORT int syn_gemm_adds(int M, int N, int K) {
+  return M >= 512 && N > 0 && K > 0 && N % 16 == 0 && K % 128 == 0 && plan_stream(STREAMED, M, N, K, 1, true, 4).tile >= 0;
+}
+SYN_EXPORT int syn_gemm_add(const void* x, const void* w, float* resid, int M, int N, int K, hipStream_t stream) {
+  SYN_CHECK(syn_gemm_adds(M, N, K), "gemm_add: no product of %d x %d rows of %d that adds", M, N, K);
+  SYN_CHECK(((uintptr_t)x | (uintptr_t)w | (uintptr_t)resid) % 16 == 0, "gemm_add: operands are not aligned");
+  const int rc = launch_large<false>((const bf16*)x, {(const bf16*)w, true}, resid, {1, SYN_ACT_SILU, 0.f, SYN_POINT_NONE, 1}, M, N, K, stream);
+  if (rc) return rc;
+  SYN_LAUNCH_CHECK("gemm_add");
+  return 0;
 }
 
 // out[M, N/2] = silu(x . Wg^T) * (x . Wu^T), bf16, where w [N, K] holds the rows of Wg and of Wu in

@@ -330,6 +330,21 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
 
 
 @functools.lru_cache(maxsize=4096)
+def gemm_adds(M, N, K) -> bool:
+    """Whether gemm_add takes M rows with a weight [N, K] in fragment order (csrc/gemm.hip: syn_gemm_adds)."""
+    return bool(load_library("core").syn_gemm_adds(M, N, K))
+
+
+def gemm_add(x, w, resid):
+    """resid[M, N] += x[M, K] . w[N, K]^T: bf16 rows and a weight in fragment order, 32-bit sums added once to the float rows."""
+    _need(x, "gemm_add.x", _BF16, (None, None))
+    M, K = x.shape
+    N = _packed_shape(w, "gemm_add.w", K)
+    _need(resid, "gemm_add.resid", _F32, (M, N))
+    _call(load_library("core"), "syn_gemm_add", _ptr(x), _ptr(w), _ptr(resid), M, N, K, _stream())
+
+
+@functools.lru_cache(maxsize=4096)
 def _f32_floats(M, N, K) -> int:
     """Floats of working memory of a 32-bit product: parts of x, and sums over parts of K."""
     fn = load_library("core").syn_gemm_f32_scratch

@@ -81,14 +81,18 @@ def as_rows(h):
 class DeferredProduct:
     """A product x . W^T over packed weights that has not been run: the norm that receives it as the delta of
     the residual rows runs it with the residual sum and its own first half as the epilogue (ops.gemm_packed,
-    resid_norm), or asks for `run()`, the float product itself."""
+    resid_norm), or asks for `run()`, the float product itself.  `many`: a product of so many rows that it adds its sums
+    into the residual rows by itself (`add_to`) and leaves the norm all of its own work."""
 
-    def __init__(self, x, w):
-        self.x, self.w, self.packed = x, w, w.packed
+    def __init__(self, x, w, many=False):
+        self.x, self.w, self.packed, self.many = x, w, w.packed, many
         self.shape = (x.shape[0], w.shape[0])
 
     def run(self):
         return linear_for_sum(self.x, self.w)
+
+    def add_to(self, resid):
+        ops.gemm_add(self.x, self.packed, resid)
 
 
 class WeightedDeltas:
@@ -206,10 +210,13 @@ def as_delta(d):
 
 
 def deferred_product(x, w):
-    """linear_for_sum, but where the product would run over few rows in one slice it is only described:
+    """linear_for_sum, but where the product would run over few rows in one slice, or over many in one, it is only described:
     the caller's result is the delta that a following norm adds to the residual rows, and that norm can take the
     product in (RmsNorm.add_apply)."""
     w = _matrix(w)
+    if (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and w.packed is not None
+            and ops.gemm_adds(x.shape[0], *w.shape) and product_slices(x.shape[0], w, x.dtype) <= 1):
+        return DeferredProduct(x, w, many=True)
     if isinstance(x, torch.Tensor) and _use_packed(x, w) and ops.packed_slices(w.shape[0], w.shape[1]) <= 1:
         return DeferredProduct(x, w)
     return linear_for_sum(x, w)

@@ -37,7 +37,7 @@ class RmsNorm(Part):
 
     def _runs_product(self, resid, delta, out_dtype, rows):
         """Whether this norm takes `delta`, a product that has not been run, in as its epilogue's residual sum."""
-        return (isinstance(delta, DeferredProduct) and rows is None and out_dtype == torch.bfloat16
+        return (isinstance(delta, DeferredProduct) and not delta.many and rows is None and out_dtype == torch.bfloat16
                 and delta.shape == tuple(resid.shape) and self.dim % 16 == 0)
 
     def add_apply(self, resid, delta, out_dtype, rows=None):
@@ -74,7 +74,11 @@ class RmsNorm(Part):
                 ss = torch.empty((resid.shape[0], self.dim // 16), dtype=torch.float32, device=resid.device)
                 ops.gemm_packed(delta.x, delta.packed, None, resid_norm=(resid, self.gain, self.gain_offset, xs, ss, *more))
                 return ScaledRows(xs, ss, self.eps, resid, self)
-            delta = delta.run()
+            if delta.many and rows is None and delta.shape == tuple(resid.shape):
+                delta.add_to(resid)          # (many rows: the product adds its own sums)
+                delta = None
+            else:
+                delta = delta.run()
         n = resid.shape[0] if rows is None else rows.shape[0]
         out = torch.empty((n, self.dim), dtype=out_dtype, device=resid.device)
         ops.add_rmsnorm(resid, delta, self.gain, self.eps, out, rows, self.gain_offset)

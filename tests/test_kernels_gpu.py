@@ -2184,3 +2184,39 @@ def test_tokens_reach_pinned_memory_as_they_reach_the_device(ops, rows):
     for bad in (torch.empty(rows, dtype=I32), torch.empty(rows + 1, dtype=I32, pin_memory=True), torch.empty(rows, dtype=torch.int64, pin_memory=True)):
         with pytest.raises(ops.KernelError):
             ops.sample_rows(x, t, u, bad)
+
+
+@pytest.mark.parametrize("M", [512, 513, 700, 1729, 2051])
+@pytest.mark.parametrize("N,K", [(1024, 1024), (4096, 4096), (2560, 4096), (2576, 1152), (48, 2048), (5120, 512)])
+def test_products_of_many_rows_add_to_the_residual_rows_what_the_norm_would(M, N, K):
+    """One product that adds its sums to the rows against the product and the norm that adds: the same sums, added once, so the same bits
+    wherever K is not cut; rows beyond M and the rows' neighbours in memory stay as they are.  All tiles that the sizes take."""
+    from synaptix_amd.kernels import ops
+    from synaptix_amd.parts import RmsNorm
+    from synaptix_amd.parts.linear import DeferredProduct, Matrix, deferred_product, linear
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=DEV).bfloat16()
+    w = Matrix((0.02 * torch.randn((N, K), generator=g, device=DEV)).bfloat16())
+    room = torch.randn((M + 2, N), generator=g, device=DEV)
+    before = room.clone()
+    assert ops.gemm_adds(M, N, K) and not ops.gemm_adds(511, N, K)
+    ops.gemm_add(x, w.packed, room[1:-1])
+    want = before[1:-1] + linear(x, w, torch.float32)
+    same_tile = ops.gemm_slices(M, N, K, torch.bfloat16) == 1
+    if same_tile:
+        assert torch.equal(room[1:-1], want)
+    # (else the plain product may go through other tiles: K / 32 roundings of the sums' size in another order)
+    assert float((room[1:-1] - want).abs().max()) <= K / 32 * 2.0 ** -23 * float((want - before[1:-1]).abs().max()) + 2.0 ** -23 * float(want.abs().max())
+    assert torch.equal(room[0], before[0]) and torch.equal(room[-1], before[-1])
+    # through the norm, which takes the product that has not been run; with rows picked it runs it and leaves the residual alone
+    norm = RmsNorm("n", N, 1e-6)
+    norm.gain = (1 + 0.1 * torch.randn((N,), generator=g, device=DEV)).bfloat16()
+    delta = deferred_product(x, w)
+    picked = torch.tensor([M - 1, 0, 5], dtype=torch.int32, device=DEV)
+    for rows in (picked, None):
+        resid = [before[1:-1].clone() for _ in range(2)]
+        got = norm.add_apply(resid[0], delta, torch.bfloat16, rows=rows)
+        ref = norm.add_apply(resid[1], linear(x, w, torch.float32), torch.bfloat16, rows=rows)
+        if same_tile:
+            assert isinstance(delta, DeferredProduct) and delta.many and torch.equal(got, ref) and torch.equal(resid[0], resid[1])
+        assert rows is None or torch.equal(resid[0], before[1:-1])
