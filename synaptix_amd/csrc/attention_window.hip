@@ -354,7 +354,14 @@ template <> __device__ __forceinline__ void load8<float>(const float* p, float (
 // results (maximum, sum, weighted values) are merged through LDS at the end.  One wave is enough where a step has many
 // tokens; single tokens over a long window get eight.
 // MAXD: the largest head size that the registers and LDS of this instantiation hold (a multiple of 64).
-template <typename T, int WAVES, int MAXD>
+// PAGES (bf16, keys and values of 128): a wave brings a block's keys, and then its values, into LDS in whole lines of 16 KB and reads its
+// lanes' rows there (slot s of row r holds piece s ^ r % 16 of a key, s ^ r / 2 % 8 of a value's row, so that 16 lanes meet every bank once).
+// Straight from memory a load takes 16 bytes of 64 rows, a line each, and eight waves' lines push one another out of the L1 before
+// their other pieces are asked for.  The same sums in the same order.  8
+// sequences, 32 query and 8 key heads: 20 keys 7.3 -> 7.2 us, 130 7.9 -> 7.9, 500 12.0 -> 9.2, 1,024 22.8 -> 18.5; one sequence 7.2 -> 7.0,
+// 7.6 -> 7.5, 11.4 -> 8.5, 21.0 -> 16.0.  (All of a lane's loads issued together from memory instead: 500 keys 13.9, 2,016 pairs 1.1 to 1.8
+// times as long.)
+template <typename T, int WAVES, int MAXD, bool PAGES = false>
 __global__ void __launch_bounds__(WAVES * SYN_WAVE)
 window_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
                         const int* __restrict__ page_table, int table_stride, const int* __restrict__ tok_seq,
@@ -365,10 +372,21 @@ window_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, 
   __shared__ float ps[WAVES][SYN_PAGE];
   __shared__ float part_o[WAVES][MAXD];
   __shared__ float part_ml[WAVES][2];
+  extern __shared__ __attribute__((aligned(16))) bf16 staged[];      // PAGES: [WAVES][64 * 128]
   const int tok = blockIdx.x, head = blockIdx.y;
-  const int wave = threadIdx.x / SYN_WAVE, lane = threadIdx.x % SYN_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SYN_WAVE), lane = threadIdx.x % SYN_WAVE;
   const int seq = tok_seq[tok], pos = tok_pos[tok];
   const int kvh = head / (nh / nkv);
+  bf16* const mine = staged + wave * (SYN_PAGE * 128);
+  // 16 KB that lie one after another, in pieces of 16 bytes: load p takes piece `from` of the wave's p-th KB to place `lane`
+  auto bring = [&](const bf16* at, auto from) {
+    const BufferView v = buffer_view(at, SYN_PAGE * 128 * sizeof(bf16));
+#pragma unroll
+    for (int p = 0; p < 16; ++p) buffer_to_lds16(v, (char*)mine + p * 1024, (unsigned)(p * 1024 + from(p) * 16), 0);
+    __builtin_amdgcn_s_waitcnt(0x0070);      // vmcnt(0), lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
   const T* qr = q + ((size_t)tok * nh + head) * dim;
   for (int d = threadIdx.x; d < dim; d += WAVES * SYN_WAVE) qs[d] = to_f32<T>(qr[d]);
   __syncthreads();
@@ -393,7 +411,23 @@ window_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, 
     const int key = kb * SYN_PAGE + lane;
     const bool valid = key <= pos && (key >= lo || key < kept);
     float s = -INFINITY;
-    if (valid) {
+    if constexpr (PAGES) {
+      // (the places past the sequence's end lie in the page as well: what they hold is read, and counts nothing)
+      asm volatile("" ::: "memory");
+      bring((const bf16*)k_pages + kbase, [&](int p) { const int r = lane / 16; return r * 16 + (lane % 16 ^ (4 * p + r) % 16); });
+      float dot = 0.f;
+#pragma unroll
+      for (int d = 0; d < 128; d += 8) {
+        const bf16x8 kv = *(const bf16x8*)(mine + lane * 128 + (d / 8 ^ lane % 16) * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf(qs[d + e], (float)kv[e], dot);
+      }
+      if (valid) s = window_score(dot, scale, terms, slope, r1, r2, pos, key);
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0): the keys are in registers, values may take their place
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      bring((const bf16*)v_pages + vbase, [&](int p) { const int r = lane / 8; return r * 8 + (lane % 8 ^ (8 * p + r) / 2 % 8); });
+    } else if (valid) {
       const T* kr = k_pages + kbase + (size_t)lane * dim;
       float dot = 0.f;
       if (dim % 8 == 0) {
@@ -429,7 +463,8 @@ window_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, 
         float acc = o[i] * alpha;
         for (int j = 0; j < SYN_PAGE; j += 8) {
           float vv[8];
-          load8<T>(vr + j, vv);
+          if constexpr (PAGES) load8<bf16>(mine + d * SYN_PAGE + (j / 8 ^ d / 2 % 8) * 8, vv);
+          else load8<T>(vr + j, vv);
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const float pj = ps[wave][j + e];
@@ -438,6 +473,11 @@ window_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, 
         }
         o[i] = acc;
       }
+    }
+    if constexpr (PAGES) {
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   if (WAVES > 1) {
@@ -508,6 +548,22 @@ SYN_EXPORT int syn_window_attention(const void* q, const void* k_pages, const vo
                                                                       page_table, table_stride, tok_seq, tok_pos, gate, \
                                                                       gate_stride, gate_bias, (T*)out, scale, nh, nkv,  \
                                                                       dim, vdim, terms)
+  // blocks through LDS (128 KB of it a workgroup) while every pair has a compute unit of its own; with two rounds of them the start counts
+  // twice: 512 pairs, 20 keys 7.8 us straight from memory and 13.0 so, 500 keys 20.8 and 18.1; 2,016 pairs, 500 keys 86 and 95
+  if (!is_f32 && dim == 128 && vdim == 128 && (long)n_tokens * nh <= syn_compute_units() &&
+      ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0) {
+    constexpr int LDS = 8 * SYN_PAGE * 128 * (int)sizeof(bf16);
+    static OncePerDevice raised;
+    const hipError_t e = once_per_device(raised, [&] {
+      return hipFuncSetAttribute((const void*)window_attention_kernel<bf16, 8, 128, true>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    });
+    SYN_CHECK(e == hipSuccess, "window_attention: %d bytes of LDS refused: %s", LDS, hipGetErrorString(e));
+    window_attention_kernel<bf16, 8, 128, true><<<grid, 8 * SYN_WAVE, LDS, stream>>>(
+        (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, page_table, table_stride, tok_seq, tok_pos, gate, gate_stride, gate_bias,
+        (bf16*)out, scale, nh, nkv, dim, vdim, terms);
+    SYN_LAUNCH_CHECK("window_attention_pages");
+    return 0;
+  }
 #define SYN_AW(T, W) do { if (large) SYN_AW2(T, W, 640); else SYN_AW2(T, W, 256); } while (0)
   if (is_f32) {
     if (many_waves) SYN_AW(float, 8); else SYN_AW(float, 1);

@@ -882,3 +882,29 @@ def test_intake_of_many_tokens_is_that_of_few(nh, nk, D, write, N, dtype):
     for a, b in zip(got[0][:2], got[1][:2]):
         assert bool(((a - b).abs() <= rel * b.abs()).all())
     assert torch.equal(got[0][2], got[1][2]) and bool(got[0][1].any()) == write
+
+
+@pytest.mark.parametrize("how", [dict(), dict(window=100, softcap=30.0), dict(chunk=70, keep_first=3), dict(window=1)])
+@pytest.mark.parametrize("B,nh,nk,D,E", [(1, 8, 8, 128, 128), (8, 32, 8, 128, 128), (9, 4, 2, 128, 128), (16, 16, 4, 128, 128), (17, 16, 4, 128, 128)])
+def test_blocks_through_lds_are_those_straight_from_memory(B, nh, nk, D, E, how):
+    """Single tokens through the kernel that brings whole blocks into LDS against the general one, which wider values lead to: the same sums in
+    the same order.  Contexts that end at and beside a page's border; places that hold no key are NaN."""
+    from synaptix_amd.kernels import ops
+    g = torch.Generator().manual_seed(B + nh + E)
+    ends = ([0, 62, 63, 64, 65, 511, 512, 700, 1300] * 7)[:B] if B > 1 else [777]
+    pages = 1300 // 64 + 1
+    table = torch.randperm(B * pages, generator=g).to(torch.int32).view(B, pages)
+    kp = torch.full((B * pages, nk, 64, D), float("nan"), dtype=torch.bfloat16)
+    vw = torch.full((B * pages, nk, D + 16, 64), float("nan"), dtype=torch.bfloat16)
+    for b, end in enumerate(ends):
+        for j in range(end // 64 + 1):
+            n = min(64, end + 1 - 64 * j)
+            kp[table[b, j], :, :n] = randn(g, nk, n, D).bfloat16()
+            vw[table[b, j], :, :, :n] = randn(g, nk, D + 16, n).bfloat16()
+    vp = vw[:, :, :E].contiguous().to(DEV)
+    q, slopes, gate = dev(randn(g, B, nh * D), torch.bfloat16), dev(torch.linspace(0.001, 0.2, nh)), dev(randn(g, B, nh))
+    out = [torch.full((B, nh * n), float("nan"), dtype=torch.bfloat16, device=DEV) for n in (E, D + 16)]
+    for o, v, n in ((out[0], vp, E), (out[1], vw.to(DEV), D + 16)):
+        ops.window_attention(q, kp.to(DEV), v, table.to(DEV), ints(range(B)), ints(ends), o, D ** -0.5, nh, nk, D, n, slopes=slopes, gate=gate,
+                             gate_per_head=True, **how)
+    assert not bool(out[0].isnan().any()) and torch.equal(out[0].view(B, nh, E), out[1].view(B, nh, D + 16)[:, :, :E])
