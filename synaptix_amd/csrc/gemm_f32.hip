@@ -333,9 +333,9 @@ struct F32Plan {
 // 24, 21, 34, 24, 43, 32, 100, 83, 142, 113; 2,560 x 9,728 39, 37, 63, 43, 133, 54, 181, 111, 265, 187; 19,456 x 2,560 56, 42, 58, 49, 78, 74, 268,
 // 201, 435, 308; 151,936 x 2,560 with 1 row 286, 275, 17 290, 290, 32 310, 300, 64 493, 376.
 static F32Plan plan_f32(int M, int N, int K) {
-  const double cus = syn_compute_units(), w = 4e-6 * N * K;
   F32Plan best = {F32_FEW, false};
-  if (M <= 64 && (int64_t)N * K <= 1 << 18) return best;
+  if (M <= 64 && (int64_t)N * K <= 1 << 18) return best;      // (asked before anything that costs the host time: a layer of few tokens plans a dozen times)
+  const double cus = syn_compute_units(), w = 4e-6 * N * K;
   double least = M <= 64 ? 3.0 + w / 2.95 * ((M + 15) / 16) * (1.0 + 0.02 * std::min(M, 16)) : 1e30;
   const int nk = (K + 31) / 32;
   for (int i = 0; i < (int)(sizeof(F32_TILES) / sizeof(F32_TILES[0])); ++i)
