@@ -329,6 +329,9 @@ def gemm(x, w, out, force_simt=False, point=None, tile=-1, rows=0):
           slices, 1 if packed else 0, point_of, tile, rows, _ptr(scratch), ctypes.c_int64(floats), _stream())
 
 
+ADDS_MIN_ROWS = 512       # (gemm_adds says no to fewer)
+
+
 @functools.lru_cache(maxsize=4096)
 def gemm_adds(M, N, K) -> bool:
     """Whether gemm_add takes M rows with a weight [N, K] in fragment order (csrc/gemm.hip: syn_gemm_adds)."""

@@ -214,7 +214,8 @@ def deferred_product(x, w):
     the caller's result is the delta that a following norm adds to the residual rows, and that norm can take the
     product in (RmsNorm.add_apply)."""
     w = _matrix(w)
-    if (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and w.packed is not None
+    # (the rows first: steps of 130 of them wait for the host, and the whole question takes it a microsecond and more a product)
+    if (x.shape[0] >= ops.ADDS_MIN_ROWS and isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16 and w.packed is not None
             and ops.gemm_adds(x.shape[0], *w.shape) and product_slices(x.shape[0], w, x.dtype) <= 1):
         return DeferredProduct(x, w, many=True)
     if isinstance(x, torch.Tensor) and _use_packed(x, w) and ops.packed_slices(w.shape[0], w.shape[1]) <= 1:

@@ -2199,7 +2199,7 @@ def test_products_of_many_rows_add_to_the_residual_rows_what_the_norm_would(M, N
     w = Matrix((0.02 * torch.randn((N, K), generator=g, device=DEV)).bfloat16())
     room = torch.randn((M + 2, N), generator=g, device=DEV)
     before = room.clone()
-    assert ops.gemm_adds(M, N, K) and not ops.gemm_adds(511, N, K)
+    assert ops.gemm_adds(M, N, K) and not ops.gemm_adds(ops.ADDS_MIN_ROWS - 1, N, K)
     ops.gemm_add(x, w.packed, room[1:-1])
     want = before[1:-1] + linear(x, w, torch.float32)
     same_tile = ops.gemm_slices(M, N, K, torch.bfloat16) == 1
